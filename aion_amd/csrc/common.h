@@ -327,8 +327,11 @@ __device__ __forceinline__ void prepare_act_block8(float v0, float v1, float v2,
 
 __device__ __forceinline__ int dot4_i8(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }
 
-// aion cpu/kernels/fast_math.zig:53-148: exp(x) = 2^n * P4(r ln2), sigmoid, tanh = 2 sigmoid(2x) - 1
+// aion cpu/kernels/fast_math.zig:53-148: exp(x) = 2^n * P4(r ln2), sigmoid, tanh = 2 sigmoid(2x) - 1. Every product and sum is
+// rounded on its own, as there: left to itself the compiler contracts them differently from kernel to kernel, and a gated value
+// that differs in its last bit can flip an int8 code behind it.
 __device__ __forceinline__ float aion_exp_approx(float x_in) {
+#pragma clang fp contract(off)
     const float x = fminf(80.f, fmaxf(-80.f, x_in));
     const float y = x * 1.4426950408889634f;
     const float nf = floorf(y + 0.5f);
@@ -337,6 +340,7 @@ __device__ __forceinline__ float aion_exp_approx(float x_in) {
     return __uint_as_float((unsigned)((int)nf + 127) << 23) * p;
 }
 __device__ __forceinline__ float aion_tanh_approx(float x) {
+#pragma clang fp contract(off)
     const float z = 2.f * x;
     const float e = aion_exp_approx(-fabsf(z));
     float sg = (z >= 0.f ? 1.f : e) / (1.f + e);
@@ -344,14 +348,18 @@ __device__ __forceinline__ float aion_tanh_approx(float x) {
     return fminf(1.f, fmaxf(-1.f, 2.f * sg - 1.f));
 }
 __device__ __forceinline__ float aion_sigmoid_approx(float x) {
+#pragma clang fp contract(off)
     const float e = aion_exp_approx(-fabsf(x));
     return fminf(1.f, fmaxf(0.f, (x >= 0.f ? 1.f : e) / (1.f + e)));
 }
-// aion cpu/exec/elementwise.zig:25-37 (gate) + cpu/kernels/gelu.zig:8-14: gelu_tanh(x) * up
-__device__ __forceinline__ float aion_gate_gelu(float x, float up) {
+// aion cpu/kernels/gelu.zig:8-14
+__device__ __forceinline__ float aion_gelu(float x) {
+#pragma clang fp contract(off)
     const float t = 0.7978845608028654f * (x + 0.044715f * (x * x * x));
-    return (0.5f * x * (1.f + aion_tanh_approx(t))) * up;
+    return 0.5f * x * (1.f + aion_tanh_approx(t));
 }
+// aion cpu/exec/elementwise.zig:25-37 (gate): gelu_tanh(x) * up
+__device__ __forceinline__ float aion_gate_gelu(float x, float up) { return aion_gelu(x) * up; }
 // sum over a 256-thread workgroup; red: 4 floats of LDS. Every thread returns the total.
 __device__ __forceinline__ float block_sum_256(float v, float *red) {
     v = wave_sum(v);

@@ -232,7 +232,7 @@ __global__ void unary_kernel(float *__restrict__ out, const float *__restrict__ 
     const float v = x[i];
     float r;
     if (OP == AIONHIP_UNARY_RELU) r = v > 0.f ? v : 0.f;
-    else if (OP == AIONHIP_UNARY_GELU) r = 0.5f * v * (1.f + aion_tanh_approx(0.7978845608028654f * (v + 0.044715f * (v * v * v))));
+    else if (OP == AIONHIP_UNARY_GELU) r = aion_gelu(v);
     else if (OP == AIONHIP_UNARY_SILU) r = v * aion_sigmoid_approx(v);
     else if (OP == AIONHIP_UNARY_SIGMOID) r = aion_sigmoid_approx(v);
     else if (OP == AIONHIP_UNARY_TANH) r = aion_tanh_approx(v);
