@@ -163,13 +163,17 @@ constexpr size_t STATIC_SCRATCH_BYTES = AIONHIP_STATIC_SCRATCH_BYTES;
     } while (0)
 
 // ---- prepared activations (aion cpu/kernels/matmul_q_i8.zig:187-264) --------------------------
+// Row-major for the GEMV kernels; `tiled` in the order the exact GEMM's operand loads want (gemm_i8_kernel.h): tiles of 32 rows (the
+// last one may hold fewer), per tile and quant block [k / 16 of the block][row][16 codes], scales per tile and block [row], no sums.
+// Either form fills the same bytes.
 struct PreparedAct {
     int8_t *q;      // [m][k]
     float *scale;   // [m][k/32]
     int *sum;       // [m][k/32]   plain sum of the 32 codes
+    bool tiled;
 };
 size_t prepared_act_bytes(size_t m, size_t k);
-PreparedAct prepared_act_carve(void *base, size_t m, size_t k);
+PreparedAct prepared_act_carve(void *base, size_t m, size_t k, bool tiled);
 int launch_prepare_act(aionhip_ctx *ctx, const float *a, size_t lda, size_t m, size_t k, PreparedAct out);
 int launch_prepare_gate(aionhip_ctx *ctx, const float *gate, const float *up, size_t m, size_t k, PreparedAct out);
 int launch_prepare_rmsnorm(aionhip_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, size_t m, size_t k, PreparedAct out);
@@ -242,12 +246,17 @@ int launch_gemv_ksplit(aionhip_ctx *ctx, const aionhip_weight *w, float *c, cons
 int launch_gemv(aionhip_ctx *ctx, const aionhip_weight *w, int m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
                       PreparedAct act, float alpha, float beta);
-int launch_gemm_i8(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
+// whether launch_gemv_batch runs m rows against these weights on the exact GEMM's kernel (it then wants the tiled preparation)
+bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m);
+// modelled time of the exact GEMM's kernel
+float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k);
+// the exact GEMM addresses a row tile of a weight with 32-bit offsets; longer rows run on the GEMV kernels, eight at a time
+constexpr size_t GEMM_I8_MAX_K = (size_t)1 << 26;
 // bf16 mode only: whether the bf16 MFMA kernel is expected to be the faster one for m rows against an n x k weight
 bool gemm_bf16_pays(const aionhip_ctx *ctx, size_t m, size_t n, size_t k);
-// the LDS-staged MFMA kernel for a handful of rows (no profile scope of its own: the caller's name stays)
 int launch_gemm_i8_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m,
                          PreparedAct act, float alpha, float beta);
+// the same kernel for a handful of rows (no profile scope of its own: the caller's name stays)
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
 // MatMulNT with an f32 [N,K] operand (matmul_nt_f32.hip): plain f32 arithmetic, any number of rows
 int launch_matmul_nt_f32(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, const float *a, size_t lda, float *c, size_t ldc, float alpha,

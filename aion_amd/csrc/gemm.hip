@@ -1,12 +1,6 @@
-// Prefill GEMM back ends (more than 8 activation rows): C[m,n] = alpha * A[m,:] . W[n,:] + beta * C.
+// Prefill GEMM, bf16 mode (AIONHIP_GEMM_BF16_MFMA; the exact mode is gemm_i8.hip): C[m,n] = alpha * A[m,:] . W[n,:] + beta * C.
 //
-// gemm_i8_lds_kernel (AIONHIP_GEMM_EXACT_I8) - aion's CPU arithmetic (cpu/kernels/matmul_q_i8.zig:
-//   384-497): activations int8 per (row, 32-block), one v_mfma_i32_16x16x32_i8 per 16x16 output
-//   tile per quant block (K=32 IS one block, so the i32 tile is the exact block dot), then
-//   acc += f32(idot) * (a_scale * w_scale) on the VALU. Operands are staged through LDS. The per-block
-//   rescale (3 VALU ops per output element per block) is what bounds it, not the MFMA pipe.
-//
-// gemm_bf16_wide_kernel (AIONHIP_GEMM_BF16_MFMA) - weights as bf16, either from a copy the context builds once per
+// gemm_bf16_wide_kernel - weights as bf16, either from a copy the context builds once per
 //   weight and owns (2 B/weight; 288 GB of HBM makes it affordable) or converted from the quant blocks while they are
 //   staged (no copy; same bits, slower), activations rounded to bf16, v_mfma_f32_32x32x16_bf16 with f32 accumulation;
 //   described at the kernel.
@@ -18,269 +12,7 @@
 namespace {
 
 using u32x2 = __attribute__((ext_vector_type(2))) unsigned int;
-using i32x4 = __attribute__((ext_vector_type(4))) int;
 using bf16x8 = __attribute__((ext_vector_type(8))) __bf16;
-
-// ------------------------------------------------------------------------------------ exact int8
-// ---- LDS-staged exact kernel: one
-// v_mfma_i32_16x16x32_i8 per 16x16 tile per quant block, then acc += f32(idot) * (a_scale * w_scale) - but
-// the operands of a K step (4 quant blocks) are staged once per workgroup in LDS with coalesced 16-byte
-// loads (a cache line per row), instead of 8-byte operand loads per lane per tile from global memory, which
-// cost several times their payload in L1 bandwidth. q4 nibbles become signed int8 while they are staged
-// (((x | 0x80) - 8) ^ 0x80 per byte), so no per-tile bias correction is left. Workgroup tile (32*WM) x 128,
-// 2 x 2 wavefronts of (16*WM) x 64 outputs; double-buffered, one barrier per K step. The rescale (3 VALU
-// operations per output per block against 32 integer MACs) bounds it at roughly 1/7 of the int8 MFMA peak.
-// KC = quant blocks per K step: 4 when the grid fills the device (two workgroups per CU hide each other's
-// staging), 8 when it does not (few activation rows: fewer, larger steps - a step then costs one memory
-// latency however little it loads).
-// up to four weights with the same K and block format against one prepared activation: column tiles first_tile[i] .. of weight i
-struct GemmSegs {
-    const uint8_t *qs[4];
-    const __half *sc[4];
-    float *c[4];
-    size_t ldc[4];
-    int n[4], first_tile[4];
-    int count;
-};
-template <int KC> struct GiCfg { static constexpr int ROW = KC * 32 + 16; };   // staged code row; +16 B: conflict-free 8-byte operand reads
-// SPLITK (few activation rows, where the tiles above would leave most CUs idle): the workgroup tile shrinks
-// to (16*WM) x 64 and its four wavefronts share it, each taking every fourth quant block of a K step; their
-// partial sums are added in wavefront order through LDS at the end, so the result does not depend on timing.
-template <int DT, int WM, int KC, bool SPLITK>
-__global__ __launch_bounds__(256, KC == 4 || SPLITK ? 2 : 1) void gemm_i8_lds_kernel(GemmSegs segs,
-                                                          const int8_t *__restrict__ aq, const float *__restrict__ a_scale,
-                                                          int M, int K, float alpha, float beta, float *__restrict__ partial, int partial_ld) {
-    constexpr bool Q8 = DT == AIONHIP_Q8_0;
-    static_assert(!SPLITK || KC == 8, "split K: two blocks per wavefront per step");
-    constexpr int BM3 = (SPLITK ? 16 : 32) * WM, BN3 = SPLITK ? 64 : 128, ROW = GiCfg<KC>::ROW;
-    constexpr int KCW = SPLITK ? KC / 4 : KC;            // blocks of a K step this wavefront works on
-    constexpr int A_BYTES = BM3 * ROW, B_BYTES = BN3 * ROW;
-    constexpr int AS_BYTES = BM3 * KC * 4, WS_BYTES = BN3 * KC * 4;
-    constexpr int STAGE = A_BYTES + B_BYTES + AS_BYTES + WS_BYTES;
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds3[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, g = lane >> 4;
-    // the weight this column tile belongs to (sibling weights over one activation share a launch)
-    int si = 0;
-#pragma unroll
-    for (int i = 1; i < 4; ++i)
-        if (i < segs.count && (int)blockIdx.x >= segs.first_tile[i]) si = i;
-    const uint8_t *__restrict__ qs = segs.qs[si];
-    const __half *__restrict__ sc = segs.sc[si];
-    float *__restrict__ c = segs.c[si];
-    const int N = segs.n[si];
-    const size_t ldc = segs.ldc[si];
-    const int m0 = blockIdx.y * BM3, n0 = ((int)blockIdx.x - segs.first_tile[si]) * BN3;
-    const int wm0 = SPLITK ? 0 : (wave >> 1) * (16 * WM), wn0 = SPLITK ? 0 : (wave & 1) * 64;
-    const int jw = SPLITK ? wave : 0, jstep = SPLITK ? 4 : 1;     // this wavefront's blocks: jw + jstep * jj
-    const int KB = K >> 5, KT = (KB + KC - 1) / KC;
-
-    f32x4 acc[WM][4];
-#pragma unroll
-    for (int mi = 0; mi < WM; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 4; ++ni) acc[mi][ni] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    // staging assignment: 16-byte chunks, 2*KC per code row of a K step (q4 weights: KC, one block each)
-    constexpr int CPR = 2 * KC;                          // chunks per int8 row
-    constexpr int NAC = BM3 * CPR / 256;                 // activation chunks per thread
-    constexpr int NBC = (Q8 ? BN3 * CPR : BN3 * KC) / 256;
-    constexpr int NAS = (BM3 * KC + 255) / 256, NWS = BN3 * KC / 256;
-    u32x4 ra[NAC], rb[NBC];
-    float ras[NAS];
-    __half rws[NWS];                                     // converted when stored: a conversion here would wait for the load
-    auto load_stage = [&](int kt) {
-        const int kb0 = kt * KC;
-#pragma unroll
-        for (int i = 0; i < NAC; ++i) {
-            const int id = tid + 256 * i, row = id / CPR, part = id % CPR;
-            const int kbyte = min(kb0 * 32 + part * 16, K - 16);
-            ra[i] = *(const u32x4 *)(aq + (size_t)min(m0 + row, M - 1) * K + kbyte);
-        }
-#pragma unroll
-        for (int i = 0; i < NBC; ++i) {
-            const int id = tid + 256 * i;
-            if (Q8) {
-                const int row = id / CPR, part = id % CPR;
-                const int kbyte = min(kb0 * 32 + part * 16, K - 16);
-                rb[i] = *(const u32x4 *)(qs + (size_t)min(n0 + row, N - 1) * K + kbyte);
-            } else {
-                const int row = id / KC, blk = min(kb0 + id % KC, KB - 1);
-                rb[i] = *(const u32x4 *)(qs + (size_t)min(n0 + row, N - 1) * (K >> 1) + (size_t)blk * 16);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < NAS; ++i) {
-            // unconditional loads at clamped addresses (a predicated load is waited for on the spot)
-            const int id = min(tid + 256 * i, BM3 * KC - 1), row = id / KC, j = id % KC;
-            ras[i] = a_scale[(size_t)min(m0 + row, M - 1) * KB + min(kb0 + j, KB - 1)];
-        }
-#pragma unroll
-        for (int i = 0; i < NWS; ++i) {
-            const int id = tid + 256 * i, row = id / KC, j = id % KC;
-            rws[i] = sc[(size_t)min(n0 + row, N - 1) * KB + min(kb0 + j, KB - 1)];
-        }
-    };
-    auto store_stage = [&](unsigned char *st, int kt) {
-        const int kb0 = kt * KC;
-#pragma unroll
-        for (int i = 0; i < NAC; ++i) {
-            const int id = tid + 256 * i, row = id / CPR, part = id % CPR;
-            *(u32x4 *)(st + row * ROW + part * 16) = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < NBC; ++i) {
-            const int id = tid + 256 * i;
-            if (Q8) {
-                const int row = id / CPR, part = id % CPR;
-                *(u32x4 *)(st + A_BYTES + row * ROW + part * 16) = rb[i];
-            } else {
-                // word w of the device layout holds elements 8w..8w+7: low nibbles 8w..8w+3, high nibbles 8w+4..8w+7
-                const int row = id / KC, j = id % KC;
-                unsigned char *dst = st + A_BYTES + row * ROW + j * 32;
-                const unsigned ws4[4] = {rb[i].x, rb[i].y, rb[i].z, rb[i].w};
-                unsigned dec[8];
-#pragma unroll
-                for (int w = 0; w < 4; ++w) {
-                    const unsigned lo = ws4[w] & 0x0F0F0F0Fu, hi = (ws4[w] >> 4) & 0x0F0F0F0Fu;
-                    dec[2 * w] = ((lo | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                    dec[2 * w + 1] = ((hi | 0x80808080u) - 0x08080808u) ^ 0x80808080u;
-                }
-                *(u32x4 *)dst = u32x4{dec[0], dec[1], dec[2], dec[3]};
-                *(u32x4 *)(dst + 16) = u32x4{dec[4], dec[5], dec[6], dec[7]};
-            }
-        }
-        float *as_l = (float *)(st + A_BYTES + B_BYTES), *ws_l = (float *)(st + A_BYTES + B_BYTES + AS_BYTES);
-#pragma unroll
-        for (int i = 0; i < NAS; ++i)                            // blocks past the end of K: scale 0, no contribution
-            if (tid + 256 * i < BM3 * KC) as_l[tid + 256 * i] = kb0 + (tid + 256 * i) % KC < KB ? ras[i] : 0.f;
-#pragma unroll
-        for (int i = 0; i < NWS; ++i) ws_l[tid + 256 * i] = kb0 + (tid + 256 * i) % KC < KB ? __half2float(rws[i]) : 0.f;
-    };
-
-    // K slices (grid z, few workgroups against a long K): slice z takes its share of the K steps and leaves raw sums in
-    // `partial` [z][M][partial_ld] for gemm_i8_slices_kernel, which adds the slices in their order
-    const int kt_per = (KT + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int kt_lo = (int)blockIdx.z * kt_per, kt_hi = min(KT, kt_lo + kt_per);
-    if (partial) {
-        partial += (size_t)blockIdx.z * M * partial_ld + (size_t)blockIdx.x * BN3;
-        c = partial - n0;                                // column n0 + j of this tile -> partial column blockIdx.x * BN3 + j
-        alpha = 1.f;
-        beta = 0.f;
-    }
-    const size_t ldo = partial ? (size_t)partial_ld : ldc;
-    const int n_hi = partial ? n0 + BN3 : N;            // (a partial tile is written whole: its padding columns are sums over clamped rows, never read)
-    load_stage(kt_lo);
-    store_stage(lds3, kt_lo);
-    __syncthreads();
-    for (int kt = kt_lo; kt < kt_hi; ++kt) {
-        const unsigned char *st = lds3 + ((kt - kt_lo) & 1) * STAGE;
-        const bool more = kt + 1 < kt_hi;
-        if (more) load_stage(kt + 1);
-        const float *as_l = (const float *)(st + A_BYTES + B_BYTES), *ws_l = (const float *)(st + A_BYTES + B_BYTES + AS_BYTES);
-        float wsc[4][KCW];
-#pragma unroll
-        for (int ni = 0; ni < 4; ++ni) {
-            if (SPLITK) {
-#pragma unroll
-                for (int jj = 0; jj < KCW; ++jj) wsc[ni][jj] = ws_l[(wn0 + ni * 16 + r) * KC + jw + 4 * jj];
-            } else {
-#pragma unroll
-                for (int q = 0; q < KC / 4; ++q) {
-                    const f32x4 v = *(const f32x4 *)(ws_l + (wn0 + ni * 16 + r) * KC + q * 4);
-                    wsc[ni][q * 4 % KCW] = v.x; wsc[ni][(q * 4 + 1) % KCW] = v.y; wsc[ni][(q * 4 + 2) % KCW] = v.z; wsc[ni][(q * 4 + 3) % KCW] = v.w;
-                }
-            }
-        }
-        // (row tile, block) steps, software-pipelined: a step's dots are issued one at a time between the
-        // rescales of the previous step's dots, so the matrix pipe runs under the vector work even with a
-        // single wavefront on the SIMD. The empty asm statements fix that order for the compiler, which
-        // otherwise issues every dot of the K step first and runs out of registers.
-        i32x4 dprev[4];
-        float asc[4][KCW];
-#pragma unroll
-        for (int t = 0; t <= WM * KCW; ++t) {
-            const int mi = t / KCW, jj = t % KCW;
-            const int pm = (t - 1) / KCW, pj = (t - 1) % KCW;
-            i32x4 dcur[4];
-            long a = 0;
-            if (t < WM * KCW) a = *(const long *)(st + (wm0 + mi * 16 + r) * ROW + (jw + jstep * jj) * 32 + g * 8);
-            if (t > 0 && pj == 0) {             // the previous row tile's activation scales
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    if (SPLITK) {
-#pragma unroll
-                        for (int q = 0; q < KCW; ++q) asc[i][q] = as_l[(wm0 + pm * 16 + g * 4 + i) * KC + jw + 4 * q];
-                    } else {
-#pragma unroll
-                        for (int q = 0; q < KC / 4; ++q) {
-                            const f32x4 v = *(const f32x4 *)(as_l + (wm0 + pm * 16 + g * 4 + i) * KC + q * 4);
-                            asc[i][q * 4 % KCW] = v.x; asc[i][(q * 4 + 1) % KCW] = v.y; asc[i][(q * 4 + 2) % KCW] = v.z; asc[i][(q * 4 + 3) % KCW] = v.w;
-                        }
-                    }
-                }
-            }
-#pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
-                if (t < WM * KCW) {
-                    const long b = *(const long *)(st + A_BYTES + (wn0 + ni * 16 + r) * ROW + (jw + jstep * jj) * 32 + g * 8);
-                    dcur[ni] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, b, i32x4{0, 0, 0, 0}, 0, 0, 0);
-                }
-                if (t > 0) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) acc[pm][ni][i] += (float)dprev[ni][i] * (asc[i][pj] * wsc[ni][pj]);
-                    asm volatile("" : "+v"(acc[pm][ni]));
-                }
-            }
-#pragma unroll
-            for (int ni = 0; ni < 4; ++ni) dprev[ni] = dcur[ni];
-        }
-        if (more) store_stage(lds3 + ((kt + 1 - kt_lo) & 1) * STAGE, kt + 1);
-        __syncthreads();
-    }
-
-    if (SPLITK) {
-        // partial sums of the four wavefronts -> LDS (the stages are free: the loop ended on a barrier), then
-        // wavefront w adds column tile w in the fixed order 0,1,2,3 and writes it
-        f32x4 *red = (f32x4 *)lds3;                      // [wave][mi][ni][lane]
-#pragma unroll
-        for (int mi = 0; mi < WM; ++mi)
-#pragma unroll
-            for (int ni = 0; ni < 4; ++ni) red[((wave * WM + mi) * 4 + ni) * 64 + lane] = acc[mi][ni];
-        __syncthreads();
-#pragma unroll
-        for (int mi = 0; mi < WM; ++mi) {
-            f32x4 sum = red[((0 * WM + mi) * 4 + wave) * 64 + lane];
-#pragma unroll
-            for (int w = 1; w < 4; ++w) sum += red[((w * WM + mi) * 4 + wave) * 64 + lane];
-            const int col = n0 + wave * 16 + r;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = m0 + mi * 16 + g * 4 + i;
-                if (row >= M || col >= n_hi) continue;
-                float *dst = c + (size_t)row * ldo + col;
-                const float v = alpha * sum[i];
-                *dst = beta == 0.f ? v : v + beta * *dst;
-            }
-        }
-        return;
-    }
-#pragma unroll
-    for (int mi = 0; mi < WM; ++mi)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int row = m0 + wm0 + mi * 16 + g * 4 + i;
-            if (row >= M) continue;
-#pragma unroll
-            for (int ni = 0; ni < 4; ++ni) {
-                const int col = n0 + wn0 + ni * 16 + r;
-                if (col >= n_hi) continue;
-                float *dst = c + (size_t)row * ldo + col;
-                const float v = alpha * acc[mi][ni][i];
-                *dst = beta == 0.f ? v : v + beta * *dst;
-            }
-        }
-}
 
 // ------------------------------------------------------------------------------------ bf16 MFMA
 constexpr int G2_TILE_K = 32;                                // k extent of a block of the tiled bf16 operands = the kernel's K step
@@ -756,137 +488,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_mixed_kernel(const unsigned sho
     else gemm_bf16_tile<4, NST, 3, BDT>(lds2, A, (const unsigned short *)wq, c, M, N, K, ldc, alpha, beta, m0, tw * 256 + idx * 192, wq, wsc);
 }
 
-// Tile choice by a small cost model fitted to measurements on one MI355X (q4, K = 2048..8192, 24..2048
-// rows): a lone workgroup of each shape costs `us_per_block` per quant block of K; workgroups beyond one
-// per CU overlap by the factor `overlap` (two resident per CU hide each other's staging).
-struct GiShape { int wm; bool split; float us_per_block, overlap; };
-constexpr GiShape GI_SHAPES[6] = {
-    {4, false, 0.81f, 1.40f}, {2, false, 0.44f, 1.25f}, {1, false, 0.284f, 1.55f},
-    {4, true, 0.253f, 1.45f}, {2, true, 0.164f, 1.50f}, {1, true, 0.121f, 1.85f},
-};
-// The K slices of gemm_i8_lds_kernel folded in slice order: C = alpha * (p[0] + p[1] + ...) + beta * C, one thread per
-// (row, four columns of a tile).
-__global__ __launch_bounds__(256) void gemm_i8_slices_kernel(GemmSegs segs, const float *__restrict__ partial, int M, int slices, int partial_ld,
-                                                             int bn, float alpha, float beta) {
-    const int quads = partial_ld >> 2;
-    const size_t id = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (id >= (size_t)M * quads) return;
-    const int row = (int)(id / quads), pc = (int)(id % quads) * 4, tile = pc / bn;
-    int si = 0;
-#pragma unroll
-    for (int i = 1; i < 4; ++i)
-        if (i < segs.count && tile >= segs.first_tile[i]) si = i;
-    const int col = pc - segs.first_tile[si] * bn;
-    if (col >= segs.n[si]) return;
-    f32x4 sum = *(const f32x4 *)(partial + (size_t)row * partial_ld + pc);
-    for (int z = 1; z < slices; ++z) sum += *(const f32x4 *)(partial + ((size_t)z * M + row) * partial_ld + pc);
-    float *dst = segs.c[si] + (size_t)row * segs.ldc[si] + col;
-    const float e[4] = {sum.x, sum.y, sum.z, sum.w};
-#pragma unroll
-    for (int t = 0; t < 4; ++t)
-        if (col + t < segs.n[si]) dst[t] = beta == 0.f ? alpha * e[t] : alpha * e[t] + beta * dst[t];
-}
-
-// How many K slices a launch of `wgs` workgroups (each able to overlap `overlap` to a CU, `us_per_block` per quant block of a
-// lone one) over `kt` K steps of `blocks` quant blocks is cut into. Slices pay when the modelled time with them, the
-// launch that adds them up included, is under three quarters of the time without (measured: 4096 x 14336 at 16 rows
-// 52 -> 22 us in 7 slices, 2048 x 8192 33 -> 15 us, 4096 x 4096 20 -> 15 us; K = 2048 never: the second launch costs what
-// the slices save).
-inline int i8_k_slices(const aionhip_ctx *ctx, float wgs, float overlap, int kt, float us_per_block, float blocks) {
-    const float cus = (float)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    const float rounds = wgs / (cus * overlap);
-    if (ctx->no_scratch_paths || rounds >= 0.75f || kt < 8) return 1;
-    int s = (int)(1.f / rounds + 0.5f);
-    s = s < kt / 4 ? s : kt / 4;                          // at least four K steps per slice
-    s = s > 8 ? 8 : s;
-    if (s < 2) return 1;
-    const float alone = us_per_block * blocks;
-    const float sliced = alone / (float)s * (rounds * (float)s > 1.f ? rounds * (float)s : 1.f) + 4.f;
-    return sliced < 0.75f * alone ? s : 1;
-}
-
-template <int DT, int WM, int KC, bool SPLITK>
-int launch_i8_lds(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m, PreparedAct act,
-                  float alpha, float beta) {
-    constexpr int BM3 = (SPLITK ? 16 : 32) * WM, BN3 = SPLITK ? 64 : 128;
-    constexpr int LDS = 2 * ((BM3 + BN3) * GiCfg<KC>::ROW + (BM3 + BN3) * KC * 4);
-    static_assert(LDS <= 160 * 1024, "two stages must fit the CU's LDS");
-    static_assert(!SPLITK || 4 * WM * 4 * 64 * 16 <= LDS, "the split-K reduction reuses the stages");
-    static bool attr = false;
-    if (!attr) {
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_lds_kernel<DT, WM, KC, SPLITK>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
-        attr = true;
-    }
-    GemmSegs segs{};
-    segs.count = count;
-    int tiles = 0;
-    for (int i = 0; i < count; ++i) {
-        segs.qs[i] = ws[i]->qs;
-        segs.sc[i] = ws[i]->sc;
-        segs.c[i] = cs[i];
-        segs.ldc[i] = ldcs[i];
-        segs.n[i] = (int)ws[i]->n;
-        segs.first_tile[i] = tiles;
-        tiles += (int)((ws[i]->n + BN3 - 1) / BN3);
-    }
-    const int m_tiles = (int)((m + BM3 - 1) / BM3), kt = (int)(((ws[0]->k >> 5) + KC - 1) / KC);
-    // Few workgroups against a long K (a short prompt or a batch of 9..64 rows on a narrow weight): the K steps are cut into
-    // slices across more workgroups and a second, small launch adds the slices in order - the same sums in the same
-    // order per slice, the slices in a fixed order, so the result does not depend on timing.
-    constexpr GiShape SHAPE = GI_SHAPES[(SPLITK ? 3 : 0) + (WM == 4 ? 0 : WM == 2 ? 1 : 2)];
-    static_assert(SHAPE.wm == WM && SHAPE.split == SPLITK, "shape table order");
-    int slices = i8_k_slices(ctx, (float)tiles * (float)m_tiles, SHAPE.overlap, kt, SHAPE.us_per_block, (float)(ws[0]->k >> 5));
-    while (slices > 1 && (kt + slices - 1) / slices * (slices - 1) >= kt) --slices;      // no empty slice
-    float *partial = nullptr;
-    const int partial_ld = tiles * BN3;
-    if (slices > 1) {
-        const int rc = ensure_scratch2(ctx, (size_t)slices * m * partial_ld * sizeof(float));
-        if (rc) return rc;
-        partial = (float *)ctx->scratch2;
-    }
-    const dim3 grid((unsigned)tiles, (unsigned)m_tiles, (unsigned)slices);
-    launch_k(ctx, gemm_i8_lds_kernel<DT, WM, KC, SPLITK>, grid, dim3(256), LDS, segs, act.q, act.scale, (int)m, (int)ws[0]->k, alpha, beta, partial, partial_ld);
-    if (slices > 1) {
-        const size_t threads = m * (size_t)(partial_ld >> 2);
-        launch_k(ctx, gemm_i8_slices_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, segs, partial, (int)m, slices, partial_ld, BN3, alpha, beta);
-    }
-    return AIONHIP_OK;
-}
-
-// the cheapest shape for m rows against an n x k weight and its modelled time per quant block of K
-int pick_i8_shape(const aionhip_ctx *ctx, size_t m, size_t n, size_t k, float *us_per_block) {
-    const float cus = (float)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    int best = 0;
-    float best_t = 0.f;
-    for (int i = 0; i < 6; ++i) {
-        const GiShape &g = GI_SHAPES[i];
-        if (g.split && k < 256) continue;                // a split-K step is 8 blocks
-        const size_t bm = (size_t)(g.split ? 16 : 32) * g.wm, bn = g.split ? 64 : 128;
-        const float wgs = (float)(((m + bm - 1) / bm) * ((n + bn - 1) / bn));
-        const float rounds = wgs / (cus * g.overlap);
-        const float t = g.us_per_block * (rounds > 1.f ? rounds : 1.f);
-        if (i == 0 || t < best_t) { best = i; best_t = t; }
-    }
-    if (us_per_block) *us_per_block = best_t;
-    return best;
-}
-// the tile shape is chosen for the columns of all the weights together (their tiles share the launch)
-template <int DT>
-int launch_i8_lds_pick(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m,
-                       PreparedAct act, float alpha, float beta) {
-    size_t n_total = 0;
-    for (int i = 0; i < count; ++i) n_total += ws[i]->n;
-    const int best = pick_i8_shape(ctx, m, n_total, ws[0]->k, nullptr);
-    switch (best) {
-    case 0: return launch_i8_lds<DT, 4, 4, false>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    case 1: return launch_i8_lds<DT, 2, 4, false>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    case 2: return launch_i8_lds<DT, 1, 4, false>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    case 3: return launch_i8_lds<DT, 4, 8, true>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    case 4: return launch_i8_lds<DT, 2, 8, true>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    default: return launch_i8_lds<DT, 1, 8, true>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    }
-}
-
 }  // namespace
 
 // In bf16 mode: is the bf16 MFMA kernel expected to beat the exact kernel for this shape? Up to a few hundred rows it
@@ -894,53 +495,15 @@ int launch_i8_lds_pick(aionhip_ctx *ctx, const aionhip_weight *const *ws, float 
 // one workgroup's K loop is a latency chain - and the exact kernel is then both the faster and the exact one.
 // Modelled times in microseconds, constants fitted to a sweep of 9..512 rows over four weight shapes.
 bool gemm_bf16_pays(const aionhip_ctx *ctx, size_t m, size_t n, size_t k) {
-    float per_block = 0.f;
-    const GiShape &g = GI_SHAPES[pick_i8_shape(ctx, m, n, k, &per_block)];
-    const float blocks = (float)(k / 32);
-    // (the exact kernel cuts a long K into slices across workgroups when its grid is sparse)
-    const size_t bm = (size_t)(g.split ? 16 : 32) * g.wm, bn = g.split ? 64 : 128;
-    const float wgs = (float)(((m + bm - 1) / bm) * ((n + bn - 1) / bn));
-    const int kc = g.split ? 8 : 4;                      // (the launcher's KC per shape)
-    const int slices = i8_k_slices(ctx, wgs, g.overlap, (int)((k / 32 + kc - 1) / kc), g.us_per_block, blocks);
-    const float cus = (float)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    const float rounds = wgs * (float)slices / (cus * g.overlap);
-    const float kernel_us = slices > 1 ? g.us_per_block * blocks / (float)slices * (rounds > 1.f ? rounds : 1.f) + 4.f : per_block * blocks;
-    const float exact_us = kernel_us + 5.f + (float)m * (float)k * 4.f / 2.0e6f;               // + the int8 preparation of A
+    const float exact_us = gemm_i8_us(ctx, AIONHIP_Q4_0, m, n, k) + 5.f + (float)m * (float)k * 4.f / 2.0e6f;   // + the int8 preparation of A
     // (constants fitted to both kernels' times over six weight shapes x 65..1024 rows, q4: the choice costs 0.3 % over
     // always taking the faster one; always exact would cost 36 %, always bf16 17 %)
     const float copy_us = (float)n * (float)k * 2.f / 3.0e6f;                                  // weight bytes at ~3 TB/s
     const float flop_us = 2.f * (float)m * (float)n * (float)k / 9.0e8f;                        // ~900 TFLOP/s
-    const float chain_us = blocks * 0.24f;                                                       // one workgroup's K loop
+    const float chain_us = (float)(k / 32) * 0.24f;                                                       // one workgroup's K loop
     const float act_us = (float)m * (float)k * 6.f / 4.0e6f;                                     // the bf16 rounding of A
     const float bf16_us = fmaxf(fmaxf(copy_us, flop_us), chain_us) + act_us;
     return bf16_us < exact_us;
-}
-
-int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {
-    return w->dtype == AIONHIP_Q8_0 ? launch_i8_lds_pick<AIONHIP_Q8_0>(ctx, &w, &c, &ldc, 1, m, act, alpha, beta)
-                                    : launch_i8_lds_pick<AIONHIP_Q4_0>(ctx, &w, &c, &ldc, 1, m, act, alpha, beta);
-}
-
-// 1..4 weights of one dtype, layout and K against the same prepared rows, one launch
-int launch_gemm_i8_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m,
-                         PreparedAct act, float alpha, float beta) {
-    if (count < 1 || count > 4) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemm: %d weights in one launch (1..4)", count);
-    const char *name = ws[0]->dtype == AIONHIP_Q8_0 ? "gemm_i8_q8" : "gemm_i8_q4";
-    ProfScope scope(ctx, name);
-    const int rc = ws[0]->dtype == AIONHIP_Q8_0 ? launch_i8_lds_pick<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
-                                                 : launch_i8_lds_pick<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-    if (rc) return rc;
-    LAUNCH_CHECK(ctx, name);
-    return AIONHIP_OK;
-}
-
-int launch_gemm_i8(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {
-    const char *name = w->dtype == AIONHIP_Q8_0 ? "gemm_i8_q8" : "gemm_i8_q4";
-    ProfScope scope(ctx, name);
-    const int rc = launch_gemm_i8_few_rows(ctx, w, m, act, c, ldc, alpha, beta);
-    if (rc) return rc;
-    LAUNCH_CHECK(ctx, name);
-    return AIONHIP_OK;
 }
 
 // The context's bf16 copy of a weight (tiled layout), built on first use: see aionhip_set_bf16_weight_copies.

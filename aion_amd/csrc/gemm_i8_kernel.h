@@ -1,0 +1,291 @@
+// The exact GEMM's kernel (see gemm_i8.hip for the launcher and the choice of shapes).
+//
+// v_mfma_i32_32x32x32_i8: the 32 of K are one quant block, so the i32 tile is the exact block dot; the vector ALU then does
+// acc += f32(dot) * (a_scale * w_scale), three operations per output per block, and that is the bound: 48 vector instructions behind
+// a 32-cycle MFMA. What the parts cost on gfx950, alone in a loop: multiply, multiply-add 1.1 ns per wavefront instruction with
+// four wavefronts on the SIMD but 2.0 .. 2.3 ns with one, conversion 1.8 ns; the MFMA 13.5 ns; the whole rescale of a tile 60 ns per
+// SIMD with two wavefronts and 115 with one. So the shape of this kernel: at least two wavefronts per SIMD at every size, and nothing that
+// makes them wait for each other. A wavefront owns a (32 MT) x (32 NT) tile and a share of K (every KS-th group of four blocks); the KS
+// wavefronts of a tile meet once, at the end, in LDS, in a fixed order. Operands go from global memory (L2) straight into the
+// MFMA's registers, two blocks ahead; there is no staging and no barrier in the loop.
+//   activations: prepared in operand order, a wavefront's load of a block is 1 KiB of consecutive memory; their scales are the one thing
+//     that passes through LDS (16 rows' scales per lane: a wavefront's private copy, 4 reads per row tile and block)
+//   weights: the row-major device layout. q8: a lane loads its row's 16 codes. q4: a lane loads 16 bytes = a whole block, the lane
+//     halves two neighbouring blocks, and two v_permlane32_swap give both halves their words of each
+// Other forms measured: f16 codes on v_mfma_f32_32x32x16_f16 (no conversion after the dot, 51 ns a tile, but the codes have to be
+// converted and the operands are twice the bytes), scale products as 4x4x1 outer products on the matrix pipe (82 ns), activation scales by
+// DPP broadcast (90 ns), an integer bias in place of the conversion (62 ns).
+// Measured (kernel alone, q4 / q8): 512 x 4096 x 4096 31 / 35 us = 550 / 490 TOP/s (LDS-staged 16 x 16 tiles with one or two
+// wavefronts per SIMD before: 46 / 47), 128 x 16384 x 2048 19 / 22 us (31), 128 x 2048 x 8192 12 / 17 us (31), 77 x 11008 x 4096 23 / 24 us
+// (38), 2048 x 14336 x 4096 365 / 415 us (450). Without the operand and scale loads the last one takes 225 us: what is left above
+// the rescale is the registers' fill from LDS and memory beside it.
+#pragma once
+#include "common.h"
+
+using i32x4 = __attribute__((ext_vector_type(4))) int;
+using i32x16 = __attribute__((ext_vector_type(16))) int;
+using f32x16 = __attribute__((ext_vector_type(16))) float;
+
+// up to four weights with the same K and block format against one prepared activation: column tiles first_tile[i] .. of weight i
+struct GemmSegs {
+    const uint8_t *qs[4];
+    const __half *sc[4];
+    float *c[4];
+    size_t ldc[4];
+    int n[4], first_tile[4];
+    int count;
+};
+
+// Prepared activation in the order the kernel's operand loads want: row tiles of 32 rows (the last one may hold fewer), per
+// tile and quant block [h = 0, 1][row][16 codes] - k = 16 h .. 16 h + 15 of the block - so that a wavefront's load of one
+// block of a full tile is 1 KiB of consecutive memory; scales per tile and block [row].
+__host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M - mt * 32 < 32 ? M - mt * 32 : 32; }
+
+template <int DT, int MT, int NT, int KS, int WGM, int WGN>
+__global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
+                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, float alpha, float beta,
+                                                                         float *__restrict__ partial, int partial_ld) {
+    constexpr bool Q8 = DT == AIONHIP_Q8_0;
+    constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 31, h = lane >> 5;
+    const int ks = wave / (WGM * WGN), wsub = wave % (WGM * WGN), wm = wsub / WGN, wn = wsub % WGN;
+    // workgroup -> tile: ids go round-robin over the 8 XCDs; every XCD takes a contiguous run of tiles, row tiles fastest, so that
+    // the workgroups that share a weight column tile run on one L2
+    const int tiles = row_tiles * col_tiles;
+    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int t = xcd * (tiles >> 3) + min(xcd, tiles & 7) + slot;
+    const int grp = t / (row_group * col_tiles), gr0 = grp * row_group, gr = min(row_group, row_tiles - gr0);
+    const int ct = (t - gr0 * col_tiles) / gr, rt = gr0 + (t - gr0 * col_tiles) - ct * gr;
+    int si = 0;
+#pragma unroll
+    for (int i = 1; i < 4; ++i)
+        if (i < segs.count && ct >= segs.first_tile[i]) si = i;
+    const uint8_t *__restrict__ qs = segs.qs[si];
+    const __half *__restrict__ sc = segs.sc[si];
+    float *__restrict__ c = segs.c[si];
+    const int N = segs.n[si];
+    size_t ldc = segs.ldc[si];
+    const int KB = K >> 5, G = (KB + 3) >> 2;
+    const int n0 = (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
+
+    // this wavefront's operand rows: activation tiles mt0 .., weight rows n0 + 32 ni + r (clamped: a clamped row's results are not
+    // stored). Every operand address is a uniform base that moves with K plus a 32-bit offset a lane keeps for good, so that a
+    // load costs the vector ALU nothing.
+    const uint8_t *ab[MT];
+    const float *asb[MT];
+    unsigned ao[MT], aso[MT];
+    int arows[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int mt = min((m0 >> 5) + i, (M - 1) >> 5);
+        arows[i] = act_tile_rows(M, mt);
+        ab[i] = aq + (size_t)mt * 32 * K;
+        ao[i] = (unsigned)(h * arows[i] + min(r, arows[i] - 1)) * 16;
+        asb[i] = a_scale + (size_t)mt * 32 * KB;
+        aso[i] = (unsigned)min(r, arows[i] - 1);
+    }
+    const int nb = min(n0, N - 1);
+    const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
+    const uint8_t *wb = qs + (size_t)nb * wpitch;
+    const __half *sb = sc + (size_t)nb * KB;
+    unsigned wo[NT], so[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) {
+        const unsigned row = (unsigned)(min(n0 + i * 32 + r, N - 1) - nb);
+        wo[i] = row * wpitch + (unsigned)h * 16;         // (q4: a lane half takes the next block, 16 bytes on)
+        so[i] = row * (unsigned)KB;
+    }
+
+    f32x16 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+
+    // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
+    const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
+    const int g_lo = (int)blockIdx.z * g_per, g_hi = min(G, g_lo + g_per);
+
+    // operand registers: block b of the sequence lives in set b & 3; requested two blocks ahead
+    i32x4 A[4][MT];
+    i32x4 W[Q8 ? 4 : 2][NT];                   // q8: a block; q4: a pair of blocks (lanes 0..31 the even one, 32..63 the odd one)
+    unsigned long sw_raw[NT];                  // four f16 scales of the lane's weight row
+    int sw_shift = 0;
+    float sa_raw[2][MT];                       // two of the group's 4 x 32 activation scales per lane
+    float *sa_lds = (float *)lds + wave * (2 * MT * 128);
+    auto load_a = [&](int set, int kb) {
+        kb = min(kb, KB - 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) A[set][i] = *(const i32x4 *)(ab[i] + (size_t)((unsigned)kb * (unsigned)(arows[i] * 32)) + ao[i]);
+    };
+    auto load_w8 = [&](int set, int kb) {
+        kb = min(kb, KB - 1);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) W[set][i] = *(const i32x4 *)(wb + (size_t)(unsigned)(kb * 32) + wo[i]);
+    };
+    auto load_w4 = [&](int set, int kb) {                // (one block past the end of K: another row's or the slack behind the weight, scale 0)
+        kb = min(kb, KB - 1);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) W[set][i] = *(const i32x4 *)(wb + (size_t)(unsigned)(kb * 16) + wo[i]);
+    };
+    struct __attribute__((packed, aligned(2))) U64 { unsigned long v; };
+    auto load_scales = [&](int g) {
+        const int kb = min(g * 4, KB - 1), base = max(0, min(kb, KB - 4));
+        sw_shift = (kb - base) * 16;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) sw_raw[i] = ((const U64 *)(sb + base + so[i]))->v;
+        const int b0 = min(kb, KB - 1), b1 = min(kb + 1, KB - 1), b2 = min(kb + 2, KB - 1), b3 = min(kb + 3, KB - 1);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            sa_raw[0][i] = asb[i][aso[i] + (unsigned)((h ? b1 : b0) * arows[i])];
+            sa_raw[1][i] = asb[i][aso[i] + (unsigned)((h ? b3 : b2) * arows[i])];
+        }
+    };
+    auto store_sa = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            sa_lds[(buf * MT + i) * 128 + lane] = sa_raw[0][i];
+            sa_lds[(buf * MT + i) * 128 + 64 + lane] = sa_raw[1][i];
+        }
+    };
+
+    // the activation scales a lane multiplies with - 16 rows of each row tile - come from the wavefront's LDS copy of the group
+    float sa[MT][16];
+    auto read_sa = [&](int i, int buf, int j) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const f32x4 v = *(const f32x4 *)(sa_lds + (buf * MT + i) * 128 + j * 32 + 8 * q + 4 * h);
+            sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
+        }
+    };
+    int g = g_lo + ks;
+    if (g < g_hi) {
+        load_scales(g);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            load_a(j, g * 4 + j);
+            if constexpr (Q8) load_w8(j, g * 4 + j);
+            else if ((j & 1) == 0) load_w4(j >> 1, g * 4 + j);
+        }
+        store_sa(0);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) read_sa(i, 0, 0);
+    }
+    int buf = 0;
+    i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
+    float sw_due = 0.f;
+    for (; g < g_hi; g += KS) {
+        const int gn = g + KS < g_hi ? g + KS : g;       // the last group's look-ahead repeats it (never used)
+        float sw[4][NT];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                const unsigned short hb = (unsigned short)((sw_raw[i] >> sw_shift) >> (16 * j));
+                sw[j][i] = g * 4 + j < KB ? __half2float(__ushort_as_half(hb)) : 0.f;
+            }
+        load_scales(gn);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            load_a((j + 2) & 3, j < 2 ? g * 4 + j + 2 : gn * 4 + j - 2);
+            if constexpr (Q8) load_w8((j + 2) & 3, j < 2 ? g * 4 + j + 2 : gn * 4 + j - 2);
+            else if (j == 0) load_w4(1, g * 4 + 2);
+            else if (j == 2) load_w4(0, gn * 4);
+            if (j == 3) store_sa(buf ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+            i32x4 B[NT];
+#pragma unroll
+            for (int i = 0; i < NT; ++i) {
+                if constexpr (Q8) {
+                    B[i] = W[j][i];
+                } else {
+                    // lanes 0..31 hold words 0..3 of the even block, lanes 32..63 of the odd one; a half needs words 2h, 2h + 1 of one block
+                    if ((j & 1) == 0) {
+                        const auto x = __builtin_amdgcn_permlane32_swap(W[j >> 1][i].x, W[j >> 1][i].z, false, false);
+                        const auto y = __builtin_amdgcn_permlane32_swap(W[j >> 1][i].y, W[j >> 1][i].w, false, false);
+                        W[j >> 1][i] = i32x4{(int)x[0], (int)y[0], (int)x[1], (int)y[1]};
+                    }
+                    const unsigned w0 = (j & 1) ? W[j >> 1][i].z : W[j >> 1][i].x, w1 = (j & 1) ? W[j >> 1][i].w : W[j >> 1][i].y;
+                    // 16 * (nibble - 8) as int8: the nibble in the upper half of its byte with the top bit flipped; the sums are divided by
+                    // 16 at the end (in the scales, the division would round where a product of scales is subnormal)
+                    B[i] = i32x4{(int)(((w0 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w0 & 0xF0F0F0F0u) ^ 0x80808080u),
+                                 (int)(((w1 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w1 & 0xF0F0F0F0u) ^ 0x80808080u)};
+                }
+            }
+            // a tile's dots are issued ahead of the previous tile's rescale (the last tile's is left to the next block); the empty
+            // asm statements keep that order. A row tile's scales of the next block are read once the block's last use of them is past.
+#pragma unroll
+            for (int tl = 0; tl < MT * NT; ++tl) {
+                const i32x16 dn = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j][tl / NT], B[tl % NT], i32x16{0}, 0, 0, 0);
+                const int pt = (tl + MT * NT - 1) % (MT * NT), pi = pt / NT, pj = pt % NT;
+                const float s = tl == 0 ? sw_due : sw[j][pj];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[pi][pj][e] += (float)d[e] * (sa[pi][e] * s);
+                asm volatile("" : "+v"(acc[pi][pj]));
+                if (pj == NT - 1) read_sa(pi, tl == 0 ? buf : (j == 3 ? buf ^ 1 : buf), tl == 0 ? j : (j + 1) & 3);
+                d = dn;
+            }
+            sw_due = sw[j][NT - 1];
+        }
+        buf ^= 1;
+    }
+    // the last block's last tile (a wavefront without a group has none)
+    if (g_lo + ks < g_hi)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
+
+    if (partial) {
+        // a K slice leaves raw sums; gemm_i8_slices_kernel adds the slices in order and applies alpha and beta
+        c = partial + (size_t)blockIdx.z * M * partial_ld + (size_t)segs.first_tile[si] * BN;
+        ldc = partial_ld;
+        alpha = 1.f;
+        beta = 0.f;
+    }
+    auto put = [&](int mi, int ni, int e, float v) {
+        const int row = m0 + mi * 32 + 8 * (e >> 2) + 4 * h + (e & 3), col = n0 + ni * 32 + r;
+        if (row >= M || col >= N) return;
+        float *dst = c + (size_t)row * ldc + col;
+        v = alpha * (Q8 ? v : 0.0625f * v);
+        *dst = beta == 0.f ? v : v + beta * *dst;
+    };
+    if constexpr (KS == 1) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) put(i, j, e, acc[i][j][e]);
+    } else {
+        // the KS partial sums of a tile through LDS, added in wavefront order by the tile's wavefronts, a share each
+        constexpr int CH = MT * NT * 4;                  // 16-byte chunks per lane
+        f32x4 *red = (f32x4 *)lds + (size_t)wsub * KS * CH * 64;
+        __syncthreads();                                 // (the staged activation scales are dead)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    red[(ks * CH + (i * NT + j) * 4 + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        __syncthreads();
+#pragma unroll
+        for (int c0 = 0; c0 < (CH + KS - 1) / KS; ++c0) {
+            const int ch = c0 * KS + ks;
+            if (ch >= CH) break;
+            f32x4 s = red[ch * 64 + lane];
+#pragma unroll
+            for (int k = 1; k < KS; ++k) s += red[(k * CH + ch) * 64 + lane];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) put((ch >> 2) / NT, (ch >> 2) % NT, (ch & 3) * 4 + e, s[e]);
+        }
+    }
+}
+
+template <int MT, int NT, int KS, int WGM, int WGN> constexpr int gemm_i8_lds_bytes() {
+    const int scales = KS * WGM * WGN * 2 * MT * 512, red = KS > 1 ? KS * WGM * WGN * MT * NT * 4096 : 0;
+    return scales > red ? scales : red;
+}

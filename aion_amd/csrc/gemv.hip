@@ -414,11 +414,27 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 
 }  // namespace
 
+// 5..8 rows against a wide, short weight (a logits head at batch 8): the 16-row MFMA tile of the LDS-staged int8
+// GEMM beats the lane-per-row kernel, whose LDS traffic grows with the rows (262144 x 2048, 8 rows: 77 against
+// 104 us for q4, 110 against 142 us for q8). Long K or few columns leave that kernel's grid too sparse.
+// q8 (twice the weight bytes per row: the lane-per-row kernel leaves its latency floor later) moves there from two
+// rows on once the weight has some 12k columns - 14336 x 4096: 22 -> 20 us at 4 rows, 26.6 -> 20.3 at 8;
+// 16384 x 2048: 15 -> 13.7 at 2-4 rows - but not against the largest weights, which the lane-per-row kernel
+// streams faster at 2-4 rows (65536 x 4096: 58-64 against 70 us).
+bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m) {
+    if (count != 1 || gemv_mfma_applies(ws, count, m)) return false;
+    const size_t n = ws[0]->n, k = ws[0]->k;
+    const bool q8w = ws[0]->dtype == AIONHIP_Q8_0;
+    const bool tile16 = (m >= 5 && n >= 16384) || (q8w && m >= 2 && n >= 12288 && n * k <= ((size_t)1 << 27)) ||
+                        (q8w && m >= 5 && n >= 8192 && k <= 2048);
+    return tile16 && k >= 256 && k <= 4096;
+}
+
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
                       PreparedAct act, float alpha, float beta) {
     if (m < 1 || m > 8) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: m=%d outside 1..8", m);
     if (count < 1 || count > 4) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: %d weights in one launch (1..4)", count);
-    if (gemv_mfma_applies(ws, count, m)) {
+    if (!act.tiled && gemv_mfma_applies(ws, count, m)) {
         const char *mname = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8_mfma" : "gemv_q4_mfma";
         ProfScope scope(ctx, mname);
         const int rc = launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
@@ -430,18 +446,7 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
     }
     const char *name = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8" : "gemv_q4";
     ProfScope scope(ctx, name);
-    // 5..8 rows against a wide, short weight (a logits head at batch 8): the 16-row MFMA tile of the LDS-staged int8
-    // GEMM beats the lane-per-row kernel, whose LDS traffic grows with the rows (262144 x 2048, 8 rows: 77 against
-    // 104 us for q4, 110 against 142 us for q8). Long K or few columns leave that kernel's grid too sparse.
-    // q8 (twice the weight bytes per row: the lane-per-row kernel leaves its latency floor later) moves there from two
-    // rows on once the weight has some 12k columns - 14336 x 4096: 22 -> 20 us at 4 rows, 26.6 -> 20.3 at 8;
-    // 16384 x 2048: 15 -> 13.7 at 2-4 rows - but not against the largest weights, which the lane-per-row kernel
-    // streams faster at 2-4 rows (65536 x 4096: 58-64 against 70 us).
-    const size_t n = ws[0]->n, k = ws[0]->k;
-    const bool q8w = ws[0]->dtype == AIONHIP_Q8_0;
-    const bool tile16 = (m >= 5 && n >= 16384) || (q8w && m >= 2 && n >= 12288 && n * k <= ((size_t)1 << 27)) ||
-                        (q8w && m >= 5 && n >= 8192 && k <= 2048);
-    if (count == 1 && tile16 && k >= 256 && k <= 4096) {
+    if (act.tiled) {
         const int rc = launch_gemm_i8_few_rows(ctx, ws[0], (size_t)m, act, cs[0], ldcs[0], alpha, beta);
         if (rc) return rc;
         LAUNCH_CHECK(ctx, name);

@@ -3,8 +3,8 @@
 // (the counterpart of cpu/exec/matmul.zig:233-296 `matvecRoute` / `gemm2D`):
 //   m == 1, k <= 4096, 16-byte aligned A  -> gemv_fused_kernel (activation prepared in the kernel)
 //   m <= 8                                -> prepare_act_kernel + gemv_kernel / gemv_rows_kernel (5..8 rows against a
-//                                            wide short weight: the 16-row tile of gemm_i8_lds_kernel)
-//   m  > 8                                -> gemm_i8_lds_kernel (exact) or gemm_bf16_wide_kernel
+//                                            wide short weight: gemm_i8_kernel)
+//   m  > 8                                -> gemm_i8_kernel (exact) or gemm_bf16_wide_kernel
 // and the decode fusions built on the single-row kernel: RMSNorm / gelu-gate prologues, the q/k/v + RoPE +
 // cache-append launch and the GeGLU block (two launches).
 #include "common.h"
@@ -64,8 +64,25 @@ static bool fused_row_pays(const Batch &b) {
 // Prepared rows against the weights of `b`: the GEMV kernels up to eight rows, except five to eight rows over a K past 4096,
 // where the GEMV walks K with all eight accumulator sets live and falls far behind the exact GEMM's 16-row tile (q8
 // 14336 x 8192 at 8 rows: 80 against 33 us, q4 65 against 29; the two meet at K = 4096 ... 5120); the GEMM beyond eight rows.
+static bool rows_on_gemv(const Batch &b, size_t m) { return m <= GEMV_MAX_M && (b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)); }
+// which form of the preparation the kernel behind launch_prepared_rows reads
+static bool rows_tiled(const Batch &b, size_t m) {
+    if (b.k > GEMM_I8_MAX_K) return false;
+    return !rows_on_gemv(b, m) || gemv_rows_on_gemm(b.w, (int)b.count, (int)m);
+}
 static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, PreparedAct act, float alpha, float beta) {
-    if (m <= GEMV_MAX_M && !(m >= 5 && b.k > FUSED_PAYS_K))
+    if (m > GEMV_MAX_M && b.k > GEMM_I8_MAX_K) {                 // rows past the GEMM's addressing
+        Batch part = b;
+        for (size_t r0 = 0; r0 < m; r0 += GEMV_MAX_M) {
+            const size_t rows = m - r0 < GEMV_MAX_M ? m - r0 : GEMV_MAX_M, kb = b.k / QK;
+            for (size_t i = 0; i < b.count; ++i) part.c[i] = b.c[i] + r0 * b.ldc[i];
+            const PreparedAct at{act.q + r0 * b.k, act.scale + r0 * kb, act.sum + r0 * kb, false};
+            const int rc = launch_gemv_batch(ctx, part.w, part.c, part.ldc, (int)part.count, (int)rows, at, alpha, beta);
+            if (rc) return rc;
+        }
+        return AIONHIP_OK;
+    }
+    if (rows_on_gemv(b, m))
         return launch_gemv_batch(ctx, b.w, b.c, b.ldc, (int)b.count, (int)m, act, alpha, beta);
     // sibling weights (q/k/v, gate/up) share one launch, four at a time
     for (size_t i = 0; i < b.count; i += 4) {
@@ -110,7 +127,7 @@ int run_rows(aionhip_ctx *ctx, const Batch &b, size_t m, const float *a, size_t 
     }
     int rc = static_scratch ? (int)AIONHIP_OK : ensure_scratch(ctx, prepared_act_bytes(m, b.k));
     if (rc) return rc;
-    PreparedAct act = prepared_act_carve(static_scratch ? ctx->static_scratch : ctx->scratch, m, b.k);
+    PreparedAct act = prepared_act_carve(static_scratch ? ctx->static_scratch : ctx->scratch, m, b.k, rows_tiled(b, m));
     rc = launch_prepare_act(ctx, a, lda, m, b.k, act);
     if (rc) return rc;
     return launch_prepared_rows(ctx, b, m, act, alpha, beta);
@@ -193,7 +210,7 @@ int aionhip_step_rmsnorm_matmul(aionhip_ctx *ctx, size_t count, const aionhip_we
     if (rows >= 2 && rows <= 0x7FFFFFFFu && !bf16_route && ((x | gamma | beta_norm) & 15) == 0) {
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
         if (rc) return rc;
-        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k);
+        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(b, rows));
         rc = launch_prepare_rmsnorm(ctx, xp, gp, bp, eps, rows, b.k, act);
         if (rc) return rc;
         return launch_prepared_rows(ctx, b, rows, act, alpha, beta);
@@ -256,7 +273,7 @@ int aionhip_step_rmsnorm_geglu_matmul(aionhip_ctx *ctx, const aionhip_weight *w_
         return set_err(ctx, AIONHIP_UNSUPPORTED, "geglu_matmul: needs k <= %zu, a hidden size that is a multiple of 32 and 16-byte aligned x/gamma/beta", FUSED_MAX_K);
     int rc = ensure_scratch(ctx, prepared_act_bytes(1, w_down->k));
     if (rc) return rc;
-    PreparedAct act = prepared_act_carve(ctx->scratch, 1, w_down->k);
+    PreparedAct act = prepared_act_carve(ctx->scratch, 1, w_down->k, false);
     FusedIn in{(const float *)(uintptr_t)x, nullptr, (const float *)(uintptr_t)gamma, (const float *)(uintptr_t)beta_norm, eps};
     rc = launch_gemv_fused_geglu(ctx, w_gate, w_up, in, act);
     if (rc) return rc;
@@ -283,7 +300,7 @@ int aionhip_step_gate_matmul(aionhip_ctx *ctx, const aionhip_weight *w, size_t r
         // gate and activation preparation in one small launch, then the GEMV (or GEMM) on the prepared rows
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
         if (rc) return rc;
-        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k);
+        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(b, rows));
         rc = launch_prepare_gate(ctx, gp, up_p, rows, b.k, act);
         if (rc) return rc;
         return launch_prepared_rows(ctx, b, rows, act, alpha, beta);

@@ -110,6 +110,21 @@ __global__ void quantize_rank2_kernel(const float *__restrict__ src, uint8_t *__
     }
 }
 
+// Where quant block kb of a row lies in the tiled form of a prepared activation (PreparedAct)
+struct TiledSlot {
+    size_t base, scale;
+    unsigned rows, r;
+    __device__ __forceinline__ TiledSlot(size_t row, size_t kb, size_t m, size_t kb_per_row) {
+        const size_t mt = row >> 5;
+        rows = (unsigned)(m - mt * 32 < 32 ? m - mt * 32 : 32);
+        r = (unsigned)(row & 31);
+        scale = mt * 32 * kb_per_row + kb * rows + r;
+        base = (mt * 32 * kb_per_row + kb * rows) * 8;
+    }
+    // 32-bit word `sub` (0..7) of the block
+    __device__ __forceinline__ size_t word(int sub) const { return base + (size_t)(((sub >> 2) * rows + r) * 4 + (sub & 3)); }
+};
+
 // Activation preparation (aion matmul_q_i8.zig:187-203): 8 lanes share one 32-element block.
 // GATE: the activation is gelu_tanh(a) * up (aion cpu/exec/elementwise.zig:25-37), not written out.
 // RMSNorm + int8 preparation, one workgroup per row of k columns (k a multiple of 32; x, gamma, beta 16-byte aligned). The sum
@@ -117,10 +132,10 @@ __global__ void quantize_rank2_kernel(const float *__restrict__ src, uint8_t *__
 // is rounded as they round it ((x * inv) * gamma + beta), so the codes, scales and code sums are those of the norm step followed
 // by the preparation launch. SHORT: rows of up to 2048 columns, every load requested before the reduction (one memory round
 // trip); otherwise two passes over the row.
-template <bool SHORT>
+template <bool SHORT, bool TILED>
 __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
                                                               size_t cols, float eps, int *__restrict__ aq, float *__restrict__ a_scale,
-                                                              int *__restrict__ a_sum) {
+                                                              int *__restrict__ a_sum, size_t m) {
     __shared__ float red[4];
     const size_t row = blockIdx.x;
     const float *xr = x + row * cols;
@@ -132,7 +147,12 @@ __global__ __launch_bounds__(256) void rmsnorm_prepare_kernel(const float *__res
         int word, sm;
         float scale;
         prepare_act_block8(y0, y1, y2, y3, word, scale, sm);         // (all eight lanes of a block take part: chunks is a multiple of 8)
-        if (live) {
+        if (!live) return;
+        if (TILED) {
+            const TiledSlot t(row, c4 >> 3, m, kb_per_row);
+            aq[t.word((int)c4 & 7)] = word;
+            if ((c4 & 7) == 0) a_scale[t.scale] = scale;
+        } else {
             aq[row * chunks + c4] = word;
             if ((c4 & 7) == 0) {
                 a_scale[row * kb_per_row + (c4 >> 3)] = scale;
@@ -207,6 +227,35 @@ __global__ __launch_bounds__(256) void prepare_act_kernel(const float *__restric
     }
 }
 
+// The tiled form: 8 lanes per block again, consecutive lane groups on consecutive rows of one 32-row tile and block, so that a
+// wavefront reads eight 128-byte lines and writes two runs of 128 bytes. 32-bit index arithmetic (m * k / 32 blocks stay below 2^32:
+// the f32 rows would be half a terabyte), the rows' divisions once per lane.
+template <bool GATE>
+__global__ __launch_bounds__(256) void prepare_act_tiled_kernel(const float *__restrict__ a, const float *__restrict__ up, size_t lda, unsigned m,
+                                                                unsigned kb_per_row, int *__restrict__ aq, float *__restrict__ a_scale) {
+    const unsigned blk = blockIdx.x * 32 + (threadIdx.x >> 3), total = m * kb_per_row, b = min(blk, total - 1);
+    const int sub = threadIdx.x & 7;
+    const unsigned mt = min(b / (32 * kb_per_row), (m - 1) >> 5), rem = b - mt * 32 * kb_per_row, rows = min(m - mt * 32, 32u);
+    const unsigned kb = rem / rows, r = rem - kb * rows;
+    const size_t at = (size_t)(mt * 32 + r) * lda + (size_t)kb * QK + sub * 4;
+    const float *p = a + at;
+    float v0 = p[0], v1 = p[1], v2 = p[2], v3 = p[3];
+    if (GATE) {
+        const float *u = up + at;
+        v0 = aion_gate_gelu(v0, u[0]);
+        v1 = aion_gate_gelu(v1, u[1]);
+        v2 = aion_gate_gelu(v2, u[2]);
+        v3 = aion_gate_gelu(v3, u[3]);
+    }
+    int word, s;
+    float scale;
+    prepare_act_block8(v0, v1, v2, v3, word, scale, s);
+    if (blk >= total) return;
+    const size_t base = (size_t)(mt * 32 * kb_per_row + kb * rows);
+    aq[base * 8 + ((sub >> 2) * rows + r) * 4 + (sub & 3)] = word;
+    if (sub == 0) a_scale[base + r] = scale;
+}
+
 }  // namespace
 
 size_t prepared_act_bytes(size_t m, size_t k) {
@@ -214,13 +263,14 @@ size_t prepared_act_bytes(size_t m, size_t k) {
     const size_t s = (m * (k / QK) * 4 + 255) & ~(size_t)255;
     return q + 2 * s;
 }
-PreparedAct prepared_act_carve(void *base, size_t m, size_t k) {
+PreparedAct prepared_act_carve(void *base, size_t m, size_t k, bool tiled) {
     const size_t q = (m * k + 255) & ~(size_t)255;
     const size_t s = (m * (k / QK) * 4 + 255) & ~(size_t)255;
     PreparedAct p;
     p.q = (int8_t *)base;
     p.scale = (float *)((char *)base + q);
     p.sum = (int *)((char *)base + q + s);
+    p.tiled = tiled;
     return p;
 }
 int launch_prepare_act(aionhip_ctx *ctx, const float *a, size_t lda, size_t m, size_t k, PreparedAct out) {
@@ -228,6 +278,8 @@ int launch_prepare_act(aionhip_ctx *ctx, const float *a, size_t lda, size_t m, s
     if (!threads) return AIONHIP_OK;
     const size_t blocks = (threads + 255) / 256;
     ProfScope scope(ctx, "prepare_act");
+    if (out.tiled) launch_k(ctx, prepare_act_tiled_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, a, nullptr, lda, (unsigned)m, (unsigned)(k / QK), (int *)out.q, out.scale);
+    else
     launch_k(ctx, prepare_act_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, a, nullptr, lda, m, k, (int *)out.q, out.scale, out.sum);
     LAUNCH_CHECK(ctx, "prepare_act");
     return AIONHIP_OK;
@@ -237,6 +289,8 @@ int launch_prepare_gate(aionhip_ctx *ctx, const float *gate, const float *up, si
     if (!threads) return AIONHIP_OK;
     const size_t blocks = (threads + 255) / 256;
     ProfScope scope(ctx, "prepare_gate");
+    if (out.tiled) launch_k(ctx, prepare_act_tiled_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, gate, up, k, (unsigned)m, (unsigned)(k / QK), (int *)out.q, out.scale);
+    else
     launch_k(ctx, prepare_act_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, gate, up, k, m, k, (int *)out.q, out.scale, out.sum);
     LAUNCH_CHECK(ctx, "prepare_gate");
     return AIONHIP_OK;
@@ -247,8 +301,9 @@ int launch_prepare_gate(aionhip_ctx *ctx, const float *gate, const float *up, si
 int launch_prepare_rmsnorm(aionhip_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, size_t m, size_t k, PreparedAct out) {
     if (!m || !k) return AIONHIP_OK;
     ProfScope scope(ctx, "prepare_rmsnorm");
-    if (k <= 2048) launch_k(ctx, rmsnorm_prepare_kernel<true>, dim3((unsigned)m), dim3(256), 0, x, gamma, beta, k, eps, (int *)out.q, out.scale, out.sum);
-    else launch_k(ctx, rmsnorm_prepare_kernel<false>, dim3((unsigned)m), dim3(256), 0, x, gamma, beta, k, eps, (int *)out.q, out.scale, out.sum);
+    auto *kern = k <= 2048 ? (out.tiled ? rmsnorm_prepare_kernel<true, true> : rmsnorm_prepare_kernel<true, false>)
+                           : (out.tiled ? rmsnorm_prepare_kernel<false, true> : rmsnorm_prepare_kernel<false, false>);
+    launch_k(ctx, kern, dim3((unsigned)m), dim3(256), 0, x, gamma, beta, k, eps, (int *)out.q, out.scale, out.sum, m);
     LAUNCH_CHECK(ctx, "prepare_rmsnorm");
     return AIONHIP_OK;
 }

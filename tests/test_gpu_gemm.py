@@ -186,6 +186,32 @@ def test_exact_gemm_k_slices(gpu, orc, dtype, layout):
     w.free(); w2.free()
 
 
+# The exact GEMM's row tiles of 32 (the last one partial, alone and behind full ones), columns that end inside a tile, K of one block, of
+# less than a group of four, and of a group and one block; each division of K (2, 4 and 8 wavefronts per tile, 4 slices).
+# Tolerance: the dots are exact, so both sides are f32 sums of K / 32 terms, within K / 32 * 2^-24 * sum|terms| of the exact value;
+# the terms are of both signs and sum|terms| < 4 sqrt(K / 32) rms here: 3e-5 at 8192, 1e-6 seen.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(9, 31, 32), (31, 33, 64), (32, 32, 96), (33, 65, 160), (97, 64, 2080), (129, 1000, 2048), (64, 4099, 544),
+                                   (10, 2050, 8192), (1025, 4097, 64)])
+def test_exact_gemm_tiles_and_k_divisions(gpu, orc, dtype, layout, m, n, k):
+    say("exact gemm tiles", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    blocks, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    blocks2, w2 = make_weight(gpu, dtype, layout, 40, k, seed=m + k + 1)
+    a = np.random.default_rng(m * k).standard_normal((m, k)).astype(np.float32)
+    got, got2 = gpu.matmul(w, a), gpu.matmul(w2, a)
+    assert rms_err(got, oracle_i8(orc, dtype, layout, a, blocks, n)) < 3e-5
+    assert rms_err(got2, oracle_i8(orc, dtype, layout, a, blocks2, 40)) < 3e-5
+    # a weight gives the same bits beside a sibling, whether the two share their division of K (and a launch) or not
+    a_buf, c, c2 = gpu.upload(a), gpu.alloc(m * n * 4), gpu.alloc(m * 40 * 4)
+    gpu.step_matmul_batch([w, w2], a_buf, m, [c, c2])
+    assert np.array_equal(gpu.download(c, np.uint32, (m, n)), got.view(np.uint32))
+    assert np.array_equal(gpu.download(c2, np.uint32, (m, 40)), got2.view(np.uint32))
+    for t in (a_buf, c, c2):
+        t.free()
+    w.free(); w2.free()
+
+
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("m,n,k", [(2048, 14336, 4096), (512, 4096, 4096), (300, 520, 1056), (1300, 11008, 4096), (70, 200, 96)])
 def test_bf16_gemm_without_weight_copies_gives_the_same_bits(gpu, orc, dtype, layout, m, n, k):
