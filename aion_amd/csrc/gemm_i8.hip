@@ -97,9 +97,11 @@ int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, in
 template <int DT, int MT, int NT, int KS, int WGM, int SHAPE>
 int launch_shape(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m, PreparedAct act,
                  float alpha, float beta, int slices) {
-    constexpr int BM = 32 * MT * WGM, BN = 32 * NT, LDS = gemm_i8_lds_bytes<MT, NT, KS, WGM, 1>();
+    constexpr int BM = 32 * MT * WGM, BN = 32 * NT, LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, NT, KS, WGM, 1>();
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
-    static_assert(LDS <= 64 * 1024, "default LDS limit of a launch");
+    static_assert(LDS <= 80 * 1024, "two workgroups per CU");
+    if (LDS > 64 * 1024)
+        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
     GemmSegs segs{};
     segs.count = count;
     int tiles = 0;

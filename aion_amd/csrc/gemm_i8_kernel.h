@@ -6,22 +6,25 @@
 // four wavefronts on the SIMD but 2.0 .. 2.3 ns with one, conversion 1.8 ns; the MFMA 13.5 ns; the whole rescale of a tile 60 ns per
 // SIMD with two wavefronts and 115 with one. So the shape of this kernel: at least two wavefronts per SIMD at every size, and nothing that
 // makes them wait for each other. A wavefront owns a (32 MT) x (32 NT) tile and a share of K (every KS-th group of four blocks); the KS
-// wavefronts of a tile meet once, at the end, in LDS, in a fixed order. Operands go from global memory (L2) straight into the
-// MFMA's registers, two blocks ahead; there is no staging and no barrier in the loop.
-//   activations: prepared in operand order, a wavefront's load of a block is 1 KiB of consecutive memory; their scales are the one thing
-//     that passes through LDS (16 rows' scales per lane: a wavefront's private copy, 4 reads per row tile and block)
-//   weights: the row-major device layout. q8: a lane loads its row's 16 codes. q4: a lane loads 16 bytes = a whole block, the lane
-//     halves two neighbouring blocks, and two v_permlane32_swap give both halves their words of each
+// wavefronts of a tile meet once, at the end, in LDS, in a fixed order. No barrier in the loop: what a wavefront stages, it stages for itself.
+//   activations: prepared in operand order, a wavefront's load of a block is 1 KiB of consecutive memory, straight to registers, three blocks
+//     ahead
+//   weights and activation scales: LDS-writing buffer loads, a group of four blocks ahead. The row-major weight puts a lane's operand bytes
+//     (its row's 16 of a block) far from its neighbours', and the L1 takes such a load lane by lane: 64 accesses, 60 .. 85 % of its cycles
+//     at 2048 x 14336 x 4096 when the operands came straight from memory. Staged, neighbouring lanes read a row's consecutive bytes: 16
+//     accesses, whole lines. The lanes take 16 rows' scales from there (4 reads per row tile and block)
 // Other forms measured: f16 codes on v_mfma_f32_32x32x16_f16 (no conversion after the dot, 51 ns a tile, but the codes have to be
 // converted and the operands are twice the bytes), scale products as 4x4x1 outer products on the matrix pipe (82 ns), activation scales by
 // DPP broadcast (90 ns), an integer bias in place of the conversion (62 ns).
-// Measured (kernel alone, q4 / q8): 512 x 4096 x 4096 31 / 35 us = 550 / 490 TOP/s (LDS-staged 16 x 16 tiles with one or two
-// wavefronts per SIMD before: 46 / 47), 128 x 16384 x 2048 19 / 22 us (31), 128 x 2048 x 8192 12 / 17 us (31), 77 x 11008 x 4096 23 / 24 us
-// (38), 2048 x 14336 x 4096 365 / 415 us (450). Without the operand and scale loads the last one takes 225 us: what is left above
-// the rescale is the registers' fill from LDS and memory beside it.
+// Measured (whole calls, weights straight from memory -> staged): q8 8 x 14336 x 4096 19.3 -> 15.5 us, 2048 x 14336 x 4096 429 -> 384,
+// 512 x 4096 x 4096 41.3 -> 37.0; q4 374 -> 366, 36.8 -> 36.0, 128 x 2048 x 8192 15.5 -> 14.8 us (q4 asks for half the bytes). What is left is
+// the vector ALU: 52 instructions a tile and block at 3.6 cycles each.
 #pragma once
 #include "common.h"
 
+#include <type_traits>
+
+using i32x2 = __attribute__((ext_vector_type(2))) int;
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 using i32x16 = __attribute__((ext_vector_type(16))) int;
 using f32x16 = __attribute__((ext_vector_type(16))) float;
@@ -41,8 +44,11 @@ struct GemmSegs {
 // block of a full tile is 1 KiB of consecutive memory; scales per tile and block [row].
 __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M - mt * 32 < 32 ? M - mt * 32 : 32; }
 
+// LDS of a wavefront: two groups of four blocks, weight codes and activation scales
+template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
+
 template <int DT, int MT, int NT, int KS, int WGM, int WGN>
-__global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
+__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
                                                                          int M, int K, int row_tiles, int row_group, int col_tiles, float alpha, float beta,
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
@@ -84,19 +90,23 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
         ab[i] = aq + (size_t)mt * 32 * K;
         ao[i] = (unsigned)(h * arows[i] + min(r, arows[i] - 1)) * 16;
         asb[i] = a_scale + (size_t)mt * 32 * KB;
-        aso[i] = (unsigned)min(r, arows[i] - 1);
+        aso[i] = (unsigned)min(r, arows[i] - 1) * 4;
     }
     const int nb = min(n0, N - 1);
     const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-    const uint8_t *wb = qs + (size_t)nb * wpitch;
+    [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch;      // (used in the device pass only)
     const __half *sb = sc + (size_t)nb * KB;
-    unsigned wo[NT], so[NT];
+    // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
+    constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
+    const int w_row = lane / LPR;
+    unsigned wo[NT][WL];
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-        const unsigned row = (unsigned)(min(n0 + i * 32 + r, N - 1) - nb);
-        wo[i] = row * wpitch + (unsigned)h * 16;         // (q4: a lane half takes the next block, 16 bytes on)
-        so[i] = row * (unsigned)KB;
-    }
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int l = 0; l < WL; ++l)
+            wo[i][l] = (unsigned)(min(n0 + i * 32 + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
+    // weight scales: with two tiles a lane half takes one tile's rows each and the halves are exchanged afterwards
+    const unsigned so = (unsigned)(min(n0 + (NT == 2 ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
 
     f32x16 acc[MT][NT];
 #pragma unroll
@@ -110,47 +120,60 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
     const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
     const int g_lo = (int)blockIdx.z * g_per, g_hi = min(G, g_lo + g_per);
 
-    // operand registers: block b of the sequence lives in set b & 3; requested two blocks ahead
+    // Registers: the four blocks of a group's activations (reloaded for the next group as each is used up), the next group's weight
+    // scales. LDS, private to the wavefront and written by the loads themselves: two groups of weight codes and activation scales.
     i32x4 A[4][MT];
-    i32x4 W[Q8 ? 4 : 2][NT];                   // q8: a block; q4: a pair of blocks (lanes 0..31 the even one, 32..63 the odd one)
-    unsigned long sw_raw[NT];                  // four f16 scales of the lane's weight row
-    int sw_shift = 0;
-    float sa_raw[2][MT];                       // two of the group's 4 x 32 activation scales per lane
-    float *sa_lds = (float *)lds + wave * (2 * MT * 128);
+    unsigned long sw_raw = 0, sw_now = 0;      // four f16 scales of a weight row: the next group's, this group's
+    int sw_shift = 0, sw_shift_now = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wb, 0, 0xFFFFFFFFu, 0x00027000);
+    __amdgpu_buffer_rsrc_t sa_rsrc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i) sa_rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void *)asb[i], 0, 0xFFFFFFFFu, 0x00027000);
+#endif
+    constexpr int LGKM0 = vmcnt_imm(63) & ~(15 << 8);        // every LDS operation has completed
+    constexpr int WBUF = NT * 32 * RB;
+    unsigned char *w_lds = lds + wave * gemm_i8_wave_lds_bytes<Q8, MT, NT>();
+    float *sa_lds = (float *)(w_lds + 2 * WBUF);
     auto load_a = [&](int set, int kb) {
         kb = min(kb, KB - 1);
 #pragma unroll
         for (int i = 0; i < MT; ++i) A[set][i] = *(const i32x4 *)(ab[i] + (size_t)((unsigned)kb * (unsigned)(arows[i] * 32)) + ao[i]);
     };
-    auto load_w8 = [&](int set, int kb) {
-        kb = min(kb, KB - 1);
+    // Row R of a tile is at R * RB, its 16-byte piece c in slot c ^ (R & 7) (q8) or c ^ ((R >> 1) & 3) (q4): the lanes of a read,
+    // consecutive rows at one piece, then cover 128 bytes of banks. (Blocks past the end of K: another row's or the slack behind the
+    // weight, scale 0.)
+    auto load_w = [&](int g, int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the builtin exists in the device pass only
 #pragma unroll
-        for (int i = 0; i < NT; ++i) W[set][i] = *(const i32x4 *)(wb + (size_t)(unsigned)(kb * 32) + wo[i]);
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int l = 0; l < WL; ++l)
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
+#endif
     };
-    auto load_w4 = [&](int set, int kb) {                // (one block past the end of K: another row's or the slack behind the weight, scale 0)
-        kb = min(kb, KB - 1);
+    const int r_slot = Q8 ? h ^ (r & 7) : (r >> 1) & 3;
+    using Codes = typename std::conditional<Q8, i32x4, i32x2>::type;    // what a lane's MFMA operand is made of: 16 codes, 16 nibbles
+    Codes Bn[NT];
+    auto read_b = [&](int buf, int j) {
 #pragma unroll
-        for (int i = 0; i < NT; ++i) W[set][i] = *(const i32x4 *)(wb + (size_t)(unsigned)(kb * 16) + wo[i]);
+        for (int i = 0; i < NT; ++i)
+            Bn[i] = *(const Codes *)(w_lds + buf * WBUF + (i * 32 + r) * RB + (Q8 ? ((2 * j) ^ r_slot) * 16 : (j ^ r_slot) * 16 + h * 8));
     };
     struct __attribute__((packed, aligned(2))) U64 { unsigned long v; };
-    auto load_scales = [&](int g) {
+    auto load_scales = [&](int g, int buf) {
         const int kb = min(g * 4, KB - 1), base = max(0, min(kb, KB - 4));
         sw_shift = (kb - base) * 16;
+        sw_raw = ((const U64 *)(sb + base + so))->v;
+#if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-        for (int i = 0; i < NT; ++i) sw_raw[i] = ((const U64 *)(sb + base + so[i]))->v;
-        const int b0 = min(kb, KB - 1), b1 = min(kb + 1, KB - 1), b2 = min(kb + 2, KB - 1), b3 = min(kb + 3, KB - 1);
+        for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            sa_raw[0][i] = asb[i][aso[i] + (unsigned)((h ? b1 : b0) * arows[i])];
-            sa_raw[1][i] = asb[i][aso[i] + (unsigned)((h ? b3 : b2) * arows[i])];
-        }
-    };
-    auto store_sa = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i) {
-            sa_lds[(buf * MT + i) * 128 + lane] = sa_raw[0][i];
-            sa_lds[(buf * MT + i) * 128 + 64 + lane] = sa_raw[1][i];
-        }
+            for (int q = 0; q < 2; ++q)                  // two blocks' scales of 32 rows
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(sa_rsrc[i], (lds_void *)(sa_lds + (buf * MT + i) * 128 + q * 64), 4,
+                                                         aso[i] + (h && g * 4 + 2 * q + 1 < KB ? (unsigned)arows[i] * 4 : 0u),
+                                                         min(g * 4 + 2 * q, KB - 1) * arows[i] * 4, 0, 0);
+#endif
     };
 
     // the activation scales a lane multiplies with - 16 rows of each row tile - come from the wavefront's LDS copy of the group
@@ -164,14 +187,15 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
     };
     int g = g_lo + ks;
     if (g < g_hi) {
-        load_scales(g);
+        load_w(g, 0);
+        load_scales(g, 0);
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            load_a(j, g * 4 + j);
-            if constexpr (Q8) load_w8(j, g * 4 + j);
-            else if ((j & 1) == 0) load_w4(j >> 1, g * 4 + j);
-        }
-        store_sa(0);
+        for (int j = 0; j < 3; ++j) load_a(j, g * 4 + j);
+        sw_now = sw_raw;
+        sw_shift_now = sw_shift;
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        asm volatile("" ::: "memory");
+        read_b(0, 0);
 #pragma unroll
         for (int i = 0; i < MT; ++i) read_sa(i, 0, 0);
     }
@@ -179,43 +203,57 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
     i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
     float sw_due = 0.f;
     for (; g < g_hi; g += KS) {
-        const int gn = g + KS < g_hi ? g + KS : g;       // the last group's look-ahead repeats it (never used)
+        const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
         float sw[4][NT];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < NT; ++i) {
-                const unsigned short hb = (unsigned short)((sw_raw[i] >> sw_shift) >> (16 * j));
-                sw[j][i] = g * 4 + j < KB ? __half2float(__ushort_as_half(hb)) : 0.f;
+        {
+            const unsigned long v = sw_now >> sw_shift_now;
+            unsigned lo[2], hi[2];
+            if constexpr (NT == 2) {
+                const auto x = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+                const auto y = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+                lo[0] = x[0]; lo[1] = x[1]; hi[0] = y[0]; hi[1] = y[1];
+            } else {
+                lo[0] = (unsigned)v; hi[0] = (unsigned)(v >> 32);
             }
-        load_scales(gn);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < NT; ++i)
+                    sw[j][i] = g * 4 + j < KB ? __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            load_a((j + 2) & 3, j < 2 ? g * 4 + j + 2 : gn * 4 + j - 2);
-            if constexpr (Q8) load_w8((j + 2) & 3, j < 2 ? g * 4 + j + 2 : gn * 4 + j - 2);
-            else if (j == 0) load_w4(1, g * 4 + 2);
-            else if (j == 2) load_w4(0, gn * 4);
-            if (j == 3) store_sa(buf ^ 1);
+            // The other buffer was last read in the previous group (those reads have returned once lgkmcnt is 0); its loads have three
+            // steps' time, and 3 MT younger ones are in flight when they are waited for. They are buffer loads: global_load_lds counts as a
+            // flat access, after which the compiler waits for every load in flight before the next use of any.
+            if (j == 0) {
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_waitcnt(LGKM0);
+                __builtin_amdgcn_sched_barrier(0);
+                load_w(gn, buf ^ 1);
+                load_scales(gn, buf ^ 1);
+            }
+            load_a((j + 3) & 3, j == 0 ? g * 4 + 3 : gn * 4 + j - 1);
             __builtin_amdgcn_sched_barrier(0);
+            if (j == 3) {
+                __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * MT));
+                asm volatile("" ::: "memory");
+            }
             i32x4 B[NT];
 #pragma unroll
             for (int i = 0; i < NT; ++i) {
                 if constexpr (Q8) {
-                    B[i] = W[j][i];
+                    B[i] = Bn[i];                        // (copied by the loop's unrolling: no instruction)
                 } else {
-                    // lanes 0..31 hold words 0..3 of the even block, lanes 32..63 of the odd one; a half needs words 2h, 2h + 1 of one block
-                    if ((j & 1) == 0) {
-                        const auto x = __builtin_amdgcn_permlane32_swap(W[j >> 1][i].x, W[j >> 1][i].z, false, false);
-                        const auto y = __builtin_amdgcn_permlane32_swap(W[j >> 1][i].y, W[j >> 1][i].w, false, false);
-                        W[j >> 1][i] = i32x4{(int)x[0], (int)y[0], (int)x[1], (int)y[1]};
-                    }
-                    const unsigned w0 = (j & 1) ? W[j >> 1][i].z : W[j >> 1][i].x, w1 = (j & 1) ? W[j >> 1][i].w : W[j >> 1][i].y;
                     // 16 * (nibble - 8) as int8: the nibble in the upper half of its byte with the top bit flipped; the sums are divided by
                     // 16 at the end (in the scales, the division would round where a product of scales is subnormal)
+                    const unsigned w0 = Bn[i].x, w1 = Bn[i].y;
                     B[i] = i32x4{(int)(((w0 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w0 & 0xF0F0F0F0u) ^ 0x80808080u),
                                  (int)(((w1 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w1 & 0xF0F0F0F0u) ^ 0x80808080u)};
                 }
             }
+            read_b(j == 3 ? buf ^ 1 : buf, (j + 1) & 3);
             // a tile's dots are issued ahead of the previous tile's rescale (the last tile's is left to the next block); the empty
             // asm statements keep that order. A row tile's scales of the next block are read once the block's last use of them is past.
 #pragma unroll
@@ -232,7 +270,10 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
             sw_due = sw[j][NT - 1];
         }
         buf ^= 1;
+        sw_now = sw_raw;
+        sw_shift_now = sw_shift;
     }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));            // no LDS-writing load may outlive the loop: its LDS is reused, or another workgroup's
     // the last block's last tile (a wavefront without a group has none)
     if (g_lo + ks < g_hi)
 #pragma unroll
@@ -285,7 +326,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, 2) void gemm_i8_kernel(GemmSeg
     }
 }
 
-template <int MT, int NT, int KS, int WGM, int WGN> constexpr int gemm_i8_lds_bytes() {
-    const int scales = KS * WGM * WGN * 2 * MT * 512, red = KS > 1 ? KS * WGM * WGN * MT * NT * 4096 : 0;
-    return scales > red ? scales : red;
+template <bool Q8, int MT, int NT, int KS, int WGM, int WGN> constexpr int gemm_i8_lds_bytes() {
+    const int operands = KS * WGM * WGN * gemm_i8_wave_lds_bytes<Q8, MT, NT>(), red = KS > 1 ? KS * WGM * WGN * MT * NT * 4096 : 0;
+    return operands > red ? operands : red;
 }
