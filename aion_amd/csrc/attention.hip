@@ -12,6 +12,7 @@
 //     split mode (few query rows: decode) - a workgroup is one 16-row tile x one key segment, its
 //       eight wavefronts interleave 32-key tiles and merge through LDS; segments merge in
 //       attn_merge_kernel (the flash-decoding split of cpu/exec/attention.zig:879-962).
+//       Where that leaves CUs idle, the value columns are divided over up to D / 64 workgroups as well.
 //     per-wavefront mode - a workgroup is four 16-row tiles, each wavefront walks its own key range; used
 //       for many query rows only when the hi+lo precise mode is on (see attn_prefill_kernel otherwise).
 // attn_prefill_kernel (attention_prefill.hip) - many query rows: 128 rows per workgroup, K/V tiles shared through LDS,
@@ -37,11 +38,12 @@ struct FlashKernelHooks {
     __device__ __forceinline__ void store_out(float *out, size_t index, f32x4 v) { *(f32x4 *)(out + index) = v; }
 };
 
-template <int KV, int D, bool SPLIT, bool HILO, bool RING = false>
+template <int KV, int D, bool SPLIT, bool HILO, bool RING = false, int DVS = 1>
 __global__ __launch_bounds__(SPLIT ? SPLIT_NW * 64 : 256) void attn_flash_kernel(AttnArgs a) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     FlashKernelHooks hooks;
-    attn_flash_body<KV, D, SPLIT, HILO, RING>(a, lds, (int)blockIdx.x, (int)blockIdx.y, hooks);
+    const int tiles = SPLIT ? (int)gridDim.x / DVS : 0, slice = DVS == 1 ? 0 : (int)blockIdx.x / tiles;
+    attn_flash_body<KV, D, SPLIT, HILO, RING, DVS>(a, lds, (int)blockIdx.x - slice * tiles, (int)blockIdx.y, hooks, slice);
 }
 
 // log-sum-exp merge of the key segments: one workgroup per (row tile, 16-wide dv slice, unit).
@@ -175,10 +177,23 @@ __global__ __launch_bounds__(256) void attn_generic_kernel(AttnArgs a, int d_k, 
     }
 }
 
+template <int KV, int D, bool HILO, bool RING, int DVS>
+int launch_flash_split(aionhip_ctx *ctx, AttnArgs &a) {
+    constexpr int LDS = FlashCfg<D, SPLIT_NW, DVS>::LDS_BYTES;
+    static bool attr_split = false;   // per kernel instantiation
+    if (!attr_split) {
+        HIP_TRY(ctx, hipFuncSetAttribute((const void *)attn_flash_kernel<KV, D, true, HILO, RING, DVS>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        attr_split = true;
+    }
+    ProfScope scope(ctx, "attn_flash_split");
+    launch_k(ctx, attn_flash_kernel<KV, D, true, HILO, RING, DVS>, dim3((unsigned)(a.row_tiles * a.nseg * DVS), (unsigned)(a.B * a.Hkv)),
+             dim3(SPLIT_NW * 64), LDS, a);
+    return AIONHIP_OK;
+}
+
 template <int KV, int D, bool HILO, bool RING = false>
 int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     using Cfg = FlashCfg<D, 4>;
-    using SplitCfg = FlashCfg<D, SPLIT_NW>;
     const int units = a.B * a.Hkv;
     // Few query rows, or so few 128-row prefill workgroups that they would occupy under a quarter of the CUs
     // (measured: one batch, one kv head, up to ~1024 positions x 8 heads): 16-row tiles spread the K/V reads
@@ -227,15 +242,17 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
             if (rc) return rc;
             a.partial = (float *)ctx->scratch2;
         }
-        static bool attr_split = false;   // per kernel instantiation
-        if (!attr_split) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)attn_flash_kernel<KV, D, true, HILO, RING>, hipFuncAttributeMaxDynamicSharedMemorySize, SplitCfg::LDS_BYTES));
-            attr_split = true;
-        }
-        {
-            ProfScope scope(ctx, "attn_flash_split");
-            launch_k(ctx, attn_flash_kernel<KV, D, true, HILO, RING>, dim3((unsigned)(a.row_tiles * nseg), (unsigned)units), dim3(SPLIT_NW * 64), SplitCfg::LDS_BYTES, a);
-        }
+        // Workgroups that leave CUs idle divide the value columns as well, down to 64 each: the scores are computed by every share,
+        // the loads of V, the second product and the merge of the wavefronts through LDS are divided. A short cache (one key
+        // segment) is a chain of latencies in one CU, of which those three were about 2 us of 9.8: one token over 144 keys, one KV
+        // head of size 256, 9.8 -> 8.0 us; over 1531 keys, 8 KV heads of size 128, 10.8 -> 10.4 with the segments' merge. Only
+        // while the shares fit one workgroup per CU: past that a second round costs more than a share saves.
+        const long wgs = (long)units * a.row_tiles * nseg;
+        int rc;
+        if (D >= 256 && wgs * (D / 64) <= cus) rc = launch_flash_split<KV, D, HILO, RING, D / 64>(ctx, a);
+        else if (D >= 128 && wgs * 2 <= cus) rc = launch_flash_split<KV, D, HILO, RING, D >= 128 ? 2 : 1>(ctx, a);
+        else rc = launch_flash_split<KV, D, HILO, RING, 1>(ctx, a);
+        if (rc) return rc;
         if (nseg > 1) {
             ProfScope scope(ctx, "attn_merge");
             launch_k(ctx, attn_merge_kernel<D>, dim3((unsigned)(a.row_tiles * (D / MERGE_DV)), (unsigned)units), dim3(256), 0, a);

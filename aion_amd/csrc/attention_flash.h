@@ -9,12 +9,13 @@ namespace attn {
 
 // NW = wavefronts per workgroup: 4 in prefill mode, 8 in split mode (a decode over a short cache
 // is one workgroup whose eight wavefronts take one 32-key tile each)
-template <int D, int NW>
+template <int D, int NW, int DVS = 1>
 struct FlashCfg {
-    static constexpr int ROW_BYTES = D * 2;                      // unpadded: the tile is filled by LDS-writing loads
+    static constexpr int DV = D / DVS;                           // the workgroup's share of a value row
+    static constexpr int ROW_BYTES = DV * 2;                     // unpadded: the tile is filled by LDS-writing loads
     static constexpr int WAVE_LDS = TILE_KEYS * ROW_BYTES;       // one V tile per wavefront
     static constexpr int WG_LDS = NW * WAVE_LDS;
-    static constexpr int MERGE_LDS = (NW * (16 * (D + 4) + 32) + 16 * NW + 32) * 4;   // split mode: NW x (acc[16][D+4], m[16], l[16]) f32 + merge factors
+    static constexpr int MERGE_LDS = (NW * (16 * (DV + 4) + 32) + 16 * NW + 32) * 4;   // split mode: NW x (acc[16][DV+4], m[16], l[16]) f32 + merge factors
     static constexpr int Q_ROW = D * 2 + 64;                     // split mode: the 16 query rows in the K/V element type
     static constexpr int Q_OFF = WG_LDS > MERGE_LDS ? WG_LDS : MERGE_LDS;
     static constexpr int LDS_BYTES = Q_OFF + 16 * Q_ROW;
@@ -26,13 +27,19 @@ constexpr int SPLIT_NW = 8;
 // q arrives as f32 (aion's cached decode: f32 q over an f16 cache). K and V are exact either way.
 // RING: the caches are rolling rings (a.ring = T). A template flag, not a run-time test: the identity instances
 // must not carry the ring's extra live values (both kernels sit at their register limit).
-template <int KV, int D, bool SPLIT, bool HILO, bool RING, class Hooks>
-__device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int block_x, const int block_y, Hooks &hooks) {
+// DVS (split mode): DVS workgroups share a row tile and key segment, each computing all of its scores and a DVS-th of the value
+// columns (the slice_dv-th); an output element is the same sum in the same order whatever DVS is.
+template <int KV, int D, bool SPLIT, bool HILO, bool RING, int DVS = 1, class Hooks>
+__device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int block_x, const int block_y, Hooks &hooks,
+                                                const int slice_dv = 0) {
     const int ring = RING ? a.ring : 0;
     constexpr int NW = SPLIT ? SPLIT_NW : 4;
-    using Cfg = FlashCfg<D, NW>;
+    using Cfg = FlashCfg<D, NW, DVS>;
+    static_assert(SPLIT || DVS == 1, "value columns are divided in split mode only");
+    constexpr int DV = Cfg::DV;
     constexpr int KK = D / 32;   // MFMA k-steps over the head dim
-    constexpr int MT = D / 16;   // 16-wide dv tiles
+    constexpr int MT = DV / 16;  // 16-wide dv tiles
+    const int dv0 = DVS == 1 ? 0 : slice_dv * DV;
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
@@ -171,20 +178,20 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     // K (MFMA operand layout, registers) of a tile is requested one tile ahead, right after the S MFMAs
     // have released the registers. V goes global -> LDS directly (global_load_lds_dwordx4, 1 KiB per
     // instruction) into this wavefront's tile, requested as soon as the previous tile's gathers are done.
-    // Tile layout: key row of D*2 bytes, 16-byte chunk c of key k at slot c ^ (2 * ((k >> 2) & 3)) ^ (8 * (k & 1)) (the
+    // Tile layout: key row of DV*2 bytes, 16-byte chunk c of key k at slot c ^ (2 * ((k >> 2) & 3)) ^ (8 * (k & 1)) (the
     // last term for rows of 256 bytes and more; 128-byte rows alternate bank halves by themselves): the sixteen keys
     // one transposing read of the second product covers (four key groups x four keys) then fall on eight distinct
     // 32-byte bank ranges, two keys each - 512 bytes in the two passes they need anyway. Keys outside the union interval are read from
     // a clamped in-range key instead (their probabilities are exact zeros, and the cache tail may hold
     // anything, so the value must only be finite).
-    constexpr int NVI = TILE_KEYS * D * 2 / 1024;
-    constexpr int KEYS_PER_VI = 1024 / (D * 2);
+    constexpr int NVI = TILE_KEYS * DV * 2 / 1024;
+    constexpr int KEYS_PER_VI = 1024 / (DV * 2);
     // Addresses: while one batch entry's cache is under 2 GiB (a uniform test) a row is reached by a 32-bit byte
     // offset from a uniform base - one 24-bit multiply-add per load instead of 64-bit arithmetic, which counts
     // when a lone workgroup issues a whole short cache's loads.
     const unsigned row_bytes = (unsigned)(kv_row * 2);
     const bool near = (size_t)a.T * kv_row * 2 < ((size_t)1 << 31) && a.T < (1 << 24) && row_bytes < (1u << 24);
-    const unsigned char *kb8 = (const unsigned char *)(kp + kv_base), *vb8 = (const unsigned char *)(vp + kv_base);
+    const unsigned char *kb8 = (const unsigned char *)(kp + kv_base), *vb8 = (const unsigned char *)(vp + kv_base + dv0);
     const int k_last = RING ? max(uni_hi - 1, 0) : a.T - 1;        // the last key a K load may name
     u32x4 kf[2][KK];
     auto load_k_as = [&](int t, auto near_c) __attribute__((always_inline)) {
@@ -205,8 +212,8 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             }
         }
     };
-    const int v_key_in = (lane * 16) / (D * 2);                      // key of this lane within one V load
-    const int v_slot = ((lane * 16) % (D * 2)) / 16;                 // its 16-byte slot within the key row
+    const int v_key_in = (lane * 16) / (DV * 2);                     // key of this lane within one V load
+    const int v_slot = ((lane * 16) % (DV * 2)) / 16;                // its 16-byte slot within the key row
     const int v_hi_key = max(uni_hi - 1, 0);
     (void)NVI; (void)KEYS_PER_VI; (void)vb8; (void)v_key_in; (void)v_slot; (void)v_hi_key;   // (used by the V loads, which exist in the device pass only)
     auto load_k = [&](int t) __attribute__((always_inline)) {
@@ -223,12 +230,12 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             const int key = i * KEYS_PER_VI + v_key_in;
             // (key >> 2) & 3 does not depend on the lane while an instruction covers at most four keys
             const int grp = KEYS_PER_VI <= 4 ? ((i * KEYS_PER_VI) >> 2) & 3 : (key >> 2) & 3;
-            const int chunk = v_slot ^ (2 * grp) ^ (D >= 128 ? 8 * (key & 1) : 0);
+            const int chunk = v_slot ^ (2 * grp) ^ (DV >= 128 ? 8 * (key & 1) : 0);
             const int kabs = tm.row(min(max(key0 + key, uni_lo), v_hi_key));
             if (near)
                 __builtin_amdgcn_global_load_lds(vb8 + (__umul24((unsigned)kabs, row_bytes) + (unsigned)chunk * 16u), (lds_void *)(vs + i * 1024), 16, 0, 0);
             else
-                __builtin_amdgcn_global_load_lds(vp + kv_base + (size_t)kabs * kv_row + chunk * 8, (lds_void *)(vs + i * 1024), 16, 0, 0);
+                __builtin_amdgcn_global_load_lds(vp + kv_base + dv0 + (size_t)kabs * kv_row + chunk * 8, (lds_void *)(vs + i * 1024), 16, 0, 0);
         }
 #endif
     };
@@ -239,7 +246,7 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     // V^T operand addresses (second product): lane = 16*g + 4*r + q reads key 4g+r (and 16+4g+r), dv 16*mt + 4q .. +3
     const int tr_r = (lane >> 2) & 3, tr_q = lane & 3;
     const unsigned v_rowaddr = (unsigned)(size_t)(lds_void *)vs + (unsigned)((4 * g + tr_r) * Cfg::ROW_BYTES + (tr_q & 1) * 8);
-    const unsigned v_slot_l = (unsigned)(((tr_q >> 1) ^ (2 * g) ^ (D >= 128 ? 8 * (tr_r & 1) : 0)) << 4);
+    const unsigned v_slot_l = (unsigned)(((tr_q >> 1) ^ (2 * g) ^ (DV >= 128 ? 8 * (tr_r & 1) : 0)) << 4);
     if (t_begin < t_end) {
         load_k(t_begin);
         load_v(t_begin);
@@ -340,9 +347,9 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             // V: the same stale row, overwritten in the wavefront's LDS tile (16-byte chunk c of key k sits in slot
             // c ^ 2 * ((k >> 2) & 3) ^ 8 * (k & 1), the last term for rows of 256 bytes and more) before any operand read
             const int rel = hooks.new_key() - key0;
-            if (t == t_begin && rel >= 0 && rel < TILE_KEYS && lane < D / 8) {
-                const int slot = lane ^ (2 * ((rel >> 2) & 3)) ^ (D >= 128 ? 8 * (rel & 1) : 0);
-                *(u32x4 *)(vs + rel * Cfg::ROW_BYTES + slot * 16) = hooks.new_v(hk * D + lane * 8);
+            if (t == t_begin && rel >= 0 && rel < TILE_KEYS && lane < DV / 8) {
+                const int slot = lane ^ (2 * ((rel >> 2) & 3)) ^ (DV >= 128 ? 8 * (rel & 1) : 0);
+                *(u32x4 *)(vs + rel * Cfg::ROW_BYTES + slot * 16) = hooks.new_v(hk * D + dv0 + lane * 8);
             }
         }
 
@@ -387,11 +394,11 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         return;
     }
 
-    // ---- split mode: merge the wavefronts through LDS. Rows are D+4 floats apart so that the sixteen
+    // ---- split mode: merge the wavefronts through LDS. Rows are DV+4 floats apart so that the sixteen
     // lanes of a row group write their 16-byte pieces to distinct banks.
     __syncthreads();
     float *mg = (float *)lds;
-    constexpr int RS = D + 4;                 // padded row stride (floats)
+    constexpr int RS = DV + 4;                // padded row stride (floats)
     constexpr int WSTRIDE = 16 * RS + 32;     // one wavefront's slot: acc[16][RS], m[16], l[16]
     {
         float *w = mg + wave * WSTRIDE;
@@ -405,8 +412,8 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     // partial slot layout in global memory (read by attn_merge_kernel): [16][D] o, [16] m, [16] l
     constexpr int PSTRIDE = 16 * D + 32;
     const size_t pslot = ((size_t)(unit * a.row_tiles + rt) * a.nseg + seg) * PSTRIDE;
-    for (int e = threadIdx.x; e < 16 * D / 4; e += NW * 64) {
-        const int row = e / (D / 4), col = (e % (D / 4)) * 4;
+    for (int e = threadIdx.x; e < 16 * DV / 4; e += NW * 64) {
+        const int row = e / (DV / 4), col = (e % (DV / 4)) * 4;
         float mw[NW];
         float m_all = -INFINITY;
 #pragma unroll
@@ -427,11 +434,11 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             if (rr < a.rows_total) {
                 const int l2 = rr / a.groups, g2 = rr % a.groups;
                 const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
-                hooks.store_out(a.out, (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g2) * D + col, o * inv);
+                hooks.store_out(a.out, (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g2) * D + dv0 + col, o * inv);
             }
         } else if (rt * 16 + row < a.rows_total) {        // (rows past the last query row are padding: nobody reads them)
-            *(f32x4 *)(a.partial + pslot + row * D + col) = o;
-            if (col == 0) {
+            *(f32x4 *)(a.partial + pslot + row * D + dv0 + col) = o;
+            if (col == 0 && dv0 == 0) {
                 a.partial[pslot + 16 * D + row] = m_all;
                 a.partial[pslot + 16 * D + 16 + row] = l_all;
             }

@@ -143,6 +143,36 @@ def test_decode_ragged_lengths_and_stale_cache_tail(gpu, orc):
     attn_err(got, ref, 2e-3)
 
 
+@pytest.mark.parametrize("D,precise", [(64, False), (128, False), (256, False), (128, True), (256, True)])
+@pytest.mark.parametrize("T", [200, 600])                         # one key segment, three
+def test_decode_value_columns_divided_or_not(gpu, orc, T, D, precise):
+    """A decode step that leaves CUs idle divides the value columns over workgroups, down to 64 each: 1, 40 and 80 sequences
+    take D / 64, 2 and 1 shares, with the same key segments. Every output is the same sum in the same order, so a sequence's
+    row is the same bits whatever batch it is in; lengths end anywhere in a key tile and the cache tails hold NaN."""
+    B, Hq, Hkv = 80 if T == 600 else 160, 8, 1
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T + D, B, 1, T, Hq, Hkv, D, "f16")
+    lens = np.random.default_rng(D).integers(1, T + 1, B).astype(np.int32)
+    lens[:3] = (T, 1, 33)
+    for b in range(B):
+        for x, f in ((k, kf), (v, vf)):
+            x[b, lens[b]:], f[b, lens[b]:] = np.nan, 0
+    pos = (lens - 1).reshape(B, 1)
+
+    def rows(s):
+        return run_attention(gpu, q[s], k[s], v[s], 1 / math.sqrt(D), qd, kd, positions=pos[s], kv_lengths=lens[s])
+
+    gpu.set_attention_precise(precise)
+    try:
+        whole = rows(slice(0, B))
+        assert gpu.last_kernel() == "attn_flash_split"
+        attn_err(whole[:8], orc.attention_f64(qf[:8], kf[:8], vf[:8], 1 / math.sqrt(D), positions=pos[:8], kv_lengths=lens[:8]), 2e-3)
+        assert np.array_equal(rows(slice(0, B // 2)), whole[: B // 2])
+        for b in (0, 1, 2, B - 1):
+            assert np.array_equal(rows(slice(b, b + 1)), whole[b: b + 1]), (b, lens[b])
+    finally:
+        gpu.set_attention_precise(False)
+
+
 @pytest.mark.parametrize("window", [(100, 0, 0), (16, 0, 64), (be.UNBOUNDED, be.UNBOUNDED, 0), (5, 3, 0)])
 def test_windows_prefill_and_decode(gpu, orc, window):
     B, L, Hq, Hkv, D = 1, 200, 4, 1, 64
