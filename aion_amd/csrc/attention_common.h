@@ -111,6 +111,36 @@ __device__ __forceinline__ int wave_max_i(int v) {
     for (int o = 32; o >= 1; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
     return v;
 }
+// Minimum / maximum over the sixteen rows of a wavefront whose lanes l, l + 16, l + 32, l + 48 hold the same value: four DPP steps on
+// the vector pipe (an LDS permute is some 60 cycles of latency each), the result in a scalar register.
+__device__ __forceinline__ int rows16_min_i(int v) {
+    v = min(v, dpp_i<DPP_QUAD_XOR1>(v));
+    v = min(v, dpp_i<DPP_QUAD_XOR2>(v));
+    v = min(v, dpp_i<DPP_ROW_HALF_MIRROR>(v));
+    v = min(v, dpp_i<DPP_ROW_MIRROR>(v));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+__device__ __forceinline__ int rows16_max_i(int v) {
+    v = max(v, dpp_i<DPP_QUAD_XOR1>(v));
+    v = max(v, dpp_i<DPP_QUAD_XOR2>(v));
+    v = max(v, dpp_i<DPP_ROW_HALF_MIRROR>(v));
+    v = max(v, dpp_i<DPP_ROW_MIRROR>(v));
+    return __builtin_amdgcn_readfirstlane(v);
+}
+// Maximum / sum over the four lanes l, l + 16, l + 32, l + 48: swapped with itself, a register's halves (rows of sixteen) end up as
+// both operands of one vector instruction. Sums are taken as ((r0 + r1) + (r2 + r3)), the order of an exchange across 16, then 32.
+__device__ __forceinline__ float groups4_max(float v) {
+    auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+    x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+}
+__device__ __forceinline__ float groups4_sum(float v) {
+    auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+    x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
 
 using u32x2 = __attribute__((ext_vector_type(2))) unsigned int;
 // f(integral_constant<int, I>) for I in [I0, E): a loop whose index is a constant expression in the body (immediate

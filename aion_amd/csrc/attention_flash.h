@@ -29,6 +29,12 @@ constexpr int SPLIT_NW = 8;
 // must not carry the ring's extra live values (both kernels sit at their register limit).
 // DVS (split mode): DVS workgroups share a row tile and key segment, each computing all of its scores and a DVS-th of the value
 // columns (the slice_dv-th); an output element is the same sum in the same order whatever DVS is.
+// What bounds it: for one token over a short cache the chain index operands -> K, V -> scores -> softmax -> product -> merge, each link
+// a latency; over a long one HBM, with the wavefronts' own chains under it. The chain is kept short: one memory round trip for the
+// index operands and the queries, reductions by DPP and lane swaps instead of LDS permutes, hardware exp2 (the arguments are <= 0 and
+// results under 2^-126 vanish in a sum that holds a 1), V in flight under the scores. One token, one KV head of size 256, 144 keys:
+// 8.0 -> 6.75 us; 1531 keys, 8 KV heads of size 128: 7.6 -> 6.0 us (+ 3.6 for the segments' merge); eight sequences over 16384 keys,
+// one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
 template <int KV, int D, bool SPLIT, bool HILO, bool RING, int DVS = 1, class Hooks>
 __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int block_x, const int block_y, Hooks &hooks,
                                                 const int slice_dv = 0) {
@@ -64,8 +70,11 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     const int *len_p = a.kv_lengths ? a.kv_lengths + b : (const int *)a.q;
     const int *pos_p = a.positions ? a.positions + ((size_t)b * a.L + li) : (const int *)a.q;
     const int len_ld = len_p[lane_zero], pos_ld = *pos_p;
-    const int kv_end_raw = a.kv_lengths ? len_ld : a.T;
-    const int pos_raw = (row_ok && a.positions) ? pos_ld : li;
+    // (chosen by masks the compiler cannot see through: a select it would turn back into a branch around the load)
+    int len_mask = a.kv_lengths ? -1 : 0, pos_mask = a.positions ? -1 : 0;
+    asm("" : "+v"(len_mask), "+v"(pos_mask));
+    const int kv_end_raw = (len_ld & len_mask) | (a.T & ~len_mask);
+    const int pos_raw = (pos_ld & pos_mask) | (li & ~pos_mask);
 
     const size_t qbase = (((size_t)b * a.L + li) * a.Hq + hq) * D;
     const bool q_f32_vec = a.q_dtype == AIONHIP_F32 && (((uintptr_t)a.q) & 15) == 0;
@@ -104,13 +113,13 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     }
 
     int kv_end = clip_kv_end(ring, a.T, kv_end_raw);
-    int lo = 0, hi = 0;
-    if (row_ok) {
-        window_keys(a.win_left, a.win_right, a.win_chunk, max(pos_raw, 0), kv_end, lo, hi);
-        clip_to_ring(ring, kv_end, lo, hi);
-    }
-    const int uni_lo = wave_min_i(hi > lo ? lo : INT_MAX);
-    const int uni_hi = wave_max_i(hi > lo ? hi : 0);
+    int lo, hi;
+    window_keys(a.win_left, a.win_right, a.win_chunk, max(pos_raw, 0), kv_end, lo, hi);
+    clip_to_ring(ring, kv_end, lo, hi);
+    lo = row_ok ? lo : 0;                                        // (a padding row's position is row 0's)
+    hi = row_ok ? hi : 0;
+    const int uni_lo = rows16_min_i(hi > lo ? lo : INT_MAX);
+    const int uni_hi = rows16_max_i(hi > lo ? hi : 0);
 
     // ---- Q^T operand: 8 consecutive d of row n per k-step, converted to the K/V element type
 #pragma unroll
@@ -186,45 +195,36 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     // anything, so the value must only be finite).
     constexpr int NVI = TILE_KEYS * DV * 2 / 1024;
     constexpr int KEYS_PER_VI = 1024 / (DV * 2);
-    // Addresses: while one batch entry's cache is under 2 GiB (a uniform test) a row is reached by a 32-bit byte
-    // offset from a uniform base - one 24-bit multiply-add per load instead of 64-bit arithmetic, which counts
-    // when a lone workgroup issues a whole short cache's loads.
+    // A row is reached by one 32 x 32 + 64-bit multiply-add; no second form for small caches, whose branch would blur the
+    // compiler's count of the loads in flight (see the tile loop).
     const unsigned row_bytes = (unsigned)(kv_row * 2);
-    const bool near = (size_t)a.T * kv_row * 2 < ((size_t)1 << 31) && a.T < (1 << 24) && row_bytes < (1u << 24);
     const unsigned char *kb8 = (const unsigned char *)(kp + kv_base), *vb8 = (const unsigned char *)(vp + kv_base + dv0);
     const int k_last = RING ? max(uni_hi - 1, 0) : a.T - 1;        // the last key a K load may name
     u32x4 kf[2][KK];
-    auto load_k_as = [&](int t, auto near_c) __attribute__((always_inline)) {
-        constexpr bool near = decltype(near_c)::value;
+    auto load_k = [&](int t) __attribute__((always_inline)) {
         const int key0 = t * TILE_KEYS;
         const TileMap tm(ring, key0);
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
             const int kabs = tm.row(min(key0 + h * 16 + n, k_last));
-            if (near) {
-                const unsigned char *krow = kb8 + (__umul24((unsigned)kabs, row_bytes) + (unsigned)g * 16u);
+            const unsigned char *krow = kb8 + (size_t)(unsigned)kabs * row_bytes + (unsigned)g * 16u;
 #pragma unroll
-                for (int kk = 0; kk < KK; ++kk) kf[h][kk] = *(const u32x4 *)(krow + kk * 64);
-            } else {
-                const unsigned short *krow = kp + kv_base + (size_t)kabs * kv_row + g * 8;
-#pragma unroll
-                for (int kk = 0; kk < KK; ++kk) kf[h][kk] = *(const u32x4 *)(krow + kk * 32);
-            }
+            for (int kk = 0; kk < KK; ++kk) kf[h][kk] = *(const u32x4 *)(krow + kk * 64);
         }
     };
     const int v_key_in = (lane * 16) / (DV * 2);                     // key of this lane within one V load
     const int v_slot = ((lane * 16) % (DV * 2)) / 16;                // its 16-byte slot within the key row
     const int v_hi_key = max(uni_hi - 1, 0);
     (void)NVI; (void)KEYS_PER_VI; (void)vb8; (void)v_key_in; (void)v_slot; (void)v_hi_key;   // (used by the V loads, which exist in the device pass only)
-    auto load_k = [&](int t) __attribute__((always_inline)) {
-        if (near) load_k_as(t, std::true_type{});
-        else load_k_as(t, std::false_type{});
-    };
-    auto load_v_as = [&](int t, auto near_c) __attribute__((always_inline)) {
+    auto load_v = [&](int t) __attribute__((always_inline)) {
 #if defined(__HIP_DEVICE_COMPILE__)   // the builtin exists in the device pass only
-        constexpr bool near = decltype(near_c)::value;
         const int key0 = t * TILE_KEYS;
         const TileMap tm(ring, key0);
+        // As buffer loads: a global LDS-writing load counts as an LDS access too, and with one in flight the compiler waits for every
+        // load before it uses any - the scores for this tile's V. Keys past the clamps fall back into the tile (it holds a visible key),
+        // so an offset from the tile's first row stays below 32 rows: < 2^31 at the largest row. A ring's rows may lie before it.
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t v_rsrc =
+            __builtin_amdgcn_make_buffer_rsrc((void *)(vb8 + (size_t)(unsigned)key0 * row_bytes), 0, 0xFFFFFFFFu, 0x00027000);
 #pragma unroll
         for (int i = 0; i < NVI; ++i) {
             const int key = i * KEYS_PER_VI + v_key_in;
@@ -232,24 +232,22 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             const int grp = KEYS_PER_VI <= 4 ? ((i * KEYS_PER_VI) >> 2) & 3 : (key >> 2) & 3;
             const int chunk = v_slot ^ (2 * grp) ^ (DV >= 128 ? 8 * (key & 1) : 0);
             const int kabs = tm.row(min(max(key0 + key, uni_lo), v_hi_key));
-            if (near)
-                __builtin_amdgcn_global_load_lds(vb8 + (__umul24((unsigned)kabs, row_bytes) + (unsigned)chunk * 16u), (lds_void *)(vs + i * 1024), 16, 0, 0);
+            if constexpr (RING)
+                __builtin_amdgcn_global_load_lds(vb8 + (size_t)(unsigned)kabs * row_bytes + (unsigned)chunk * 16u, (lds_void *)(vs + i * 1024), 16, 0, 0);
             else
-                __builtin_amdgcn_global_load_lds(vp + kv_base + dv0 + (size_t)kabs * kv_row + chunk * 8, (lds_void *)(vs + i * 1024), 16, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(v_rsrc, (lds_void *)(vs + i * 1024), 16, (int)((unsigned)(kabs - key0) * row_bytes + (unsigned)chunk * 16u), 0, 0, 0);
         }
 #endif
-    };
-    auto load_v = [&](int t) __attribute__((always_inline)) {
-        if (near) load_v_as(t, std::true_type{});
-        else load_v_as(t, std::false_type{});
     };
     // V^T operand addresses (second product): lane = 16*g + 4*r + q reads key 4g+r (and 16+4g+r), dv 16*mt + 4q .. +3
     const int tr_r = (lane >> 2) & 3, tr_q = lane & 3;
     const unsigned v_rowaddr = (unsigned)(size_t)(lds_void *)vs + (unsigned)((4 * g + tr_r) * Cfg::ROW_BYTES + (tr_q & 1) * 8);
     const unsigned v_slot_l = (unsigned)(((tr_q >> 1) ^ (2 * g) ^ (DV >= 128 ? 8 * (tr_r & 1) : 0)) << 4);
+    // The queries go through LDS between the requests for K and those for V: they arrived with the index operands, and behind the
+    // LDS-writing loads the compiler would wait for V before it reads them back. Late queries arrive behind both.
     if (t_begin < t_end) {
         load_k(t_begin);
-        load_v(t_begin);
+        if (Hooks::Q_LATE) load_v(t_begin);
     }
     if (q_shared) {
         unsigned char *qsm = lds + Cfg::Q_OFF;
@@ -261,7 +259,8 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         if (qs_row < 16)
             *(u32x4 *)(qsm + qs_row * Cfg::Q_ROW + qs_col * 2) =
                 u32x4{pack2<KV>(qs0.x, qs0.y), pack2<KV>(qs0.z, qs0.w), pack2<KV>(qs1.x, qs1.y), pack2<KV>(qs1.z, qs1.w)};
-        __syncthreads();
+        if (Hooks::Q_LATE) __syncthreads();
+        else asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // (no wait for the K loads in flight)
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) qf[kk] = *(const u32x4 *)(qsm + n * Cfg::Q_ROW + kk * 64 + g * 16);
     }
@@ -278,66 +277,66 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
                 }
         }
     }
-    for (int t = t_begin; t < t_end; t += t_step) {
+    // MORE: another tile of this wavefront follows. Two copies of the body rather than a test in one: every path then requests K
+    // and V in the same order, and the compiler's count of the loads in flight behind K (which lets V of the same tile arrive under
+    // the scores and the softmax) holds; with the test in the body it waited for everything at every tile.
+    auto tile = [&](int t, auto more_c) __attribute__((always_inline)) {
+        constexpr bool more = decltype(more_c)::value;
         const int key0 = t * TILE_KEYS;
-        const bool more = t + t_step < t_end;      // wavefront-uniform
         // -- S^T = K . Q^T for two 16-key halves
-        f32x4 s[2];
+        f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            f32x4 c = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int kk = 0; kk < KK; ++kk)
 #pragma unroll
-            for (int kk = 0; kk < KK; ++kk) {
-                c = mfma16<KV>(kf[h][kk], qf[kk], c);
-                if (HILO) c = mfma16<KV>(kf[h][kk], qf_lo[kk], c);
+            for (int h = 0; h < 2; ++h) {
+                s[h] = mfma16<KV>(kf[h][kk], qf[kk], s[h]);
+                if (HILO) s[h] = mfma16<KV>(kf[h][kk], qf_lo[kk], s[h]);
             }
-            s[h] = c;
+        if (more) {
+            load_k(t + t_step);
+            asm volatile("" ::: "memory");         // requested here, ahead of the counted wait for V below
         }
-        if (more) load_k(t + t_step);
         // -- scale, soft cap, interval mask; lane holds keys key0 + h*16 + g*4 + i of row n
         float p[8];
         float mx = -INFINITY;
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int j = 0; j < 8; ++j) p[j] = s[j >> 2][j & 3] * a.scale;
+        if (a.soft_cap > 0.f) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = key0 + h * 16 + g * 4 + i;
-                float x = s[h][i] * a.scale;
-                if (a.soft_cap > 0.f) x = a.soft_cap * tanhf(x / a.soft_cap);
-                const bool ok = key >= lo && key < hi;
-                x = ok ? x : -INFINITY;
-                p[h * 4 + i] = x;
-                mx = fmaxf(mx, x);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+            for (int j = 0; j < 8; ++j) p[j] = a.soft_cap * tanhf(p[j] / a.soft_cap);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const int key = key0 + (j >> 2) * 16 + g * 4 + (j & 3);
+            p[j] = key >= lo && key < hi ? p[j] : -INFINITY;
+            mx = fmaxf(mx, p[j]);
+        }
+        mx = groups4_max(mx);
         const float m_new = fmaxf(m_run, mx);
         float alpha = 1.f, rowsum = 0.f;
         if (m_new > -INFINITY) {
-            alpha = m_run > -INFINITY ? exp2f((m_run - m_new) * LOG2E) : 1.f;
+            alpha = m_run > -INFINITY ? __builtin_amdgcn_exp2f((m_run - m_new) * LOG2E) : 1.f;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                p[j] = p[j] > -INFINITY ? exp2f((p[j] - m_new) * LOG2E) : 0.f;
+                p[j] = p[j] > -INFINITY ? __builtin_amdgcn_exp2f((p[j] - m_new) * LOG2E) : 0.f;
                 rowsum += p[j];
             }
         } else {
 #pragma unroll
             for (int j = 0; j < 8; ++j) p[j] = 0.f;
         }
-        rowsum += __shfl_xor(rowsum, 16, 64);
-        rowsum += __shfl_xor(rowsum, 32, 64);
+        rowsum = groups4_sum(rowsum);
         l_run = l_run * alpha + rowsum;
         m_run = m_new;
-        unsigned short ph[8], pl[8];
+        const u32x4 pf = u32x4{pack2<KV>(p[0], p[1]), pack2<KV>(p[2], p[3]), pack2<KV>(p[4], p[5]), pack2<KV>(p[6], p[7])};
+        u32x4 pf_lo = u32x4{0u, 0u, 0u, 0u};
+        if (HILO) {
+            const unsigned ph[4] = {pf.x, pf.y, pf.z, pf.w};
+            float lo8[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            ph[j] = to_half_bits<KV>(p[j]);
-            pl[j] = HILO ? to_half_bits<KV>(p[j] - from_half_bits<KV>(ph[j])) : (unsigned short)0;
+            for (int j = 0; j < 8; ++j) lo8[j] = p[j] - from_half_bits<KV>((unsigned short)(ph[j >> 1] >> (16 * (j & 1))));
+            pf_lo = u32x4{pack2<KV>(lo8[0], lo8[1]), pack2<KV>(lo8[2], lo8[3]), pack2<KV>(lo8[4], lo8[5]), pack2<KV>(lo8[6], lo8[7])};
         }
-        const u32x4 pf = u32x4{(unsigned)ph[0] | ((unsigned)ph[1] << 16), (unsigned)ph[2] | ((unsigned)ph[3] << 16),
-                               (unsigned)ph[4] | ((unsigned)ph[5] << 16), (unsigned)ph[6] | ((unsigned)ph[7] << 16)};
-        const u32x4 pf_lo = u32x4{(unsigned)pl[0] | ((unsigned)pl[1] << 16), (unsigned)pl[2] | ((unsigned)pl[3] << 16),
-                                  (unsigned)pl[4] | ((unsigned)pl[5] << 16), (unsigned)pl[6] | ((unsigned)pl[7] << 16)};
 
         // -- this tile's V has landed in the wavefront's LDS tile once only the younger K loads are
         //    outstanding (loads complete in order); the tile is written and read by this wavefront only
@@ -359,7 +358,7 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         // 4r+q supplies the address of 4 consecutive dv of key r, lane i receives keys 0..3 of dv i): keys 4g+r and
         // 16+4g+r of row-major V, dv 16*mt + 4q .. +3, which is the slot order above. Written as assembly and waited for
         // by count: as a builtin the compiler would wait for every load in flight - the next tile's K - before the first.
-        constexpr int VA = 2;                                        // operands requested ahead
+        constexpr int VA = HILO ? 2 : MT < 4 ? MT : 4;               // operands requested ahead
         u32x4 vop[VA];
         auto v_operand = [&](auto mt_c) __attribute__((always_inline)) {
             constexpr int mt = decltype(mt_c)::value;
@@ -381,7 +380,16 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
             acc[mt] = c;
             if constexpr (mt + VA < MT) vop[mt % VA] = v_operand(std::integral_constant<int, mt + VA>{});
         });
-        if (more) load_v(t + t_step);      // the operand reads above are complete: each was waited for before its MFMA
+        if (more) {
+            asm volatile("" ::: "memory");         // the operand reads above are complete: each was waited for before its MFMA
+            load_v(t + t_step);
+        }
+    };
+    if (t_begin < t_end) {
+        if (!Hooks::Q_LATE) load_v(t_begin);
+        int t = t_begin;
+        for (; t + t_step < t_end; t += t_step) tile(t, std::true_type{});
+        tile(t, std::false_type{});
     }
 
     if (!SPLIT) {
@@ -425,7 +433,7 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         float l_all = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float f = mw[w] > -INFINITY ? exp2f((mw[w] - m_all) * LOG2E) : 0.f;
+            const float f = mw[w] > -INFINITY ? __builtin_amdgcn_exp2f((mw[w] - m_all) * LOG2E) : 0.f;
             l_all += mg[w * WSTRIDE + 16 * RS + 16 + row] * f;
             o += *(const f32x4 *)(mg + w * WSTRIDE + row * RS + col) * f;
         }

@@ -173,6 +173,27 @@ def test_decode_value_columns_divided_or_not(gpu, orc, T, D, precise):
         gpu.set_attention_precise(False)
 
 
+@pytest.mark.parametrize("kind,tol", [("f16", 2e-3), ("bf16", 1e-2)])
+@pytest.mark.parametrize("D,Hkv", [(64, 1), (128, 2), (256, 1)])
+@pytest.mark.parametrize("T,left", [(1400, 333), (1400, 5000), (333, 31), (40, 7)])   # window starts inside a key tile, or no limit
+def test_decode_reads_no_row_outside_the_window(gpu, orc, T, left, D, Hkv, kind, tol):
+    """Rows in front of the window and behind the cache length hold NaN patterns; key tiles straddle both ends and are read in
+    clamped rows. Sequences of three lengths, one of them inside the first tile."""
+    B, Hq, cap = 3, 8, T + 90
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T + left + D, B, 1, cap, Hq, Hkv, D, kind)
+    lens = np.array([T, T - 17, 5], np.int32)
+    nan = np.float16(np.nan) if kind == "f16" else np.uint16(0x7FC1)
+    for b in range(B):
+        first = max(0, lens[b] - 1 - left)
+        for x, f in ((k, kf), (v, vf)):
+            x[b, :first], x[b, lens[b]:] = nan, nan
+            f[b, :first], f[b, lens[b]:] = 0, 0
+    pos = (lens - 1).reshape(B, 1)
+    got = run_attention(gpu, q, k, v, 1 / math.sqrt(D), qd, kd, positions=pos, kv_lengths=lens, window=(left, 0, 0))
+    assert gpu.last_kernel() == "attn_flash_split"
+    attn_err(got, orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D), positions=pos, kv_lengths=lens, window=(left, 0, 0)), tol)
+
+
 @pytest.mark.parametrize("window", [(100, 0, 0), (16, 0, 64), (be.UNBOUNDED, be.UNBOUNDED, 0), (5, 3, 0)])
 def test_windows_prefill_and_decode(gpu, orc, window):
     B, L, Hq, Hkv, D = 1, 200, 4, 1, 64
