@@ -414,20 +414,23 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 
 }  // namespace
 
-// 5..8 rows against a wide, short weight (a logits head at batch 8): the 16-row MFMA tile of the LDS-staged int8
-// GEMM beats the lane-per-row kernel, whose LDS traffic grows with the rows (262144 x 2048, 8 rows: 77 against
-// 104 us for q4, 110 against 142 us for q8). Long K or few columns leave that kernel's grid too sparse.
-// q8 (twice the weight bytes per row: the lane-per-row kernel leaves its latency floor later) moves there from two
-// rows on once the weight has some 12k columns - 14336 x 4096: 22 -> 20 us at 4 rows, 26.6 -> 20.3 at 8;
-// 16384 x 2048: 15 -> 13.7 at 2-4 rows - but not against the largest weights, which the lane-per-row kernel
-// streams faster at 2-4 rows (65536 x 4096: 58-64 against 70 us).
+// Rows against one weight that the exact GEMM's kernel (32 x 32 tiles) multiplies faster than the lane-per-row kernel, whose work
+// and LDS traffic grow with the rows; weights of few columns leave the GEMM too few tiles. Both kernels timed over 63 shapes
+// (K = 512 ... 14336, N = 512 ... 131072) at 2, 3, 4, 5 and 8 rows, both block formats, preparation included:
+//   5..8 rows:  from max(1024, K) columns on. q4 8192 x 512 10.6 against 7.1 us, 4096 x 2048 9.1 against 7.9, 8192 x 4096 13.2 against
+//               9.6; q8 8192 x 4096 16.4 against 11.7. Narrower the GEMM loses: q4 2048 x 4096 9.2 against 9.7, q8 9.8 against 11.0.
+//   2..4 rows:  q8 from 8192 columns on (8192 x 8192 19.7 against 17.3, 16384 x 14336 53.7 against 39.8), up to 2^28 weights: beyond,
+//               the lane-per-row kernel streams faster (32768 x 14336 80 against 96). q4 with half the bytes per weight keeps that
+//               lead from 16384 columns on (32768 x 4096 18.4 against 21.5) and, at 2 rows, up to K = 4096 (8192 x 4096 10.0 against
+//               9.9; 8192 x 14336 21.3 against 20.4); between, 3..4 rows: 8192 x 4096 10.7 against 9.7, 16384 x 14336 35.7 against 32.4.
+// Five rows and more over a K past 4096 take the GEMM before this rule is asked.
 bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m) {
-    if (count != 1 || gemv_mfma_applies(ws, count, m)) return false;
+    if (count != 1 || m < 2 || gemv_mfma_applies(ws, count, m)) return false;
     const size_t n = ws[0]->n, k = ws[0]->k;
-    const bool q8w = ws[0]->dtype == AIONHIP_Q8_0;
-    const bool tile16 = (m >= 5 && n >= 16384) || (q8w && m >= 2 && n >= 12288 && n * k <= ((size_t)1 << 27)) ||
-                        (q8w && m >= 5 && n >= 8192 && k <= 2048);
-    return tile16 && k >= 256 && k <= 4096;
+    if (k < 256 || k > GEMM_I8_MAX_K) return false;
+    if (m >= 5) return k <= 4096 && n >= (k > 1024 ? k : 1024);
+    if (n < 8192 || n * k > ((size_t)1 << 28)) return false;
+    return ws[0]->dtype == AIONHIP_Q8_0 || (n <= 16384 && (m >= 3 || k > 4096));
 }
 
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,

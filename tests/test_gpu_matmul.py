@@ -357,6 +357,23 @@ def test_decode_gemv_two_to_eight_rows(gpu, orc, dtype, layout, m, n, k):
     w.free()
 
 
+# both sides of the lines between the lane-per-row kernel and the exact GEMM's: columns against K at 5..8 rows, 8192 and 16384
+# columns at 2..4 rows; widths that end inside a tile
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(5, 1023, 512), (8, 1024, 512), (8, 1040, 224), (6, 2049, 2048), (7, 2047, 2048), (5, 4100, 4096), (8, 3999, 4000),
+                                   (2, 8191, 512), (2, 8195, 512), (4, 8192, 1056), (3, 16385, 1024), (2, 8200, 4128), (4, 9001, 8192)])
+def test_few_rows_on_either_side_of_the_gemm_line(gpu, orc, dtype, layout, m, n, k):
+    say("few rows", dtype, layout, m, n, k)
+    blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 17 + n + k, std=0.05)
+    a = np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float32)
+    on_gemm = k >= 256 and (n >= max(1024, k) if m >= 5 else n >= 8192 and (dtype == be.Q8_0 or n <= 16384 and (m >= 3 or k > 4096)))
+    got = gpu.matmul(w, a)
+    assert ("gemm_i8" in gpu.last_launch()["kernel"]) == on_gemm
+    want = oracle_matmul(orc, dtype, layout, a, blocks, n)
+    assert norm_err(got, want) < TOL and rms_err(got, want) < RMS_TOL
+    w.free()
+
+
 def test_linearity_in_alpha_and_row_independence(gpu, orc):
     # size-independent properties: rows of A never interact (the one-row and the several-row kernels give a row
     # the same int8 codes and block dots; only the order of the f32 additions over lanes may differ); alpha
