@@ -415,22 +415,27 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 }  // namespace
 
 // Rows against one weight that the exact GEMM's kernel (32 x 32 tiles) multiplies faster than the lane-per-row kernel, whose work
-// and LDS traffic grow with the rows; weights of few columns leave the GEMM too few tiles. Both kernels timed over 63 shapes
-// (K = 512 ... 14336, N = 512 ... 131072) at 2, 3, 4, 5 and 8 rows, both block formats, preparation included:
+// and LDS traffic grow with the rows; weights of few columns leave the GEMM too few tiles, and 8200 ... 12000 columns leave its second
+// round of workgroups nearly empty. Both kernels timed over 230 shapes (K = 512 ... 14336, N = 512 ... 131072) at 2 ... 8 rows, both
+// block formats, preparation included:
 //   5..8 rows:  from max(1024, K) columns on. q4 8192 x 512 10.6 against 7.1 us, 4096 x 2048 9.1 against 7.9, 8192 x 4096 13.2 against
 //               9.6; q8 8192 x 4096 16.4 against 11.7. Narrower the GEMM loses: q4 2048 x 4096 9.2 against 9.7, q8 9.8 against 11.0.
-//   2..4 rows:  q8 from 8192 columns on (8192 x 8192 19.7 against 17.3, 16384 x 14336 53.7 against 39.8), up to 2^28 weights: beyond,
-//               the lane-per-row kernel streams faster (32768 x 14336 80 against 96). q4 with half the bytes per weight keeps that
-//               lead from 16384 columns on (32768 x 4096 18.4 against 21.5) and, at 2 rows, up to K = 4096 (8192 x 4096 10.0 against
-//               9.9; 8192 x 14336 21.3 against 20.4); between, 3..4 rows: 8192 x 4096 10.7 against 9.7, 16384 x 14336 35.7 against 32.4.
+//   2..4 rows:  one round of tiles (8192 columns on 256 CUs: q8 x 8192 19.7 against 17.3, q4 14.9 against 13.9) or one and a half and
+//               more (q8 16384 x 14336 53.7 against 39.8, q4 35.7 against 32.4); q8 in between too (9664 x 4096 14.8 against 13.7)
+//               except over K = 5120 ... 8192 (9664 x 7392 21.0 against 22.2; q4 17.7 against 19.9). Beyond 2^28 weights the lane-per-row
+//               kernel streams faster (q8 32768 x 14336 80 against 96), for q4, with half the bytes a weight, from three rounds on
+//               (32768 x 4096 18.4 against 21.5). Two rows of q4: up to two rounds and K from 4096 on (12288 x 4096 14.2 against 13.3,
+//               x 2048 9.1 against 9.5).
 // Five rows and more over a K past 4096 take the GEMM before this rule is asked.
 bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m) {
     if (count != 1 || m < 2 || gemv_mfma_applies(ws, count, m)) return false;
     const size_t n = ws[0]->n, k = ws[0]->k;
+    const bool q8 = ws[0]->dtype == AIONHIP_Q8_0;
     if (k < 256 || k > GEMM_I8_MAX_K) return false;
     if (m >= 5) return k <= 4096 && n >= (k > 1024 ? k : 1024);
-    if (n < 8192 || n * k > ((size_t)1 << 28)) return false;
-    return ws[0]->dtype == AIONHIP_Q8_0 || (n <= 16384 && (m >= 3 || k > 4096));
+    if (n <= 7680 || n * k > ((size_t)1 << 28)) return false;
+    if (n > 8192 && n < 12288 && !(q8 && (k <= 5120 || k > 8192))) return false;
+    return q8 || (m >= 3 ? n <= 24576 : n <= 16384 && k >= 4096);
 }
 
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,

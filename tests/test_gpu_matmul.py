@@ -357,16 +357,22 @@ def test_decode_gemv_two_to_eight_rows(gpu, orc, dtype, layout, m, n, k):
     w.free()
 
 
-# both sides of the lines between the lane-per-row kernel and the exact GEMM's: columns against K at 5..8 rows, 8192 and 16384
-# columns at 2..4 rows; widths that end inside a tile
+# both sides of the lines between the lane-per-row kernel and the exact GEMM's: columns against K at 5..8 rows, rounds
+# of the GEMM's tiles on 256 CUs at 2..4 rows; widths that end inside a tile
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("m,n,k", [(5, 1023, 512), (8, 1024, 512), (8, 1040, 224), (6, 2049, 2048), (7, 2047, 2048), (5, 4100, 4096), (8, 3999, 4000),
-                                   (2, 8191, 512), (2, 8195, 512), (4, 8192, 1056), (3, 16385, 1024), (2, 8200, 4128), (4, 9001, 8192)])
+                                   (2, 8191, 512), (2, 8195, 512), (4, 7680, 1056), (4, 8192, 1056), (3, 16385, 1024), (2, 8200, 4128), (4, 9001, 8192),
+                                   (2, 12287, 4096), (2, 12290, 4096), (3, 24577, 512), (2, 16385, 4096)])
 def test_few_rows_on_either_side_of_the_gemm_line(gpu, orc, dtype, layout, m, n, k):
     say("few rows", dtype, layout, m, n, k)
     blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 17 + n + k, std=0.05)
     a = np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float32)
-    on_gemm = k >= 256 and (n >= max(1024, k) if m >= 5 else n >= 8192 and (dtype == be.Q8_0 or n <= 16384 and (m >= 3 or k > 4096)))
+    q8 = dtype == be.Q8_0
+    if m >= 5:
+        on_gemm = n >= max(1024, k)
+    else:
+        on_gemm = (7680 < n <= 8192 or n >= 12288 or (q8 and n > 8192 and not 5120 < k <= 8192)) and (q8 or (n <= 24576 if m >= 3 else n <= 16384 and k >= 4096))
+    on_gemm = on_gemm and k >= 256
     got = gpu.matmul(w, a)
     assert ("gemm_i8" in gpu.last_launch()["kernel"]) == on_gemm
     want = oracle_matmul(orc, dtype, layout, a, blocks, n)
