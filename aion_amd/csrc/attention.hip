@@ -200,9 +200,11 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     // over many CUs, which outweighs re-reading K/V per row tile from L2.
     const int cus0 = ctx->cu_count > 0 ? ctx->cu_count : 256;
     // (the smaller the head, the longer the 16-row kernel stays ahead: per key it re-reads less. Crossovers measured over
-    // five head layouts x L = 128 .. 2048: about 80 / 40 / 32 workgroups of the 128-row kernel at head size 64 / 128 / 256)
+    // five head layouts x L = 32 .. 2048, one and two sequences: about 112 / 40 / 32 workgroups of the 128-row kernel at head size 64 /
+    // 128 / 256. 16 q / 4 kv heads x 64: 768 queries, 96 workgroups, 14.0 against 19.2 us; 1024, 128 workgroups, 19.3 against 19.3;
+    // two sequences of 768, 192 workgroups, 23.5 against 19.5. 32 / 8 x 128: 128 queries 6.1 against 8.1, 192 10.6 against 9.2)
     const long pf_wgs = (long)units * ((a.rows_total + PF_ROWS - 1) / PF_ROWS);
-    const long pf_min = D <= 64 ? (long)cus0 * 5 / (2 * PF_FLASH_BELOW) : D <= 128 ? (long)cus0 * 5 / (4 * PF_FLASH_BELOW) : (long)cus0 / PF_FLASH_BELOW;
+    const long pf_min = D <= 64 ? (long)cus0 * 7 / (2 * PF_FLASH_BELOW) : D <= 128 ? (long)cus0 * 5 / (4 * PF_FLASH_BELOW) : (long)cus0 / PF_FLASH_BELOW;
     bool split = a.rows_total <= 64 || (!HILO && pf_wgs <= pf_min) ||
                  (!HILO && !prefill_takes(a, D));      // e.g. a softmax scale that is not positive: the 16-row kernel takes any
     // A chunk of queries over a cache at least four times its length (chunked prompts, speculative batches): the crossover
