@@ -185,6 +185,16 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
         }
     };
+    // Blocks past the end of K in the last group: activation scale 0 as well as weight scale 0, where a real block's infinite scale
+    // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first block's.
+    auto clear_tail = [&](int g, int buf) {
+        if (g * 4 + 4 <= KB) return;
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 1; j < 4; ++j)
+                if (g * 4 + j >= KB && lane < 32) sa_lds[(buf * MT + i) * 128 + j * 32 + lane] = 0.f;
+    };
     int g = g_lo + ks;
     if (g < g_hi) {
         load_w(g, 0);
@@ -197,8 +207,10 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         asm volatile("" ::: "memory");
         read_b(0, 0);
 #pragma unroll
-        for (int i = 0; i < MT; ++i) read_sa(i, 0, 0);
+        for (int i = 0; i < MT - 1; ++i) read_sa(i, 0, 0);
     }
+#pragma unroll
+    for (int e = 0; e < 16; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
     int buf = 0;
     i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
     float sw_due = 0.f;
@@ -231,6 +243,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                 __builtin_amdgcn_sched_barrier(0);
                 __builtin_amdgcn_s_waitcnt(LGKM0);
                 __builtin_amdgcn_sched_barrier(0);
+                clear_tail(g, buf);
                 load_w(gn, buf ^ 1);
                 load_scales(gn, buf ^ 1);
             }

@@ -292,3 +292,27 @@ def test_bf16_mode_runs_the_bf16_kernel_only_where_it_pays(gpu, orc):
     finally:
         gpu.set_gemm_mode(be.GEMM_EXACT_I8)
     w.free()
+
+
+# A row with an infinite element has one block of scale inf, whose codes are 0 but for -127 at that element (the clamp of 0 * inf): each sum
+# is inf against the sign of the weight there, NaN where that weight is 0. Only what the block multiplies may leave the finite range:
+# the rescale that starts a wavefront's pipeline, and the blocks a last group has past the end of K, must not meet it with a zero. The
+# block is the first, the last and one in the middle; K ends inside a group of four blocks and at its end.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(40, 100, 160), (33, 96, 2080), (9, 40, 8224), (8, 1056, 992), (150, 4128, 2048)])
+def test_exact_gemm_infinite_activations(gpu, orc, dtype, layout, m, n, k):
+    say("inf", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    blocks, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    a = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    a[0, 3], a[1, k - 5], a[m - 2, k // 64 * 32 + 7] = np.inf, np.inf, -np.inf
+    got = gpu.matmul(w, a)
+    assert "gemm_i8" in gpu.last_launch()["kernel"]
+    for r, col in ((0, 3), (1, k - 5), (m - 2, k // 64 * 32 + 7)):
+        one = np.zeros((1, k), np.float32)
+        one[0, col] = 1
+        sign = np.sign(gpu.matmul(w, one)[0])
+        assert np.array_equal(got[r], np.where(sign == 0, np.nan, np.where(sign > 0, -np.inf, np.inf)), equal_nan=True), r
+    rows = [r for r in range(m) if r not in (0, 1, m - 2)]
+    assert rms_err(got[rows], oracle_i8(orc, dtype, layout, a[rows], blocks, n)) < 3e-5      # (bound: test_exact_gemm_tiles_and_k_divisions)
+    w.free()
