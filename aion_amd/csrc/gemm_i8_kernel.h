@@ -76,221 +76,248 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
     const int KB = K >> 5, G = (KB + 3) >> 2;
     const int n0 = (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
 
-    // this wavefront's operand rows: activation tiles mt0 .., weight rows n0 + 32 ni + r (clamped: a clamped row's results are not
-    // stored). Every operand address is a uniform base that moves with K plus a 32-bit offset a lane keeps for good, so that a
-    // load costs the vector ALU nothing.
-    const uint8_t *ab[MT];
-    const float *asb[MT];
-    unsigned ao[MT], aso[MT];
-    int arows[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-        const int mt = min((m0 >> 5) + i, (M - 1) >> 5);
-        arows[i] = act_tile_rows(M, mt);
-        ab[i] = aq + (size_t)mt * 32 * K;
-        ao[i] = (unsigned)(h * arows[i] + min(r, arows[i] - 1)) * 16;
-        asb[i] = a_scale + (size_t)mt * 32 * KB;
-        aso[i] = (unsigned)min(r, arows[i] - 1) * 4;
-    }
-    const int nb = min(n0, N - 1);
-    const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-    [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch;      // (used in the device pass only)
-    const __half *sb = sc + (size_t)nb * KB;
-    // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
-    constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
-    const int w_row = lane / LPR;
-    unsigned wo[NT][WL];
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int l = 0; l < WL; ++l)
-            wo[i][l] = (unsigned)(min(n0 + i * 32 + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
-    // weight scales: with two tiles a lane half takes one tile's rows each and the halves are exchanged afterwards
-    const unsigned so = (unsigned)(min(n0 + (NT == 2 ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
-
     f32x16 acc[MT][NT];
+    // q4 dots are 16 times the codes' dots. The 1/16 is taken from the sums, where it is exact down to subnormal products of scales; sums past
+    // 2^124 leave the f32 range that way (a row that holds the lowest f32 as a mask), so a wavefront with one that is not finite runs
+    // its share again with the 1/16 in the weight scales. (Codes without the 16 cost eight vector instructions a tile and block.)
+    float code_scale = 1.f, sum_scale = Q8 ? 1.f : 0.0625f;
+    for (;;) {
+        // (the addresses of a second walk are computed again: kept, they would cost the first one registers)
+        int lane_now = lane;
+        asm volatile("" : "+v"(lane_now));
+        const int lane = lane_now, r = lane & 31, h = lane >> 5;
+        // this wavefront's operand rows: activation tiles mt0 .., weight rows n0 + 32 ni + r (clamped: a clamped row's results are not
+        // stored). Every operand address is a uniform base that moves with K plus a 32-bit offset a lane keeps for good, so that a
+        // load costs the vector ALU nothing.
+        const uint8_t *ab[MT];
+        const float *asb[MT];
+        unsigned ao[MT], aso[MT];
+        int arows[MT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int j = 0; j < NT; ++j)
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-
-    // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
-    const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
-    const int g_lo = (int)blockIdx.z * g_per, g_hi = min(G, g_lo + g_per);
-
-    // Registers: the four blocks of a group's activations (reloaded for the next group as each is used up), the next group's weight
-    // scales. LDS, private to the wavefront and written by the loads themselves: two groups of weight codes and activation scales.
-    i32x4 A[4][MT];
-    unsigned long sw_raw = 0, sw_now = 0;      // four f16 scales of a weight row: the next group's, this group's
-    int sw_shift = 0, sw_shift_now = 0;
-#if defined(__HIP_DEVICE_COMPILE__)
-    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wb, 0, 0xFFFFFFFFu, 0x00027000);
-    __amdgpu_buffer_rsrc_t sa_rsrc[MT];
-#pragma unroll
-    for (int i = 0; i < MT; ++i) sa_rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void *)asb[i], 0, 0xFFFFFFFFu, 0x00027000);
-#endif
-    constexpr int LGKM0 = vmcnt_imm(63) & ~(15 << 8);        // every LDS operation has completed
-    constexpr int WBUF = NT * 32 * RB;
-    unsigned char *w_lds = lds + wave * gemm_i8_wave_lds_bytes<Q8, MT, NT>();
-    float *sa_lds = (float *)(w_lds + 2 * WBUF);
-    auto load_a = [&](int set, int kb) {
-        kb = min(kb, KB - 1);
-#pragma unroll
-        for (int i = 0; i < MT; ++i) A[set][i] = *(const i32x4 *)(ab[i] + (size_t)((unsigned)kb * (unsigned)(arows[i] * 32)) + ao[i]);
-    };
-    // Row R of a tile is at R * RB, its 16-byte piece c in slot c ^ (R & 7) (q8) or c ^ ((R >> 1) & 3) (q4): the lanes of a read,
-    // consecutive rows at one piece, then cover 128 bytes of banks. (Blocks past the end of K: another row's or the slack behind the
-    // weight, scale 0.)
-    auto load_w = [&](int g, int buf) {
-#if defined(__HIP_DEVICE_COMPILE__)   // the builtin exists in the device pass only
+        for (int i = 0; i < MT; ++i) {
+            const int mt = min((m0 >> 5) + i, (M - 1) >> 5);
+            arows[i] = act_tile_rows(M, mt);
+            ab[i] = aq + (size_t)mt * 32 * K;
+            ao[i] = (unsigned)(h * arows[i] + min(r, arows[i] - 1)) * 16;
+            asb[i] = a_scale + (size_t)mt * 32 * KB;
+            aso[i] = (unsigned)min(r, arows[i] - 1) * 4;
+        }
+        const int nb = min(n0, N - 1);
+        const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
+        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch;      // (used in the device pass only)
+        const __half *sb = sc + (size_t)nb * KB;
+        // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
+        constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
+        const int w_row = lane / LPR;
+        unsigned wo[NT][WL];
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
             for (int l = 0; l < WL; ++l)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
-#endif
-    };
-    const int r_slot = Q8 ? h ^ (r & 7) : (r >> 1) & 3;
-    using Codes = typename std::conditional<Q8, i32x4, i32x2>::type;    // what a lane's MFMA operand is made of: 16 codes, 16 nibbles
-    Codes Bn[NT];
-    auto read_b = [&](int buf, int j) {
+                wo[i][l] = (unsigned)(min(n0 + i * 32 + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
+        // weight scales: with two tiles a lane half takes one tile's rows each and the halves are exchanged afterwards
+        const unsigned so = (unsigned)(min(n0 + (NT == 2 ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
+
+        // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
+        const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
+        const int g_lo = (int)blockIdx.z * g_per, g_hi = min(G, g_lo + g_per);
+
+        // Registers: the four blocks of a group's activations (reloaded for the next group as each is used up), the next group's weight
+        // scales. LDS, private to the wavefront and written by the loads themselves: two groups of weight codes and activation scales.
+        i32x4 A[4][MT];
+        unsigned long sw_raw = 0, sw_now = 0;      // four f16 scales of a weight row: the next group's, this group's
+        int sw_shift = 0, sw_shift_now = 0;
+#if defined(__HIP_DEVICE_COMPILE__)
+        const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wb, 0, 0xFFFFFFFFu, 0x00027000);
+        __amdgpu_buffer_rsrc_t sa_rsrc[MT];
 #pragma unroll
-        for (int i = 0; i < NT; ++i)
-            Bn[i] = *(const Codes *)(w_lds + buf * WBUF + (i * 32 + r) * RB + (Q8 ? ((2 * j) ^ r_slot) * 16 : (j ^ r_slot) * 16 + h * 8));
-    };
-    struct __attribute__((packed, aligned(2))) U64 { unsigned long v; };
-    auto load_scales = [&](int g, int buf) {
-        const int kb = min(g * 4, KB - 1), base = max(0, min(kb, KB - 4));
-        sw_shift = (kb - base) * 16;
-        sw_raw = ((const U64 *)(sb + base + so))->v;
+        for (int i = 0; i < MT; ++i) sa_rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void *)asb[i], 0, 0xFFFFFFFFu, 0x00027000);
+#endif
+        constexpr int LGKM0 = vmcnt_imm(63) & ~(15 << 8);        // every LDS operation has completed
+        constexpr int WBUF = NT * 32 * RB;
+        unsigned char *w_lds = lds + wave * gemm_i8_wave_lds_bytes<Q8, MT, NT>();
+        float *sa_lds = (float *)(w_lds + 2 * WBUF);
+        auto load_a = [&](int set, int kb) {
+            kb = min(kb, KB - 1);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) A[set][i] = *(const i32x4 *)(ab[i] + (size_t)((unsigned)kb * (unsigned)(arows[i] * 32)) + ao[i]);
+        };
+        // Row R of a tile is at R * RB, its 16-byte piece c in slot c ^ (R & 7) (q8) or c ^ ((R >> 1) & 3) (q4): the lanes of a read,
+        // consecutive rows at one piece, then cover 128 bytes of banks. (Blocks past the end of K: another row's or the slack behind the
+        // weight, scale 0.)
+        auto load_w = [&](int g, int buf) {
+#if defined(__HIP_DEVICE_COMPILE__)   // the builtin exists in the device pass only
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+#pragma unroll
+                for (int l = 0; l < WL; ++l)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
+#endif
+        };
+        const int r_slot = Q8 ? h ^ (r & 7) : (r >> 1) & 3;
+        using Codes = typename std::conditional<Q8, i32x4, i32x2>::type;    // what a lane's MFMA operand is made of: 16 codes, 16 nibbles
+        Codes Bn[NT];
+        auto read_b = [&](int buf, int j) {
+#pragma unroll
+            for (int i = 0; i < NT; ++i)
+                Bn[i] = *(const Codes *)(w_lds + buf * WBUF + (i * 32 + r) * RB + (Q8 ? ((2 * j) ^ r_slot) * 16 : (j ^ r_slot) * 16 + h * 8));
+        };
+        struct __attribute__((packed, aligned(2))) U64 { unsigned long v; };
+        auto load_scales = [&](int g, int buf) {
+            const int kb = min(g * 4, KB - 1), base = max(0, min(kb, KB - 4));
+            sw_shift = (kb - base) * 16;
+            sw_raw = ((const U64 *)(sb + base + so))->v;
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int q = 0; q < 2; ++q)                  // two blocks' scales of 32 rows
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(sa_rsrc[i], (lds_void *)(sa_lds + (buf * MT + i) * 128 + q * 64), 4,
-                                                         aso[i] + (h && g * 4 + 2 * q + 1 < KB ? (unsigned)arows[i] * 4 : 0u),
-                                                         min(g * 4 + 2 * q, KB - 1) * arows[i] * 4, 0, 0);
+                for (int q = 0; q < 2; ++q)                  // two blocks' scales of 32 rows
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(sa_rsrc[i], (lds_void *)(sa_lds + (buf * MT + i) * 128 + q * 64), 4,
+                                                             aso[i] + (h && g * 4 + 2 * q + 1 < KB ? (unsigned)arows[i] * 4 : 0u),
+                                                             min(g * 4 + 2 * q, KB - 1) * arows[i] * 4, 0, 0);
 #endif
-    };
+        };
 
-    // the activation scales a lane multiplies with - 16 rows of each row tile - come from the wavefront's LDS copy of the group
-    float sa[MT][16];
-    auto read_sa = [&](int i, int buf, int j) {
+        // the activation scales a lane multiplies with - 16 rows of each row tile - come from the wavefront's LDS copy of the group
+        float sa[MT][16];
+        auto read_sa = [&](int i, int buf, int j) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const f32x4 v = *(const f32x4 *)(sa_lds + (buf * MT + i) * 128 + j * 32 + 8 * q + 4 * h);
-            sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
-        }
-    };
-    // Blocks past the end of K in the last group: activation scale 0 as well as weight scale 0, where a real block's infinite scale
-    // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first block's.
-    auto clear_tail = [&](int g, int buf) {
-        if (g * 4 + 4 <= KB) return;
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 v = *(const f32x4 *)(sa_lds + (buf * MT + i) * 128 + j * 32 + 8 * q + 4 * h);
+                sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
+            }
+        };
+        // Blocks past the end of K in the last group: activation scale 0 as well as weight scale 0, where a real block's infinite scale
+        // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first block's.
+        auto clear_tail = [&](int g, int buf) {
+            if (g * 4 + 4 <= KB) return;
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 1; j < 4; ++j)
+                    if (g * 4 + j >= KB && lane < 32) sa_lds[(buf * MT + i) * 128 + j * 32 + lane] = 0.f;
+        };
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int j = 1; j < 4; ++j)
-                if (g * 4 + j >= KB && lane < 32) sa_lds[(buf * MT + i) * 128 + j * 32 + lane] = 0.f;
-    };
-    int g = g_lo + ks;
-    if (g < g_hi) {
-        load_w(g, 0);
-        load_scales(g, 0);
+            for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int j = 0; j < 3; ++j) load_a(j, g * 4 + j);
-        sw_now = sw_raw;
-        sw_shift_now = sw_shift;
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-        asm volatile("" ::: "memory");
-        read_b(0, 0);
+                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+        int g = g_lo + ks;
+        if (g < g_hi) {
+            load_w(g, 0);
+            load_scales(g, 0);
 #pragma unroll
-        for (int i = 0; i < MT - 1; ++i) read_sa(i, 0, 0);
-    }
+            for (int j = 0; j < 3; ++j) load_a(j, g * 4 + j);
+            sw_now = sw_raw;
+            sw_shift_now = sw_shift;
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+            asm volatile("" ::: "memory");
+            read_b(0, 0);
 #pragma unroll
-    for (int e = 0; e < 16; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
-    int buf = 0;
-    i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
-    float sw_due = 0.f;
-    for (; g < g_hi; g += KS) {
-        const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
-        float sw[4][NT];
-        {
-            const unsigned long v = sw_now >> sw_shift_now;
-            unsigned lo[2], hi[2];
-            if constexpr (NT == 2) {
-                const auto x = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
-                const auto y = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
-                lo[0] = x[0]; lo[1] = x[1]; hi[0] = y[0]; hi[1] = y[1];
-            } else {
-                lo[0] = (unsigned)v; hi[0] = (unsigned)(v >> 32);
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-#pragma unroll
-                for (int i = 0; i < NT; ++i)
-                    sw[j][i] = g * 4 + j < KB ? __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
+            for (int i = 0; i < MT - 1; ++i) read_sa(i, 0, 0);
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            // The other buffer was last read in the previous group (those reads have returned once lgkmcnt is 0); its loads have three
-            // steps' time, and 3 MT younger ones are in flight when they are waited for. They are buffer loads: global_load_lds counts as a
-            // flat access, after which the compiler waits for every load in flight before the next use of any.
-            if (j == 0) {
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_sched_barrier(0);
-                __builtin_amdgcn_s_waitcnt(LGKM0);
-                __builtin_amdgcn_sched_barrier(0);
-                clear_tail(g, buf);
-                load_w(gn, buf ^ 1);
-                load_scales(gn, buf ^ 1);
-            }
-            load_a((j + 3) & 3, j == 0 ? g * 4 + 3 : gn * 4 + j - 1);
-            __builtin_amdgcn_sched_barrier(0);
-            if (j == 3) {
-                __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * MT));
-                asm volatile("" ::: "memory");
-            }
-            i32x4 B[NT];
-#pragma unroll
-            for (int i = 0; i < NT; ++i) {
-                if constexpr (Q8) {
-                    B[i] = Bn[i];                        // (copied by the loop's unrolling: no instruction)
+        for (int e = 0; e < 16; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
+        int buf = 0;
+        i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
+        float sw_due = 0.f;
+        for (; g < g_hi; g += KS) {
+            const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
+            float sw[4][NT];
+            {
+                const unsigned long v = sw_now >> sw_shift_now;
+                unsigned lo[2], hi[2];
+                if constexpr (NT == 2) {
+                    const auto x = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+                    const auto y = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
+                    lo[0] = x[0]; lo[1] = x[1]; hi[0] = y[0]; hi[1] = y[1];
                 } else {
-                    // 16 * (nibble - 8) as int8: the nibble in the upper half of its byte with the top bit flipped; the sums are divided by
-                    // 16 at the end (in the scales, the division would round where a product of scales is subnormal)
-                    const unsigned w0 = Bn[i].x, w1 = Bn[i].y;
-                    B[i] = i32x4{(int)(((w0 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w0 & 0xF0F0F0F0u) ^ 0x80808080u),
-                                 (int)(((w1 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w1 & 0xF0F0F0F0u) ^ 0x80808080u)};
+                    lo[0] = (unsigned)v; hi[0] = (unsigned)(v >> 32);
                 }
-            }
-            read_b(j == 3 ? buf ^ 1 : buf, (j + 1) & 3);
-            // a tile's dots are issued ahead of the previous tile's rescale (the last tile's is left to the next block); the empty
-            // asm statements keep that order. A row tile's scales of the next block are read once the block's last use of them is past.
 #pragma unroll
-            for (int tl = 0; tl < MT * NT; ++tl) {
-                const i32x16 dn = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j][tl / NT], B[tl % NT], i32x16{0}, 0, 0, 0);
-                const int pt = (tl + MT * NT - 1) % (MT * NT), pi = pt / NT, pj = pt % NT;
-                const float s = tl == 0 ? sw_due : sw[j][pj];
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[pi][pj][e] += (float)d[e] * (sa[pi][e] * s);
-                asm volatile("" : "+v"(acc[pi][pj]));
-                if (pj == NT - 1) read_sa(pi, tl == 0 ? buf : (j == 3 ? buf ^ 1 : buf), tl == 0 ? j : (j + 1) & 3);
-                d = dn;
+                    for (int i = 0; i < NT; ++i)
+                        sw[j][i] = g * 4 + j < KB ? code_scale * __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
             }
-            sw_due = sw[j][NT - 1];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                // The other buffer was last read in the previous group (those reads have returned once lgkmcnt is 0); its loads have three
+                // steps' time, and 3 MT younger ones are in flight when they are waited for. They are buffer loads: global_load_lds counts as a
+                // flat access, after which the compiler waits for every load in flight before the next use of any.
+                if (j == 0) {
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+                    __builtin_amdgcn_s_waitcnt(LGKM0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    clear_tail(g, buf);
+                    load_w(gn, buf ^ 1);
+                    load_scales(gn, buf ^ 1);
+                }
+                load_a((j + 3) & 3, j == 0 ? g * 4 + 3 : gn * 4 + j - 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (j == 3) {
+                    __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * MT));
+                    asm volatile("" ::: "memory");
+                }
+                i32x4 B[NT];
+#pragma unroll
+                for (int i = 0; i < NT; ++i) {
+                    if constexpr (Q8) {
+                        B[i] = Bn[i];                        // (copied by the loop's unrolling: no instruction)
+                    } else {
+                        // 16 * (nibble - 8) as int8: the nibble in the upper half of its byte with the top bit flipped
+                        const unsigned w0 = Bn[i].x, w1 = Bn[i].y;
+                        B[i] = i32x4{(int)(((w0 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w0 & 0xF0F0F0F0u) ^ 0x80808080u),
+                                     (int)(((w1 << 4) & 0xF0F0F0F0u) ^ 0x80808080u), (int)((w1 & 0xF0F0F0F0u) ^ 0x80808080u)};
+                    }
+                }
+                read_b(j == 3 ? buf ^ 1 : buf, (j + 1) & 3);
+                // a tile's dots are issued ahead of the previous tile's rescale (the last tile's is left to the next block); the empty
+                // asm statements keep that order. A row tile's scales of the next block are read once the block's last use of them is past.
+#pragma unroll
+                for (int tl = 0; tl < MT * NT; ++tl) {
+                    const i32x16 dn = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j][tl / NT], B[tl % NT], i32x16{0}, 0, 0, 0);
+                    const int pt = (tl + MT * NT - 1) % (MT * NT), pi = pt / NT, pj = pt % NT;
+                    const float s = tl == 0 ? sw_due : sw[j][pj];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) acc[pi][pj][e] += (float)d[e] * (sa[pi][e] * s);
+                    asm volatile("" : "+v"(acc[pi][pj]));
+                    if (pj == NT - 1) read_sa(pi, tl == 0 ? buf : (j == 3 ? buf ^ 1 : buf), tl == 0 ? j : (j + 1) & 3);
+                    d = dn;
+                }
+                sw_due = sw[j][NT - 1];
+            }
+            buf ^= 1;
+            sw_now = sw_raw;
+            sw_shift_now = sw_shift;
         }
-        buf ^= 1;
-        sw_now = sw_raw;
-        sw_shift_now = sw_shift;
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));            // no LDS-writing load may outlive the loop: its LDS is reused, or another workgroup's
-    // the last block's last tile (a wavefront without a group has none)
-    if (g_lo + ks < g_hi)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));            // no LDS-writing load may outlive the loop: its LDS is reused, or another workgroup's
+        // the last block's last tile (a wavefront without a group has none)
+        if (g_lo + ks < g_hi)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
+            for (int e = 0; e < 16; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
+
+        if constexpr (Q8) break;
+        if (code_scale != 1.f) break;
+        float finite = 0.f;                                  // NaN if a sum is not finite
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) finite += acc[i][j][e] * 0.f;
+        if (!__any(finite != finite)) break;
+        code_scale = 0.0625f;
+        sum_scale = 1.f;
+    }
+    if constexpr (!Q8) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] *= sum_scale;
+    }
 
     if (partial) {
         // a K slice leaves raw sums; gemm_i8_slices_kernel adds the slices in order and applies alpha and beta
@@ -303,7 +330,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         const int row = m0 + mi * 32 + 8 * (e >> 2) + 4 * h + (e & 3), col = n0 + ni * 32 + r;
         if (row >= M || col >= N) return;
         float *dst = c + (size_t)row * ldc + col;
-        v = alpha * (Q8 ? v : 0.0625f * v);
+        v *= alpha;
         *dst = beta == 0.f ? v : v + beta * *dst;
     };
     if constexpr (KS == 1) {

@@ -316,3 +316,23 @@ def test_exact_gemm_infinite_activations(gpu, orc, dtype, layout, m, n, k):
     rows = [r for r in range(m) if r not in (0, 1, m - 2)]
     assert rms_err(got[rows], oracle_i8(orc, dtype, layout, a[rows], blocks, n)) < 3e-5      # (bound: test_exact_gemm_tiles_and_k_divisions)
     w.free()
+
+
+# Sums stay finite up to the f32 range: the lowest f32, as a mask leaves it, in four blocks of a row gives sums of 1e37 .. 1e38. Beside it
+# rows of ordinary values. (test_gpu_prepare_act.py holds the other end: products of subnormal scales keep their bits.)
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(40, 100, 160), (33, 96, 2080), (9, 40, 8224), (8, 1056, 992), (150, 4128, 2048)])
+def test_exact_gemm_lowest_activations(gpu, orc, dtype, layout, m, n, k):
+    say("lowest", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    blocks, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    a = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    lowest = np.finfo(np.float32).min
+    a[3, [0, 40, 70, k - 1]] = lowest
+    a[m - 1, [5, 33, 100, k - 32]] = lowest
+    got = gpu.matmul(w, a)
+    assert "gemm_i8" in gpu.last_launch()["kernel"]
+    want = oracle_i8(orc, dtype, layout, a, blocks, n)
+    assert np.abs(want[[3, m - 1]]).max() > 2.2e37 and np.isfinite(want).all() and np.isfinite(got).all()
+    assert max(rms_err(g, x) for g, x in zip(got, want)) < 3e-5          # (bound: test_exact_gemm_tiles_and_k_divisions)
+    w.free()
