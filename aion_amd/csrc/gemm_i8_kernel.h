@@ -47,12 +47,14 @@ __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M 
 // LDS of a wavefront: two groups of four blocks, weight codes and activation scales
 template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
 
-template <int DT, int MT, int NT, int KS, int WGM, int WGN>
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE>
 __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
                                                                          int M, int K, int row_tiles, int row_group, int col_tiles, float alpha, float beta,
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
+    static_assert(RQ == 4 || MT * WGM == 1, "fewer rows than a tile: one row tile");
+    using Acc = __attribute__((ext_vector_type(4 * RQ))) float;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 31, h = lane >> 5;
@@ -76,7 +78,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
     const int KB = K >> 5, G = (KB + 3) >> 2;
     const int n0 = (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
 
-    f32x16 acc[MT][NT];
+    Acc acc[MT][NT];
     // q4 dots are 16 times the codes' dots. The 1/16 is taken from the sums, where it is exact down to subnormal products of scales; sums past
     // 2^124 leave the f32 range that way (a row that holds the lowest f32 as a mask), so a wavefront with one that is not finite runs
     // its share again with the 1/16 in the weight scales. (Codes without the 16 cost eight vector instructions a tile and block.)
@@ -138,7 +140,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         unsigned char *w_lds = lds + wave * gemm_i8_wave_lds_bytes<Q8, MT, NT>();
         float *sa_lds = (float *)(w_lds + 2 * WBUF);
         auto load_a = [&](int set, int kb) {
-            kb = min(kb, KB - 1);
+            if (!WHOLE) kb = min(kb, KB - 1);
 #pragma unroll
             for (int i = 0; i < MT; ++i) A[set][i] = *(const i32x4 *)(ab[i] + (size_t)((unsigned)kb * (unsigned)(arows[i] * 32)) + ao[i]);
         };
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         };
         struct __attribute__((packed, aligned(2))) U64 { unsigned long v; };
         auto load_scales = [&](int g, int buf) {
-            const int kb = min(g * 4, KB - 1), base = max(0, min(kb, KB - 4));
+            const int kb = WHOLE ? g * 4 : min(g * 4, KB - 1), base = WHOLE ? kb : max(0, min(kb, KB - 4));
             sw_shift = (kb - base) * 16;
             sw_raw = ((const U64 *)(sb + base + so))->v;
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -173,24 +175,25 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
                 for (int q = 0; q < 2; ++q)                  // two blocks' scales of 32 rows
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(sa_rsrc[i], (lds_void *)(sa_lds + (buf * MT + i) * 128 + q * 64), 4,
-                                                             aso[i] + (h && g * 4 + 2 * q + 1 < KB ? (unsigned)arows[i] * 4 : 0u),
-                                                             min(g * 4 + 2 * q, KB - 1) * arows[i] * 4, 0, 0);
+                                                             aso[i] + (h && (WHOLE || g * 4 + 2 * q + 1 < KB) ? (unsigned)arows[i] * 4 : 0u),
+                                                             (WHOLE ? g * 4 + 2 * q : min(g * 4 + 2 * q, KB - 1)) * arows[i] * 4, 0, 0);
 #endif
         };
 
         // the activation scales a lane multiplies with - 16 rows of each row tile - come from the wavefront's LDS copy of the group
-        float sa[MT][16];
+        float sa[MT][4 * RQ];
         auto read_sa = [&](int i, int buf, int j) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
+            for (int q = 0; q < RQ; ++q) {
                 const f32x4 v = *(const f32x4 *)(sa_lds + (buf * MT + i) * 128 + j * 32 + 8 * q + 4 * h);
                 sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
             }
         };
         // Blocks past the end of K in the last group: activation scale 0 as well as weight scale 0, where a real block's infinite scale
-        // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first block's.
+        // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first
+        // block's. (Writes in every group, all but the last to words nobody reads, in place of the branch: 1 % slower.)
         auto clear_tail = [&](int g, int buf) {
-            if (g * 4 + 4 <= KB) return;
+            if (WHOLE || g * 4 + 4 <= KB) return;
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -202,7 +205,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+                for (int e = 0; e < 4 * RQ; ++e) acc[i][j][e] = 0.f;
         int g = g_lo + ks;
         if (g < g_hi) {
             load_w(g, 0);
@@ -218,7 +221,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             for (int i = 0; i < MT - 1; ++i) read_sa(i, 0, 0);
         }
 #pragma unroll
-        for (int e = 0; e < 16; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
+        for (int e = 0; e < 4 * RQ; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
         int buf = 0;
         i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
         float sw_due = 0.f;
@@ -239,7 +242,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
                     for (int i = 0; i < NT; ++i)
-                        sw[j][i] = g * 4 + j < KB ? code_scale * __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
+                        sw[j][i] = WHOLE || g * 4 + j < KB ? code_scale * __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -282,7 +285,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                     const int pt = (tl + MT * NT - 1) % (MT * NT), pi = pt / NT, pj = pt % NT;
                     const float s = tl == 0 ? sw_due : sw[j][pj];
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) acc[pi][pj][e] += (float)d[e] * (sa[pi][e] * s);
+                    for (int e = 0; e < 4 * RQ; ++e) acc[pi][pj][e] += (float)d[e] * (sa[pi][e] * s);
                     asm volatile("" : "+v"(acc[pi][pj]));
                     if (pj == NT - 1) read_sa(pi, tl == 0 ? buf : (j == 3 ? buf ^ 1 : buf), tl == 0 ? j : (j + 1) & 3);
                     d = dn;
@@ -297,7 +300,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         // the last block's last tile (a wavefront without a group has none)
         if (g_lo + ks < g_hi)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
+            for (int e = 0; e < 4 * RQ; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
 
         if constexpr (Q8) break;
         if (code_scale != 1.f) break;
@@ -307,7 +310,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) finite += acc[i][j][e] * 0.f;
+                for (int e = 0; e < 4 * RQ; ++e) finite += acc[i][j][e] * 0.f;
         if (!__any(finite != finite)) break;
         code_scale = 0.0625f;
         sum_scale = 1.f;
@@ -339,10 +342,10 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) put(i, j, e, acc[i][j][e]);
+                for (int e = 0; e < 4 * RQ; ++e) put(i, j, e, acc[i][j][e]);
     } else {
         // the KS partial sums of a tile through LDS, added in wavefront order by the tile's wavefronts, a share each
-        constexpr int CH = MT * NT * 4;                  // 16-byte chunks per lane
+        constexpr int CH = MT * NT * RQ;                 // 16-byte chunks per lane
         f32x4 *red = (f32x4 *)lds + (size_t)wsub * KS * CH * 64;
         __syncthreads();                                 // (the staged activation scales are dead)
 #pragma unroll
@@ -350,8 +353,8 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
             for (int j = 0; j < NT; ++j)
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    red[(ks * CH + (i * NT + j) * 4 + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+                for (int q = 0; q < RQ; ++q)
+                    red[(ks * CH + (i * NT + j) * RQ + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
         __syncthreads();
 #pragma unroll
         for (int c0 = 0; c0 < (CH + KS - 1) / KS; ++c0) {
@@ -361,12 +364,12 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
 #pragma unroll
             for (int k = 1; k < KS; ++k) s += red[(k * CH + ch) * 64 + lane];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) put((ch >> 2) / NT, (ch >> 2) % NT, (ch & 3) * 4 + e, s[e]);
+            for (int e = 0; e < 4; ++e) put(ch / RQ / NT, ch / RQ % NT, ch % RQ * 4 + e, s[e]);
         }
     }
 }
 
-template <bool Q8, int MT, int NT, int KS, int WGM, int WGN> constexpr int gemm_i8_lds_bytes() {
-    const int operands = KS * WGM * WGN * gemm_i8_wave_lds_bytes<Q8, MT, NT>(), red = KS > 1 ? KS * WGM * WGN * MT * NT * 4096 : 0;
+template <bool Q8, int MT, int NT, int KS, int WGM, int WGN, int RQ> constexpr int gemm_i8_lds_bytes() {
+    const int operands = KS * WGM * WGN * gemm_i8_wave_lds_bytes<Q8, MT, NT>(), red = KS > 1 ? KS * WGM * WGN * MT * NT * RQ * 1024 : 0;
     return operands > red ? operands : red;
 }
