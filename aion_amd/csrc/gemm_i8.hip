@@ -38,7 +38,9 @@ __global__ __launch_bounds__(256) void gemm_i8_slices_kernel(GemmSegs segs, cons
 //   2 wavefronts: from 1024 rows and two 128 x 64 tiles per CU on (2048 x 14336 x 2048: q4 188 against 213 us, q8 210 against 243;
 //                 512 x 14336 x 4096 the other way, 101 against 95)
 //   4 slices:     few tiles against a long K, a second launch adds them in order (q4 16 x 2048 x 8192: 9.7 against 10.7 us,
-//                 16 x 2048 x 14336: 11.8 against 15.0; q8 11.0 against 13.9 and 13.5 against 19.1)
+//                 16 x 2048 x 14336: 11.8 against 15.0; q8, twice the bytes a tile, from K = 6144 and up to half a tile per CU on:
+//                 16 x 2048 x 6144 14.9 -> 12.4 us, 16 x 4096 x 8192 20.2 -> 17.1, 16 x 3072 x 11008 25.3 -> 18.8; past K = 11008 up to
+//                 three quarters: 16 x 6144 x 11008 28.8 -> 26.6, 64 x 3072 x 14336 31.1 -> 28.7)
 struct KSplit {
     int wavefronts, slices;
     bool operator==(const KSplit &o) const { return wavefronts == o.wavefronts && slices == o.slices; }
@@ -46,7 +48,9 @@ struct KSplit {
 KSplit k_split(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
     const size_t cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256, blocks = k / QK;
     const size_t small = ((m + 31) / 32) * ((n + 31) / 32), large = ((m + 127) / 128) * ((n + 63) / 64);
-    const int slices = !ctx->no_scratch_paths && ((blocks >= 256 && small <= cus / 4) || (blocks >= 448 && small <= cus / 2)) ? 4 : 1;
+    const bool sliced = dtype == AIONHIP_Q4_0 ? (blocks >= 256 && small <= cus / 4) || (blocks >= 448 && small <= cus / 2)
+                                              : (blocks >= 192 && small <= cus / 2) || (blocks >= 344 && small <= cus * 3 / 4);
+    const int slices = !ctx->no_scratch_paths && sliced ? 4 : 1;
     if (dtype == AIONHIP_Q4_0 && blocks >= 64 && small <= cus) return KSplit{8, slices};
     if (m >= 1024 && large >= 2 * cus) return KSplit{2, slices};
     return KSplit{4, slices};

@@ -336,3 +336,20 @@ def test_exact_gemm_lowest_activations(gpu, orc, dtype, layout, m, n, k):
     assert np.abs(want[[3, m - 1]]).max() > 2.2e37 and np.isfinite(want).all() and np.isfinite(got).all()
     assert max(rms_err(g, x) for g, x in zip(got, want)) < 3e-5          # (bound: test_exact_gemm_tiles_and_k_divisions)
     w.free()
+
+
+# Division of a long K over workgroups: either side of the lines (K = 6144, half a 32 x 32 tile per CU; K = 11008, three quarters; q4 8192 and
+# a quarter), seen as the second launch that adds the slices. Tolerance as in test_exact_gemm_tiles_and_k_divisions: 3e-5 at K = 11008.
+@pytest.mark.parametrize("m,n,k,q8_sliced,q4_sliced", [(9, 4096, 6144, True, False), (9, 4097, 6144, False, False), (16, 2048, 6112, False, False),
+                                                       (33, 2050, 8192, False, False), (40, 1024, 8192, True, True), (10, 6144, 11008, True, False),
+                                                       (10, 6145, 11008, False, False)])
+def test_exact_gemm_k_slices(gpu, orc, m, n, k, q8_sliced, q4_sliced):
+    for dtype, layout, sliced in ((be.Q8_0, be.ROWS_NK, q8_sliced), (be.Q4_0, be.KMAJOR_KN, q4_sliced)):
+        say("slices", dtype, m, n, k)
+        gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+        blocks, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+        a = np.random.default_rng(m * k).standard_normal((m, k)).astype(np.float32)
+        got = gpu.matmul(w, a)
+        assert ("slices" in gpu.last_launch()["kernel"]) == sliced
+        assert rms_err(got, oracle_i8(orc, dtype, layout, a, blocks, n)) < 3e-5
+        w.free()
