@@ -30,82 +30,133 @@ __global__ __launch_bounds__(256) void gemm_i8_slices_kernel(GemmSegs segs, cons
         if (col + t < segs.n[si]) dst[t] = beta == 0.f ? alpha * e[t] : alpha * e[t] + beta * dst[t];
 }
 
-// How the K of a weight is divided, which fixes the order its sums are taken in: across the 2, 4 or 8 wavefronts of a workgroup that
-// share a tile, and across `slices` workgroups. It depends on the rows, K and the weight's own columns alone, so that a weight that
-// shares a launch with siblings gives the bits it gives by itself; the tile is chosen freely below.
-//   8 wavefronts: q4 against a grid of at most one 32 x 32 tile per CU, K >= 2048 (16 x 4096 x 4096: 7.0 us against 8.6 with 4; q8,
-//                 twice the bytes per block, is level or better with 4)
-//   2 wavefronts: from 1024 rows and two 128 x 64 tiles per CU on (2048 x 14336 x 2048: q4 188 against 213 us, q8 210 against 243;
-//                 512 x 14336 x 4096 the other way, 101 against 95)
-//   4 slices:     few tiles against a long K, a second launch adds them in order (q4 16 x 2048 x 8192: 9.7 against 10.7 us,
-//                 16 x 2048 x 14336: 11.8 against 15.0; q8, twice the bytes a tile, from K = 6144 and up to half a tile per CU on:
-//                 16 x 2048 x 6144 14.9 -> 12.4 us, 16 x 4096 x 8192 20.2 -> 17.1, 16 x 3072 x 11008 25.3 -> 18.8; past K = 11008 up to
-//                 three quarters: 16 x 6144 x 11008 28.8 -> 26.6, 64 x 3072 x 14336 31.1 -> 28.7)
+// How the K of a weight is divided, which fixes the order its sums are taken in: across the 1, 2, 4 or 8 wavefronts of a workgroup that
+// share a tile, and across `slices` workgroups. It depends on the rows, the weight itself, the device's CUs and on whether the call may use
+// scratch memory, not on the weights beside it, so that a weight that shares a launch with siblings gives the bits it gives by itself;
+// the tile is chosen freely below.
 struct KSplit {
     int wavefronts, slices;
-    bool operator==(const KSplit &o) const { return wavefronts == o.wavefronts && slices == o.slices; }
+    bool fewer;                                  // fewer wavefronts than a longer K would get, see k_split
+    bool operator==(const KSplit &o) const { return wavefronts == o.wavefronts && slices == o.slices && fewer == o.fewer; }
 };
-KSplit k_split(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
-    const size_t cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256, blocks = k / QK;
-    const size_t small = ((m + 31) / 32) * ((n + 31) / 32), large = ((m + 127) / 128) * ((n + 63) / 64);
-    const bool sliced = dtype == AIONHIP_Q4_0 ? (blocks >= 256 && small <= cus / 4) || (blocks >= 448 && small <= cus / 2)
-                                              : (blocks >= 192 && small <= cus / 2) || (blocks >= 344 && small <= cus * 3 / 4);
-    const int slices = !ctx->no_scratch_paths && sliced ? 4 : 1;
-    if (dtype == AIONHIP_Q4_0 && blocks >= 64 && small <= cus) return KSplit{8, slices};
-    if (m >= 1024 && large >= 2 * cus) return KSplit{2, slices};
-    return KSplit{4, slices};
-}
 
-// The workgroup shapes, and a model of their times: t = t0 + blocks * us * max(1, b * ((1 - q) * r + q * whole)), where r is the
+// The workgroup shapes, and a model of their times: t = t0 + (blocks + e) * us * max(1, b * ((1 - q) * r + q * whole)), where r is the
 // workgroups per CU and `whole` the same in whole rounds of `resident` workgroups per CU - a lone workgroup costs us per quant
-// block of K, a filled device b * us per workgroup and CU. Fitted per block format to a sweep of 5 .. 2048 rows x N = 1024 ..
-// 32768 x K = 1024 .. 14336 (rms 4 .. 11 % a shape); choosing by it costs 1 % on average over always taking the fastest.
+// block of K, a filled device b * us per workgroup and CU, and what a tile costs beside its K counts as e blocks. Three sets of constants
+// per block format (no t0: not a shape of that set):
+//   [0]  launches alone, from a sweep of 5 .. 2048 rows x N = 1024 .. 32768 x K = 1024 .. 14336 (rms 4 .. 11 % a shape); the tiles whose K
+//        is shared as far as it pays for a long K are chosen by it
+//   [1]  whole calls of more than 16 rows, up to 2048, x N = 1024 .. 131072 x K = 512, 1056, 2048 (rms 8 %); [2] the same up to 16 rows.
+//        They weigh those tiles against wide tiles whose wavefronts share K less (the last four shapes): at a short K a tile's start
+//        and end weigh as much as its K, and these halve them. 512 x 32768 x 512 q4 61.9 -> 42.9 us with 128 x 128 tiles, 512 x 131072 x
+//        1056 q8 386 -> 280; 8 x 131072 x 512 q8 26.3 -> 20.5 with 32 x 256.
 struct I8Shape {
-    int bm, bn, ks, resident;
-    float t0[2], us[2], b[2], q[2];              // [0] q4_0, [1] q8_0
+    int bm, bn, ks;
 };
 constexpr I8Shape I8_SHAPES[] = {
-    {32, 32, 8, 2, {3.43f, 3.27f}, {0.0300f, 0.0468f}, {1.446f, 1.267f}, {0.00f, 0.09f}},
-    {32, 32, 4, 4, {3.12f, 2.85f}, {0.0437f, 0.0449f}, {0.903f, 1.213f}, {0.07f, 0.05f}},
-    {64, 32, 4, 3, {3.61f, 3.54f}, {0.0709f, 0.0686f}, {0.858f, 1.082f}, {0.15f, 0.10f}},
-    {96, 32, 4, 2, {4.03f, 4.01f}, {0.1034f, 0.0993f}, {0.938f, 1.082f}, {0.16f, 0.07f}},
-    {64, 64, 4, 2, {4.32f, 4.41f}, {0.1240f, 0.1187f}, {0.941f, 1.135f}, {0.28f, 0.18f}},
-    {128, 64, 2, 2, {5.71f, 5.61f}, {0.2479f, 0.2357f}, {0.875f, 1.050f}, {0.27f, 0.10f}},
+    {32, 32, 8}, {32, 32, 4}, {64, 32, 4}, {96, 32, 4}, {64, 64, 4}, {128, 64, 2}, {32, 64, 2}, {128, 128, 1}, {32, 128, 2}, {32, 256, 1}, {32, 64, 4},
 };
-constexpr int I8_COUNT = (int)(sizeof(I8_SHAPES) / sizeof(I8_SHAPES[0]));
+constexpr int I8_COUNT = 10;                     // (shapes that the model chooses from)
+constexpr int I8_WIDE4 = 10;                     // see pick_shape
+struct I8Fit {
+    int resident;
+    float t0, us, b, q, e;
+};
+constexpr size_t SHORT_BLOCKS = 80;              // between the measured K = 2080 and 4096
+constexpr I8Fit I8_FITS[3][2][I8_COUNT] = {      // [set][q4_0, q8_0][shape]
+    {{{2, 3.43f, 0.0300f, 1.446f, 0.00f, 0.f}, {4, 3.12f, 0.0437f, 0.903f, 0.07f, 0.f}, {3, 3.61f, 0.0709f, 0.858f, 0.15f, 0.f},
+      {2, 4.03f, 0.1034f, 0.938f, 0.16f, 0.f}, {2, 4.32f, 0.1240f, 0.941f, 0.28f, 0.f}, {2, 5.71f, 0.2479f, 0.875f, 0.27f, 0.f}},
+     {{}, {4, 2.85f, 0.0449f, 1.213f, 0.05f, 0.f}, {3, 3.54f, 0.0686f, 1.082f, 0.10f, 0.f},
+      {2, 4.01f, 0.0993f, 1.082f, 0.07f, 0.f}, {2, 4.41f, 0.1187f, 1.135f, 0.18f, 0.f}, {2, 5.61f, 0.2357f, 1.050f, 0.10f, 0.f}}},
+    {{{1, 5.15f, 0.0330f, 1.156f, 0.67f, 26.2f}, {1, 5.34f, 0.0486f, 0.738f, 0.87f, 12.5f}, {3, 5.52f, 0.0721f, 0.785f, 0.29f, 16.6f},
+      {2, 5.45f, 0.1022f, 0.852f, 0.44f, 19.4f}, {1, 6.13f, 0.1308f, 0.811f, 0.68f, 17.7f}, {1, 7.01f, 0.2614f, 0.764f, 0.75f, 11.8f},
+      {4, 5.21f, 0.0998f, 0.743f, 0.24f, 6.9f}, {1, 5.78f, 0.5707f, 0.696f, 0.77f, 7.6f}, {3, 5.45f, 0.1580f, 0.794f, 0.32f, 8.8f},
+      {3, 3.18f, 0.3581f, 0.894f, 0.29f, 8.5f}},
+     {{}, {4, 5.24f, 0.0503f, 0.843f, 0.22f, 9.2f}, {3, 5.82f, 0.0739f, 0.878f, 0.24f, 12.7f},
+      {1, 5.70f, 0.1183f, 0.847f, 0.68f, 15.f}, {1, 6.23f, 0.1498f, 0.824f, 0.72f, 13.5f}, {4, 5.57f, 0.2778f, 0.743f, 0.17f, 12.9f},
+      {3, 5.17f, 0.1094f, 0.892f, 0.31f, 3.3f}, {1, 5.45f, 0.5846f, 0.708f, 0.66f, 8.1f}, {3, 4.42f, 0.1938f, 0.838f, 0.25f, 10.5f},
+      {4, 5.27f, 0.3547f, 1.232f, 0.14f, 3.2f}}},
+    {{{1, 5.12f, 0.0264f, 1.467f, 0.50f, 17.f}, {4, 4.86f, 0.0426f, 0.818f, 0.24f, 10.3f}, {}, {}, {}, {}, {3, 4.99f, 0.0804f, 0.938f, 0.34f, 2.1f},
+      {}, {4, 4.72f, 0.1529f, 0.933f, 0.11f, 4.6f}, {2, 5.18f, 0.2571f, 1.286f, 0.22f, 2.f}},
+     {{}, {3, 5.10f, 0.0416f, 1.259f, 0.22f, 7.6f}, {}, {}, {}, {}, {3, 4.91f, 0.0829f, 1.253f, 0.25f, 4.1f},
+      {}, {3, 3.33f, 0.1636f, 1.093f, 0.26f, 10.5f}, {1, 6.76f, 0.1922f, 2.286f, 0.43f, 0.1f}}},
+};
 constexpr float I8_SLICE_US = 4.5f;              // the launch that adds K slices
 
-// the fastest shape of a K split for m rows against weights of ns[0 .. count - 1] columns
-int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k, KSplit split, float *us) {
-    const float cus = (float)(ctx->cu_count > 0 ? ctx->cu_count : 256), blocks = (float)(k / QK) / (float)split.slices;
-    const int f = dtype == AIONHIP_Q8_0;
+float shape_us(const aionhip_ctx *ctx, int i, const I8Fit &f, size_t m, const size_t *ns, int count, size_t k, int slices) {
+    const I8Shape &s = I8_SHAPES[i];
+    const float cus = (float)(ctx->cu_count > 0 ? ctx->cu_count : 256), blocks = (float)(k / QK) / (float)slices;
+    size_t tiles = 0;
+    for (int w = 0; w < count; ++w) tiles += (ns[w] + s.bn - 1) / s.bn;
+    const float r = (float)(tiles * ((m + s.bm - 1) / s.bm) * (size_t)slices) / cus;
+    const float whole = ceilf(r / (float)f.resident) * (float)f.resident;
+    return f.t0 + (blocks + f.e) * f.us * fmaxf(1.f, f.b * ((1.f - f.q) * r + f.q * whole)) + (slices > 1 ? I8_SLICE_US : 0.f);
+}
+
+// the fastest shape of a K split (-1: there is none) for m rows against weights of ns[0 .. count - 1] columns
+int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k, const KSplit &split, float *us) {
+    const I8Fit *fits = I8_FITS[!split.fewer ? 0 : m > 16 ? 1 : 2][dtype == AIONHIP_Q8_0];
     int best = -1;
     float best_us = 0.f;
     for (int i = 0; i < I8_COUNT; ++i) {
-        const I8Shape &s = I8_SHAPES[i];
-        if (s.ks != split.wavefronts) continue;
-        size_t tiles = 0;
-        for (int w = 0; w < count; ++w) tiles += (ns[w] + s.bn - 1) / s.bn;
-        const float r = (float)(tiles * ((m + s.bm - 1) / s.bm) * (size_t)split.slices) / cus;
-        const float whole = ceilf(r / (float)s.resident) * (float)s.resident;
-        const float t = s.t0[f] + blocks * s.us[f] * fmaxf(1.f, s.b[f] * ((1.f - s.q[f]) * r + s.q[f] * whole)) + (split.slices > 1 ? I8_SLICE_US : 0.f);
+        if (fits[i].t0 == 0.f || I8_SHAPES[i].ks != split.wavefronts) continue;
+        const float t = shape_us(ctx, i, fits[i], m, ns, count, k, split.slices);
         if (best < 0 || t < best_us) {
             best = i;
             best_us = t;
         }
     }
     if (us) *us = best_us;
+    // Few rows and three 32 x 32 tiles per CU or more: two of them to a wavefront, half the starts and ends and half the reads of the activation
+    // (16 x 32768 x 8192: q4 50.9 -> 46.1 us, q8 69.2 -> 61.0; x 4096 27.9 -> 25.9, 39.1 -> 36.0; x 2080 19.4 -> 18.4, 24.9 -> 23.9; level at two
+    // tiles per CU, and at K = 512).
+    if (best == 1 && (k / QK > SHORT_BLOCKS ? m <= 32 : m <= 16 && k >= 1024)) {
+        size_t tiles = 0;
+        for (int w = 0; w < count; ++w) tiles += (ns[w] + 31) / 32;
+        if (tiles >= 3 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256)) best = I8_WIDE4;
+    }
     return best;
 }
 
-template <int DT, int MT, int NT, int KS, int WGM, int SHAPE, bool WHOLE>
+//   8 wavefronts: q4 against a grid of at most one 32 x 32 tile per CU, K >= 2048 (16 x 4096 x 4096: 7.0 us against 8.6 with 4; q8,
+//                 twice the bytes per block, is level or better with 4)
+//   2 wavefronts: from 1024 rows and two 128 x 64 tiles per CU on (2048 x 14336 x 2048: q4 188 against 213 us, q8 210 against 243;
+//                 512 x 14336 x 4096 the other way, 101 against 95)
+//   fewer:        a K of up to SHORT_BLOCKS, where the model finds that 5 % ahead (never more: siblings of different widths seldom differ)
+//   4 slices:     few tiles against a long K, a second launch adds them in order (q4 16 x 2048 x 8192: 9.7 against 10.7 us,
+//                 16 x 2048 x 14336: 11.8 against 15.0; q8, twice the bytes a tile, from K = 6144 and up to half a tile per CU on:
+//                 16 x 2048 x 6144 14.9 -> 12.4 us, 16 x 4096 x 8192 20.2 -> 17.1, 16 x 3072 x 11008 25.3 -> 18.8; past K = 11008 up to
+//                 three quarters: 16 x 6144 x 11008 28.8 -> 26.6, 64 x 3072 x 14336 31.1 -> 28.7)
+KSplit k_split(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
+    const size_t cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256, blocks = k / QK;
+    const size_t small = ((m + 31) / 32) * ((n + 31) / 32), large = ((m + 127) / 128) * ((n + 63) / 64);
+    const bool sliced = dtype == AIONHIP_Q4_0 ? (blocks >= 256 && small <= cus / 4) || (blocks >= 448 && small <= cus / 2)
+                                              : (blocks >= 192 && small <= cus / 2) || (blocks >= 344 && small <= cus * 3 / 4);
+    const int slices = !ctx->no_scratch_paths && sliced ? 4 : 1;
+    KSplit split{dtype == AIONHIP_Q4_0 && blocks >= 64 && small <= cus ? 8 : m >= 1024 && large >= 2 * cus ? 2 : 4, slices, false};
+    if (blocks > SHORT_BLOCKS) return split;
+    const I8Fit *fits = I8_FITS[m > 16 ? 1 : 2][dtype == AIONHIP_Q8_0];
+    const int own = pick_shape(ctx, dtype, m, &n, 1, k, split, nullptr);
+    if (fits[own].t0 == 0.f) return split;
+    float best_us = 0.95f * shape_us(ctx, own, fits[own], m, &n, 1, k, 1);
+    for (int ks = split.wavefronts / 2; ks >= 1; ks /= 2) {
+        const KSplit fewer{ks, 1, true};
+        float us = 0.f;
+        if (pick_shape(ctx, dtype, m, &n, 1, k, fewer, &us) < 0 || us >= best_us) continue;
+        split = fewer;
+        best_us = us;
+    }
+    return split;
+}
+
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int SHAPE, int RQ, bool WHOLE>
 int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m, PreparedAct act,
                  float alpha, float beta, int slices) {
-    constexpr int BM = 32 * MT * WGM, BN = 32 * NT, LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, NT, KS, WGM, 1, 4>();
+    constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN, LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, NT, KS, WGM, WGN, RQ>();
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
     if (LDS > 64 * 1024)
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, 1, 4, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
     GemmSegs segs{};
     segs.count = count;
     int tiles = 0;
@@ -127,10 +178,10 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
         if (rc) return rc;
         partial = (float *)ctx->scratch2;
     }
-    // Tiles are dealt out in groups of 512 or 1024 rows, columns within: the activation rows and weight columns that run on an XCD
+    // Tiles are dealt out in groups of eight row tiles (256 .. 1024 rows), columns within: the activation rows and weight columns that run on an XCD
     // at the same time then fit its L2 (2048 x 14336 x 4096, 64 x 64 tiles: 409 -> 387 us for q4, 524 -> 465 for q8).
     const int row_group = row_tiles < 8 ? row_tiles : 8;
-    launch_k(ctx, gemm_i8_kernel<DT, MT, NT, KS, WGM, 1, 4, WHOLE>, dim3((unsigned)(tiles * row_tiles), 1, (unsigned)slices), dim3(64 * KS * WGM), LDS, segs,
+    launch_k(ctx, gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, dim3((unsigned)(tiles * row_tiles), 1, (unsigned)slices), dim3(64 * KS * WGM * WGN), LDS, segs,
              (const uint8_t *)act.q, (const float *)act.scale, (int)m, (int)ws[0]->k, row_tiles, row_group, tiles, alpha, beta, partial, partial_ld);
     if (slices > 1) {
         const size_t threads = m * (size_t)(partial_ld >> 2);
@@ -141,11 +192,19 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
 
 // WHOLE: K is whole groups of four blocks, as the projections of models are. The checks for blocks past the end of K cost a lone wavefront
 // up to 80 ns a group (32 x 1024 x 4096 q8 11.0 -> 11.7 us, 256 x 1024 x 8192 20.0 -> 21.5).
-template <int DT, int MT, int NT, int KS, int WGM, int SHAPE>
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int SHAPE, int RQ = 4>
 int launch_shape(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m, PreparedAct act,
                  float alpha, float beta, int slices) {
-    if (ws[0]->k % (4 * QK) == 0) return launch_kernel<DT, MT, NT, KS, WGM, SHAPE, true>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
-    return launch_kernel<DT, MT, NT, KS, WGM, SHAPE, false>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    if (ws[0]->k % (4 * QK) == 0) return launch_kernel<DT, MT, NT, KS, WGM, WGN, SHAPE, RQ, true>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    return launch_kernel<DT, MT, NT, KS, WGM, WGN, SHAPE, RQ, false>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+}
+
+// a shape of one row tile: up to 16 rows its kernel keeps half the sums
+template <int DT, int NT, int KS, int WGN, int SHAPE>
+int launch_rows32(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m, PreparedAct act,
+                  float alpha, float beta, int slices) {
+    if (m <= 16) return launch_shape<DT, 1, NT, KS, 1, WGN, SHAPE, 2>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    return launch_shape<DT, 1, NT, KS, 1, WGN, SHAPE>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
 }
 
 template <int DT>
@@ -153,14 +212,23 @@ int launch_split(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const
                  float alpha, float beta, KSplit split) {
     size_t ns[4];
     for (int i = 0; i < count; ++i) ns[i] = ws[i]->n;
+    const int slices = split.slices;
     switch (pick_shape(ctx, DT, m, ns, count, ws[0]->k, split, nullptr)) {
-    case 0: return launch_shape<DT, 1, 1, 8, 1, 0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
-    case 1: return launch_shape<DT, 1, 1, 4, 1, 1>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
-    case 2: return launch_shape<DT, 2, 1, 4, 1, 2>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
-    case 3: return launch_shape<DT, 3, 1, 4, 1, 3>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
-    case 4: return launch_shape<DT, 2, 2, 4, 1, 4>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
-    default: return launch_shape<DT, 2, 2, 2, 2, 5>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, split.slices);
+    case 0:
+        if constexpr (DT == AIONHIP_Q4_0) return launch_rows32<DT, 1, 8, 1, 0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+        break;
+    case 1: return launch_rows32<DT, 1, 4, 1, 1>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 2: return launch_shape<DT, 2, 1, 4, 1, 1, 2>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 3: return launch_shape<DT, 3, 1, 4, 1, 1, 3>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 4: return launch_shape<DT, 2, 2, 4, 1, 1, 4>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 5: return launch_shape<DT, 2, 2, 2, 2, 1, 5>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 6: return launch_rows32<DT, 1, 2, 2, 6>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 7: return launch_shape<DT, 2, 2, 1, 2, 2, 7>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 8: return launch_rows32<DT, 2, 2, 2, 8>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case 9: return launch_rows32<DT, 2, 1, 4, 9>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
+    case I8_WIDE4: return launch_rows32<DT, 2, 4, 1, I8_WIDE4>(ctx, ws, cs, ldcs, count, m, act, alpha, beta, slices);
     }
+    return set_err(ctx, AIONHIP_EXECUTION_FAILED, "gemm: no tile shape for m=%zu, n=%zu, k=%zu", m, ns[0], (size_t)ws[0]->k);
 }
 
 // one launch for the weights of each K split (siblings of one model nearly always share it)

@@ -353,3 +353,24 @@ def test_exact_gemm_k_slices(gpu, orc, m, n, k, q8_sliced, q4_sliced):
         assert ("slices" in gpu.last_launch()["kernel"]) == sliced
         assert rms_err(got, oracle_i8(orc, dtype, layout, a, blocks, n)) < 3e-5
         w.free()
+
+
+# A short K against a wide grid: wide tiles whose wavefronts share K less (1 or 2 to a tile instead of 4), rows and columns that end inside a
+# tile and inside a wavefront's part of it, K of one block, inside a group and of whole groups, both numbers of rows a tile keeps.
+# Tolerance as in test_exact_gemm_tiles_and_k_divisions (K / 32 terms: far below its 3e-5).
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k,most", [(257, 33000, 32, 2), (384, 32900, 96, 2), (300, 32900, 96, 2), (129, 131072, 128, 2), (1000, 16500, 160, 1), (9, 131100, 544, 2),
+                                        (16, 131073, 512, 2), (17, 131110, 64, 2), (96, 33001, 512, 2), (5, 100000, 544, 2)])
+def test_exact_gemm_short_k_wide_grid(gpu, orc, dtype, layout, m, n, k, most):
+    say("short k", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    blocks, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    a = np.random.default_rng(m * k).standard_normal((m, k)).astype(np.float32)
+    got = gpu.matmul(w, a)
+    instance = [x.strip() for x in gpu.last_launch()["kernel"].split("<")[1].split(">")[0].split(",")]
+    assert int(instance[3]) <= most, instance                      # wavefronts that share a tile's K
+    rows = sorted({0, 1, 2, 15, 16, 31, 32, 63, 64, 127, 128, m - 2, m - 1} & set(range(m)))
+    assert rms_err(got[rows], oracle_i8(orc, dtype, layout, a[rows], blocks, n)) < 3e-5
+    again = gpu.matmul(w, a)
+    assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
+    w.free()
