@@ -4,6 +4,7 @@
 // launches.
 #include "gemm_i8_kernel.h"
 
+#include <atomic>
 #include <cmath>
 
 namespace {
@@ -155,8 +156,14 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN, LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, NT, KS, WGM, WGN, RQ>();
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
-    if (LDS > 64 * 1024)
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+    if (LDS > 64 * 1024) {
+        static std::atomic<uint64_t> attr{0};                // devices (by number, of the first 64) that have it; per instance
+        const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
+        if (!(attr.load() & bit)) {
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+            attr.fetch_or(bit);
+        }
+    }
     GemmSegs segs{};
     segs.count = count;
     int tiles = 0;
