@@ -238,16 +238,15 @@ int rope_table(aionhip_ctx *ctx, int pairs, float freq_step, float scale_factor,
 // one activation row against one weight with a long reduction axis: K cut into slices, one launch (gemv_ksplit.hip)
 // 3..8 prepared rows against a weight with very many rows, the dots on the matrix pipe (gemv_mfma.hip); launch returns -1 when
 // the shape does not suit the kernel after all
-bool gemv_mfma_applies(const aionhip_weight *const *ws, int count, int m);
+bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m);
 int launch_gemv_mfma(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
                      float alpha, float beta);
 bool gemv_ksplit_applies(const aionhip_ctx *ctx, const aionhip_weight *w, const float *x);
 int launch_gemv_ksplit(aionhip_ctx *ctx, const aionhip_weight *w, float *c, const float *x, float alpha, float beta);
-int launch_gemv(aionhip_ctx *ctx, const aionhip_weight *w, int m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
                       PreparedAct act, float alpha, float beta);
 // whether launch_gemv_batch runs m rows against these weights on the exact GEMM's kernel (it then wants the tiled preparation)
-bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m);
+bool gemv_rows_on_gemm(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m);
 // modelled time of the exact GEMM's kernel
 float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k);
 // the exact GEMM addresses a row tile of a weight with 32-bit offsets; longer rows run on the GEMV kernels, eight at a time

@@ -414,35 +414,40 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 
 }  // namespace
 
-// Rows against one weight that the exact GEMM's kernel (32 x 32 tiles) multiplies faster than the lane-per-row kernel, whose work
-// and LDS traffic grow with the rows; weights of few columns leave the GEMM too few tiles, and 8200 ... 12000 columns leave its second
-// round of workgroups nearly empty. Both kernels timed over 230 shapes (K = 512 ... 14336, N = 512 ... 131072) at 2 ... 8 rows, both
-// block formats, preparation included:
-//   5..8 rows:  from max(1024, K) columns on. q4 8192 x 512 10.6 against 7.1 us, 4096 x 2048 9.1 against 7.9, 8192 x 4096 13.2 against
-//               9.6; q8 8192 x 4096 16.4 against 11.7. Narrower the GEMM loses: q4 2048 x 4096 9.2 against 9.7, q8 9.8 against 11.0.
-//   2..4 rows:  one round of tiles (8192 columns on 256 CUs: q8 x 8192 19.7 against 17.3, q4 14.9 against 13.9) or one and a half and
-//               more (q8 16384 x 14336 53.7 against 39.8, q4 35.7 against 32.4); q8 in between too (9664 x 4096 14.8 against 13.7)
-//               except over K = 5120 ... 8192 (9664 x 7392 21.0 against 22.2; q4 17.7 against 19.9). Beyond 2^28 weights the lane-per-row
-//               kernel streams faster (q8 32768 x 14336 80 against 96), for q4, with half the bytes a weight, from three rounds on
-//               (32768 x 4096 18.4 against 21.5). Two rows of q4: up to two rounds and K from 4096 on (12288 x 4096 14.2 against 13.3,
-//               x 2048 9.1 against 9.5).
+// Rows against one weight that the exact GEMM's kernel (tiles of 32 columns and up) multiplies faster than the lane-per-row kernel, whose
+// work and LDS traffic grow with the rows; weights of few columns leave the GEMM too few tiles. A round is 32 columns per CU. All kernels
+// timed over 130 shapes (K = 512 ... 14336, N = 1024 ... 262144) at 2, 4, 5 and 8 rows, both block formats, preparation included, weights
+// rotated past the memory-side cache (lane-per-row against GEMM, us; columns for 256 CUs):
+//   5..8 rows:  from max(1024, K) columns on. q4 8192 x 512 10.5 against 6.2, 4096 x 2048 9.6 against 8.7, 8192 x 4096 14 against 11; q8
+//               8192 x 4096 18 against 14. Narrower the GEMM loses: q8 2048 x 4096 10 against 12.
+//   2..4 rows:  one nearly full round (7681 ... 8192 columns: q8 x 8192 22 against 22, q4 16 against 14), or one and a half (12288
+//               columns) and more; q8 between them too up to K = 5120 (9664 x 4096 level; x 6144 1.11 times, x 8192 1.10) and where
+//               only two of the lane-per-row kernel's workgroups, which hold their rows' K in LDS, fit a CU (4 x 9664 x 14336 49 against
+//               44; of two rows four fit: 35 against 43). Upper ends: four rounds for q8 (65536 x 1024 19.5 against 22.5, 32768 x 4096
+//               level; of two rows past K = 8192 two: 20480 x 14336 60 against 69), three for q4, with half the bytes a weight (32768 x 4096 20.6 against 24), two for two rows of q4, from K = 4096
+//               on (12288 x 4096 14.2 against 13.3, x 2048 9.1 against 9.5). Beyond 2^28 weights the lane-per-row kernel streams faster
+//               whatever the CUs (q8 32768 x 14336 80 against 96).
 // Five rows and more over a K past 4096 take the GEMM before this rule is asked.
-bool gemv_rows_on_gemm(const aionhip_weight *const *ws, int count, int m) {
-    if (count != 1 || m < 2 || gemv_mfma_applies(ws, count, m)) return false;
-    const size_t n = ws[0]->n, k = ws[0]->k;
+bool gemv_rows_on_gemm(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m) {
+    if (count != 1 || m < 2 || gemv_mfma_applies(ctx, ws, count, m)) return false;
+    const size_t n = ws[0]->n, k = ws[0]->k, round = 32 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256);
     const bool q8 = ws[0]->dtype == AIONHIP_Q8_0;
     if (k < 256 || k > GEMM_I8_MAX_K) return false;
     if (m >= 5) return k <= 4096 && n >= (k > 1024 ? k : 1024);
-    if (n <= 7680 || n * k > ((size_t)1 << 28)) return false;
-    if (n > 8192 && n < 12288 && !(q8 && (k <= 5120 || k > 8192))) return false;
-    return q8 || (m >= 3 ? n <= 24576 : n <= 16384 && k >= 4096);
+    if (n * 16 <= round * 15 || n * k > ((size_t)1 << 28)) return false;
+    if (n > round && n * 2 < round * 3) {
+        const bool two_per_cu = (size_t)(m == 2 ? 2 : 4) * 40 * (k / QK) * 3 > 160 * 1024;
+        if (!(q8 && (k <= 5120 || two_per_cu))) return false;
+    }
+    if (q8) return n <= round * (m == 2 && k > 8192 ? 2 : 4);
+    return m >= 3 ? n <= round * 3 : n <= round * 2 && k >= 4096;
 }
 
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
                       PreparedAct act, float alpha, float beta) {
     if (m < 1 || m > 8) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: m=%d outside 1..8", m);
     if (count < 1 || count > 4) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: %d weights in one launch (1..4)", count);
-    if (!act.tiled && gemv_mfma_applies(ws, count, m)) {
+    if (!act.tiled && gemv_mfma_applies(ctx, ws, count, m)) {
         const char *mname = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8_mfma" : "gemv_q4_mfma";
         ProfScope scope(ctx, mname);
         const int rc = launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
@@ -465,8 +470,4 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
     if (rc) return rc;
     LAUNCH_CHECK(ctx, name);
     return AIONHIP_OK;
-}
-
-int launch_gemv(aionhip_ctx *ctx, const aionhip_weight *w, int m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {
-    return launch_gemv_batch(ctx, &w, &c, &ldc, 1, m, act, alpha, beta);
 }

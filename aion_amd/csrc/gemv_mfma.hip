@@ -342,28 +342,32 @@ int launch_mf_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const
 
 }  // namespace
 
-// Where this kernel is ahead of the vector-ALU rows kernel (and of the exact GEMM's 16-row tile), from a sweep of 3..8 rows over
-// N = 14336 ... 262144 x K = 2048 ... 8192, both weight types: it needs many row tiles to amortise its longer start (ring fill
-// behind the activation copy), and it gains most where the vector ALU is the rows kernel's bound - q4 from five rows on.
-//   q4, 5..8 rows, N >= 14336: 14336 x 4096 19.3 against 20.1 us, 24576 x 4096 20.8 / 25.0, 65536 x 4096 33.0 / 41.9,
-//                               262144 x 2048 60.0 / 83.6 (8 rows)
-//   q4, 3..4 rows, N >= 65536: 65536 x 2048 20.5 / 23.5, 131072 x 2048 31.1 / 39.0, 262144 x 2048 62.2 / 66.6 (4 rows);
-//                               below that the rows kernel leads (32768 x 4096: 22.3 / 21.1)
-//   q8, 3..8 rows, N >= 65536 and up to 300 M weights: 65536 x 2048 28.5 / 31.1, 131072 x 2048 49.0 / 53.5, 65536 x 4096
-//                               52.0 / 59.5; past that size the rows kernel streams faster (262144 x 2048: 107 / 99)
-// K: whole 256-code stages, 2048 ... 4096 (at 8192 the rows kernel is far ahead at 3..4 rows, the exact GEMM even at 5..8).
+// Where this kernel is ahead of the vector-ALU rows kernel and of the exact GEMM's, from sweeps of 3..8 rows over N = 14336 ... 262144 x
+// K = 1024 ... 8192, both weight types (us, this kernel against the faster of the other two; columns for 256 CUs): it needs many row
+// tiles to amortise its longer start (ring fill behind the activation copy), and it gains most where the vector ALU is the rows kernel's
+// bound - q4 from five rows on.
+//   q4, 5..8 rows, 56 columns a CU:  65536 x 2048 22 / 25.5, 65536 x 4096 37 / 43, 262144 x 2048 66 / 84; siblings (q/k/v, gate/up) have
+//                      the rows kernel only: 14336 x 4096 19.3 / 19.5, 24576 x 4096 22 / 28. A single weight of up to 32768 rows is
+//                      faster on the exact GEMM's kernel (14336 x 4096 14.2, 24576 x 4096 20.8, 32768 x 4096 level)
+//     K under 2048, 192:              262144 x 1024 36 / 44, 131072 x 1536 0.61 / 0.67 of the rows kernel, 49152 level; 32768 x 1024 0.85 / 0.74
+//   q4, 3..4 rows, 256:  65536 x 2048 21 / 23, x 1024 14.9 / 15.5, 262144 x 1024 35 / 39; x 2048 65 / 63, 65536 x 4096 level; 32768 x 4096 22.3 / 20.6
+//   q8, 5..8 rows, 256:  65536 x 2048 32 / 34, 262144 x 2048 106 / 117, x 1024 level; 49152 x 4096 51 / 51
+//   q8, 3..4 rows, 256 and up to 300 M weights, K from 2048 on: level with the rows kernel (65536 x 2048 31 / 30, 131072 x 2048 54.4 / 52.5);
+//                      past that size the rows kernel streams faster (262144 x 2048 102 / 96)
+// K: whole 256-code stages, 1024 ... 4096 (at 8192 the rows kernel is far ahead at 3..4 rows, the exact GEMM at 5..8).
 // N counts the rows of all weights of the call (siblings share the launch).
-bool gemv_mfma_applies(const aionhip_weight *const *ws, int count, int m) {
+bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m) {
     if (m < 3 || m > 8 || count < 1 || count > 4) return false;
-    const size_t k = ws[0]->k;
-    if (k % (MF_SB * 32) != 0 || k < 2048 || k > 4096) return false;
+    const size_t k = ws[0]->k, cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256;
+    if (k % (MF_SB * 32) != 0 || k < 1024 || k > 4096) return false;
     size_t rows = 0;
     for (int i = 0; i < count; ++i) {
         if (ws[i]->k != k || ws[i]->dtype != ws[0]->dtype || ws[i]->n < 1) return false;
         rows += ws[i]->n;
     }
-    if (ws[0]->dtype == AIONHIP_Q4_0) return rows >= (m >= 5 ? (size_t)14336 : (size_t)65536);
-    if (ws[0]->dtype == AIONHIP_Q8_0) return rows >= 65536 && rows * k <= (size_t)300 * 1000 * 1000;
+    const bool short_k = k < 2048;
+    if (ws[0]->dtype == AIONHIP_Q4_0) return rows >= cus * (m < 5 ? 256 : short_k ? 192 : 56);
+    if (ws[0]->dtype == AIONHIP_Q8_0) return rows >= cus * 256 && (m >= 5 || (!short_k && rows * k <= (size_t)300 * 1000 * 1000));
     return false;
 }
 

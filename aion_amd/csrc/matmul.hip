@@ -66,9 +66,9 @@ static bool fused_row_pays(const Batch &b) {
 // 14336 x 8192 at 8 rows: 80 against 33 us, q4 65 against 29; the two meet at K = 4096 ... 5120); the GEMM beyond eight rows.
 static bool rows_on_gemv(const Batch &b, size_t m) { return m <= GEMV_MAX_M && (b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)); }
 // which form of the preparation the kernel behind launch_prepared_rows reads
-static bool rows_tiled(const Batch &b, size_t m) {
+static bool rows_tiled(const aionhip_ctx *ctx, const Batch &b, size_t m) {
     if (b.k > GEMM_I8_MAX_K) return false;
-    return !rows_on_gemv(b, m) || gemv_rows_on_gemm(b.w, (int)b.count, (int)m);
+    return !rows_on_gemv(b, m) || gemv_rows_on_gemm(ctx, b.w, (int)b.count, (int)m);
 }
 static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, PreparedAct act, float alpha, float beta) {
     if (m > GEMV_MAX_M && b.k > GEMM_I8_MAX_K) {                 // rows past the GEMM's addressing
@@ -127,7 +127,7 @@ int run_rows(aionhip_ctx *ctx, const Batch &b, size_t m, const float *a, size_t 
     }
     int rc = static_scratch ? (int)AIONHIP_OK : ensure_scratch(ctx, prepared_act_bytes(m, b.k));
     if (rc) return rc;
-    PreparedAct act = prepared_act_carve(static_scratch ? ctx->static_scratch : ctx->scratch, m, b.k, rows_tiled(b, m));
+    PreparedAct act = prepared_act_carve(static_scratch ? ctx->static_scratch : ctx->scratch, m, b.k, rows_tiled(ctx, b, m));
     rc = launch_prepare_act(ctx, a, lda, m, b.k, act);
     if (rc) return rc;
     return launch_prepared_rows(ctx, b, m, act, alpha, beta);
@@ -210,7 +210,7 @@ int aionhip_step_rmsnorm_matmul(aionhip_ctx *ctx, size_t count, const aionhip_we
     if (rows >= 2 && rows <= 0x7FFFFFFFu && !bf16_route && ((x | gamma | beta_norm) & 15) == 0) {
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
         if (rc) return rc;
-        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(b, rows));
+        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(ctx, b, rows));
         rc = launch_prepare_rmsnorm(ctx, xp, gp, bp, eps, rows, b.k, act);
         if (rc) return rc;
         return launch_prepared_rows(ctx, b, rows, act, alpha, beta);
@@ -300,7 +300,7 @@ int aionhip_step_gate_matmul(aionhip_ctx *ctx, const aionhip_weight *w, size_t r
         // gate and activation preparation in one small launch, then the GEMV (or GEMM) on the prepared rows
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
         if (rc) return rc;
-        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(b, rows));
+        PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, rows_tiled(ctx, b, rows));
         rc = launch_prepare_gate(ctx, gp, up_p, rows, b.k, act);
         if (rc) return rc;
         return launch_prepared_rows(ctx, b, rows, act, alpha, beta);

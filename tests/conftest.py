@@ -75,12 +75,14 @@ def row_rms_err(got, ref):
 
 
 def rows_kernel(q8, m, n, k):
-    """The kernel 2..8 activation rows against an [n, k] weight run on (what aionhip_last_kernel reports): the matrix-pipe GEMV for
-    many weight rows and a K of 2048..4096 in whole 256-code stages (q4: from 14336 rows at 5..8 activation rows, from 65536 at
-    3..4; q8: from 65536 rows up to 300 M weights), the exact GEMM's 16-row tile for 5..8 rows over a K past 4096, else the
-    vector-ALU rows kernel."""
+    """The kernel 2..8 activation rows against an [n, k] weight run on (what aionhip_last_kernel reports), for 256 CUs: the matrix-pipe
+    GEMV for many weight rows and a K of 1024..4096 in whole 256-code stages (q4: from 14336 rows at 5..8 activation rows - 49152 below
+    K = 2048 -, from 65536 at 3..4; q8: from 65536 rows, at 3..4 activation rows from K = 2048 on and up to 300 M weights), the exact
+    GEMM for 5..8 rows over a K past 4096, else the vector-ALU rows kernel or, under the same name, the exact GEMM's kernel."""
     tag = "q8" if q8 else "q4"
-    if 3 <= m <= 8 and 2048 <= k <= 4096 and k % 256 == 0:
-        if (not q8 and n >= (14336 if m >= 5 else 65536)) or (q8 and n >= 65536 and n * k <= 300_000_000):
-            return "gemv_%s_mfma" % tag
+    if 3 <= m <= 8 and 1024 <= k <= 4096 and k % 256 == 0:
+        if not q8 and n >= (65536 if m < 5 else 49152 if k < 2048 else 14336):
+            return "gemv_q4_mfma"
+        if q8 and n >= 65536 and (m >= 5 or (k >= 2048 and n * k <= 300_000_000)):
+            return "gemv_q8_mfma"
     return ("gemm_i8_" if m >= 5 and k > 4096 else "gemv_") + tag

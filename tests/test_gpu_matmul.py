@@ -333,10 +333,9 @@ def test_exact_gemm_shapes_and_edges(gpu, orc, dtype, layout, m, n, k):
 
 # 2..8 activation rows (gemv_rows_kernel): row counts that fill a 2-, 4- or 8-row instance only partly, N that is
 # not a multiple of the rows a wavefront works on, K of one LDS pass, K that needs most of a CU's LDS (16384 at 4 rows) and K
-# long enough to run as several K-range launches (32768 at 3 rows), alpha/beta on a pre-filled C. Three shapes (5..8 rows, at
-# least 16384 columns, K up to 4096) run on the 16-row tile of the LDS-staged MFMA kernel instead: ragged N, K of one and of
-# many steps. Five to eight rows over a K past 4096 take the exact GEMM (its 16-row tile is far ahead there). Many weight rows
-# over a K of 2048 ... 4096 take the matrix-pipe GEMV (gemv_mfma_kernel; conftest.rows_kernel states where): one wavefront per
+# long enough to run as several K-range launches (32768 at 3 rows), alpha/beta on a pre-filled C. Some shapes (5..8 rows, many
+# columns, K up to 4096) run on the exact GEMM's kernel under the same name: ragged N, K of two and of many groups. Five to eight
+# rows over a K past 4096 take the exact GEMM (it is far ahead there). Many weight rows over a K of 1024 ... 4096 take the matrix-pipe GEMV (gemv_mfma_kernel; conftest.rows_kernel states where): one wavefront per
 # 16-row tile and two sharing a tile's K (14400 rows), ragged N, K of 8 / 9 / 16 stages, 3 ... 8 rows, both weight types.
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("m,n,k", [(2, 70, 96), (3, 1001, 1056), (5, 333, 2048), (8, 1030, 14336), (7, 4100, 7200), (4, 9000, 512),
@@ -357,12 +356,30 @@ def test_decode_gemv_two_to_eight_rows(gpu, orc, dtype, layout, m, n, k):
     w.free()
 
 
+# The matrix-pipe GEMV's lines on 256 CUs: the smallest K and its next stage, columns on either side, q8 past 300 M weights (from five
+# rows on). Below a line the vector-ALU rows kernel or the exact GEMM's kernel runs, under the name gemv_q*.
+@pytest.mark.parametrize("m,n,k,q4_mfma,q8_mfma", [(5, 65540, 1024, True, True), (8, 49153, 1280, True, False), (8, 49151, 1024, False, False),
+                                                   (4, 65537, 1024, True, False), (3, 65535, 1280, False, False), (8, 131073, 2304, True, True),
+                                                   (4, 131073, 2304, True, False)])
+def test_matrix_pipe_gemv_lines(gpu, orc, m, n, k, q4_mfma, q8_mfma):
+    for dtype, layout, mfma in ((be.Q4_0, be.KMAJOR_KN, q4_mfma), (be.Q8_0, be.ROWS_NK, q8_mfma)):
+        say("matrix-pipe lines", dtype, m, n, k)
+        blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m + n + k, std=0.05)
+        a = np.random.default_rng(m + n).standard_normal((m, k)).astype(np.float32)
+        got = gpu.matmul(w, a)
+        assert gpu.last_kernel() == "gemv_%s%s" % ("q8" if dtype == be.Q8_0 else "q4", "_mfma" if mfma else "")
+        want = oracle_matmul(orc, dtype, layout, a, blocks, n)
+        assert norm_err(got, want) < TOL and rms_err(got, want) < RMS_TOL
+        w.free()
+
+
 # both sides of the lines between the lane-per-row kernel and the exact GEMM's: columns against K at 5..8 rows, rounds
 # of the GEMM's tiles on 256 CUs at 2..4 rows; widths that end inside a tile
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("m,n,k", [(5, 1023, 512), (8, 1024, 512), (8, 1040, 224), (6, 2049, 2048), (7, 2047, 2048), (5, 4100, 4096), (8, 3999, 4000),
                                    (2, 8191, 512), (2, 8195, 512), (4, 7680, 1056), (4, 8192, 1056), (3, 16385, 1024), (2, 8200, 4128), (4, 9001, 8192),
-                                   (2, 12287, 4096), (2, 12290, 4096), (3, 24577, 512), (2, 16385, 4096)])
+                                   (2, 12287, 4096), (2, 12290, 4096), (3, 24577, 512), (2, 16385, 4096), (4, 9664, 14336), (2, 9664, 14336),
+                                   (4, 32800, 1024), (2, 16390, 8224)])
 def test_few_rows_on_either_side_of_the_gemm_line(gpu, orc, dtype, layout, m, n, k):
     say("few rows", dtype, layout, m, n, k)
     blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 17 + n + k, std=0.05)
@@ -371,7 +388,9 @@ def test_few_rows_on_either_side_of_the_gemm_line(gpu, orc, dtype, layout, m, n,
     if m >= 5:
         on_gemm = n >= max(1024, k)
     else:
-        on_gemm = (7680 < n <= 8192 or n >= 12288 or (q8 and n > 8192 and not 5120 < k <= 8192)) and (q8 or (n <= 24576 if m >= 3 else n <= 16384 and k >= 4096))
+        between = q8 and n > 8192 and (k <= 5120 or (m > 2 and k > 10922))      # (past 10922 the rows of K take a third of a CU's LDS)
+        upper = (16384 if m == 2 and k > 8192 else 32768) if q8 else (24576 if m >= 3 else 16384 if k >= 4096 else 0)
+        on_gemm = (7680 < n <= 8192 or n >= 12288 or between) and n <= upper
     on_gemm = on_gemm and k >= 256
     got = gpu.matmul(w, a)
     assert ("gemm_i8" in gpu.last_launch()["kernel"]) == on_gemm
