@@ -247,12 +247,12 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
                       PreparedAct act, float alpha, float beta);
 // whether launch_gemv_batch runs m rows against these weights on the exact GEMM's kernel (it then wants the tiled preparation)
 bool gemv_rows_on_gemm(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m);
-// modelled time of the exact GEMM's kernel
+// modelled time of a call on the exact GEMM, preparation included
 float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k);
 // the exact GEMM addresses a row tile of a weight with 32-bit offsets; longer rows run on the GEMV kernels, eight at a time
 constexpr size_t GEMM_I8_MAX_K = (size_t)1 << 26;
 // bf16 mode only: whether the bf16 MFMA kernel is expected to be the faster one for m rows against an n x k weight
-bool gemm_bf16_pays(const aionhip_ctx *ctx, size_t m, size_t n, size_t k);
+bool gemm_bf16_pays(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k);
 int launch_gemm_i8_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, size_t m,
                          PreparedAct act, float alpha, float beta);
 // the same kernel for a handful of rows (no profile scope of its own: the caller's name stays)

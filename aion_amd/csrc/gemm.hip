@@ -493,15 +493,15 @@ __global__ __launch_bounds__(256) void gemm_bf16_mixed_kernel(const unsigned sho
 // In bf16 mode: is the bf16 MFMA kernel expected to beat the exact kernel for this shape? Up to a few hundred rows it
 // is not - it streams a 2-byte copy of every weight (3.5x the q4 bytes), its 256-column tiles leave most CUs idle and
 // one workgroup's K loop is a latency chain - and the exact kernel is then both the faster and the exact one.
-// Modelled times in microseconds, constants fitted to a sweep of 9..512 rows over four weight shapes.
-bool gemm_bf16_pays(const aionhip_ctx *ctx, size_t m, size_t n, size_t k) {
-    const float exact_us = gemm_i8_us(ctx, AIONHIP_Q4_0, m, n, k) + 5.f + (float)m * (float)k * 4.f / 2.0e6f;   // + the int8 preparation of A
-    // (constants fitted to both kernels' times over six weight shapes x 65..1024 rows, q4: the choice costs 0.3 % over
-    // always taking the faster one; always exact would cost 36 %, always bf16 17 %)
-    const float copy_us = (float)n * (float)k * 2.f / 3.0e6f;                                  // weight bytes at ~3 TB/s
-    const float flop_us = 2.f * (float)m * (float)n * (float)k / 9.0e8f;                        // ~900 TFLOP/s
-    const float chain_us = (float)(k / 32) * 0.24f;                                                       // one workgroup's K loop
-    const float act_us = (float)m * (float)k * 6.f / 4.0e6f;                                     // the bf16 rounding of A
+// Modelled times of whole calls in microseconds, the constants below fitted to the bf16 kernel's over ten weight shapes x 16 .. 2048 rows
+// (rms 20 %). Over those, both block formats, the choice costs 1.2 % over always taking the faster kernel; always exact would cost 10 %,
+// always bf16 58 %. (512 x 4096 x 14336 q4: exact 97 us, bf16 168; 2048 x 14336 x 4096 the other way, 356 and 215.)
+bool gemm_bf16_pays(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
+    const float exact_us = gemm_i8_us(ctx, dtype, m, n, k);
+    const float copy_us = (float)n * (float)k * 2.f / 2.7e6f;                                  // weight bytes at ~2.7 TB/s
+    const float flop_us = 2.f * (float)m * (float)n * (float)k / 9.3e8f;                        // ~930 TFLOP/s
+    const float chain_us = (float)(k / 32) * 0.31f;                                            // one workgroup's K loop
+    const float act_us = (float)m * (float)k * 2.0e-6f;                                         // the bf16 rounding of A
     const float bf16_us = fmaxf(fmaxf(copy_us, flop_us), chain_us) + act_us;
     return bf16_us < exact_us;
 }

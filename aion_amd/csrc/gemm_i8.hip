@@ -267,8 +267,9 @@ int launch_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
 
 float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
     float us = 0.f;
-    pick_shape(ctx, dtype, m, &n, 1, k, k_split(ctx, dtype, m, n, k), &us);
-    return us;
+    const KSplit split = k_split(ctx, dtype, m, n, k);
+    pick_shape(ctx, dtype, m, &n, 1, k, split, &us);
+    return split.fewer ? us : us + 2.f;          // + the preparation's launch, which the first set of constants leaves out
 }
 
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {

@@ -116,7 +116,7 @@ int run_rows(aionhip_ctx *ctx, const Batch &b, size_t m, const float *a, size_t 
         // the bf16 kernel where it is expected to win (or always, if so asked), the exact kernel (below) for the rest
         bool all_bf16 = true;
         if (ctx->gemm_mode == AIONHIP_GEMM_BF16_MFMA)
-            for (size_t i = 0; i < b.count; ++i) all_bf16 = all_bf16 && gemm_bf16_pays(ctx, m, b.w[i]->n, b.k);
+            for (size_t i = 0; i < b.count; ++i) all_bf16 = all_bf16 && gemm_bf16_pays(ctx, b.w[i]->dtype, m, b.w[i]->n, b.k);
         if (all_bf16) {
             for (size_t i = 0; i < b.count; ++i) {
                 int rc = launch_gemm_bf16(ctx, b.w[i], m, a, lda, b.c[i], b.ldc[i], alpha, beta);
@@ -206,7 +206,7 @@ int aionhip_step_rmsnorm_matmul(aionhip_ctx *ctx, size_t count, const aionhip_we
     // into slices that prepare their own part), and so does a call that the bf16 kernel takes (it wants the f32 rows).
     bool bf16_route = rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8;
     if (bf16_route && ctx->gemm_mode == AIONHIP_GEMM_BF16_MFMA)
-        for (size_t i = 0; i < b.count; ++i) bf16_route = bf16_route && gemm_bf16_pays(ctx, rows, b.w[i]->n, b.k);
+        for (size_t i = 0; i < b.count; ++i) bf16_route = bf16_route && gemm_bf16_pays(ctx, b.w[i]->dtype, rows, b.w[i]->n, b.k);
     if (rows >= 2 && rows <= 0x7FFFFFFFu && !bf16_route && ((x | gamma | beta_norm) & 15) == 0) {
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
         if (rc) return rc;
@@ -295,7 +295,7 @@ int aionhip_step_gate_matmul(aionhip_ctx *ctx, const aionhip_weight *w, size_t r
         return launch_gemv_fused(ctx, b.w, b.c, b.ldc, 1, PRO_GATE, FusedIn{gp, up_p, nullptr, nullptr, 0.f}, alpha, beta);
     // more rows, on the exact kernels (always, or where the bf16 kernel would not pay): the same two launches, the GEMM last
     const bool bf16_route = rows > GEMV_MAX_M && (ctx->gemm_mode == AIONHIP_GEMM_BF16_MFMA_ALWAYS ||
-                                                  (ctx->gemm_mode == AIONHIP_GEMM_BF16_MFMA && gemm_bf16_pays(ctx, rows, b.w[0]->n, b.k)));
+                                                  (ctx->gemm_mode == AIONHIP_GEMM_BF16_MFMA && gemm_bf16_pays(ctx, b.w[0]->dtype, rows, b.w[0]->n, b.k)));
     if (!bf16_route && rows <= 0x7FFFFFFFu) {
         // gate and activation preparation in one small launch, then the GEMV (or GEMM) on the prepared rows
         rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
