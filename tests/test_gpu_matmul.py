@@ -356,6 +356,54 @@ def test_decode_gemv_two_to_eight_rows(gpu, orc, dtype, layout, m, n, k):
     w.free()
 
 
+# Rows of K past 2^26, which the exact GEMM cannot address: they run on the GEMV kernels, eight at a time (nine rows: eight and one, each
+# with its part of the preparation and of C), five to eight of them as well. Two weights, alpha and beta. Reference: the integer codes and
+# scales in float64, on the rows at the ends of the parts. Tolerance: an output is K / 32 = 2.1 M products summed by 64 lanes, 33 k f32
+# additions one after the other (q4: 9.1 k launches that add to C), whose rounding grows like a random walk: sqrt(33 k) 2^-24 = 1.1e-5 of
+# the sum, ten times that allowed.
+@pytest.mark.parametrize("dtype,layout", [(be.Q8_0, be.ROWS_NK), (be.Q4_0, be.KMAJOR_KN)])
+@pytest.mark.parametrize("m,rows", [(9, (0, 7, 8)), (6, (5,))])
+def test_rows_past_the_gemms_addressing(gpu, orc, dtype, layout, m, rows):
+    k, ns = (1 << 26) + 32, (2, 1)
+    say("long rows", dtype, m, k)
+    rng = np.random.default_rng(m)
+    pool = rng.standard_normal((1 << 20) + 7).astype(np.float32)
+    a = np.empty((m, k), np.float32)
+    for r in range(m):
+        a[r] = np.resize(np.roll(pool, 1000 * r), k)
+    made = []
+    for n in ns:
+        shape = (n, k) if layout == be.ROWS_NK else (k, n)
+        w = np.resize(rng.standard_normal((1 << 19) + 3).astype(np.float32) * np.float32(0.02), n * k).reshape(shape)
+        blocks = be.quantize_blocks(dtype, w, 1 if layout == be.ROWS_NK else 0)
+        made.append((blocks, gpu.upload_weight(dtype, layout, n, k, blocks)))
+    a_buf = gpu.upload(a)
+    c0 = [rng.standard_normal((m, n)).astype(np.float32) for n in ns]
+    c_bufs = [gpu.upload(c) for c in c0]
+    gpu.step_matmul_batch([w for _b, w in made], a_buf, m, c_bufs, alpha=0.5, beta=-2.0)
+    gpu.sync()
+    for (blocks, _w), cb, c, n in zip(made, c_bufs, c0, ns):
+        got = gpu.download(cb, np.float32, (m, n))
+        b = blocks.reshape(n, k // 32, -1) if layout == be.ROWS_NK else blocks.reshape(k // 32, n, -1).transpose(1, 0, 2)
+        for r in rows:
+            codes, scales = orc.prepare_a(a[r:r + 1])[:2]
+            codes, scales = codes.reshape(-1, 32).astype(np.int32), scales.reshape(-1).astype(np.float64)
+            for j in range(n):
+                ws = np.ascontiguousarray(b[j, :, :2]).view(np.float16)[:, 0].astype(np.float64)
+                if dtype == be.Q8_0:
+                    wc = np.ascontiguousarray(b[j, :, 2:]).view(np.int8).astype(np.int32)
+                else:
+                    nib = np.ascontiguousarray(b[j, :, 2:])
+                    wc = np.stack([nib & 15, nib >> 4], axis=2).reshape(-1, 32).astype(np.int32) - 8
+                want = 0.5 * float(((codes * wc).sum(1) * (scales * ws)).sum()) - 2.0 * float(c[r, j])
+                size = 0.5 * float(np.sqrt((((codes * wc).sum(1) * (scales * ws)) ** 2).sum()))
+                assert abs(got[r, j] - want) < 1e-4 * max(size, abs(want)), (r, j, got[r, j], want)
+    for t in [a_buf] + c_bufs:
+        t.free()
+    for _b, w in made:
+        w.free()
+
+
 # The matrix-pipe GEMV's lines on 256 CUs: the smallest K and its next stage, columns on either side, q8 past 300 M weights (from five
 # rows on). Below a line the vector-ALU rows kernel or the exact GEMM's kernel runs, under the name gemv_q*.
 @pytest.mark.parametrize("m,n,k,q4_mfma,q8_mfma", [(5, 65540, 1024, True, True), (8, 49153, 1280, True, False), (8, 49151, 1024, False, False),
