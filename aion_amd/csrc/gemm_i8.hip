@@ -156,6 +156,7 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN, LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, NT, KS, WGM, WGN, RQ>();
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
+    static_assert((uint64_t)32 * NT * GEMM_I8_MAX_K <= (uint64_t)1 << 32, "a lane's weight offset and the group's behind it fit 32 bits");
     if (LDS > 64 * 1024) {
         static std::atomic<uint64_t> attr{0};                // devices (by number, of the first 64) that have it; per instance
         const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;

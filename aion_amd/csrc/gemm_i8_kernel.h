@@ -4,9 +4,10 @@
 // acc += f32(dot) * (a_scale * w_scale), three operations per output per block, and that is the bound: 48 vector instructions behind
 // a 32-cycle MFMA. What the parts cost on gfx950, alone in a loop: multiply, multiply-add 1.1 ns per wavefront instruction with
 // four wavefronts on the SIMD but 2.0 .. 2.3 ns with one, conversion 1.8 ns; the MFMA 13.5 ns; the whole rescale of a tile 60 ns per
-// SIMD with two wavefronts and 115 with one. So the shape of this kernel: at least two wavefronts per SIMD at every size, and nothing that
-// makes them wait for each other. A wavefront owns a (32 MT) x (32 NT) tile and a share of K (every KS-th group of four blocks); the KS
-// wavefronts of a tile meet once, at the end, in LDS, in a fixed order. No barrier in the loop: what a wavefront stages, it stages for itself.
+// SIMD with two wavefronts and 115 with one. So the shape of this kernel: wavefronts that never wait for each other, two or more per SIMD
+// as soon as there are two workgroups per CU (a grid of at most one runs one per SIMD, q4 from K = 2048 on two: eight wavefronts to a
+// workgroup). A wavefront owns a (32 MT) x (32 NT) tile and a share of K (every KS-th group of four blocks); the KS wavefronts of a tile
+// meet once, at the end, in LDS, in a fixed order. No barrier in the loop: what a wavefront stages, it stages for itself.
 //   activations: prepared in operand order, a wavefront's load of a block is 1 KiB of consecutive memory, straight to registers, three blocks
 //     ahead
 //   weights and activation scales: LDS-writing buffer loads, a group of four blocks ahead. The row-major weight puts a lane's operand bytes
@@ -16,6 +17,8 @@
 // Other forms measured: f16 codes on v_mfma_f32_32x32x16_f16 (no conversion after the dot, 51 ns a tile, but the codes have to be
 // converted and the operands are twice the bytes), scale products as 4x4x1 outer products on the matrix pipe (82 ns), activation scales by
 // DPP broadcast (90 ns), an integer bias in place of the conversion (62 ns).
+// RQ: of a tile's 32 rows the first 8 RQ are kept (2: calls of up to 16 rows, half the rescale; 131072 x 512 at 9 rows q4 22.7 -> 20.3 us).
+// WHOLE: K is a multiple of 128, see the launcher.
 // Measured (whole calls, weights straight from memory -> staged): q8 8 x 14336 x 4096 19.3 -> 15.5 us, 2048 x 14336 x 4096 429 -> 384,
 // 512 x 4096 x 4096 41.3 -> 37.0; q4 374 -> 366, 36.8 -> 36.0, 128 x 2048 x 8192 15.5 -> 14.8 us (q4 asks for half the bytes). What is left is
 // the vector ALU: 52 instructions a tile and block at 3.6 cycles each.

@@ -62,8 +62,9 @@ static bool fused_row_pays(const Batch &b) {
 }
 
 // Prepared rows against the weights of `b`: the GEMV kernels up to eight rows, except five to eight rows over a K past 4096,
-// where the GEMV walks K with all eight accumulator sets live and falls far behind the exact GEMM's 16-row tile (q8
-// 14336 x 8192 at 8 rows: 80 against 33 us, q4 65 against 29; the two meet at K = 4096 ... 5120); the GEMM beyond eight rows.
+// where the GEMV walks K with all eight accumulator sets live and falls far behind the exact GEMM (8 x 14336 x 8192: q8 78 against 31 us,
+// q4 65 against 25; 8 x 6144 x 4128 20 / 15, 18 / 11; q8 up to 4096 columns is level there or, below 3072, up to a fifth ahead on the
+// GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2); the GEMM beyond eight rows.
 static bool rows_on_gemv(const Batch &b, size_t m) { return m <= GEMV_MAX_M && (b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)); }
 // which form of the preparation the kernel behind launch_prepared_rows reads
 static bool rows_tiled(const aionhip_ctx *ctx, const Batch &b, size_t m) {

@@ -337,8 +337,8 @@ def run_gemm_headline(gpu, be):
              "f32-activation oracle, NMSE <= 1e-4 vs aion's int8-activation CPU path)"),
             (be.GEMM_EXACT_I8, "gemm_i8_q4", "int8", "exact_i8",
              "aion's arithmetic (int8 activations per 32-block, exact i32 block dots, f32 scale-accumulate): tolerance class 2e-3, "
-             "observed 1e-6. The parity path, not the throughput path: both operands carry a scale per 32-block, so every 16x16x32 "
-             "MFMA is followed by 12 VALU instructions of rescaling, which bounds it near 15 % of the int8 peak")):
+             "observed 1e-6. The parity path, not the throughput path: both operands carry a scale per 32-block, so every 32x32x32 "
+             "MFMA is followed by 48 VALU instructions of rescaling, which bounds it near 15 % of the int8 peak")):
         gpu.set_gemm_mode(mode)
         gpu.step_matmul(w, x, m, y)
         settle(gpu, lambda i: gpu.step_matmul(w, x, m, y))
@@ -464,7 +464,7 @@ def run_sweep(gpu, be, q4_blocks):
             for m in (1, 4, 8):
                 x = gpu.upload(rng.standard_normal((m, k)).astype(np.float32))
                 y = gpu.alloc(m * n * 4)
-                # five to eight rows over a K past 4096 run on the exact GEMM's 16-row tile, everything else on a GEMV kernel
+                # five to eight rows over a K past 4096 run on the exact GEMM, everything else under a GEMV kernel's name
                 ms = time_kernel(gpu, ws, x, y, m, (kname, "gemm_i8_" + kname[-2:]) if m >= 5 and k > 4096 else kname)
                 by = algorithmic_bytes(bb, n, k, m)
                 ll = gpu.last_launch()

@@ -2,7 +2,7 @@
 against the CPU oracle - and the persistent row-group loop of every one-row kernel variant on cheap shapes.
 
 This shape is where the one-row kernel runs its largest grid (8192 workgroups), the 2..4-row kernel its persistent grid, and
-where 5..8 rows run on the 16-row tile of the exact GEMM at a size no other test reaches. The loop in which a wavefront
+where 5..8 rows run on the matrix-pipe GEMV at a size no other test reaches. The loop in which a wavefront
 walks several row groups (`gwave += wave_stride`, new row addresses, new first loads) starts beyond the grid caps: the
 second test enters it with every prologue variant on weights that are long but thin.
 Bar: max|err| <= 1e-5 * rms(ref) and the 2e-3 elementwise bound (floored), as for every exact-integer-dot kernel.
