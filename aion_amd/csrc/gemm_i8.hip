@@ -128,12 +128,18 @@ int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, in
 //                 16 x 2048 x 14336: 11.8 against 15.0; q8, twice the bytes a tile, from K = 6144 and up to half a tile per CU on:
 //                 16 x 2048 x 6144 14.9 -> 12.4 us, 16 x 4096 x 8192 20.2 -> 17.1, 16 x 3072 x 11008 25.3 -> 18.8; past K = 11008 up to
 //                 three quarters: 16 x 6144 x 11008 28.8 -> 26.6, 64 x 3072 x 14336 31.1 -> 28.7)
+//   3, 2 slices:  up to 32 rows against a little more than one tile per CU, where a few CUs have two and the rest wait (up to five quarters:
+//                 8 x 9664 x 14336 q4 37.1 -> 31.9 us, q8 48.1 -> 40.9, 16 x 9664 x 8192 25.1 -> 23.6, 30.1 -> 28.6; up to six quarters 16 x 11008 x
+//                 11008 33.1 -> 30.8, 42.8 -> 38.9, x 8192 level; at two tiles per CU slices cost 7 % and more)
 KSplit k_split(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
     const size_t cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256, blocks = k / QK;
     const size_t small = ((m + 31) / 32) * ((n + 31) / 32), large = ((m + 127) / 128) * ((n + 63) / 64);
     const bool sliced = dtype == AIONHIP_Q4_0 ? (blocks >= 256 && small <= cus / 4) || (blocks >= 448 && small <= cus / 2)
                                               : (blocks >= 192 && small <= cus / 2) || (blocks >= 344 && small <= cus * 3 / 4);
-    const int slices = !ctx->no_scratch_paths && sliced ? 4 : 1;
+    const bool uneven = m <= 32 && small > cus;
+    const int slices = ctx->no_scratch_paths ? 1 : sliced ? 4
+                       : uneven && small * 4 <= cus * 5 && blocks >= (dtype == AIONHIP_Q4_0 ? 256 : 204) ? 3
+                       : uneven && small * 2 <= cus * 3 && blocks >= 344 ? 2 : 1;
     KSplit split{dtype == AIONHIP_Q4_0 && blocks >= 64 && small <= cus ? 8 : m >= 1024 && large >= 2 * cus ? 2 : 4, slices, false};
     if (blocks > SHORT_BLOCKS) return split;
     const I8Fit *fits = I8_FITS[m > 16 ? 1 : 2][dtype == AIONHIP_Q8_0];

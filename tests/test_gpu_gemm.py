@@ -339,10 +339,12 @@ def test_exact_gemm_lowest_activations(gpu, orc, dtype, layout, m, n, k):
 
 
 # Division of a long K over workgroups: either side of the lines (K = 6144, half a 32 x 32 tile per CU; K = 11008, three quarters; q4 8192 and
-# a quarter), seen as the second launch that adds the slices. Tolerance as in test_exact_gemm_tiles_and_k_divisions: 3e-5 at K = 11008.
+# a quarter; up to 32 rows five quarters from K = 6528, q4 8192, and six from 11008), seen as the second launch that adds the slices. Tolerance as in test_exact_gemm_tiles_and_k_divisions: 3e-5 at K = 11008.
 @pytest.mark.parametrize("m,n,k,q8_sliced,q4_sliced", [(9, 4096, 6144, True, False), (9, 4097, 6144, False, False), (16, 2048, 6112, False, False),
                                                        (33, 2050, 8192, False, False), (40, 1024, 8192, True, True), (10, 6144, 11008, True, False),
-                                                       (10, 6145, 11008, False, False)])
+                                                       (10, 6145, 11008, False, False), (9, 9664, 11008, True, True), (9, 9665, 6528, True, False),
+                                                       (32, 10240, 6496, False, False), (9, 12288, 11008, True, True), (9, 12289, 11008, False, False),
+                                                       (33, 4900, 11008, False, False)])
 def test_exact_gemm_k_slices(gpu, orc, m, n, k, q8_sliced, q4_sliced):
     for dtype, layout, sliced in ((be.Q8_0, be.ROWS_NK, q8_sliced), (be.Q4_0, be.KMAJOR_KN, q4_sliced)):
         say("slices", dtype, m, n, k)
