@@ -20,8 +20,9 @@
 // RQ: of a tile's 32 rows the first 8 RQ are kept (2: calls of up to 16 rows, half the rescale; 131072 x 512 at 9 rows q4 22.7 -> 20.3 us).
 // WHOLE: K is a multiple of 128, see the launcher.
 // Measured (whole calls, weights straight from memory -> staged): q8 8 x 14336 x 4096 19.3 -> 15.5 us, 2048 x 14336 x 4096 429 -> 384,
-// 512 x 4096 x 4096 41.3 -> 37.0; q4 374 -> 366, 36.8 -> 36.0, 128 x 2048 x 8192 15.5 -> 14.8 us (q4 asks for half the bytes). What is left is
-// the vector ALU: 52 instructions a tile and block at 3.6 cycles each.
+// 512 x 4096 x 4096 41.3 -> 37.0; q4 374 -> 366, 36.8 -> 36.0, 128 x 2048 x 8192 15.5 -> 14.8 us (q4 asks for half the bytes). Since K of whole groups
+// runs without checks: 2048 x 14336 x 4096 q8 368, q4 350, 8 x 14336 x 4096 14.4 us. What is left is
+// the vector ALU: 53 .. 57 instructions a tile and block at 2048 rows, at four cycles each 97 % of the launch.
 #pragma once
 #include "common.h"
 
