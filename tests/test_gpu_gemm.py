@@ -318,6 +318,27 @@ def test_exact_gemm_infinite_activations(gpu, orc, dtype, layout, m, n, k):
     w.free()
 
 
+# The same with an infinite block in each place of K in turn, a row for each: whatever a wavefront's buffers held two groups earlier, the
+# blocks that a last group has past the end of K (one to three here) multiply as zero.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("n,k", [(64, 544), (96, 1120), (40, 2080), (4096, 992), (33, 4000)])
+def test_exact_gemm_infinite_block_anywhere(gpu, dtype, layout, n, k):
+    say("inf anywhere", dtype, layout, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    _, w = make_weight(gpu, dtype, layout, n, k, seed=n + k)
+    m = k // 32
+    one = np.zeros((m, k), np.float32)
+    one[np.arange(m), np.arange(m) * 32 + 9] = 1
+    a = np.random.default_rng(k).standard_normal((m, k)).astype(np.float32)
+    a[one == 1] = np.inf
+    for rows in (m, 12):                             # (the last rows: the last blocks of K)
+        sign = np.sign(gpu.matmul(w, one[-rows:]))
+        got = gpu.matmul(w, a[-rows:])
+        assert "gemm_i8" in gpu.last_launch()["kernel"]
+        assert np.array_equal(got, np.where(sign == 0, np.nan, np.where(sign > 0, -np.inf, np.inf)), equal_nan=True), rows
+    w.free()
+
+
 # Sums stay finite up to the f32 range: the lowest f32, as a mask leaves it, in four blocks of a row gives sums of 1e37 .. 1e38. Beside it
 # rows of ordinary values. (test_gpu_prepare_act.py holds the other end: products of subnormal scales keep their bits.)
 @pytest.mark.parametrize("dtype,layout", CASES)
