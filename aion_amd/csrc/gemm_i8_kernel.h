@@ -1,10 +1,15 @@
 // The exact GEMM's kernel (see gemm_i8.hip for the launcher and the choice of shapes).
 //
-// v_mfma_i32_32x32x32_i8: the 32 of K are one quant block, so the i32 tile is the exact block dot; the vector ALU then does
-// acc += f32(dot) * (a_scale * w_scale), three operations per output per block, and that is the bound: 48 vector instructions behind
-// a 32-cycle MFMA. What the parts cost on gfx950, alone in a loop: multiply, multiply-add 1.1 ns per wavefront instruction with
-// four wavefronts on the SIMD but 2.0 .. 2.3 ns with one, conversion 1.8 ns; the MFMA 13.5 ns; the whole rescale of a tile 60 ns per
-// SIMD with two wavefronts and 115 with one. So the shape of this kernel: wavefronts that never wait for each other, two or more per SIMD
+// v_mfma_i32_32x32x32_i8: the 32 of K are one quant block, so the i32 tile is the exact block dot; then
+// acc += f32(dot) * (a_scale * w_scale), three operations per output and block, and that is the bound. Of the three the vector ALU does
+// the conversion and the multiply-add; the products of scales come from v_mfma_f32_32x32x1_2b_f32, two tiles' outer products an instruction
+// (one product a term, rounded as v_mul_f32 rounds it: the same bits, subnormals and infinities included), except where a wavefront has one
+// tile or half of one. What the parts cost on gfx950: 48 vector instructions of a tile's rescale 52 ns a SIMD with four wavefronts on it, 57
+// with two, 94 with one; with the i8 MFMA (14 ns alone) in front 62, 69, 89: the two pipes hardly overlap once both are in demand. The
+// outer products cost 13.5 ns a tile, less than the 16 multiplies and four 16-byte LDS reads of a lane's 16 row scales that they replace (2 x 2
+// tiles: 2048 x 4096 x 4096 q4 112.5 -> 106.0 us, q8 116.8 -> 111.0; 512 x 4096 x 4096 35.5 -> 33.9, 37.6 -> 36.1; 2048 x 14336 x 512 63.4 -> 60.9, 66 ->
+// 61; 3 x 1 level; a lone tile, which takes them for two blocks at a time, loses 2 .. 4 %: 32 x 32768 x 2048, q8 64 x 4096 x 4096).
+// So the shape of this kernel: wavefronts that never wait for each other, two or more per SIMD
 // as soon as there are two workgroups per CU (a grid of at most one runs one per SIMD, q4 from K = 2048 on two: eight wavefronts to a
 // workgroup). A wavefront owns a (32 MT) x (32 NT) tile and a share of K (every KS-th group of four blocks); the KS wavefronts of a tile
 // meet once, at the end, in LDS, in a fixed order. No barrier in the loop: what a wavefront stages, it stages for itself.
@@ -13,16 +18,17 @@
 //   weights and activation scales: LDS-writing buffer loads, a group of four blocks ahead. The row-major weight puts a lane's operand bytes
 //     (its row's 16 of a block) far from its neighbours', and the L1 takes such a load lane by lane: 64 accesses, 60 .. 85 % of its cycles
 //     at 2048 x 14336 x 4096 when the operands came straight from memory. Staged, neighbouring lanes read a row's consecutive bytes: 16
-//     accesses, whole lines. The lanes take 16 rows' scales from there (4 reads per row tile and block)
+//     accesses, whole lines. The scales are read from there, one word a lane and block (a lone tile: 16 rows', 4 reads)
 // Other forms measured: f16 codes on v_mfma_f32_32x32x16_f16 (no conversion after the dot, 51 ns a tile, but the codes have to be
-// converted and the operands are twice the bytes), scale products as 4x4x1 outer products on the matrix pipe (82 ns), activation scales by
+// converted and the operands are twice the bytes), scale products as 4x4x1 outer products (82 ns) and as sums of bf16 parts (the sums of six products round up to 2 ulp off), codes as fp6 digits (exact dots
+// in f32, but what the conversion cost the unpacking of nibbles costs), activation scales by
 // DPP broadcast (90 ns), an integer bias in place of the conversion (62 ns).
 // RQ: of a tile's 32 rows the first 8 RQ are kept (2: calls of up to 16 rows, half the rescale; 131072 x 512 at 9 rows q4 22.7 -> 20.3 us).
 // WHOLE: K is a multiple of 128, see the launcher.
 // Measured (whole calls, weights straight from memory -> staged): q8 8 x 14336 x 4096 19.3 -> 15.5 us, 2048 x 14336 x 4096 429 -> 384,
 // 512 x 4096 x 4096 41.3 -> 37.0; q4 374 -> 366, 36.8 -> 36.0, 128 x 2048 x 8192 15.5 -> 14.8 us (q4 asks for half the bytes). Since K of whole groups
-// runs without checks: 2048 x 14336 x 4096 q8 368, q4 350, 8 x 14336 x 4096 14.4 us. What is left is
-// the vector ALU: 53 .. 57 instructions a tile and block at 2048 rows, at four cycles each 97 % of the launch.
+// runs without checks: 8 x 14336 x 4096 14.4 us. What is left is the vector ALU, 37 .. 41 instructions a tile and block at 2048 rows, and what the loads
+// take beside it: with neither loads nor LDS reads in the loop 512 x 4096 x 4096 took 25 of 35 us.
 #pragma once
 #include "common.h"
 
@@ -32,6 +38,7 @@ using i32x2 = __attribute__((ext_vector_type(2))) int;
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 using i32x16 = __attribute__((ext_vector_type(16))) int;
 using f32x16 = __attribute__((ext_vector_type(16))) float;
+using f32x32 = __attribute__((ext_vector_type(32))) float;
 
 // up to four weights with the same K and block format against one prepared activation: column tiles first_tile[i] .. of weight i
 struct GemmSegs {
@@ -57,6 +64,8 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
+    constexpr bool OUTER = RQ == 4 && MT * NT > 1;        // scale products from the matrix pipe
+    static_assert(OUTER || MT == 1, "one row tile");
     static_assert(RQ == 4 || MT * WGM == 1, "fewer rows than a tile: one row tile");
     using Acc = __attribute__((ext_vector_type(4 * RQ))) float;
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
@@ -193,6 +202,16 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                 sa[i][4 * q] = v.x; sa[i][4 * q + 1] = v.y; sa[i][4 * q + 2] = v.z; sa[i][4 * q + 3] = v.w;
             }
         };
+        // Scale products from the matrix pipe: v_mfma_f32_32x32x1_2b gives the products of two 32 x 32 tiles, here neighbouring tiles of a block
+        // or, of an odd tile, two blocks. Lane half h holds the rows' scales of the pair's tile (or block) h.
+        constexpr int PAIRS = MT * NT / 2;
+        constexpr bool ODD = (MT * NT) % 2 == 1;
+        float sp = 0.f, sp_odd = 0.f;
+        auto read_sp = [&](int buf, int j) {
+            if constexpr (PAIRS > 0) sp = sa_lds[(buf * MT + (MT > 1 ? h : 0)) * 128 + j * 32 + r];
+            if constexpr (ODD)
+                if (j % 2 == 0) sp_odd = sa_lds[(buf * MT + MT - 1) * 128 + (j + h) * 32 + r];
+        };
         // Blocks past the end of K in the last group: activation scale 0 as well as weight scale 0, where a real block's infinite scale
         // would make a NaN of the product. Called as the group begins: its loads have landed, and what has been read ahead is its first
         // block's. (Writes in every group, all but the last to words nobody reads, in place of the branch: 1 % slower.)
@@ -221,8 +240,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
             asm volatile("" ::: "memory");
             read_b(0, 0);
-#pragma unroll
-            for (int i = 0; i < MT - 1; ++i) read_sa(i, 0, 0);
+            if constexpr (OUTER) read_sp(0, 0);
         }
 #pragma unroll
         for (int e = 0; e < 4 * RQ; ++e) sa[MT - 1][e] = 0.f;      // the first rescale has no block behind it: 0 * 0, and no real block's scale
@@ -231,23 +249,31 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         float sw_due = 0.f;
         for (; g < g_hi; g += KS) {
             const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
-            float sw[4][NT];
+            constexpr int SW = OUTER ? 1 : NT;           // (a lane's own column is what a pair of column tiles wants of it)
+            float sw[4][SW];
+            [[maybe_unused]] float sw_odd[2];
             {
                 const unsigned long v = sw_now >> sw_shift_now;
                 unsigned lo[2], hi[2];
-                if constexpr (NT == 2) {
+                if constexpr (SW == 2) {
                     const auto x = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
                     const auto y = __builtin_amdgcn_permlane32_swap((unsigned)(v >> 32), (unsigned)(v >> 32), false, false);
                     lo[0] = x[0]; lo[1] = x[1]; hi[0] = y[0]; hi[1] = y[1];
                 } else {
                     lo[0] = (unsigned)v; hi[0] = (unsigned)(v >> 32);
                 }
+                auto scale = [&](unsigned bits) { return code_scale * __half2float(__ushort_as_half((unsigned short)bits)); };
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
 #pragma unroll
-                    for (int i = 0; i < NT; ++i)
-                        sw[j][i] = WHOLE || g * 4 + j < KB ? code_scale * __half2float(__ushort_as_half((unsigned short)((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))))) : 0.f;
+                    for (int i = 0; i < SW; ++i)
+                        sw[j][i] = WHOLE || g * 4 + j < KB ? scale((j < 2 ? lo[i] : hi[i]) >> (16 * (j & 1))) : 0.f;
+                if constexpr (OUTER && ODD) {
+                    sw_odd[0] = WHOLE || g * 4 + h < KB ? scale(lo[0] >> (16 * h)) : 0.f;
+                    sw_odd[1] = WHOLE || g * 4 + 2 + h < KB ? scale(hi[0] >> (16 * h)) : 0.f;
+                }
             }
+            [[maybe_unused]] f32x32 s_odd;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 // The other buffer was last read in the previous group (those reads have returned once lgkmcnt is 0); its loads have three
@@ -259,6 +285,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                     __builtin_amdgcn_s_waitcnt(LGKM0);
                     __builtin_amdgcn_sched_barrier(0);
                     clear_tail(g, buf);
+                    if constexpr (OUTER && ODD && !WHOLE) read_sp(buf, 0);       // (its second block may be past the end)
                     load_w(gn, buf ^ 1);
                     load_scales(gn, buf ^ 1);
                 }
@@ -281,6 +308,33 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                     }
                 }
                 read_b(j == 3 ? buf ^ 1 : buf, (j + 1) & 3);
+                if constexpr (OUTER) {
+                    f32x32 zero;
+#pragma unroll
+                    for (int e = 0; e < 32; ++e) zero[e] = 0.f;
+                    const float sp_now = sp, sp_odd_now = sp_odd;
+                    read_sp(j == 3 ? buf ^ 1 : buf, (j + 1) & 3);
+                    auto dot = [&](int tl) { return __builtin_amdgcn_mfma_i32_32x32x32_i8(A[j][tl / NT], B[tl % NT], i32x16{0}, 0, 0, 0); };
+#pragma unroll
+                    for (int p = 0; p < PAIRS; ++p) {
+                        const int t0 = 2 * p, t1 = 2 * p + 1;
+                        // (2 x 2 tiles: the rows of tile p for both)
+                        const f32x32 s = MT * NT < 4 ? __builtin_amdgcn_mfma_f32_32x32x1f32(sp_now, sw[j][0], zero, 0, 0, 0)
+                                         : p == 0    ? __builtin_amdgcn_mfma_f32_32x32x1f32(sp_now, sw[j][0], zero, 1, 0, 0)
+                                                     : __builtin_amdgcn_mfma_f32_32x32x1f32(sp_now, sw[j][0], zero, 1, 1, 0);
+                        const i32x16 d0 = dot(t0), d1 = dot(t1);
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[t0 / NT][t0 % NT][e] += (float)d0[e] * s[e];
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[t1 / NT][t1 % NT][e] += (float)d1[e] * s[16 + e];
+                    }
+                    if constexpr (ODD) {
+                        if (j % 2 == 0) s_odd = __builtin_amdgcn_mfma_f32_32x32x1f32(sp_odd_now, sw_odd[j / 2], zero, 0, 0, 0);
+                        const i32x16 d0 = dot(MT * NT - 1);
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) acc[MT - 1][NT - 1][e] += (float)d0[e] * s_odd[(j & 1) * 16 + e];
+                    }
+                } else {
                 // a tile's dots are issued ahead of the previous tile's rescale (the last tile's is left to the next block); the empty
                 // asm statements keep that order. A row tile's scales of the next block are read once the block's last use of them is past.
 #pragma unroll
@@ -295,6 +349,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                     d = dn;
                 }
                 sw_due = sw[j][NT - 1];
+                }
             }
             buf ^= 1;
             sw_now = sw_raw;
@@ -302,9 +357,10 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         }
         __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));            // no LDS-writing load may outlive the loop: its LDS is reused, or another workgroup's
         // the last block's last tile (a wavefront without a group has none)
-        if (g_lo + ks < g_hi)
+        if constexpr (!OUTER)
+            if (g_lo + ks < g_hi)
 #pragma unroll
-            for (int e = 0; e < 4 * RQ; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
+                for (int e = 0; e < 4 * RQ; ++e) acc[MT - 1][NT - 1][e] += (float)d[e] * (sa[MT - 1][e] * sw_due);
 
         if constexpr (Q8) break;
         if (code_scale != 1.f) break;

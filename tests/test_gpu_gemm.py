@@ -397,3 +397,26 @@ def test_exact_gemm_short_k_wide_grid(gpu, orc, dtype, layout, m, n, k, most):
     again = gpu.matmul(w, a)
     assert np.array_equal(got.view(np.uint32), again.view(np.uint32))
     w.free()
+
+
+# Wavefronts of more than one tile take the products of scales from the matrix pipe, calls of up to 16 rows multiply. With one block of a row's K
+# that is not zero a sum is one rounded product, so every row has the bits that it has in a call of 12: row scales from 2^-100 to 2^40 beside
+# each other, column tiles and row tiles with ends, every place of K.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(512, 4096, 2048), (500, 4070, 2080), (1030, 8200, 1024), (77, 11008, 672), (300, 5000, 1056), (700, 14330, 544),
+                                   (90, 2100, 4096), (24, 32800, 2048), (24, 32800, 4128)])
+def test_exact_gemm_scale_products_keep_their_bits(gpu, orc, dtype, layout, m, n, k):
+    say("scale products", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    _, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    rng = np.random.default_rng(k)
+    a = np.zeros((m, k // 32, 32), np.float32)
+    at = np.arange(m) * 7 % (k // 32)
+    a[np.arange(m), at] = rng.standard_normal((m, 32)) * 2.0 ** rng.integers(-100, 41, (m, 1))
+    a = a.reshape(m, k)
+    got = gpu.matmul(w, a)
+    assert "gemm_i8" in gpu.last_launch()["kernel"]
+    for rows in ([0, 1, m // 2, m - 1, *rng.integers(0, m, 8)], rng.integers(0, m, 12)):
+        assert np.array_equal(got[rows].view(np.uint32), gpu.matmul(w, a[rows]).view(np.uint32)), rows
+        assert "gemm_i8" in gpu.last_launch()["kernel"]
+    w.free()
