@@ -195,8 +195,11 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
     // Tiles are dealt out in groups of eight row tiles (256 .. 1024 rows), columns within: the activation rows and weight columns that run on an XCD
     // at the same time then fit its L2 (2048 x 14336 x 4096, 64 x 64 tiles: 409 -> 387 us for q4, 524 -> 465 for q8).
     const int row_group = row_tiles < 8 ? row_tiles : 8;
+    // All workgroups at once, two per CU at most: wavefronts give way to those behind them, see the kernel (128 x 16384 x 2048 q4 22.0 -> 21.3 us, q8
+    // 24.2 -> 23.1; q8 512 x 4096 x 4096 35.9 -> 35.0, 256 x 4096 x 4096 23.4 -> 22.8; 48 x 9000 x 2080 q4 14.8 -> 13.9).
+    const int one_round = (size_t)tiles * row_tiles * slices <= 2 * (size_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
     launch_k(ctx, gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, dim3((unsigned)(tiles * row_tiles), 1, (unsigned)slices), dim3(64 * KS * WGM * WGN), LDS, segs,
-             (const uint8_t *)act.q, (const float *)act.scale, (int)m, (int)ws[0]->k, row_tiles, row_group, tiles, alpha, beta, partial, partial_ld);
+             (const uint8_t *)act.q, (const float *)act.scale, (int)m, (int)ws[0]->k, row_tiles, row_group, tiles, one_round, alpha, beta, partial, partial_ld);
     if (slices > 1) {
         const size_t threads = m * (size_t)(partial_ld >> 2);
         launch_k(ctx, gemm_i8_slices_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, segs, partial, (int)m, slices, partial_ld, BN, alpha, beta);

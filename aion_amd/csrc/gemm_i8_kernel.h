@@ -60,7 +60,7 @@ template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wav
 
 template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE>
 __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
-                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, float alpha, float beta,
+                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
@@ -247,7 +247,17 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         int buf = 0;
         i32x16 d = i32x16{0};                      // the dots whose rescale is due: tile (MT - 1, NT - 1) of the previous block
         float sw_due = 0.f;
+        // Of two wavefronts on a SIMD the older goes first wherever both could, ends a quarter of its time ahead and leaves the other to run alone,
+        // at little more than half the SIMD's rate (512 x 4096 x 4096: workgroups end between 19 and 25 us). So a wavefront's priority falls as it
+        // proceeds. Where more workgroups follow that would hold up the ones about to end: 2048 x 14336 x 512 q8 61.2 -> 66.7 us.
+        const int quarter = (g_hi - g + 4 * KS - 1) / (4 * KS) * KS, second = g + quarter, third = second + quarter, fourth = third + quarter;
+        if (MT * NT > 1 && one_round) __builtin_amdgcn_s_setprio(3);
         for (; g < g_hi; g += KS) {
+            if (MT * NT > 1 && one_round) {
+                if (g == second) __builtin_amdgcn_s_setprio(2);
+                if (g == third) __builtin_amdgcn_s_setprio(1);
+                if (g == fourth) __builtin_amdgcn_s_setprio(0);
+            }
             const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
             constexpr int SW = OUTER ? 1 : NT;           // (a lane's own column is what a pair of column tiles wants of it)
             float sw[4][SW];
