@@ -44,39 +44,43 @@ struct KSplit {
 // The workgroup shapes, and a model of their times: t = t0 + (blocks + e) * us * max(1, b * ((1 - q) * r + q * whole)), where r is the
 // workgroups per CU and `whole` the same in whole rounds of `resident` workgroups per CU - a lone workgroup costs us per quant
 // block of K, a filled device b * us per workgroup and CU, and what a tile costs beside its K counts as e blocks. Three sets of constants
-// per block format (no t0: not a shape of that set):
-//   [0]  launches alone, from a sweep of 5 .. 2048 rows x N = 1024 .. 32768 x K = 1024 .. 14336 (rms 4 .. 11 % a shape); the tiles whose K
-//        is shared as far as it pays for a long K are chosen by it
-//   [1]  whole calls of more than 16 rows, up to 2048, x N = 1024 .. 131072 x K = 512, 1056, 2048 (rms 8 %); [2] the same up to 16 rows.
-//        They weigh those tiles against wide tiles whose wavefronts share K less (the last four shapes): at a short K a tile's start
-//        and end weigh as much as its K, and these halve them. 512 x 32768 x 512 q4 61.9 -> 42.9 us with 128 x 128 tiles, 512 x 131072 x
-//        1056 q8 386 -> 280; 8 x 131072 x 512 q8 26.3 -> 20.5 with 32 x 256.
+// per block format (no t0: not a shape of that set), all of whole calls:
+//   [0]  K past SHORT_BLOCKS, from a sweep of every shape over 17 .. 2048 rows x N = 1024 .. 32768 x K = 4096 .. 14336 (rms 3 .. 10 % a shape); the
+//        tiles whose K is shared as far as it pays for a long K are chosen by it
+//   [1]  a shorter K, the same rows and columns x K = 512, 1056, 2048 (rms 6 .. 9 %); [2] up to 16 rows x N = 1024 .. 131072. Here those tiles are
+//        weighed against wide tiles whose wavefronts share K less as well: at a short K a tile's start and end weigh as much as its K, and
+//        these halve them. 512 x 32768 x 512 q4 61.9 -> 42.9 us with 128 x 128 tiles, 512 x 131072 x 1056 q8 386 -> 280; 8 x 131072 x 512 q8
+//        26.3 -> 20.5 with 32 x 256.
+// Choosing by them costs 0.9 % over the fastest shape of each of the 1806 measured cells. The constants before these were fitted to the kernel that
+// multiplied its scales on the vector ALU and did not weigh 32 x 64 tiles past 32 rows, three wavefronts to a SIMD now: 2.4 %, 356 cells more than 3 %
+// slower and 31 faster (160 x 6144 x 14336 q4 69.3 -> 52.5 us, 160 x 22016 x 2048 39.8 -> 31.7, q8 41.5 -> 33.8; 700 x 11008 x 512 q8 31.0 -> 24.6).
 struct I8Shape {
     int bm, bn, ks;
 };
 constexpr I8Shape I8_SHAPES[] = {
     {32, 32, 8}, {32, 32, 4}, {64, 32, 4}, {96, 32, 4}, {64, 64, 4}, {128, 64, 2}, {32, 64, 2}, {128, 128, 1}, {32, 128, 2}, {32, 256, 1}, {32, 64, 4},
 };
-constexpr int I8_COUNT = 10;                     // (shapes that the model chooses from)
-constexpr int I8_WIDE4 = 10;                     // see pick_shape
+constexpr int I8_COUNT = 11;
+constexpr int I8_LONE4 = 1, I8_WIDE4 = 10;       // see pick_shape
 struct I8Fit {
     int resident;
     float t0, us, b, q, e;
 };
 constexpr size_t SHORT_BLOCKS = 80;              // between the measured K = 2080 and 4096
 constexpr I8Fit I8_FITS[3][2][I8_COUNT] = {      // [set][q4_0, q8_0][shape]
-    {{{2, 3.43f, 0.0300f, 1.446f, 0.00f, 0.f}, {4, 3.12f, 0.0437f, 0.903f, 0.07f, 0.f}, {3, 3.61f, 0.0709f, 0.858f, 0.15f, 0.f},
-      {2, 4.03f, 0.1034f, 0.938f, 0.16f, 0.f}, {2, 4.32f, 0.1240f, 0.941f, 0.28f, 0.f}, {2, 5.71f, 0.2479f, 0.875f, 0.27f, 0.f}},
-     {{}, {4, 2.85f, 0.0449f, 1.213f, 0.05f, 0.f}, {3, 3.54f, 0.0686f, 1.082f, 0.10f, 0.f},
-      {2, 4.01f, 0.0993f, 1.082f, 0.07f, 0.f}, {2, 4.41f, 0.1187f, 1.135f, 0.18f, 0.f}, {2, 5.61f, 0.2357f, 1.050f, 0.10f, 0.f}}},
-    {{{1, 5.15f, 0.0330f, 1.156f, 0.67f, 26.2f}, {1, 5.34f, 0.0486f, 0.738f, 0.87f, 12.5f}, {3, 5.52f, 0.0721f, 0.785f, 0.29f, 16.6f},
-      {2, 5.45f, 0.1022f, 0.852f, 0.44f, 19.4f}, {1, 6.13f, 0.1308f, 0.811f, 0.68f, 17.7f}, {1, 7.01f, 0.2614f, 0.764f, 0.75f, 11.8f},
-      {4, 5.21f, 0.0998f, 0.743f, 0.24f, 6.9f}, {1, 5.78f, 0.5707f, 0.696f, 0.77f, 7.6f}, {3, 5.45f, 0.1580f, 0.794f, 0.32f, 8.8f},
-      {3, 3.18f, 0.3581f, 0.894f, 0.29f, 8.5f}},
-     {{}, {4, 5.24f, 0.0503f, 0.843f, 0.22f, 9.2f}, {3, 5.82f, 0.0739f, 0.878f, 0.24f, 12.7f},
-      {1, 5.70f, 0.1183f, 0.847f, 0.68f, 15.f}, {1, 6.23f, 0.1498f, 0.824f, 0.72f, 13.5f}, {4, 5.57f, 0.2778f, 0.743f, 0.17f, 12.9f},
-      {3, 5.17f, 0.1094f, 0.892f, 0.31f, 3.3f}, {1, 5.45f, 0.5846f, 0.708f, 0.66f, 8.1f}, {3, 4.42f, 0.1938f, 0.838f, 0.25f, 10.5f},
-      {4, 5.27f, 0.3547f, 1.232f, 0.14f, 3.2f}}},
+    {{{2, 5.43f, 0.0300f, 1.446f, 0.00f, 0.f}, {1, 6.60f, 0.0435f, 0.709f, 0.82f, 0.0f}, {1, 7.06f, 0.0659f, 0.777f, 0.69f, 0.1f},
+      {1, 5.95f, 0.0957f, 0.765f, 0.78f, 15.8f}, {1, 6.93f, 0.1099f, 0.832f, 0.74f, 10.9f}, {1, 10.00f, 0.2451f, 0.755f, 0.75f, 3.2f}, {}, {}, {}, {},
+      {1, 7.15f, 0.0648f, 0.802f, 0.76f, 0.8f}},
+     {{}, {1, 6.38f, 0.0418f, 0.820f, 0.96f, 0.0f}, {1, 6.85f, 0.0647f, 0.853f, 0.74f, 0.0f}, {1, 6.35f, 0.0937f, 0.837f, 0.68f, 8.1f},
+      {1, 7.58f, 0.1109f, 0.877f, 0.67f, 5.2f}, {1, 10.00f, 0.2428f, 0.773f, 0.66f, 2.9f}, {}, {}, {}, {}, {1, 6.81f, 0.0645f, 0.910f, 0.78f, 0.6f}}},
+    {{{1, 5.15f, 0.0330f, 1.156f, 0.67f, 26.2f}, {1, 6.03f, 0.0388f, 0.769f, 0.79f, 14.4f}, {1, 6.06f, 0.0633f, 0.805f, 0.71f, 15.7f},
+      {1, 5.56f, 0.0962f, 0.791f, 0.84f, 21.5f}, {1, 5.71f, 0.1124f, 0.832f, 0.77f, 20.0f}, {1, 5.72f, 0.2286f, 0.805f, 0.82f, 13.0f},
+      {1, 6.20f, 0.0824f, 0.752f, 0.80f, 6.2f}, {1, 5.74f, 0.4557f, 0.827f, 0.82f, 6.7f}, {1, 6.57f, 0.1289f, 0.831f, 0.82f, 6.8f},
+      {1, 6.55f, 0.2661f, 0.834f, 0.78f, 3.3f}, {1, 6.08f, 0.0633f, 0.811f, 0.78f, 14.7f}},
+     {{}, {1, 6.24f, 0.0361f, 0.854f, 0.61f, 12.4f}, {1, 6.25f, 0.0629f, 0.847f, 0.61f, 14.3f}, {1, 5.69f, 0.0940f, 0.821f, 0.76f, 19.4f},
+      {2, 6.15f, 0.1091f, 0.910f, 0.39f, 16.4f}, {1, 5.89f, 0.2293f, 0.819f, 0.76f, 12.1f}, {1, 6.30f, 0.0771f, 0.842f, 0.65f, 4.4f},
+      {1, 5.31f, 0.4575f, 0.817f, 0.77f, 7.2f}, {1, 5.70f, 0.1319f, 0.848f, 0.79f, 12.0f}, {2, 6.34f, 0.2526f, 0.929f, 0.37f, 3.7f},
+      {2, 5.74f, 0.0612f, 0.896f, 0.38f, 21.3f}}},
     {{{1, 5.12f, 0.0264f, 1.467f, 0.50f, 17.f}, {4, 4.86f, 0.0426f, 0.818f, 0.24f, 10.3f}, {}, {}, {}, {}, {3, 4.99f, 0.0804f, 0.938f, 0.34f, 2.1f},
       {}, {4, 4.72f, 0.1529f, 0.933f, 0.11f, 4.6f}, {2, 5.18f, 0.2571f, 1.286f, 0.22f, 2.f}},
      {{}, {3, 5.10f, 0.0416f, 1.259f, 0.22f, 7.6f}, {}, {}, {}, {}, {3, 4.91f, 0.0829f, 1.253f, 0.25f, 4.1f},
@@ -94,9 +98,11 @@ float shape_us(const aionhip_ctx *ctx, int i, const I8Fit &f, size_t m, const si
     return f.t0 + (blocks + f.e) * f.us * fmaxf(1.f, f.b * ((1.f - f.q) * r + f.q * whole)) + (slices > 1 ? I8_SLICE_US : 0.f);
 }
 
+int fit_set(size_t m, size_t k) { return k / QK > SHORT_BLOCKS ? 0 : m > 16 ? 1 : 2; }
+
 // the fastest shape of a K split (-1: there is none) for m rows against weights of ns[0 .. count - 1] columns
 int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k, const KSplit &split, float *us) {
-    const I8Fit *fits = I8_FITS[!split.fewer ? 0 : m > 16 ? 1 : 2][dtype == AIONHIP_Q8_0];
+    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
     int best = -1;
     float best_us = 0.f;
     for (int i = 0; i < I8_COUNT; ++i) {
@@ -107,15 +113,16 @@ int pick_shape(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, in
             best_us = t;
         }
     }
-    if (us) *us = best_us;
-    // Few rows and three 32 x 32 tiles per CU or more: two of them to a wavefront, half the starts and ends and half the reads of the activation
-    // (16 x 32768 x 8192: q4 50.9 -> 46.1 us, q8 69.2 -> 61.0; x 4096 27.9 -> 25.9, 39.1 -> 36.0; x 2080 19.4 -> 18.4, 24.9 -> 23.9; level at two
-    // tiles per CU, and at K = 512).
-    if (best == 1 && (k / QK > SHORT_BLOCKS ? m <= 32 : m <= 16 && k >= 1024)) {
+    // Up to 16 rows the kernel keeps half of a tile, which the sets for more rows do not price. Three 32 x 32 tiles per CU or more: two of them to a
+    // wavefront, half the starts and ends and half the reads of the activation (16 x 32768 x 8192: q4 50.9 -> 46.1 us, q8 69.2 -> 61.0; x 4096 27.9 -> 25.9,
+    // 39.1 -> 36.0; x 2080 19.4 -> 18.4, 24.9 -> 23.9; level at two tiles per CU, and at K = 512).
+    if (m <= 16 && split.wavefronts == 4 && !split.fewer) {
         size_t tiles = 0;
         for (int w = 0; w < count; ++w) tiles += (ns[w] + 31) / 32;
-        if (tiles >= 3 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256)) best = I8_WIDE4;
+        best = k >= 1024 && tiles >= 3 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256) ? I8_WIDE4 : I8_LONE4;
+        best_us = shape_us(ctx, I8_LONE4, fits[I8_LONE4], m, ns, count, k, split.slices);
     }
+    if (us) *us = best_us;
     return best;
 }
 
@@ -142,7 +149,7 @@ KSplit k_split(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) 
                        : uneven && small * 2 <= cus * 3 && blocks >= 344 ? 2 : 1;
     KSplit split{dtype == AIONHIP_Q4_0 && blocks >= 64 && small <= cus ? 8 : m >= 1024 && large >= 2 * cus ? 2 : 4, slices, false};
     if (blocks > SHORT_BLOCKS) return split;
-    const I8Fit *fits = I8_FITS[m > 16 ? 1 : 2][dtype == AIONHIP_Q8_0];
+    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
     const int own = pick_shape(ctx, dtype, m, &n, 1, k, split, nullptr);
     if (fits[own].t0 == 0.f) return split;
     float best_us = 0.95f * shape_us(ctx, own, fits[own], m, &n, 1, k, 1);
@@ -277,9 +284,8 @@ int launch_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
 
 float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
     float us = 0.f;
-    const KSplit split = k_split(ctx, dtype, m, n, k);
-    pick_shape(ctx, dtype, m, &n, 1, k, split, &us);
-    return split.fewer ? us : us + 2.f;          // + the preparation's launch, which the first set of constants leaves out
+    pick_shape(ctx, dtype, m, &n, 1, k, k_split(ctx, dtype, m, n, k), &us);
+    return us;
 }
 
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {
