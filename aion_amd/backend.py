@@ -237,6 +237,17 @@ class HipBackend:
             self._ctx, w_gate.ptr, w_up.ptr, w_down.ptr, x.handle, gamma.handle, beta_norm.handle if beta_norm is not None else 0, eps,
             c_buf.handle, alpha, beta))
 
+    def step_rmsnorm_geglu_matmul_rows(self, w_gate, w_up, w_down, x, gamma, rows, eps, c_buf, alpha=1.0, beta=0.0, beta_norm=None):
+        """The same for many rows, three launches. False, with nothing issued, where the library wants the separate steps
+        (step_rmsnorm_matmul, step_gate_matmul) for these rows."""
+        rc = self._lib.aionhip_step_rmsnorm_geglu_matmul_rows(
+            self._ctx, w_gate.ptr, w_up.ptr, w_down.ptr, rows, x.handle, gamma.handle, beta_norm.handle if beta_norm is not None else 0, eps,
+            c_buf.handle, 0, alpha, beta)
+        if rc == hip.UNSUPPORTED:
+            return False
+        self._check(rc)
+        return True
+
     # ---- a run of decoder blocks as one launch (one new token of one sequence)
     def decoder_stack_create(self, layers, hidden, heads, kv_heads, head_dim, ffn, t_cap, eps1, eps2, attn_scale, rope_base=10000.0,
                              rope_scale=1.0, rope_proportion=1.0, soft_cap=0.0, window=CAUSAL, rolling=False):

@@ -257,6 +257,12 @@ int launch_gemm_i8_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, floa
                          PreparedAct act, float alpha, float beta);
 // the same kernel for a handful of rows (no profile scope of its own: the caller's name stays)
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
+// how the exact GEMM divides a K among a workgroup's wavefronts (false: it is also cut into slices), and whether four of them to a tile of two
+// weights' columns are better given 64 rows than 32
+bool gemm_i8_pair_plan(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts, bool *tall);
+// gate and up projections of m prepared rows, the gate and the preparation of its rows as one launch (gemm_i8_gate.hip); both prepared forms tiled
+bool gemm_i8_gate_applies(const aionhip_ctx *ctx, const aionhip_weight *gate, size_t m);
+int launch_gemm_i8_gate(aionhip_ctx *ctx, const aionhip_weight *gate, const aionhip_weight *up, size_t m, PreparedAct in, PreparedAct out);
 // MatMulNT with an f32 [N,K] operand (matmul_nt_f32.hip): plain f32 arithmetic, any number of rows
 int launch_matmul_nt_f32(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, const float *a, size_t lda, float *c, size_t ldc, float alpha,
                          float beta);
@@ -331,6 +337,23 @@ __device__ __forceinline__ void prepare_act_block8(float v0, float v1, float v2,
     s += dpp_i<DPP_QUAD_XOR2>(s);
     s += dpp_i<DPP_ROW_HALF_MIRROR>(s);
     sum = s;
+}
+
+// the same with a lane to an element: 32 lanes (half a wavefront) share one block
+__device__ __forceinline__ void prepare_act_lane32(float v, int &code, float &scale) {
+    float amax = fabsf(v);
+    amax = fmaxf(amax, dpp_f<DPP_QUAD_XOR1>(amax));
+    amax = fmaxf(amax, dpp_f<DPP_QUAD_XOR2>(amax));
+    amax = fmaxf(amax, dpp_f<DPP_ROW_HALF_MIRROR>(amax));
+    amax = fmaxf(amax, dpp_f<DPP_ROW_MIRROR>(amax));
+    amax = fmaxf(amax, __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(amax), 0x401F)));      // lane ^ 16
+    code = 0;
+    scale = 0.f;
+    if (amax != 0.f) {
+        scale = amax / 127.f;
+        const float inv = 127.f / amax;
+        code = (int)fminf(127.f, fmaxf(-127.f, roundf(v * inv)));
+    }
 }
 
 __device__ __forceinline__ int dot4_i8(int a, int b, int c) { return __builtin_amdgcn_sdot4(a, b, c, false); }

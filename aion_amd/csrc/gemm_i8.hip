@@ -61,7 +61,7 @@ constexpr I8Shape I8_SHAPES[] = {
     {32, 32, 8}, {32, 32, 4}, {64, 32, 4}, {96, 32, 4}, {64, 64, 4}, {128, 64, 2}, {32, 64, 2}, {128, 128, 1}, {32, 128, 2}, {32, 256, 1}, {32, 64, 4},
 };
 constexpr int I8_COUNT = 11;
-constexpr int I8_LONE4 = 1, I8_WIDE4 = 10;       // see pick_shape
+constexpr int I8_LONE4 = 1, I8_SQUARE4 = 4, I8_WIDE4 = 10;
 struct I8Fit {
     int resident;
     float t0, us, b, q, e;
@@ -286,6 +286,15 @@ float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k
     float us = 0.f;
     pick_shape(ctx, dtype, m, &n, 1, k, k_split(ctx, dtype, m, n, k), &us);
     return us;
+}
+
+bool gemm_i8_pair_plan(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts, bool *tall) {
+    const KSplit split = k_split(ctx, dtype, m, n, k);
+    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
+    const size_t ns[2] = {n, n};
+    *wavefronts = split.wavefronts;
+    *tall = m > 32 && shape_us(ctx, I8_SQUARE4, fits[I8_SQUARE4], m, ns, 2, k, 1) < shape_us(ctx, I8_WIDE4, fits[I8_WIDE4], m, ns, 2, k, 1);
+    return split.slices == 1;
 }
 
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {

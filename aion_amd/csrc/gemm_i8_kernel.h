@@ -58,12 +58,15 @@ __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M 
 // LDS of a wavefront: two groups of four blocks, weight codes and activation scales
 template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
 
-template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE>
+// GATE: the two column tiles of a wavefront are the same columns of weights 0 and 1 (gate and up), and what leaves is gelu(gate) * up prepared for
+// the next matmul: its codes to segs.c[0], its scales to segs.c[1], in the order above.
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, bool GATE = false>
 __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
                                                                          int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
-    constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
+    constexpr int BM = 32 * MT * WGM, BN = GATE ? 32 : 32 * NT * WGN;
+    static_assert(!GATE || (NT == 2 && WGN == 1), "gate and up side by side");
     constexpr bool OUTER = RQ == 4 && MT * NT > 1;        // scale products from the matrix pipe
     static_assert(OUTER || MT == 1, "one row tile");
     static_assert(RQ == 4 || MT * WGM == 1, "fewer rows than a tile: one row tile");
@@ -82,14 +85,14 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
     int si = 0;
 #pragma unroll
     for (int i = 1; i < 4; ++i)
-        if (i < segs.count && ct >= segs.first_tile[i]) si = i;
+        if (!GATE && i < segs.count && ct >= segs.first_tile[i]) si = i;
     const uint8_t *__restrict__ qs = segs.qs[si];
     const __half *__restrict__ sc = segs.sc[si];
     float *__restrict__ c = segs.c[si];
     const int N = segs.n[si];
     size_t ldc = segs.ldc[si];
     const int KB = K >> 5, G = (KB + 3) >> 2;
-    const int n0 = (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
+    const int n0 = GATE ? ct * 32 : (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
 
     Acc acc[MT][NT];
     // q4 dots are 16 times the codes' dots. The 1/16 is taken from the sums, where it is exact down to subnormal products of scales; sums past
@@ -119,8 +122,8 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         }
         const int nb = min(n0, N - 1);
         const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch;      // (used in the device pass only)
-        const __half *sb = sc + (size_t)nb * KB;
+        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = GATE ? segs.qs[1] + (size_t)nb * wpitch : wb;      // (used in the device pass only)
+        const __half *sb = (GATE && h ? segs.sc[1] : sc) + (size_t)nb * KB;
         // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
         constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
         const int w_row = lane / LPR;
@@ -129,9 +132,9 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         for (int i = 0; i < NT; ++i)
 #pragma unroll
             for (int l = 0; l < WL; ++l)
-                wo[i][l] = (unsigned)(min(n0 + i * 32 + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
+                wo[i][l] = (unsigned)(min(n0 + (GATE ? 0 : i * 32) + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
         // weight scales: with two tiles a lane half takes one tile's rows each and the halves are exchanged afterwards
-        const unsigned so = (unsigned)(min(n0 + (NT == 2 ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
+        const unsigned so = (unsigned)(min(n0 + (NT == 2 && !GATE ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
 
         // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
         const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
@@ -144,6 +147,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         int sw_shift = 0, sw_shift_now = 0;
 #if defined(__HIP_DEVICE_COMPILE__)
         const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)wb, 0, 0xFFFFFFFFu, 0x00027000);
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t w_rsrc1 = __builtin_amdgcn_make_buffer_rsrc((void *)wb1, 0, 0xFFFFFFFFu, 0x00027000);
         __amdgpu_buffer_rsrc_t sa_rsrc[MT];
 #pragma unroll
         for (int i = 0; i < MT; ++i) sa_rsrc[i] = __builtin_amdgcn_make_buffer_rsrc((void *)asb[i], 0, 0xFFFFFFFFu, 0x00027000);
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             for (int i = 0; i < NT; ++i)
 #pragma unroll
                 for (int l = 0; l < WL; ++l)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(GATE && i ? w_rsrc1 : w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
 #endif
         };
         const int r_slot = Q8 ? h ^ (r & 7) : (r >> 1) & 3;
@@ -406,7 +410,31 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         v *= alpha;
         *dst = beta == 0.f ? v : v + beta * *dst;
     };
-    if constexpr (KS == 1) {
+    // GATE: a lane has four rows of a column of both weights; a quant block of the gated rows is the 32 lanes of its half
+    [[maybe_unused]] auto put_gated = [&](int i, int q, f32x4 g, f32x4 u) {
+        const int kb = n0 >> 5, KBN = N >> 5, mt = (m0 >> 5) + i, rows = act_tile_rows(M, mt);
+        uint8_t *codes = (uint8_t *)segs.c[0] + ((size_t)mt * 32 * KBN + (size_t)kb * rows) * 32 + (r >> 4) * rows * 16 + (r & 15);
+        float *scales = segs.c[1] + (size_t)mt * 32 * KBN + (size_t)kb * rows;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = 8 * q + 4 * h + e;
+            int code;
+            float scale;
+            prepare_act_lane32(aion_gate_gelu(g[e], u[e]), code, scale);
+            if (row >= rows) continue;
+            codes[row * 16] = (uint8_t)code;
+            if (r == 0) scales[row] = scale;
+        }
+    };
+    if constexpr (GATE && KS == 1) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int q = 0; q < RQ; ++q) {
+                const Acc &g = acc[i][0], &u = acc[i][1];
+                put_gated(i, q, f32x4{g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]}, f32x4{u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]});
+            }
+    } else if constexpr (KS == 1) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -426,6 +454,21 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                 for (int q = 0; q < RQ; ++q)
                     red[(ks * CH + (i * NT + j) * RQ + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
         __syncthreads();
+        if constexpr (GATE) {
+#pragma unroll
+            for (int p0 = 0; p0 < (MT * RQ + KS - 1) / KS; ++p0) {
+                const int p = p0 * KS + ks, i = p / RQ, q = p % RQ, ch = i * 2 * RQ + q;
+                if (p >= MT * RQ) break;
+                f32x4 g = red[ch * 64 + lane], u = red[(ch + RQ) * 64 + lane];
+#pragma unroll
+                for (int k = 1; k < KS; ++k) {
+                    g += red[(k * CH + ch) * 64 + lane];
+                    u += red[(k * CH + ch + RQ) * 64 + lane];
+                }
+                put_gated(i, q, g, u);
+            }
+            return;
+        }
 #pragma unroll
         for (int c0 = 0; c0 < (CH + KS - 1) / KS; ++c0) {
             const int ch = c0 * KS + ks;

@@ -283,6 +283,33 @@ int aionhip_step_rmsnorm_geglu_matmul(aionhip_ctx *ctx, const aionhip_weight *w_
     return launch_gemv_batch(ctx, &w_down, &cp, &ldc, 1, 1, act, alpha, beta);
 }
 
+int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weight *w_gate, const aionhip_weight *w_up, const aionhip_weight *w_down,
+                                           size_t rows, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
+                                           aionhip_handle c, size_t ldc, float alpha, float beta) {
+    if (!ctx) return AIONHIP_INVALID_ARGUMENT;
+    if (rows == 0) return AIONHIP_OK;
+    const aionhip_weight *gu[2] = {w_gate, w_up};
+    const aionhip_handle unused[2] = {4, 4};                  // (neither projection is written out)
+    Batch in, down;
+    int rc = check_batch(ctx, "geglu_matmul_rows", 2, gu, unused, nullptr, in);
+    if (!rc) rc = check_batch(ctx, "geglu_matmul_rows", 1, &w_down, &c, &ldc, down);
+    if (rc) return rc;
+    if (!x || !gamma) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "geglu_matmul_rows: null x or gamma");
+    if (!(eps > 0.f) || !(eps < INFINITY)) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "geglu_matmul_rows: eps must be positive and finite");
+    if (w_gate->n != w_up->n || down.k != w_gate->n) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "geglu_matmul_rows: gate and up must match, down must take their outputs");
+    if (((x | gamma | beta_norm) & 15) || (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || rows > 0x7FFFFFFFu ||
+        !rows_tiled(ctx, in, rows) || !rows_tiled(ctx, down, rows) || !gemm_i8_gate_applies(ctx, w_gate, rows))
+        return set_err(ctx, AIONHIP_UNSUPPORTED, "geglu_matmul_rows: %zu rows against %zu x %zu do not run on the exact GEMM's gate instances", rows, (size_t)w_gate->n, in.k);
+    const size_t in_bytes = (prepared_act_bytes(rows, in.k) + 255) & ~(size_t)255;
+    rc = ensure_scratch(ctx, in_bytes + prepared_act_bytes(rows, down.k));
+    if (rc) return rc;
+    const PreparedAct act = prepared_act_carve(ctx->scratch, rows, in.k, true), gated = prepared_act_carve((char *)ctx->scratch + in_bytes, rows, down.k, true);
+    rc = launch_prepare_rmsnorm(ctx, (const float *)(uintptr_t)x, (const float *)(uintptr_t)gamma, (const float *)(uintptr_t)beta_norm, eps, rows, in.k, act);
+    if (!rc) rc = launch_gemm_i8_gate(ctx, w_gate, w_up, rows, act, gated);
+    if (rc) return rc;
+    return launch_prepared_rows(ctx, down, rows, gated, alpha, beta);
+}
+
 int aionhip_step_gate_matmul(aionhip_ctx *ctx, const aionhip_weight *w, size_t rows, aionhip_handle gate, aionhip_handle up,
                              aionhip_handle c, size_t ldc, float alpha, float beta) {
     if (!ctx || !w) return AIONHIP_INVALID_ARGUMENT;

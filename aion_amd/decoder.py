@@ -184,7 +184,9 @@ class Decoder:
                 # one row: RMSNorm -> MatMul gate, up -> gate(gelu) -> MatMul down (beta = 1), two launches
                 g.step_rmsnorm_geglu_matmul(self.w[p + "wgate"], self.w[p + "wup"], self.w[p + "wdown"], b["x"], self.gamma, c.eps,
                                             b["x"], beta=1.0)
-            else:
+            # many rows: the same, three launches, where the exact GEMM runs all three matmuls
+            elif not g.step_rmsnorm_geglu_matmul_rows(self.w[p + "wgate"], self.w[p + "wup"], self.w[p + "wdown"], b["x"], self.gamma, s, c.eps,
+                                                      b["x"], beta=1.0):
                 g.step_rmsnorm_matmul([self.w[p + "wgate"], self.w[p + "wup"]], b["x"], self.gamma, s, [b["gate"], b["up"]], c.eps)
                 # gate(gelu) -> MatMul down, beta = 1
                 g.step_gate_matmul(self.w[p + "wdown"], b["gate"], b["up"], s, b["x"], beta=1.0)

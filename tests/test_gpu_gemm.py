@@ -420,3 +420,35 @@ def test_exact_gemm_scale_products_keep_their_bits(gpu, orc, dtype, layout, m, n
         assert np.array_equal(got[rows].view(np.uint32), gpu.matmul(w, a[rows]).view(np.uint32)), rows
         assert "gemm_i8" in gpu.last_launch()["kernel"]
     w.free()
+
+
+# A GeGLU block of many rows with the gate and the preparation of its rows in the gate / up launch: the bits of the two calls it stands for, at
+# the edges of the 32-, 64- and 128-row tiles and for widths and K that end inside a group of four blocks; a row of zeros among them.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("rows,hidden,ffn", [(9, 256, 512), (16, 2048, 4128), (17, 2080, 8192), (32, 2048, 544), (33, 96, 8224), (64, 1056, 2048), (65, 2048, 8192),
+                                             (100, 256, 11008), (128, 2048, 8192), (129, 4096, 1056), (300, 672, 2080), (1100, 512, 16416), (2048, 2048, 8192)])
+def test_geglu_block_of_many_rows_is_the_separate_calls(gpu, dtype, layout, rows, hidden, ffn):
+    say("geglu rows", dtype, layout, rows, hidden, ffn)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    rng = np.random.default_rng(rows + ffn)
+    wg, wu, wd = (make_weight(gpu, dtype, layout, n, k, seed=n + s)[1] for s, (n, k) in enumerate(((ffn, hidden), (ffn, hidden), (hidden, ffn))))
+    x = rng.standard_normal((rows, hidden)).astype(np.float32)
+    x[rows // 2] = 0
+    gamma, beta = (gpu.upload(rng.standard_normal(hidden).astype(np.float32)) for _ in range(2))
+    xb, gate, up = gpu.upload(x), gpu.alloc(4 * rows * ffn), gpu.alloc(4 * rows * ffn)
+    for norm_beta, alpha, b in ((None, 1.0, 1.0), (beta, 0.5, 0.0)):
+        c = [gpu.upload(np.full((rows, hidden), 0.25, np.float32)) for _ in range(2)]
+        gpu.step_rmsnorm_matmul([wg, wu], xb, gamma, rows, [gate, up], 1e-6, beta_norm=norm_beta)
+        gpu.step_gate_matmul(wd, gate, up, rows, c[0], alpha=alpha, beta=b)
+        ran = gpu.step_rmsnorm_geglu_matmul_rows(wg, wu, wd, xb, gamma, rows, 1e-6, c[1], alpha=alpha, beta=b, beta_norm=norm_beta)
+        assert ran or (rows, hidden) == (33, 96)             # (one or two wavefronts to a K, and a row tile to spare)
+        want, got = (gpu.download(t, np.float32, (rows, hidden)) for t in c)
+        if ran:
+            assert np.isfinite(want).all() and np.array_equal(want.view(np.uint32), got.view(np.uint32))
+        else:
+            assert (got == 0.25).all()
+        for t in c:
+            t.free()
+    for t in (wg, wu, wd, gamma, beta, xb, gate, up):
+        t.free()
+    say("ran" if ran else "refused")
