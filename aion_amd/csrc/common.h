@@ -241,6 +241,10 @@ int rope_table(aionhip_ctx *ctx, int pairs, float freq_step, float scale_factor,
 bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m);
 int launch_gemv_mfma(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
                      float alpha, float beta);
+// 2..8 prepared rows against weights of few rows, K divided among the wavefronts of workgroups of 16 (gemv_slim.hip)
+bool gemv_slim_applies(const aionhip_ctx *ctx, const aionhip_weight *w, int m);
+int launch_gemv_slim(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
+                     float alpha, float beta);
 bool gemv_ksplit_applies(const aionhip_ctx *ctx, const aionhip_weight *w, const float *x);
 int launch_gemv_ksplit(aionhip_ctx *ctx, const aionhip_weight *w, float *c, const float *x, float alpha, float beta);
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,

@@ -450,17 +450,32 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
     if (!act.tiled && gemv_mfma_applies(ctx, ws, count, m)) {
         const char *mname = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8_mfma" : "gemv_q4_mfma";
         ProfScope scope(ctx, mname);
-        const int rc = launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+        // q4 from five rows on, up to six workgroups of gemv_slim.hip per CU: its 16-row workgroups start sooner than ones that copy all rows' K to LDS (8 x
+        // 14336 x 2048 1.47 times as fast, x 4096 1.34, 5 x 20480 x 4096 1.21; 32768 x 3072 0.92)
+        size_t tiles = 0;
+        for (int i = 0; i < count; ++i) tiles += (ws[i]->n + 15) / 16;
+        const bool slim = ws[0]->dtype == AIONHIP_Q4_0 && m >= 5 && ws[0]->k >= 2048 && tiles <= 6 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256);
+        const int rc = slim ? launch_gemv_slim(ctx, ws, cs, ldcs, count, m, act, alpha, beta) : launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
         if (rc == AIONHIP_OK) {
             LAUNCH_CHECK(ctx, mname);
             return AIONHIP_OK;
         }
         if (rc != -1) return rc;
     }
-    const char *name = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8" : "gemv_q4";
+    // (five rows and more over a long K go by the name of the exact GEMM, which takes those that gemv_slim.hip leaves)
+    const bool q8 = ws[0]->dtype == AIONHIP_Q8_0, long_k = m >= 5 && ws[0]->k > FUSED_PAYS_K && ws[0]->k <= GEMM_I8_MAX_K;
+    const char *name = long_k ? (q8 ? "gemm_i8_q8" : "gemm_i8_q4") : q8 ? "gemv_q8" : "gemv_q4";
     ProfScope scope(ctx, name);
     if (act.tiled) {
         const int rc = launch_gemm_i8_few_rows(ctx, ws[0], (size_t)m, act, cs[0], ldcs[0], alpha, beta);
+        if (rc) return rc;
+        LAUNCH_CHECK(ctx, name);
+        return AIONHIP_OK;
+    }
+    bool slim = true;
+    for (int i = 0; i < count; ++i) slim = slim && gemv_slim_applies(ctx, ws[i], m);
+    if (slim) {
+        const int rc = launch_gemv_slim(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
         if (rc) return rc;
         LAUNCH_CHECK(ctx, name);
         return AIONHIP_OK;

@@ -62,14 +62,19 @@ static bool fused_row_pays(const Batch &b) {
 }
 
 // Prepared rows against the weights of `b`: the GEMV kernels up to eight rows, except five to eight rows over a K past 4096,
-// where the GEMV walks K with all eight accumulator sets live and falls far behind the exact GEMM (8 x 14336 x 8192: q8 78 against 31 us,
+// where gemv_rows_kernel walks K with all eight accumulator sets live and falls far behind the exact GEMM (8 x 14336 x 8192: q8 78 against 31 us,
 // q4 65 against 25; 8 x 6144 x 4128 20 / 15, 18 / 11; q8 up to 4096 columns is level there or, below 3072, up to a fifth ahead on the
-// GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2); the GEMM beyond eight rows.
-static bool rows_on_gemv(const Batch &b, size_t m) { return m <= GEMV_MAX_M && (b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)); }
+// GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2) and gemv_slim_kernel does not apply; the GEMM beyond eight rows.
+static bool rows_on_gemv(const aionhip_ctx *ctx, const Batch &b, size_t m) {
+    if (m > GEMV_MAX_M || b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)) return m <= GEMV_MAX_M;
+    for (size_t i = 0; i < b.count; ++i)
+        if (!gemv_slim_applies(ctx, b.w[i], (int)m)) return false;
+    return true;
+}
 // which form of the preparation the kernel behind launch_prepared_rows reads
 static bool rows_tiled(const aionhip_ctx *ctx, const Batch &b, size_t m) {
     if (b.k > GEMM_I8_MAX_K) return false;
-    return !rows_on_gemv(b, m) || gemv_rows_on_gemm(ctx, b.w, (int)b.count, (int)m);
+    return !rows_on_gemv(ctx, b, m) || gemv_rows_on_gemm(ctx, b.w, (int)b.count, (int)m);
 }
 static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, PreparedAct act, float alpha, float beta) {
     if (m > GEMV_MAX_M && b.k > GEMM_I8_MAX_K) {                 // rows past the GEMM's addressing
@@ -83,7 +88,7 @@ static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, Prep
         }
         return AIONHIP_OK;
     }
-    if (rows_on_gemv(b, m))
+    if (rows_on_gemv(ctx, b, m))
         return launch_gemv_batch(ctx, b.w, b.c, b.ldc, (int)b.count, (int)m, act, alpha, beta);
     // sibling weights (q/k/v, gate/up) share one launch, four at a time
     for (size_t i = 0; i < b.count; i += 4) {

@@ -684,3 +684,43 @@ def test_an_f32_weight_is_a_matmul_nt_operand_only(gpu):
     for t in (x, g, c, ab, cb):
         t.free()
     w.free()
+
+
+# Both sides of the lines of the kernel for few weight rows: its workgroups have 16 of them and 16, 8 or 4 wavefronts to a K (256, 512, 768 workgroups
+# on 256 CUs); K of fewer stages than wavefronts, of one more and of several runs of scales; widths that end inside a tile, every row count.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k,q8_slim,q4_slim", [(3, 70, 512, 1, 1), (3, 1001, 640, 1, 1), (4, 4096, 14336, 1, 1), (4, 4097, 2176, 1, 1), (3, 8400, 1024, 0, 1),
+                                                   (2, 12280, 8192, 1, 1), (2, 12289, 8192, 0, 0), (2, 4096, 4096, 0, 0), (5, 40, 4096, 1, 1), (7, 1000, 2048, 1, 1),
+                                                   (8, 1023, 896, 1, 1), (6, 4096, 8320, 1, 1), (8, 6000, 4224, 1, 0), (5, 8208, 16384, 1, 1), (5, 300, 16512, 0, 0),
+                                                   (2, 33, 33024, 1, 1), (4, 500, 480, 0, 0), (8, 14400, 2048, 0, 1)])
+def test_few_weight_rows(gpu, orc, dtype, layout, m, n, k, q8_slim, q4_slim):
+    say("few weight rows", dtype, layout, m, n, k)
+    blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 13 + n + k, std=0.05)
+    rng = np.random.default_rng(m + n + k)
+    a = rng.standard_normal((m, k)).astype(np.float32)
+    a[m - 1, :64] = 0                                                   # (two blocks of zeros)
+    c0 = rng.standard_normal((m, n)).astype(np.float32)
+    got = gpu.matmul(w, a)
+    assert ("gemv_slim" in gpu.last_launch()["kernel"]) == bool(q8_slim if dtype == be.Q8_0 else q4_slim)
+    want = oracle_matmul(orc, dtype, layout, a, blocks, n)
+    assert norm_err(got, want) < TOL and rms_err(got, want) < RMS_TOL
+    assert rms_err(gpu.matmul(w, a, alpha=-1.5, beta=0.25, c=c0), -1.5 * want + 0.25 * c0) < RMS_TOL
+    w.free()
+
+
+# The same with siblings in one launch, the tiles of all weights counted together (4300, 9000, 4812 rows: 8, 4 and 8 wavefronts to a K)
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,ns", [(3, (4000, 300)), (4, (4000, 5000)), (8, (300, 4000, 512))])
+def test_few_weight_rows_siblings(gpu, orc, dtype, layout, m, ns):
+    k = 8192
+    made = [make_weight(gpu, orc, dtype, layout, n, k, seed=n + i, std=0.05) for i, n in enumerate(ns)]
+    a = np.random.default_rng(m).standard_normal((m, k)).astype(np.float32)
+    a_buf, c_bufs = gpu.upload(a), [gpu.alloc(m * n * 4) for n in ns]
+    gpu.step_matmul_batch([w for _b, w in made], a_buf, m, c_bufs)
+    assert ("gemv_slim" in gpu.last_launch()["kernel"]) == (max(ns) <= 4096 or m < 5 or dtype == be.Q8_0)
+    for (blocks, w), n, c in zip(made, ns, c_bufs):
+        got, want = gpu.download(c, np.float32, (m, n)), oracle_matmul(orc, dtype, layout, a, blocks, n)
+        assert norm_err(got, want) < TOL and rms_err(got, want) < RMS_TOL
+        c.free()
+        w.free()
+    a_buf.free()
