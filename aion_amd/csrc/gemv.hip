@@ -419,7 +419,8 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 // timed over 130 shapes (K = 512 ... 14336, N = 1024 ... 262144) at 2, 4, 5 and 8 rows, both block formats, preparation included, weights
 // rotated past the memory-side cache (lane-per-row against GEMM, us; columns for 256 CUs):
 //   5..8 rows:  from max(1024, K) columns on. q4 8192 x 512 10.5 against 6.2, 4096 x 2048 9.6 against 8.7, 8192 x 4096 14 against 11; q8
-//               8192 x 4096 18 against 14. Narrower the GEMM loses: q8 2048 x 4096 10 against 12.
+//               8192 x 4096 18 against 14. Narrower the GEMM loses: q8 2048 x 4096 10 against 12. Past one round, from K = 2048 on, gemv_slim_kernel
+//               takes those within its range (GEMM against it: q8 8 x 12288 x 4096 17.6 against 14.9, q4 8 x 9664 x 4096 1.16 times, 5 x 9000 x 2048 1.04)
 //   2..4 rows:  one nearly full round (7681 ... 8192 columns: q8 x 8192 22 against 22, q4 16 against 14), or one and a half (12288
 //               columns) and more; q8 between them too up to K = 5120 (9664 x 4096 level; x 6144 1.11 times, x 8192 1.10) and where
 //               only two of the lane-per-row kernel's workgroups, which hold their rows' K in LDS, fit a CU (4 x 9664 x 14336 49 against
@@ -427,13 +428,13 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
 //               level; of two rows past K = 8192 two: 20480 x 14336 60 against 69), three for q4, with half the bytes a weight (32768 x 4096 20.6 against 24), two for two rows of q4, from K = 4096
 //               on (12288 x 4096 14.2 against 13.3, x 2048 9.1 against 9.5). Beyond 2^28 weights the lane-per-row kernel streams faster
 //               whatever the CUs (q8 32768 x 14336 80 against 96).
-// Five rows and more over a K past 4096 take the GEMM before this rule is asked.
+// Five rows and more over a K past 4096 take the GEMM, or gemv_slim_kernel, before this rule is asked.
 bool gemv_rows_on_gemm(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m) {
     if (count != 1 || m < 2 || gemv_mfma_applies(ctx, ws, count, m)) return false;
     const size_t n = ws[0]->n, k = ws[0]->k, round = 32 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256);
     const bool q8 = ws[0]->dtype == AIONHIP_Q8_0;
     if (k < 256 || k > GEMM_I8_MAX_K) return false;
-    if (m >= 5) return k <= 4096 && n >= (k > 1024 ? k : 1024);
+    if (m >= 5) return k <= 4096 && n >= (k > 1024 ? k : 1024) && !(n > round && k >= 2048 && gemv_slim_applies(ctx, ws[0], m));
     if (n * 16 <= round * 15 || n * k > ((size_t)1 << 28)) return false;
     if (n > round && n * 2 < round * 3) {
         const bool two_per_cu = (size_t)(m == 2 ? 2 : 4) * 40 * (k / QK) * 3 > 160 * 1024;

@@ -692,7 +692,8 @@ def test_an_f32_weight_is_a_matmul_nt_operand_only(gpu):
 @pytest.mark.parametrize("m,n,k,q8_slim,q4_slim", [(3, 70, 512, 1, 1), (3, 1001, 640, 1, 1), (4, 4096, 14336, 1, 1), (4, 4097, 2176, 1, 1), (3, 8400, 1024, 0, 1),
                                                    (2, 12280, 8192, 1, 1), (2, 12289, 8192, 0, 0), (2, 4096, 4096, 0, 0), (5, 40, 4096, 1, 1), (7, 1000, 2048, 1, 1),
                                                    (8, 1023, 896, 1, 1), (6, 4096, 8320, 1, 1), (8, 6000, 4224, 1, 0), (5, 8208, 16384, 1, 1), (5, 300, 16512, 0, 0),
-                                                   (2, 33, 33024, 1, 1), (4, 500, 480, 0, 0), (8, 14400, 2048, 0, 1)])
+                                                   (2, 33, 33024, 1, 1), (4, 500, 480, 0, 0), (8, 14400, 2048, 0, 1), (8, 8208, 2048, 1, 1), (6, 8208, 1920, 0, 0),
+                                                   (5, 12290, 4096, 0, 0)])
 def test_few_weight_rows(gpu, orc, dtype, layout, m, n, k, q8_slim, q4_slim):
     say("few weight rows", dtype, layout, m, n, k)
     blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 13 + n + k, std=0.05)
