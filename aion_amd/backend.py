@@ -237,6 +237,18 @@ class HipBackend:
             self._ctx, w_gate.ptr, w_up.ptr, w_down.ptr, x.handle, gamma.handle, beta_norm.handle if beta_norm is not None else 0, eps,
             c_buf.handle, alpha, beta))
 
+    def step_rmsnorm_qkv_rope_append_rows(self, wq, wk, wv, x, gamma, eps, q_out, k_cache, v_cache, positions, write_index, b, s, t_cap, h_q, h_kv, d,
+                                          base=10000.0, scale_factor=1.0, proportion=1.0, beta_norm=None):
+        """RMSNorm -> q, k, v -> RoPE(q, k) -> f16 -> append for b sequences of s tokens, two launches. False, with nothing issued, where the
+        library wants the separate steps (step_rmsnorm_matmul, step_rope_append)."""
+        rc = self._lib.aionhip_step_rmsnorm_qkv_rope_append_rows(
+            self._ctx, wq.ptr, wk.ptr, wv.ptr, b, s, x.handle, gamma.handle, beta_norm.handle if beta_norm is not None else 0, eps, q_out.handle,
+            k_cache.handle, v_cache.handle, positions.handle, write_index.handle, t_cap, h_q, h_kv, d, base, scale_factor, proportion)
+        if rc == hip.UNSUPPORTED:
+            return False
+        self._check(rc)
+        return True
+
     def step_rmsnorm_geglu_matmul_rows(self, w_gate, w_up, w_down, x, gamma, rows, eps, c_buf, alpha=1.0, beta=0.0, beta_norm=None):
         """The same for many rows, three launches. False, with nothing issued, where the library wants the separate steps
         (step_rmsnorm_matmul, step_gate_matmul) for these rows."""

@@ -261,12 +261,22 @@ int launch_gemm_i8_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, floa
                          PreparedAct act, float alpha, float beta);
 // the same kernel for a handful of rows (no profile scope of its own: the caller's name stays)
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta);
-// how the exact GEMM divides a K among a workgroup's wavefronts (false: it is also cut into slices), and whether four of them to a tile of two
-// weights' columns are better given 64 rows than 32
-bool gemm_i8_pair_plan(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts, bool *tall);
-// gate and up projections of m prepared rows, the gate and the preparation of its rows as one launch (gemm_i8_gate.hip); both prepared forms tiled
+// how the exact GEMM divides a K among a workgroup's wavefronts (false: it is also cut into slices), and whether four of them to a tile of 64
+// columns are better given 64 rows than 32
+bool gemm_i8_unsliced(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts);
+bool gemm_i8_tall(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k);
+// gate and up projections of m prepared rows, the gate and the preparation of its rows as one launch (gemm_i8_pair.hip); both prepared forms tiled
 bool gemm_i8_gate_applies(const aionhip_ctx *ctx, const aionhip_weight *gate, size_t m);
 int launch_gemm_i8_gate(aionhip_ctx *ctx, const aionhip_weight *gate, const aionhip_weight *up, size_t m, PreparedAct in, PreparedAct out);
+// q, k and v projections of m prepared rows (tiled), the rotation of q and k and the append of k and v to their f16 caches as one launch
+struct RopeAppend {
+    __half *kcache, *vcache;
+    const int *positions, *write_index;
+    const float *freq;
+    int s_len, t_cap, h_q, h_kv, d, rope_pairs;
+};
+bool gemm_i8_rope_applies(const aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, size_t d);
+int launch_gemm_i8_rope(aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, PreparedAct in, float *q_out, RopeAppend rope);
 // MatMulNT with an f32 [N,K] operand (matmul_nt_f32.hip): plain f32 arithmetic, any number of rows
 int launch_matmul_nt_f32(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, const float *a, size_t lda, float *c, size_t ldc, float alpha,
                          float beta);

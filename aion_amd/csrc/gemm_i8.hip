@@ -288,13 +288,14 @@ float gemm_i8_us(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k
     return us;
 }
 
-bool gemm_i8_pair_plan(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts, bool *tall) {
+bool gemm_i8_unsliced(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts) {
     const KSplit split = k_split(ctx, dtype, m, n, k);
-    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
-    const size_t ns[2] = {n, n};
     *wavefronts = split.wavefronts;
-    *tall = m > 32 && shape_us(ctx, I8_SQUARE4, fits[I8_SQUARE4], m, ns, 2, k, 1) < shape_us(ctx, I8_WIDE4, fits[I8_WIDE4], m, ns, 2, k, 1);
     return split.slices == 1;
+}
+bool gemm_i8_tall(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k) {
+    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
+    return m > 32 && shape_us(ctx, I8_SQUARE4, fits[I8_SQUARE4], m, ns, count, k, 1) < shape_us(ctx, I8_WIDE4, fits[I8_WIDE4], m, ns, count, k, 1);
 }
 
 int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, PreparedAct act, float *c, size_t ldc, float alpha, float beta) {

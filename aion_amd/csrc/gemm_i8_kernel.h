@@ -50,6 +50,21 @@ struct GemmSegs {
     int count;
 };
 
+// What leaves the kernel (EPI). Past GEMM_PLAIN the two column tiles of a wavefront belong together:
+//   GEMM_GATE  the same columns of weights 0 and 1 (gate and up): gelu(gate) * up, prepared for the next matmul, its codes to c[0], its scales to
+//              c[1], in the order below
+//   GEMM_ROPE  the two halves of a head's columns of weight 0, 1 or 2 (q, k, v): q and k rotated, q to q_out, k and v as f16 to their caches
+constexpr int GEMM_PLAIN = 0, GEMM_GATE = 1, GEMM_ROPE = 2;
+struct GemmRopeSegs : GemmSegs {
+    float *q_out;
+    __half *kcache, *vcache;
+    const int *positions, *write_index;
+    const float *freq;
+    int s_len, t_cap, h_q, h_kv, d, rope_pairs;
+};
+template <int EPI> struct GemmSegsOf { using type = GemmSegs; };
+template <> struct GemmSegsOf<GEMM_ROPE> { using type = GemmRopeSegs; };
+
 // Prepared activation in the order the kernel's operand loads want: row tiles of 32 rows (the last one may hold fewer), per
 // tile and quant block [h = 0, 1][row][16 codes] - k = 16 h .. 16 h + 15 of the block - so that a wavefront's load of one
 // block of a full tile is 1 KiB of consecutive memory; scales per tile and block [row].
@@ -58,15 +73,14 @@ __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M 
 // LDS of a wavefront: two groups of four blocks, weight codes and activation scales
 template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
 
-// GATE: the two column tiles of a wavefront are the same columns of weights 0 and 1 (gate and up), and what leaves is gelu(gate) * up prepared for
-// the next matmul: its codes to segs.c[0], its scales to segs.c[1], in the order above.
-template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, bool GATE = false>
-__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI = GEMM_PLAIN>
+__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(typename GemmSegsOf<EPI>::type segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
                                                                          int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
                                                                          float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
-    constexpr int BM = 32 * MT * WGM, BN = GATE ? 32 : 32 * NT * WGN;
-    static_assert(!GATE || (NT == 2 && WGN == 1), "gate and up side by side");
+    constexpr bool PAIR = EPI != GEMM_PLAIN, GATE = EPI == GEMM_GATE;
+    constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
+    static_assert(!PAIR || (NT == 2 && WGN == 1), "a pair of tiles side by side");
     constexpr bool OUTER = RQ == 4 && MT * NT > 1;        // scale products from the matrix pipe
     static_assert(OUTER || MT == 1, "one row tile");
     static_assert(RQ == 4 || MT * WGM == 1, "fewer rows than a tile: one row tile");
@@ -92,7 +106,17 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
     const int N = segs.n[si];
     size_t ldc = segs.ldc[si];
     const int KB = K >> 5, G = (KB + 3) >> 2;
-    const int n0 = GATE ? ct * 32 : (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
+    // (a head's columns: pair tile `head_tile` is its columns 32 head_tile .. and the same of its second half)
+    [[maybe_unused]] int head = 0, head_tile = 0, pair_col = ct * 32;
+    size_t second = 0;                           // weight rows from a column of the first tile to its partner's
+    if constexpr (EPI == GEMM_ROPE) {
+        const int per_head = segs.d >> 6;
+        head = (ct - segs.first_tile[si]) / per_head;
+        head_tile = ct - segs.first_tile[si] - head * per_head;
+        second = (size_t)segs.d >> 1;
+        pair_col = head * segs.d + head_tile * 32;
+    }
+    const int n0 = PAIR ? pair_col : (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
 
     Acc acc[MT][NT];
     // q4 dots are 16 times the codes' dots. The 1/16 is taken from the sums, where it is exact down to subnormal products of scales; sums past
@@ -122,8 +146,8 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         }
         const int nb = min(n0, N - 1);
         const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = GATE ? segs.qs[1] + (size_t)nb * wpitch : wb;      // (used in the device pass only)
-        const __half *sb = (GATE && h ? segs.sc[1] : sc) + (size_t)nb * KB;
+        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = (GATE ? segs.qs[1] : qs) + ((size_t)nb + second) * wpitch;      // (used in the device pass only)
+        const __half *sb = (GATE && h ? segs.sc[1] : sc) + ((size_t)nb + (EPI == GEMM_ROPE && h ? second : 0)) * KB;
         // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
         constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
         const int w_row = lane / LPR;
@@ -132,9 +156,9 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         for (int i = 0; i < NT; ++i)
 #pragma unroll
             for (int l = 0; l < WL; ++l)
-                wo[i][l] = (unsigned)(min(n0 + (GATE ? 0 : i * 32) + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
+                wo[i][l] = (unsigned)(min(n0 + (PAIR ? 0 : i * 32) + l * (64 / LPR) + w_row, N - 1) - nb) * wpitch + (unsigned)((lane % LPR) ^ (Q8 ? w_row & 7 : (w_row >> 1) & 3)) * 16;
         // weight scales: with two tiles a lane half takes one tile's rows each and the halves are exchanged afterwards
-        const unsigned so = (unsigned)(min(n0 + (NT == 2 && !GATE ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
+        const unsigned so = (unsigned)(min(n0 + (NT == 2 && !PAIR ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
 
         // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
         const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
@@ -170,7 +194,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             for (int i = 0; i < NT; ++i)
 #pragma unroll
                 for (int l = 0; l < WL; ++l)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(GATE && i ? w_rsrc1 : w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(PAIR && i ? w_rsrc1 : w_rsrc, (lds_void *)(w_lds + buf * WBUF + (i * WL + l) * 1024), 16, wo[i][l], g * RB, 0, 0);
 #endif
         };
         const int r_slot = Q8 ? h ^ (r & 7) : (r >> 1) & 3;
@@ -410,8 +434,39 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
         v *= alpha;
         *dst = beta == 0.f ? v : v + beta * *dst;
     };
-    // GATE: a lane has four rows of a column of both weights; a quant block of the gated rows is the 32 lanes of its half
-    [[maybe_unused]] auto put_gated = [&](int i, int q, f32x4 g, f32x4 u) {
+    // A lane has four rows of a column of both tiles. GEMM_GATE: a quant block of the gated rows is the 32 lanes of its half.
+    [[maybe_unused]] auto put_pair = [&](int i, int q, f32x4 g, f32x4 u) {
+        if constexpr (EPI == GEMM_ROPE) {
+            // (rope_append_kernel's arithmetic and bounds)
+            const int pair = head_tile * 32 + r;
+            const bool rot = si < 2 && pair < segs.rope_pairs;
+            const float fr = rot ? segs.freq[pair] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = m0 + i * 32 + 8 * q + 4 * h + e;
+                if (row >= M) continue;
+                const float xl = alpha * g[e], xh = alpha * u[e];
+                float yl = xl, yh = xh;
+                if (rot) {
+                    float sn, cs;
+                    sincosf((float)segs.positions[row] * fr, &sn, &cs);
+                    rope_rotate(xl, xh, sn, cs, yl, yh);
+                }
+                if (si == 0) {
+                    float *dst = segs.q_out + ((size_t)row * segs.h_q + head) * segs.d + pair;
+                    dst[0] = yl;
+                    dst[second] = yh;
+                    continue;
+                }
+                const int b = row / segs.s_len;
+                const long t = (long)segs.write_index[b] + (long)(row - b * segs.s_len);
+                if (t < 0 || t >= segs.t_cap) continue;
+                __half *dst = (si == 1 ? segs.kcache : segs.vcache) + (((size_t)b * segs.t_cap + (size_t)t) * segs.h_kv + head) * segs.d + pair;
+                dst[0] = __float2half_rn(yl);
+                dst[second] = __float2half_rn(yh);
+            }
+            return;
+        }
         const int kb = n0 >> 5, KBN = N >> 5, mt = (m0 >> 5) + i, rows = act_tile_rows(M, mt);
         uint8_t *codes = (uint8_t *)segs.c[0] + ((size_t)mt * 32 * KBN + (size_t)kb * rows) * 32 + (r >> 4) * rows * 16 + (r & 15);
         float *scales = segs.c[1] + (size_t)mt * 32 * KBN + (size_t)kb * rows;
@@ -426,13 +481,13 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             if (r == 0) scales[row] = scale;
         }
     };
-    if constexpr (GATE && KS == 1) {
+    if constexpr (PAIR && KS == 1) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int q = 0; q < RQ; ++q) {
                 const Acc &g = acc[i][0], &u = acc[i][1];
-                put_gated(i, q, f32x4{g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]}, f32x4{u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]});
+                put_pair(i, q, f32x4{g[4 * q], g[4 * q + 1], g[4 * q + 2], g[4 * q + 3]}, f32x4{u[4 * q], u[4 * q + 1], u[4 * q + 2], u[4 * q + 3]});
             }
     } else if constexpr (KS == 1) {
 #pragma unroll
@@ -454,7 +509,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                 for (int q = 0; q < RQ; ++q)
                     red[(ks * CH + (i * NT + j) * RQ + q) * 64 + lane] = f32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
         __syncthreads();
-        if constexpr (GATE) {
+        if constexpr (PAIR) {
 #pragma unroll
             for (int p0 = 0; p0 < (MT * RQ + KS - 1) / KS; ++p0) {
                 const int p = p0 * KS + ks, i = p / RQ, q = p % RQ, ch = i * 2 * RQ + q;
@@ -465,7 +520,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
                     g += red[(k * CH + ch) * 64 + lane];
                     u += red[(k * CH + ch + RQ) * 64 + lane];
                 }
-                put_gated(i, q, g, u);
+                put_pair(i, q, g, u);
             }
             return;
         }

@@ -265,6 +265,47 @@ int aionhip_step_rmsnorm_qkv_rope_append(aionhip_ctx *ctx, const aionhip_weight 
     return launch_gemv_fused_rope(ctx, ws, (float *)(uintptr_t)q_out, in, epi);
 }
 
+int aionhip_step_rmsnorm_qkv_rope_append_rows(aionhip_ctx *ctx, const aionhip_weight *wq, const aionhip_weight *wk, const aionhip_weight *wv,
+                                              size_t b, size_t s, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
+                                              aionhip_handle q_out, aionhip_handle k_cache, aionhip_handle v_cache, aionhip_handle positions,
+                                              aionhip_handle write_index, size_t t_cap, size_t h_q, size_t h_kv, size_t d, float base_frequency,
+                                              float scale_factor, float rope_proportion) {
+    if (!ctx) return AIONHIP_INVALID_ARGUMENT;
+    const aionhip_weight *qkv[3] = {wq, wk, wv};
+    const aionhip_handle unused[3] = {4, 4, 4};               // (no projection is written out as it is)
+    Batch in;
+    int rc = check_batch(ctx, "qkv_rope_append_rows", 3, qkv, unused, nullptr, in);
+    if (rc) return rc;
+    if (!x || !gamma || !q_out || !k_cache || !v_cache || !positions || !write_index)
+        return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "qkv_rope_append_rows: null operand");
+    if (!(eps > 0.f) || !(eps < INFINITY)) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "qkv_rope_append_rows: eps must be positive and finite");
+    if (!(base_frequency > 0.f) || !(base_frequency < INFINITY) || !(scale_factor > 0.f) || !(scale_factor < INFINITY) ||
+        !(rope_proportion >= 0.f && rope_proportion <= 1.f))
+        return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "qkv_rope_append_rows: base/scale must be positive and finite, proportion in [0,1]");
+    if (d == 0 || d % 2 != 0 || d > 65534 || h_q == 0 || h_kv == 0 || h_q > 65535 || h_kv > 65535 || wq->n != h_q * d || wk->n != h_kv * d || wv->n != h_kv * d)
+        return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "qkv_rope_append_rows: weight rows must be heads x head size, head size even");
+    if (s > t_cap) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "qkv_rope_append_rows: %zu new tokens exceed the cache capacity %zu", s, t_cap);
+    if (b == 0 || s == 0) return AIONHIP_OK;
+    const size_t rows = b * s;
+    if (((x | gamma | beta_norm) & 15) || (q_out & 3) || ((k_cache | v_cache) & 1) || rows / b != s || rows > 0x7FFFFFFFu || t_cap > 0x7FFFFFFFu ||
+        (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_tiled(ctx, in, rows) || !gemm_i8_rope_applies(ctx, qkv, rows, d))
+        return set_err(ctx, AIONHIP_UNSUPPORTED, "qkv_rope_append_rows: %zu rows of K %zu and heads of %zu do not run on the exact GEMM's rope instances", rows, in.k, d);
+    const size_t half = d / 2;
+    size_t rope_pairs = (size_t)floorf(rope_proportion * (float)half);
+    if (rope_pairs > half) rope_pairs = half;
+    const float freq_step = (float)pow((double)base_frequency, (double)(-2.0f / (float)d));
+    const float *freq = nullptr;
+    rc = rope_table(ctx, (int)rope_pairs, freq_step, scale_factor, &freq);
+    if (!rc) rc = ensure_scratch(ctx, prepared_act_bytes(rows, in.k));
+    if (rc) return rc;
+    const PreparedAct act = prepared_act_carve(ctx->scratch, rows, in.k, true);
+    rc = launch_prepare_rmsnorm(ctx, (const float *)(uintptr_t)x, (const float *)(uintptr_t)gamma, (const float *)(uintptr_t)beta_norm, eps, rows, in.k, act);
+    if (rc) return rc;
+    const RopeAppend rope{(__half *)(uintptr_t)k_cache, (__half *)(uintptr_t)v_cache, (const int *)(uintptr_t)positions, (const int *)(uintptr_t)write_index,
+                          freq, (int)s, (int)t_cap, (int)h_q, (int)h_kv, (int)d, (int)rope_pairs};
+    return launch_gemm_i8_rope(ctx, qkv, rows, act, (float *)(uintptr_t)q_out, rope);
+}
+
 int aionhip_step_rmsnorm_geglu_matmul(aionhip_ctx *ctx, const aionhip_weight *w_gate, const aionhip_weight *w_up, const aionhip_weight *w_down,
                                       aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
                                       aionhip_handle c, float alpha, float beta) {

@@ -168,7 +168,10 @@ class Decoder:
                 g.step_rmsnorm_qkv_rope_append(self.w[p + "wq"], self.w[p + "wk"], self.w[p + "wv"], b["x"], self.gamma, c.eps,
                                                b["qr"], self.kc[l], self.vc[l], b["positions"], b["write_index"],
                                                c.max_seq, c.heads, c.kv_heads, c.head_dim, base=c.rope_base)
-            else:
+            # many tokens: the same, two launches, where the exact GEMM runs the projections
+            elif not g.step_rmsnorm_qkv_rope_append_rows(self.w[p + "wq"], self.w[p + "wk"], self.w[p + "wv"], b["x"], self.gamma, c.eps, b["qr"],
+                                                         self.kc[l], self.vc[l], b["positions"], b["write_index"], 1, s, c.max_seq, c.heads,
+                                                         c.kv_heads, c.head_dim, base=c.rope_base):
                 # RMSNorm -> MatMul q, k, v (one call: the norm is not materialised)
                 g.step_rmsnorm_matmul([self.w[p + "wq"], self.w[p + "wk"], self.w[p + "wv"]], b["x"], self.gamma, s,
                                       [b["q"], b["k"], b["v"]], c.eps)

@@ -97,6 +97,9 @@ _SIGS = {
                                                        C.c_size_t, C.c_float, C.c_float, C.c_float, C.c_int]),
     "aionhip_step_rmsnorm_geglu_matmul": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_uint64, C.c_uint64, C.c_uint64, C.c_float,
                                                     C.c_uint64, C.c_float, C.c_float]),
+    "aionhip_step_rmsnorm_qkv_rope_append_rows": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_size_t, C.c_uint64, C.c_uint64,
+                                                            C.c_uint64, C.c_float, C.c_uint64, C.c_uint64, C.c_uint64, C.c_uint64, C.c_uint64, C.c_size_t,
+                                                            C.c_size_t, C.c_size_t, C.c_size_t, C.c_float, C.c_float, C.c_float]),
     "aionhip_step_rmsnorm_geglu_matmul_rows": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t, C.c_uint64, C.c_uint64, C.c_uint64,
                                                          C.c_float, C.c_uint64, C.c_size_t, C.c_float, C.c_float]),
     "aionhip_step_gate_matmul": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t, C.c_uint64, C.c_uint64, C.c_uint64, C.c_size_t, C.c_float, C.c_float]),

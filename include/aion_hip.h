@@ -173,6 +173,15 @@ int aionhip_step_rmsnorm_qkv_rope_append(aionhip_ctx *ctx, const aionhip_weight 
                                          aionhip_handle q_out, aionhip_handle k_cache, aionhip_handle v_cache,
                                          aionhip_handle positions, aionhip_handle write_index, size_t t_cap, size_t h_q, size_t h_kv,
                                          size_t d, float base_frequency, float scale_factor, float rope_proportion, int rolling);
+/* The same for b sequences of s new tokens each on the exact GEMM, linear caches, in two launches (positions [b, s], write_index [b], as
+ * aionhip_step_rope_append takes them): the results are those of aionhip_step_rmsnorm_matmul + aionhip_step_rope_append to the bit; k, v and the
+ * unrotated q are not written out. AIONHIP_UNSUPPORTED, with nothing launched, where the projections would run on another kernel (a few rows,
+ * the bf16 modes, a K that is cut into slices) or the head size is no multiple of 64: issue the two calls. */
+int aionhip_step_rmsnorm_qkv_rope_append_rows(aionhip_ctx *ctx, const aionhip_weight *wq, const aionhip_weight *wk, const aionhip_weight *wv,
+                                              size_t b, size_t s, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
+                                              aionhip_handle q_out, aionhip_handle k_cache, aionhip_handle v_cache, aionhip_handle positions,
+                                              aionhip_handle write_index, size_t t_cap, size_t h_q, size_t h_kv, size_t d, float base_frequency,
+                                              float scale_factor, float rope_proportion);
 /* Decode fusion of a GeGLU feed-forward block for ONE activation row: RMSNorm(x) -> gate and up matmuls ->
  * gate(gelu_tanh) * up (cpu/exec/elementwise.zig:25-37) -> int8 activation preparation -> down matmul,
  * C[1, n_down] = alpha * (...) + beta * C, in two launches; the gate / up / gated rows never reach memory.

@@ -452,3 +452,43 @@ def test_geglu_block_of_many_rows_is_the_separate_calls(gpu, dtype, layout, rows
     for t in (wg, wu, wd, gamma, beta, xb, gate, up):
         t.free()
     say("ran" if ran else "refused")
+
+
+# RMSNorm, q, k, v, the rotation and the cache appends of many tokens as two launches: the bits of the two calls they stand for, at the edges of
+# the row tiles, over head sizes and layouts, for several sequences at their own write indices (one of them past the end of its cache: not
+# written) and a partial rotation.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("b,s,hidden,heads,kv_heads,d,t_cap", [(1, 9, 512, 8, 1, 64, 40), (1, 128, 2048, 8, 1, 256, 256), (2, 33, 1056, 6, 2, 128, 100),
+                                                              (1, 65, 4096, 32, 8, 128, 65), (3, 50, 640, 4, 4, 192, 300), (1, 700, 512, 32, 8, 128, 1024),
+                                                              (1, 17, 2080, 16, 4, 64, 17)])
+def test_qkv_rope_append_of_many_tokens_is_the_separate_calls(gpu, dtype, layout, b, s, hidden, heads, kv_heads, d, t_cap):
+    say("qkv rope rows", dtype, layout, b, s, hidden, heads, kv_heads, d)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    rng = np.random.default_rng(s + hidden)
+    rows = b * s
+    ws = [make_weight(gpu, dtype, layout, n * d, hidden, seed=n * d + i)[1] for i, n in enumerate((heads, kv_heads, kv_heads))]
+    x, gamma = gpu.upload(rng.standard_normal((rows, hidden)).astype(np.float32)), gpu.upload(rng.standard_normal(hidden).astype(np.float32))
+    at = np.minimum(np.arange(b) * 7, t_cap - s).astype(np.int32)
+    if b > 1:
+        at[-1] = t_cap - s + 2
+    pos, widx = gpu.upload((at[:, None] + np.arange(s)).astype(np.int32)), gpu.upload(at)
+    q, k, v = (gpu.alloc(4 * rows * n * d) for n in (heads, kv_heads, kv_heads))
+    for proportion in (1.0, 0.4):
+        outs = []
+        for fused in (False, True):
+            qr = gpu.zeros(4 * rows * heads * d)
+            kc, vc = (gpu.upload(np.full((b, t_cap, kv_heads, d), 3.0, np.float16)) for _ in range(2))
+            if fused:
+                ran = gpu.step_rmsnorm_qkv_rope_append_rows(*ws, x, gamma, 1e-6, qr, kc, vc, pos, widx, b, s, t_cap, heads, kv_heads, d, proportion=proportion)
+            else:
+                gpu.step_rmsnorm_matmul(ws, x, gamma, rows, [q, k, v], 1e-6)
+                gpu.step_rope_append(qr, q, k, v, kc, vc, pos, widx, b, s, t_cap, heads, kv_heads, d, proportion=proportion)
+            outs.append([gpu.download(qr, np.uint32, (rows * heads * d,))] + [gpu.download(t, np.uint16, (b * t_cap * kv_heads * d,)) for t in (kc, vc)])
+            for t in (qr, kc, vc):
+                t.free()
+        say("ran" if ran else "refused")
+        for want, got in zip(*outs):
+            assert np.array_equal(want, got) if ran else np.unique(got).size == 1
+    assert ran or (b, s, hidden) in ((1, 65, 4096), (1, 700, 512))       # (the K of q and of k, v divided differently)
+    for t in ws + [x, gamma, pos, widx, q, k, v]:
+        t.free()
