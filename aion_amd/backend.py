@@ -383,6 +383,20 @@ class HipBackend:
                           1 if rolling else 0)
         self._check(self._lib.aionhip_step_attention(self._ctx, C.byref(p)))
 
+    def step_attention_matmul(self, w, q, k, v, shape, scale, c_buf, q_dtype=F32, kv_dtype=F16, window=CAUSAL, soft_cap=0.0,
+                              query_positions=None, kv_lengths=None, rolling=False, alpha=1.0, beta=0.0):
+        """Attention and the matmul of its rows, two launches. False, with nothing issued, where the library wants the separate steps
+        (step_attention, step_matmul)."""
+        p = hip.Attention(0, q.handle, k.handle, v.handle,
+                          query_positions.handle if query_positions is not None else 0,
+                          kv_lengths.handle if kv_lengths is not None else 0,
+                          *shape, q_dtype, kv_dtype, scale, soft_cap, *window, 1 if rolling else 0)
+        rc = self._lib.aionhip_step_attention_matmul(self._ctx, C.byref(p), w.ptr, c_buf.handle, 0, alpha, beta)
+        if rc == hip.UNSUPPORTED:
+            return False
+        self._check(rc)
+        return True
+
     def step_rmsnorm(self, out, x, gamma, rows, cols, eps, beta=None, residual=None):
         self._check(self._lib.aionhip_step_rmsnorm(self._ctx, out.handle, x.handle, gamma.handle,
                                                    beta.handle if beta is not None else 0,

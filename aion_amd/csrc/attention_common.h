@@ -25,6 +25,8 @@ struct AttnArgs {
     int q_dtype, kv_dtype;
     float scale, soft_cap;
     unsigned win_left, win_right, win_chunk;
+    int *codes;               // not null: the output leaves as rows prepared for the exact GEMM (PreparedAct::tiled) in place of `out`
+    float *code_scales;
 };
 
 __device__ __forceinline__ unsigned short f32_to_bf16_bits(float x) {

@@ -277,6 +277,9 @@ struct RopeAppend {
 };
 bool gemm_i8_rope_applies(const aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, size_t d);
 int launch_gemm_i8_rope(aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, PreparedAct in, float *q_out, RopeAppend rope);
+// the attention step, its output prepared (tiled) for the matmul behind it in place of p->out, or AIONHIP_UNSUPPORTED with nothing launched where the
+// kernel that the step runs on cannot (attention.hip); `prepared` null: the step
+int run_attention(aionhip_ctx *ctx, const aionhip_attention *p, const PreparedAct *prepared);
 // MatMulNT with an f32 [N,K] operand (matmul_nt_f32.hip): plain f32 arithmetic, any number of rows
 int launch_matmul_nt_f32(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, const float *a, size_t lda, float *c, size_t ldc, float alpha,
                          float beta);

@@ -356,6 +356,25 @@ int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weigh
     return launch_prepared_rows(ctx, down, rows, gated, alpha, beta);
 }
 
+int aionhip_step_attention_matmul(aionhip_ctx *ctx, const aionhip_attention *p, const aionhip_weight *w, aionhip_handle c, size_t ldc, float alpha,
+                                  float beta) {
+    if (!ctx || !p || !w) return AIONHIP_INVALID_ARGUMENT;
+    Batch b;
+    int rc = check_batch(ctx, "attention_matmul", 1, &w, &c, &ldc, b);
+    if (rc) return rc;
+    if (p->h_q > 65535 || p->d_v > 65535 || p->h_q * p->d_v != b.k) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "attention_matmul: K must be heads x head size");
+    if (p->batch == 0 || p->l_q == 0) return AIONHIP_OK;
+    const size_t rows = p->batch * p->l_q;
+    if (rows / p->batch != p->l_q || rows > 0x7FFFFFFFu / b.k || (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_tiled(ctx, b, rows))
+        return set_err(ctx, AIONHIP_UNSUPPORTED, "attention_matmul: %zu rows of K %zu do not run on the exact GEMM", rows, b.k);
+    rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
+    if (rc) return rc;
+    const PreparedAct act = prepared_act_carve(ctx->scratch, rows, b.k, true);
+    rc = run_attention(ctx, p, &act);
+    if (rc) return rc;
+    return launch_prepared_rows(ctx, b, rows, act, alpha, beta);
+}
+
 int aionhip_step_gate_matmul(aionhip_ctx *ctx, const aionhip_weight *w, size_t rows, aionhip_handle gate, aionhip_handle up,
                              aionhip_handle c, size_t ldc, float alpha, float beta) {
     if (!ctx || !w) return AIONHIP_INVALID_ARGUMENT;

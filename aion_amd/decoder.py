@@ -178,11 +178,13 @@ class Decoder:
                 # RoPE1D(q), RoPE1D(k) -> f16 -> append, v -> f16 -> append
                 g.step_rope_append(b["qr"], b["q"], b["k"], b["v"], self.kc[l], self.vc[l], b["positions"], b["write_index"],
                                    1, s, c.max_seq, c.heads, c.kv_heads, c.head_dim, base=c.rope_base)
-            g.step_attention(b["att"], b["qr"], self.kc[l], self.vc[l], (1, s, c.max_seq, c.heads, c.kv_heads, c.head_dim, c.head_dim),
-                             scale, q_dtype=be.F32, kv_dtype=be.F16, window=be.CAUSAL,
-                             query_positions=b["positions"], kv_lengths=b["kv_len"])
-            # MatMul o with beta = 1: x = x + att @ Wo (the residual add rides on the matmul's beta)
-            g.step_matmul(self.w[p + "wo"], b["att"], s, b["x"], beta=1.0)
+            # attention, then MatMul o with beta = 1: x = x + att @ Wo (the residual add rides on the matmul's beta); a prompt's attention leaves
+            # its rows as the exact GEMM reads them
+            shape = (1, s, c.max_seq, c.heads, c.kv_heads, c.head_dim, c.head_dim)
+            options = {"q_dtype": be.F32, "kv_dtype": be.F16, "window": be.CAUSAL, "query_positions": b["positions"], "kv_lengths": b["kv_len"]}
+            if s == 1 or not g.step_attention_matmul(self.w[p + "wo"], b["qr"], self.kc[l], self.vc[l], shape, scale, b["x"], beta=1.0, **options):
+                g.step_attention(b["att"], b["qr"], self.kc[l], self.vc[l], shape, scale, **options)
+                g.step_matmul(self.w[p + "wo"], b["att"], s, b["x"], beta=1.0)
             if s == 1 and c.hidden <= 8192 and c.ffn % 32 == 0:
                 # one row: RMSNorm -> MatMul gate, up -> gate(gelu) -> MatMul down (beta = 1), two launches
                 g.step_rmsnorm_geglu_matmul(self.w[p + "wgate"], self.w[p + "wup"], self.w[p + "wdown"], b["x"], self.gamma, c.eps,

@@ -11,6 +11,7 @@ import sys
 
 import numpy as np
 import pytest
+import torch
 
 from aion_amd import backend as be
 from conftest import norm_err, rms_err
@@ -492,3 +493,44 @@ def test_qkv_rope_append_of_many_tokens_is_the_separate_calls(gpu, dtype, layout
     assert ran or (b, s, hidden) in ((1, 65, 4096), (1, 700, 512))       # (the K of q and of k, v divided differently)
     for t in ws + [x, gamma, pos, widx, q, k, v]:
         t.free()
+
+
+# Attention whose rows leave as the exact GEMM reads them: the bits of the attention step and the matmul, at the edges of the 32-row tiles, over head
+# sizes, layouts, types and windows and for sequences of several lengths; refused, with nothing written, where the attention runs on another kernel or
+# in segments, or the rows are few.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("b,s,t,heads,kv_heads,d,n,q_type,kv_type,window,runs", [
+    (1, 9, 40, 8, 1, 64, 320, "f32", "f16", None, True), (1, 128, 256, 8, 1, 256, 2048, "f32", "f16", None, True), (2, 33, 100, 6, 2, 128, 500, "f16", "f16", None, True),
+    (1, 65, 200, 32, 8, 128, 1024, "bf16", "bf16", (40, 0, 0), True), (3, 17, 64, 2, 2, 256, 96, "f32", "bf16", None, True), (1, 31, 31, 16, 4, 64, 33, "f32", "f16", (8, 3, 0), True),
+    (1, 300, 2000, 8, 1, 128, 512, "f32", "f16", None, False), (1, 1000, 1000, 16, 4, 64, 512, "f32", "f16", None, False), (1, 64, 1500, 4, 1, 64, 512, "f32", "f16", None, False),
+    (1, 4, 64, 8, 1, 64, 512, "f32", "f16", None, False)])
+def test_attention_and_its_matmul_is_the_separate_calls(gpu, dtype, layout, b, s, t, heads, kv_heads, d, n, q_type, kv_type, window, runs):
+    say("attention matmul", dtype, layout, b, s, t, heads, kv_heads, d, n, q_type, kv_type, window)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    gen = torch.Generator().manual_seed(s + t)
+    types = {"f32": (torch.float32, be.F32), "f16": (torch.float16, be.F16), "bf16": (torch.bfloat16, be.BF16)}
+
+    def operand(kind, *shape):
+        return gpu.upload(torch.randn(shape, generator=gen).to(types[kind][0]).contiguous().view(torch.uint8).numpy())
+
+    q, k, v = operand(q_type, b, s, heads, d), operand(kv_type, b, t, kv_heads, d), operand(kv_type, b, t, kv_heads, d)
+    lengths = np.array([max(s, t - 5 * i) for i in range(b)], np.int32)
+    pos, lens = gpu.upload((lengths[:, None] - s + np.arange(s)).astype(np.int32)), gpu.upload(lengths)
+    w = make_weight(gpu, dtype, layout, n, heads * d, seed=n)[1]
+    rows, shape = b * s, (b, s, t, heads, kv_heads, d, d)
+    options = {"q_dtype": types[q_type][1], "kv_dtype": types[kv_type][1], "window": window or be.CAUSAL, "query_positions": pos, "kv_lengths": lens}
+    out = gpu.alloc(4 * rows * heads * d)
+    for alpha, beta in ((1.0, 1.0), (0.5, 0.0)):
+        c = [gpu.upload(np.full((rows, n), 0.25, np.float32)) for _ in range(2)]
+        gpu.step_attention(out, q, k, v, shape, d ** -0.5, **options)
+        gpu.step_matmul(w, out, rows, c[0], alpha=alpha, beta=beta)
+        assert gpu.step_attention_matmul(w, q, k, v, shape, d ** -0.5, c[1], alpha=alpha, beta=beta, **options) == runs
+        want, got = (gpu.download(x, np.float32, (rows, n)) for x in c)
+        if runs:
+            assert np.isfinite(want).all() and np.array_equal(want.view(np.uint32), got.view(np.uint32))
+        else:
+            assert (got == 0.25).all()
+        for x in c:
+            x.free()
+    for x in (q, k, v, pos, lens, w, out):
+        x.free()
