@@ -257,7 +257,7 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         const float prefill_us = (nseg_p > 1 ? 16.f : 12.f) + (float)((tiles64 + nseg_p - 1) / nseg_p) * per_tile * (float)rounds_p;
         if (prefill_us < split_us) split = false;
     }
-    if (a.codes && (!split || HILO || RING)) return AIONHIP_UNSUPPORTED;
+    if (a.codes && (HILO || RING)) return AIONHIP_UNSUPPORTED;
     if (split) {
         // key segments: one 32-key tile per wavefront while that leaves the device under-filled,
         // more tiles per wavefront beyond one workgroup per CU (its LDS tiles fill a CU)

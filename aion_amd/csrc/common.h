@@ -332,6 +332,7 @@ __device__ __forceinline__ float wave_max(float v) {
 // codes and scale 0; else scale = amax / 127, inv = 127 / amax, code = clamp(round-half-away(v * inv), -127, 127).
 // Every lane of the 8 returns its four codes packed into `word`, the block scale and the plain sum of the 32 codes.
 // The one definition every kernel that prepares activations calls, so that they cannot drift apart.
+__device__ __forceinline__ int prepare_act_code(float v, float inv) { return (int)fminf(127.f, fmaxf(-127.f, roundf(v * inv))); }
 __device__ __forceinline__ void prepare_act_block8(float v0, float v1, float v2, float v3, int &word, float &scale, int &sum) {
     float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
     amax = fmaxf(amax, dpp_f<DPP_QUAD_XOR1>(amax));
@@ -343,10 +344,10 @@ __device__ __forceinline__ void prepare_act_block8(float v0, float v1, float v2,
     if (amax != 0.f) {
         scale = amax / 127.f;
         const float inv = 127.f / amax;
-        const int q0 = (int)fminf(127.f, fmaxf(-127.f, roundf(v0 * inv)));
-        const int q1 = (int)fminf(127.f, fmaxf(-127.f, roundf(v1 * inv)));
-        const int q2 = (int)fminf(127.f, fmaxf(-127.f, roundf(v2 * inv)));
-        const int q3 = (int)fminf(127.f, fmaxf(-127.f, roundf(v3 * inv)));
+        const int q0 = prepare_act_code(v0, inv);
+        const int q1 = prepare_act_code(v1, inv);
+        const int q2 = prepare_act_code(v2, inv);
+        const int q3 = prepare_act_code(v3, inv);
         word = (q0 & 0xFF) | ((q1 & 0xFF) << 8) | ((q2 & 0xFF) << 16) | ((q3 & 0xFF) << 24);
         s = q0 + q1 + q2 + q3;
     }
@@ -369,7 +370,7 @@ __device__ __forceinline__ void prepare_act_lane32(float v, int &code, float &sc
     if (amax != 0.f) {
         scale = amax / 127.f;
         const float inv = 127.f / amax;
-        code = (int)fminf(127.f, fmaxf(-127.f, roundf(v * inv)));
+        code = prepare_act_code(v, inv);
     }
 }
 

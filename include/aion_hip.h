@@ -256,8 +256,8 @@ typedef struct aionhip_attention {
 int aionhip_step_attention(aionhip_ctx *ctx, const aionhip_attention *p);
 /* aionhip_step_attention and the matmul of its output rows (w: k = h_q * d_v, C [batch * l_q, n] with row pitch ldc, 0: n) on the exact GEMM, in two
  * launches: the attention kernel writes the rows as the GEMM reads them; p->out is not used. The results are those of the two calls to the bit.
- * AIONHIP_UNSUPPORTED, with nothing launched, where the step or the matmul would run on another kernel (long prompts, few queries over a long
- * cache, a few rows, the bf16 modes): issue the two calls. */
+ * AIONHIP_UNSUPPORTED, with nothing launched, where the step would cut its keys into segments (long prompts of few heads, few queries over a long
+ * cache) or run on the generic kernel, or the matmul on another one (a few rows, the bf16 modes): issue the two calls. */
 int aionhip_step_attention_matmul(aionhip_ctx *ctx, const aionhip_attention *p, const aionhip_weight *w, aionhip_handle c, size_t ldc, float alpha,
                                   float beta);
 /* f32 queries over an f16/bf16 cache: off (default) = q rounded to the cache element type, one MFMA

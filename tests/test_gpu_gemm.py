@@ -496,14 +496,15 @@ def test_qkv_rope_append_of_many_tokens_is_the_separate_calls(gpu, dtype, layout
 
 
 # Attention whose rows leave as the exact GEMM reads them: the bits of the attention step and the matmul, at the edges of the 32-row tiles, over head
-# sizes, layouts, types and windows and for sequences of several lengths; refused, with nothing written, where the attention runs on another kernel or
-# in segments, or the rows are few.
+# sizes, layouts, types and windows, on both kernels of a prompt and for sequences of several lengths; refused, with nothing written, where the
+# attention runs in segments or the rows are few.
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("b,s,t,heads,kv_heads,d,n,q_type,kv_type,window,runs", [
     (1, 9, 40, 8, 1, 64, 320, "f32", "f16", None, True), (1, 128, 256, 8, 1, 256, 2048, "f32", "f16", None, True), (2, 33, 100, 6, 2, 128, 500, "f16", "f16", None, True),
     (1, 65, 200, 32, 8, 128, 1024, "bf16", "bf16", (40, 0, 0), True), (3, 17, 64, 2, 2, 256, 96, "f32", "bf16", None, True), (1, 31, 31, 16, 4, 64, 33, "f32", "f16", (8, 3, 0), True),
     (1, 300, 2000, 8, 1, 128, 512, "f32", "f16", None, False), (1, 1000, 1000, 16, 4, 64, 512, "f32", "f16", None, False), (1, 64, 1500, 4, 1, 64, 512, "f32", "f16", None, False),
-    (1, 4, 64, 8, 1, 64, 512, "f32", "f16", None, False)])
+    (1, 4, 64, 8, 1, 64, 512, "f32", "f16", None, False), (1, 512, 512, 32, 8, 128, 2048, "f32", "f16", None, True), (2, 300, 300, 8, 2, 256, 320, "f32", "f16", None, True),
+    (4, 200, 260, 32, 32, 128, 96, "f16", "f16", (70, 0, 0), True), (2, 500, 501, 16, 16, 64, 512, "f32", "bf16", None, True)])
 def test_attention_and_its_matmul_is_the_separate_calls(gpu, dtype, layout, b, s, t, heads, kv_heads, d, n, q_type, kv_type, window, runs):
     say("attention matmul", dtype, layout, b, s, t, heads, kv_heads, d, n, q_type, kv_type, window)
     gpu.set_gemm_mode(be.GEMM_EXACT_I8)
@@ -515,7 +516,10 @@ def test_attention_and_its_matmul_is_the_separate_calls(gpu, dtype, layout, b, s
 
     q, k, v = operand(q_type, b, s, heads, d), operand(kv_type, b, t, kv_heads, d), operand(kv_type, b, t, kv_heads, d)
     lengths = np.array([max(s, t - 5 * i) for i in range(b)], np.int32)
-    pos, lens = gpu.upload((lengths[:, None] - s + np.arange(s)).astype(np.int32)), gpu.upload(lengths)
+    pos = gpu.upload((lengths[:, None] - s + np.arange(s)).astype(np.int32))
+    if b == 4:
+        lengths[-1] = 0                                      # (a sequence that sees no key: rows of zeros)
+    lens = gpu.upload(lengths)
     w = make_weight(gpu, dtype, layout, n, heads * d, seed=n)[1]
     rows, shape = b * s, (b, s, t, heads, kv_heads, d, d)
     options = {"q_dtype": types[q_type][1], "kv_dtype": types[kv_type][1], "window": window or be.CAUSAL, "query_positions": pos, "kv_lengths": lens}
