@@ -245,6 +245,10 @@ int launch_gemv_mfma(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *c
 bool gemv_slim_applies(const aionhip_ctx *ctx, const aionhip_weight *w, int m);
 int launch_gemv_slim(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
                      float alpha, float beta);
+// weights that the exact GEMM takes and weights that gemv_slim.hip takes, one launch (applies: to the former); `act` tiled
+bool gemm_slim_applies(const aionhip_ctx *ctx, const aionhip_weight *const *gemm, int count, int m);
+int launch_gemm_slim(aionhip_ctx *ctx, const aionhip_weight *const *gemm, float *const *gemm_cs, const size_t *gemm_ldcs, int gemm_count, const aionhip_weight *const *slim,
+                     float *const *slim_cs, const size_t *slim_ldcs, int slim_count, int m, PreparedAct act, float alpha, float beta);
 bool gemv_ksplit_applies(const aionhip_ctx *ctx, const aionhip_weight *w, const float *x);
 int launch_gemv_ksplit(aionhip_ctx *ctx, const aionhip_weight *w, float *c, const float *x, float alpha, float beta);
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,

@@ -73,10 +73,10 @@ __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M 
 // LDS of a wavefront: two groups of four blocks, weight codes and activation scales
 template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
 
+// workgroup `bid` of the kernel's grid (the K slices, if any, are the grid's z)
 template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI = GEMM_PLAIN>
-__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(typename GemmSegsOf<EPI>::type segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
-                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
-                                                                         float *__restrict__ partial, int partial_ld) {
+__device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::type &segs, int bid, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int M, int K,
+                                             int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta, float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
     constexpr bool PAIR = EPI != GEMM_PLAIN, GATE = EPI == GEMM_GATE;
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
     // workgroup -> tile: ids go round-robin over the 8 XCDs; every XCD takes a contiguous run of tiles, row tiles fastest, so that
     // the workgroups that share a weight column tile run on one L2
     const int tiles = row_tiles * col_tiles;
-    const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
+    const int xcd = bid & 7, slot = bid >> 3;
     const int t = xcd * (tiles >> 3) + min(xcd, tiles & 7) + slot;
     const int grp = t / (row_group * col_tiles), gr0 = grp * row_group, gr = min(row_group, row_tiles - gr0);
     const int ct = (t - gr0 * col_tiles) / gr, rt = gr0 + (t - gr0 * col_tiles) - ct * gr;
@@ -535,6 +535,13 @@ __global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gem
             for (int e = 0; e < 4; ++e) put(ch / RQ / NT, ch / RQ % NT, ch % RQ * 4 + e, s[e]);
         }
     }
+}
+
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI = GEMM_PLAIN>
+__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(typename GemmSegsOf<EPI>::type segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
+                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
+                                                                         float *__restrict__ partial, int partial_ld) {
+    gemm_i8_body<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE, EPI>(segs, (int)blockIdx.x, aq, a_scale, M, K, row_tiles, row_group, col_tiles, one_round, alpha, beta, partial, partial_ld);
 }
 
 template <bool Q8, int MT, int NT, int KS, int WGM, int WGN, int RQ> constexpr int gemm_i8_lds_bytes() {

@@ -391,6 +391,9 @@ void launch_r(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
     else launch_k(ctx, gemv_kernel<DT, B, 1>, grid, block, 0, batch, aq, act.scale, act.sum, K, m, alpha, beta);
 }
 
+int rows_instance(int m) { return m == 2 ? 2 : (m <= 4 ? 4 : 8); }
+bool rows_outgrow_lds(int m, size_t k) { return (size_t)rows_instance(m) * 40 * (k >> 5) > ROWS_LDS_CAP; }
+
 template <int DT>
 int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
              PreparedAct act, float alpha, float beta) {
@@ -400,8 +403,8 @@ int launch_b(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs
     }
     // q8 with a K too long for one LDS-resident pass: the activation bytes per weight byte are half of q4's, and
     // operands through L1 (gemv_kernel) then beat two sliced launches (measured at 4096 x 14336, 8 rows)
-    const int bb = m == 2 ? 2 : (m <= 4 ? 4 : 8);
-    if (DT == AIONHIP_Q8_0 && (size_t)bb * 40 * (ws[0]->k >> 5) > ROWS_LDS_CAP) {
+    const int bb = rows_instance(m);
+    if (DT == AIONHIP_Q8_0 && rows_outgrow_lds(m, ws[0]->k)) {
         if (bb == 2) launch_r<DT, 2>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
         else if (bb == 4) launch_r<DT, 4>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
         else launch_r<DT, 8>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
@@ -463,26 +466,34 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
         }
         if (rc != -1) return rc;
     }
-    // (five rows and more over a long K go by the name of the exact GEMM, which takes those that gemv_slim.hip leaves)
+    // (five rows and more over a long K go by the name of the exact GEMM, which takes those that gemv_slim.hip leaves; here they are gemv_slim.hip's)
     const bool q8 = ws[0]->dtype == AIONHIP_Q8_0, long_k = m >= 5 && ws[0]->k > FUSED_PAYS_K && ws[0]->k <= GEMM_I8_MAX_K;
     const char *name = long_k ? (q8 ? "gemm_i8_q8" : "gemm_i8_q4") : q8 ? "gemv_q8" : "gemv_q4";
     ProfScope scope(ctx, name);
-    if (act.tiled) {
+    if (act.tiled && !long_k) {
         const int rc = launch_gemm_i8_few_rows(ctx, ws[0], (size_t)m, act, cs[0], ldcs[0], alpha, beta);
         if (rc) return rc;
         LAUNCH_CHECK(ctx, name);
         return AIONHIP_OK;
     }
-    bool slim = true;
-    for (int i = 0; i < count; ++i) slim = slim && gemv_slim_applies(ctx, ws[i], m);
-    if (slim) {
-        const int rc = launch_gemv_slim(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-        if (rc) return rc;
-        LAUNCH_CHECK(ctx, name);
-        return AIONHIP_OK;
+    // gemv_slim.hip takes all siblings or none where the sums of gemv_rows_kernel, which shares a row among as many lanes as all weights of the call
+    // leave it, depend on them anyway. gemv_kernel's depend on the weight alone, and so do gemv_slim.hip's: there each weight goes its own way.
+    const aionhip_weight *w[2][4];
+    float *c[2][4];
+    size_t ld[2][4];
+    int cnt[2] = {0, 0};                                         // [gemv_slim.hip, the other]
+    bool slim[4], all = true;
+    for (int i = 0; i < count; ++i) all = (slim[i] = gemv_slim_applies(ctx, ws[i], m)) && all;
+    for (int i = 0; i < count; ++i) {
+        const int to = slim[i] && (all || (q8 && rows_outgrow_lds(m, ws[i]->k))) ? 0 : 1;
+        w[to][cnt[to]] = ws[i];
+        c[to][cnt[to]] = cs[i];
+        ld[to][cnt[to]++] = ldcs[i];
     }
-    const int rc = ws[0]->dtype == AIONHIP_Q8_0 ? launch_b<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
-                                                : launch_b<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+    int rc = AIONHIP_OK;
+    if (cnt[0]) rc = launch_gemv_slim(ctx, w[0], c[0], ld[0], cnt[0], m, act, alpha, beta);
+    if (!rc && cnt[1]) rc = q8 ? launch_b<AIONHIP_Q8_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta)
+                               : launch_b<AIONHIP_Q4_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta);
     if (rc) return rc;
     LAUNCH_CHECK(ctx, name);
     return AIONHIP_OK;

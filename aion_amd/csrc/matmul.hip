@@ -61,21 +61,28 @@ static bool fused_row_pays(const Batch &b) {
     return b.k <= FUSED_MAX_K && n >= 16384 && bytes <= ((size_t)1 << 30);
 }
 
-// Prepared rows against the weights of `b`: the GEMV kernels up to eight rows, except five to eight rows over a K past 4096,
-// where gemv_rows_kernel walks K with all eight accumulator sets live and falls far behind the exact GEMM (8 x 14336 x 8192: q8 78 against 31 us,
-// q4 65 against 25; 8 x 6144 x 4128 20 / 15, 18 / 11; q8 up to 4096 columns is level there or, below 3072, up to a fifth ahead on the
-// GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2) and gemv_slim_kernel does not apply; the GEMM beyond eight rows.
-static bool rows_on_gemv(const aionhip_ctx *ctx, const Batch &b, size_t m) {
-    if (m > GEMV_MAX_M || b.k > GEMM_I8_MAX_K || !(m >= 5 && b.k > FUSED_PAYS_K)) return m <= GEMV_MAX_M;
-    for (size_t i = 0; i < b.count; ++i)
-        if (!gemv_slim_applies(ctx, b.w[i], (int)m)) return false;
-    return true;
+// Five to eight rows over a K past 4096: gemv_rows_kernel walks K with all eight accumulator sets live and falls far behind the exact GEMM
+// (8 x 14336 x 8192: q8 78 against 31 us, q4 65 against 25; 8 x 6144 x 4128 20 / 15, 18 / 11; q8 up to 4096 columns is level there or, below 3072, up to a
+// fifth ahead on the GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2), so they run on gemv_slim_kernel where it applies and on the exact GEMM
+// elsewhere. Which of the two is decided weight by weight: the sums of both depend on the weight alone, and a weight has the same bits by itself and
+// beside any siblings. Siblings of both kinds share the preparation, tiled, and are two launches.
+static bool rows_over_long_k(const Batch &b, size_t m) { return m >= 5 && m <= GEMV_MAX_M && b.k > FUSED_PAYS_K && b.k <= GEMM_I8_MAX_K; }
+static size_t slim_weights(const aionhip_ctx *ctx, const Batch &b, size_t m) {
+    size_t slim = 0;
+    for (size_t i = 0; i < b.count; ++i) slim += gemv_slim_applies(ctx, b.w[i], (int)m);
+    return slim;
 }
-// which form of the preparation the kernel behind launch_prepared_rows reads
-static bool rows_tiled(const aionhip_ctx *ctx, const Batch &b, size_t m) {
+// whether every weight runs on the exact GEMM's kernel
+static bool rows_on_gemm(const aionhip_ctx *ctx, const Batch &b, size_t m) {
     if (b.k > GEMM_I8_MAX_K) return false;
-    return !rows_on_gemv(ctx, b, m) || gemv_rows_on_gemm(ctx, b.w, (int)b.count, (int)m);
+    if (rows_over_long_k(b, m)) return slim_weights(ctx, b, m) == 0;
+    return m > GEMV_MAX_M || gemv_rows_on_gemm(ctx, b.w, (int)b.count, (int)m);
 }
+// which form of the preparation the kernels behind launch_prepared_rows read
+static bool rows_tiled(const aionhip_ctx *ctx, const Batch &b, size_t m) {
+    return rows_over_long_k(b, m) ? slim_weights(ctx, b, m) < b.count : rows_on_gemm(ctx, b, m);
+}
+// prepared rows against the weights of `b`: the GEMV kernels up to eight rows (but see above), the GEMM beyond
 static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, PreparedAct act, float alpha, float beta) {
     if (m > GEMV_MAX_M && b.k > GEMM_I8_MAX_K) {                 // rows past the GEMM's addressing
         Batch part = b;
@@ -88,8 +95,22 @@ static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, Prep
         }
         return AIONHIP_OK;
     }
-    if (rows_on_gemv(ctx, b, m))
-        return launch_gemv_batch(ctx, b.w, b.c, b.ldc, (int)b.count, (int)m, act, alpha, beta);
+    if (rows_over_long_k(b, m)) {
+        Batch slim, rest;
+        for (size_t i = 0; i < b.count; ++i) {
+            Batch &to = gemv_slim_applies(ctx, b.w[i], (int)m) ? slim : rest;
+            to.w[to.count] = b.w[i];
+            to.c[to.count] = b.c[i];
+            to.ldc[to.count++] = b.ldc[i];
+        }
+        if (rest.count && slim.count && gemm_slim_applies(ctx, rest.w, (int)rest.count, (int)m))
+            return launch_gemm_slim(ctx, rest.w, rest.c, rest.ldc, (int)rest.count, slim.w, slim.c, slim.ldc, (int)slim.count, (int)m, act, alpha, beta);
+        int rc = AIONHIP_OK;
+        if (rest.count) rc = launch_gemm_i8_batch(ctx, rest.w, rest.c, rest.ldc, (int)rest.count, m, act, alpha, beta);
+        if (!rc && slim.count) rc = launch_gemv_batch(ctx, slim.w, slim.c, slim.ldc, (int)slim.count, (int)m, act, alpha, beta);
+        return rc;
+    }
+    if (m <= GEMV_MAX_M) return launch_gemv_batch(ctx, b.w, b.c, b.ldc, (int)b.count, (int)m, act, alpha, beta);
     // sibling weights (q/k/v, gate/up) share one launch, four at a time
     for (size_t i = 0; i < b.count; i += 4) {
         const size_t cnt = b.count - i < 4 ? b.count - i : 4;
@@ -288,7 +309,7 @@ int aionhip_step_rmsnorm_qkv_rope_append_rows(aionhip_ctx *ctx, const aionhip_we
     if (b == 0 || s == 0) return AIONHIP_OK;
     const size_t rows = b * s;
     if (((x | gamma | beta_norm) & 15) || (q_out & 3) || ((k_cache | v_cache) & 1) || rows / b != s || rows > 0x7FFFFFFFu || t_cap > 0x7FFFFFFFu ||
-        (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_tiled(ctx, in, rows) || !gemm_i8_rope_applies(ctx, qkv, rows, d))
+        (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_on_gemm(ctx, in, rows) || !gemm_i8_rope_applies(ctx, qkv, rows, d))
         return set_err(ctx, AIONHIP_UNSUPPORTED, "qkv_rope_append_rows: %zu rows of K %zu and heads of %zu do not run on the exact GEMM's rope instances", rows, in.k, d);
     const size_t half = d / 2;
     size_t rope_pairs = (size_t)floorf(rope_proportion * (float)half);
@@ -344,7 +365,7 @@ int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weigh
     if (!(eps > 0.f) || !(eps < INFINITY)) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "geglu_matmul_rows: eps must be positive and finite");
     if (w_gate->n != w_up->n || down.k != w_gate->n) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "geglu_matmul_rows: gate and up must match, down must take their outputs");
     if (((x | gamma | beta_norm) & 15) || (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || rows > 0x7FFFFFFFu ||
-        !rows_tiled(ctx, in, rows) || !rows_tiled(ctx, down, rows) || !gemm_i8_gate_applies(ctx, w_gate, rows))
+        !rows_on_gemm(ctx, in, rows) || !rows_on_gemm(ctx, down, rows) || !gemm_i8_gate_applies(ctx, w_gate, rows))
         return set_err(ctx, AIONHIP_UNSUPPORTED, "geglu_matmul_rows: %zu rows against %zu x %zu do not run on the exact GEMM's gate instances", rows, (size_t)w_gate->n, in.k);
     const size_t in_bytes = (prepared_act_bytes(rows, in.k) + 255) & ~(size_t)255;
     rc = ensure_scratch(ctx, in_bytes + prepared_act_bytes(rows, down.k));
@@ -365,7 +386,7 @@ int aionhip_step_attention_matmul(aionhip_ctx *ctx, const aionhip_attention *p, 
     if (p->h_q > 65535 || p->d_v > 65535 || p->h_q * p->d_v != b.k) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "attention_matmul: K must be heads x head size");
     if (p->batch == 0 || p->l_q == 0) return AIONHIP_OK;
     const size_t rows = p->batch * p->l_q;
-    if (rows / p->batch != p->l_q || rows > 0x7FFFFFFFu / b.k || (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_tiled(ctx, b, rows))
+    if (rows / p->batch != p->l_q || rows > 0x7FFFFFFFu / b.k || (rows > GEMV_MAX_M && ctx->gemm_mode != AIONHIP_GEMM_EXACT_I8) || !rows_on_gemm(ctx, b, rows))
         return set_err(ctx, AIONHIP_UNSUPPORTED, "attention_matmul: %zu rows of K %zu do not run on the exact GEMM", rows, b.k);
     rc = ensure_scratch(ctx, prepared_act_bytes(rows, b.k));
     if (rc) return rc;

@@ -431,7 +431,7 @@ aionhip_handle aionhip_session::residual_target(const aionhip_step *steps, size_
 }
 
 // A pattern starting at step i run as one call: returns the number of steps consumed (0 = none matched, run step i alone).
-// Every pattern's entry point gives the separate steps' results to the bit; one that answers AIONHIP_UNSUPPORTED has
+// Every pattern's entry point gives the separate steps' results (MatMuls that share a launch: see aionhip_step_matmul_batch); one that answers AIONHIP_UNSUPPORTED has
 // launched nothing, and the steps then run one by one.
 size_t aionhip_session::try_fused(const aionhip_step *steps, size_t count, size_t i, int *rc_out) {
     const aionhip_step &st = steps[i];

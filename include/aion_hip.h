@@ -154,8 +154,12 @@ int aionhip_step_matmul_static(aionhip_ctx *ctx, const aionhip_weight *b, size_t
 /* Several matmul steps that read the SAME activation (q/k/v, gate/up) as one call: the activation
  * is prepared once and, for m <= 8, all weights stream through one launch. aion keeps such
  * siblings as separate MatMul/MatMulNT steps (graph/opt/weight_layout.zig:72-115 re-lays but never
- * concatenates); every C[i] is what the separate step would have produced. count <= 4; weights
- * share k and dtype; ldc may be NULL (each n). */
+ * concatenates); every C[i] is what the separate step would have produced: to the bit for more than
+ * eight rows (exact mode, k up to 2^26) and for five to eight over a k of 4097 .. 2^26, whose sums are taken in an order that
+ * depends on the weight alone, and for one row over a k of up to 4096. For other calls the order of a
+ * weight's f32 block sums (the same terms) may depend on all weights of the launch: last bits then
+ * differ. In the bf16 mode all weights of a call run on one kernel, the bf16 one only if it suits each.
+ * count <= 4; weights share k and dtype; ldc may be NULL (each n). */
 int aionhip_step_matmul_batch(aionhip_ctx *ctx, size_t count, const aionhip_weight *const *b, size_t m,
                               aionhip_handle a, size_t lda, const aionhip_handle *c, const size_t *ldc,
                               float alpha, float beta);
@@ -499,7 +503,8 @@ typedef struct aionhip_session aionhip_session;
 /* Backend.createSession (backend/backend.zig:46-52). A session belongs to one context and one thread, and is destroyed before
  * its context (it frees its re-laid weights through it). */
 int aionhip_session_create(aionhip_ctx *ctx, aionhip_session **out);
-/* Which step patterns a session may run as one call (default: both). Results are the separate steps' to the bit either way.
+/* Which step patterns a session may run as one call (default: both). Results are the separate steps', to the bit where
+ * aionhip_step_matmul_batch says so of MatMuls that share a launch, within the rounding of a reordered f32 sum elsewhere.
  * AIONHIP_FUSE_SIBLINGS: consecutive MatMul / MatMulNT steps reading one activation share its preparation and, up to eight
  * rows, one launch (aionhip_step_matmul_batch); every tensor of the list is still written.
  * AIONHIP_FUSE_WORKSPACE: a step whose output is an AIONHIP_TENSOR_WORKSPACE tensor read only by the step(s) right behind

@@ -725,3 +725,28 @@ def test_few_weight_rows_siblings(gpu, orc, dtype, layout, m, ns):
         c.free()
         w.free()
     a_buf.free()
+
+
+# A weight's results do not depend on its siblings in the call: beside others of few and of many rows - all on the slim kernel with 16, 8 and 4
+# wavefronts to a K, some on it and some on the exact GEMM's kernel (five rows and more) or, q8 over a K that outgrows LDS, on gemv_kernel -
+# every output has the bits that the weight gives by itself. K of fewer stages than runs (11 at 1408), of odd counts, and of many.
+@pytest.mark.parametrize("dtype,layout,m,ns,k", [(be.Q8_0, be.ROWS_NK, 8, (4096, 1024, 1024), 8192), (be.Q8_0, be.KMAJOR_KN, 5, (5120, 1024, 1000), 5120),
+                                                 (be.Q8_0, be.ROWS_NK, 6, (12300, 300, 4100), 4224), (be.Q4_0, be.KMAJOR_KN, 5, (5120, 1024, 1024), 5120),
+                                                 (be.Q4_0, be.KMAJOR_KN, 8, (300, 12300, 8208), 6272), (be.Q4_0, be.KMAJOR_KN, 7, (4000, 4000, 90, 40), 11008),
+                                                 (be.Q8_0, be.ROWS_NK, 3, (6000, 40, 12300), 14848), (be.Q8_0, be.ROWS_NK, 4, (4000, 700), 15104),
+                                                 (be.Q4_0, be.KMAJOR_KN, 3, (4000, 5000, 300), 1408)])
+def test_few_weight_rows_keep_their_bits_beside_siblings(gpu, orc, dtype, layout, m, ns, k):
+    say("slim siblings' bits", dtype, layout, m, ns, k)
+    made = [make_weight(gpu, orc, dtype, layout, n, k, seed=n + i, std=0.05)[1] for i, n in enumerate(ns)]
+    a_buf = gpu.upload(np.random.default_rng(m + k).standard_normal((m, k)).astype(np.float32))
+    gamma, c_bufs = gpu.upload(np.ones(k, np.float32)), [gpu.alloc(m * n * 4) for n in ns]
+    for call in (lambda ws, cs: gpu.step_matmul_batch(ws, a_buf, m, cs), lambda ws, cs: gpu.step_rmsnorm_matmul(ws, a_buf, gamma, m, cs, 1e-6)):
+        call(made, c_bufs)
+        batch = [gpu.download(c, np.uint32, (m, n)) for c, n in zip(c_bufs, ns)]
+        for w, n, c, want in zip(made, ns, c_bufs, batch):
+            if m < 5 and n >= 12288:                             # (two to four rows: by itself on the exact GEMM's kernel)
+                continue
+            call([w], [c])
+            assert np.array_equal(gpu.download(c, np.uint32, (m, n)), want), n
+    for t in made + [a_buf, gamma] + c_bufs:
+        t.free()

@@ -321,8 +321,8 @@ pub const HipBackend = struct {
         }
     };
 
-    // What aionhip_session_execute folds (each gives the separate steps' results bit for bit; AIONHIP_FUSE_* of
-    // aionhip_session_set_fusion switches them off):
+    // What aionhip_session_execute folds (each gives the separate steps' results, last bits of MatMuls that share a
+    // launch aside: aionhip_step_matmul_batch; AIONHIP_FUSE_* of aionhip_session_set_fusion switches them off):
     //   RMSNorm, MatMul x3 (q,k,v), RoPE1D x2, Cast f16 x2, SequenceAppend x2, one token -> aionhip_step_rmsnorm_qkv_rope_append
     //   RMSNorm, MatMul x2 (gate, up), gate(gelu), MatMul (down), one row              -> aionhip_step_rmsnorm_geglu_matmul
     //   RMSNorm, MatMul(s)                                                             -> aionhip_step_rmsnorm_matmul
