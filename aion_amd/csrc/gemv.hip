@@ -451,26 +451,26 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
                       PreparedAct act, float alpha, float beta) {
     if (m < 1 || m > 8) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: m=%d outside 1..8", m);
     if (count < 1 || count > 4) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "gemv: %d weights in one launch (1..4)", count);
+    const bool q8 = ws[0]->dtype == AIONHIP_Q8_0;
     if (!act.tiled && gemv_mfma_applies(ctx, ws, count, m)) {
-        const char *mname = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8_mfma" : "gemv_q4_mfma";
-        ProfScope scope(ctx, mname);
         // q4 from five rows on, up to six workgroups of gemv_slim.hip per CU: its 16-row workgroups start sooner than ones that copy all rows' K to LDS (8 x
         // 14336 x 2048 1.47 times as fast, x 4096 1.34, 5 x 20480 x 4096 1.21; 32768 x 3072 0.92)
         size_t tiles = 0;
         for (int i = 0; i < count; ++i) tiles += (ws[i]->n + 15) / 16;
-        const bool slim = ws[0]->dtype == AIONHIP_Q4_0 && m >= 5 && ws[0]->k >= 2048 && tiles <= 6 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256);
-        const int rc = slim ? launch_gemv_slim(ctx, ws, cs, ldcs, count, m, act, alpha, beta) : launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+        if (!q8 && m >= 5 && ws[0]->k >= 2048 && tiles <= 6 * (ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256))
+            return launch_gemv_slim(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+        const char *mname = q8 ? "gemv_q8_mfma" : "gemv_q4_mfma";
+        ProfScope scope(ctx, mname);
+        const int rc = launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
         if (rc == AIONHIP_OK) {
             LAUNCH_CHECK(ctx, mname);
             return AIONHIP_OK;
         }
         if (rc != -1) return rc;
     }
-    // (five rows and more over a long K go by the name of the exact GEMM, which takes those that gemv_slim.hip leaves; here they are gemv_slim.hip's)
-    const bool q8 = ws[0]->dtype == AIONHIP_Q8_0, long_k = m >= 5 && ws[0]->k > FUSED_PAYS_K && ws[0]->k <= GEMM_I8_MAX_K;
-    const char *name = long_k ? (q8 ? "gemm_i8_q8" : "gemm_i8_q4") : q8 ? "gemv_q8" : "gemv_q4";
+    const char *name = q8 ? "gemv_q8" : "gemv_q4";
     ProfScope scope(ctx, name);
-    if (act.tiled && !long_k) {
+    if (act.tiled) {
         const int rc = launch_gemm_i8_few_rows(ctx, ws[0], (size_t)m, act, cs[0], ldcs[0], alpha, beta);
         if (rc) return rc;
         LAUNCH_CHECK(ctx, name);
@@ -492,8 +492,8 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
     }
     int rc = AIONHIP_OK;
     if (cnt[0]) rc = launch_gemv_slim(ctx, w[0], c[0], ld[0], cnt[0], m, act, alpha, beta);
-    if (!rc && cnt[1]) rc = q8 ? launch_b<AIONHIP_Q8_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta)
-                               : launch_b<AIONHIP_Q4_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta);
+    if (rc || !cnt[1]) return rc;
+    rc = q8 ? launch_b<AIONHIP_Q8_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta) : launch_b<AIONHIP_Q4_0>(ctx, w[1], c[1], ld[1], cnt[1], m, act, alpha, beta);
     if (rc) return rc;
     LAUNCH_CHECK(ctx, name);
     return AIONHIP_OK;

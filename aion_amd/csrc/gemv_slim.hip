@@ -278,8 +278,13 @@ static int launch_slim(aionhip_ctx *ctx, const aionhip_weight *const *ws, float 
 }
 
 int launch_gemv_slim(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act, float alpha, float beta) {
-    return ws[0]->dtype == AIONHIP_Q8_0 ? launch_slim<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
-                                        : launch_slim<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+    const char *name = ws[0]->dtype == AIONHIP_Q8_0 ? "gemv_q8_slim" : "gemv_q4_slim";
+    ProfScope scope(ctx, name);
+    const int rc = ws[0]->dtype == AIONHIP_Q8_0 ? launch_slim<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
+                                                : launch_slim<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+    if (rc) return rc;
+    LAUNCH_CHECK(ctx, name);
+    return AIONHIP_OK;
 }
 
 bool gemm_slim_applies(const aionhip_ctx *ctx, const aionhip_weight *const *gemm, int count, int m) {
@@ -296,9 +301,9 @@ int launch_gemm_slim(aionhip_ctx *ctx, const aionhip_weight *const *gemm, float 
     static_assert(LDS <= 64 * 1024, "no attribute to set");
     GemmSegs segs, slim_segs;
     const int gemm_tiles = fill_segs(segs, gemm, gemm_cs, gemm_ldcs, gemm_count, 32), slim_tiles = fill_segs(slim_segs, slim, slim_cs, slim_ldcs, slim_count, SL_ROWS);
-    ProfScope scope(ctx, "gemm_i8_q4");
+    ProfScope scope(ctx, "gemm_i8_q4_slim");
     launch_k(ctx, gemm_slim_q4_kernel, dim3((unsigned)(gemm_tiles + slim_tiles)), dim3(64 * GS_KS), LDS, segs, slim_segs, (const uint8_t *)act.q, (const float *)act.scale,
              (int)gemm[0]->k, m, gemm_tiles, alpha, beta);
-    LAUNCH_CHECK(ctx, "gemm_i8_q4");
+    LAUNCH_CHECK(ctx, "gemm_i8_q4_slim");
     return AIONHIP_OK;
 }

@@ -2,8 +2,9 @@
 // graph/program/compiler.zig:189-239,337-357), activation preparation, kernel routing
 // (the counterpart of cpu/exec/matmul.zig:233-296 `matvecRoute` / `gemm2D`):
 //   m == 1, k <= 4096, 16-byte aligned A  -> gemv_fused_kernel (activation prepared in the kernel)
-//   m <= 8                                -> prepare_act_kernel + gemv_kernel / gemv_rows_kernel (gemm_i8_kernel
-//                                            where gemv_rows_on_gemm says so)
+//   m == 1, longer k                      -> gemv_ksplit_kernel (one weight), else prepare_act_kernel + gemv_kernel
+//   m <= 8                                -> prepare_act_kernel + gemv_mfma_kernel (many weight rows), gemv_slim_kernel (few), gemv_rows_kernel /
+//                                            gemv_kernel (the rest) or gemm_i8_kernel (gemv_rows_on_gemm; five rows and more over k > 4096)
 //   m  > 8                                -> gemm_i8_kernel (exact) or gemm_bf16_wide_kernel
 // and the decode fusions built on the single-row kernel: RMSNorm / gelu-gate prologues, the q/k/v + RoPE +
 // cache-append launch and the GeGLU block (two launches).
@@ -107,7 +108,7 @@ static int launch_prepared_rows(aionhip_ctx *ctx, const Batch &b, size_t m, Prep
             return launch_gemm_slim(ctx, rest.w, rest.c, rest.ldc, (int)rest.count, slim.w, slim.c, slim.ldc, (int)slim.count, (int)m, act, alpha, beta);
         int rc = AIONHIP_OK;
         if (rest.count) rc = launch_gemm_i8_batch(ctx, rest.w, rest.c, rest.ldc, (int)rest.count, m, act, alpha, beta);
-        if (!rc && slim.count) rc = launch_gemv_batch(ctx, slim.w, slim.c, slim.ldc, (int)slim.count, (int)m, act, alpha, beta);
+        if (!rc && slim.count) rc = launch_gemv_slim(ctx, slim.w, slim.c, slim.ldc, (int)slim.count, (int)m, act, alpha, beta);
         return rc;
     }
     if (m <= GEMV_MAX_M) return launch_gemv_batch(ctx, b.w, b.c, b.ldc, (int)b.count, (int)m, act, alpha, beta);

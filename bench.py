@@ -464,7 +464,7 @@ def run_sweep(gpu, be, q4_blocks):
             for m in (1, 4, 8):
                 x = gpu.upload(rng.standard_normal((m, k)).astype(np.float32))
                 y = gpu.alloc(m * n * 4)
-                # five to eight rows over a K past 4096 run on the exact GEMM, everything else under a GEMV kernel's name
+                # five to eight rows over a K past 4096 may run on the exact GEMM, everything else runs under a GEMV kernel's name
                 ms = time_kernel(gpu, ws, x, y, m, (kname, "gemm_i8_" + kname[-2:]) if m >= 5 and k > 4096 else kname)
                 by = algorithmic_bytes(bb, n, k, m)
                 ll = gpu.last_launch()

@@ -231,7 +231,9 @@ int aionhip_set_bf16_weight_copies(aionhip_ctx *ctx, int on);
 void aionhip_weight_drop_bf16(aionhip_ctx *ctx, aionhip_weight *w);       /* waits for the context's stream */
 int aionhip_bf16_copy_stats(aionhip_ctx *ctx, uint64_t *weights, uint64_t *bytes);
 /* Name of the kernel the last matmul/attention step launched (the reference's tests assert
- * which kernel ran after a parity check, backend/gpu/test_gpu_backend.zig:1116-1162). */
+ * which kernel ran after a parity check, backend/gpu/test_gpu_backend.zig:1116-1162). A call of up to eight
+ * rows whose single weight runs on the exact GEMM's kernel by the GEMV's routing reports gemv_q4 / gemv_q8 (aionhip_last_launch
+ * has the instance). */
 const char *aionhip_last_kernel(aionhip_ctx *ctx);
 /* The last launch a matmul or fused step made, for reports that are matched against a kernel trace: the kernel instance's
  * name as a trace prints it (demangled, template arguments included, no parameter list), its grid in workgroups, its

@@ -108,8 +108,7 @@ def test_gemv_small_and_ragged_shapes(gpu, orc, dtype, layout, m):
         got = gpu.matmul(w, a)
         want = oracle_matmul(orc, dtype, layout, a, blocks, n)
         assert norm_err(got, want) < TOL and rms_err(got, want) < RMS_TOL, (n, k, norm_err(got, want), rms_err(got, want))
-        want_kernel = "gemv_q8" if dtype == be.Q8_0 else "gemv_q4"
-        assert gpu.last_kernel() == (want_kernel + "_fused" if m == 1 else want_kernel)
+        assert gpu.last_kernel() == ("gemv_%s_fused" % ("q8" if dtype == be.Q8_0 else "q4") if m == 1 else rows_kernel(dtype == be.Q8_0, m, n, k))
         w.free()
 
 
@@ -241,7 +240,7 @@ def test_single_row_q4_eight_alternating_slices(gpu, orc):
 
 # Sibling weights at 3..8 rows whose rows together reach the matrix-pipe GEMV's range (gate / up of a feed-forward block, a short
 # prompt): one launch walks the tiles of all weights; ragged column counts, a sibling far smaller than the others, alpha / beta.
-@pytest.mark.parametrize("dtype,m,ns,k", [(be.Q4_0, 6, (8200, 8192), 2048), (be.Q4_0, 5, (14000, 40, 1000), 4096), (be.Q4_0, 3, (40000, 30000), 2304),
+@pytest.mark.parametrize("dtype,m,ns,k", [(be.Q4_0, 6, (16400, 16384), 2048), (be.Q4_0, 5, (24000, 40, 1000), 4096), (be.Q4_0, 3, (40000, 30000), 2304),
                                           (be.Q8_0, 4, (33000, 33000), 2048)])
 def test_sibling_weights_share_a_matrix_pipe_gemv_launch(gpu, orc, dtype, m, ns, k):
     say("sibling gemv mfma", dtype, m, ns, k)
@@ -334,13 +333,15 @@ def test_exact_gemm_shapes_and_edges(gpu, orc, dtype, layout, m, n, k):
 # 2..8 activation rows (gemv_rows_kernel): row counts that fill a 2-, 4- or 8-row instance only partly, N that is
 # not a multiple of the rows a wavefront works on, K of one LDS pass, K that needs most of a CU's LDS (16384 at 4 rows) and K
 # long enough to run as several K-range launches (32768 at 3 rows), alpha/beta on a pre-filled C. Some shapes (5..8 rows, many
-# columns, K up to 4096) run on the exact GEMM's kernel under the same name: ragged N, K of two and of many groups. Five to eight
-# rows over a K past 4096 take the exact GEMM (it is far ahead there). Many weight rows over a K of 1024 ... 4096 take the matrix-pipe GEMV (gemv_mfma_kernel; conftest.rows_kernel states where): one wavefront per
-# 16-row tile and two sharing a tile's K (14400 rows), ragged N, K of 8 / 9 / 16 stages, 3 ... 8 rows, both weight types.
+# columns, K up to 4096) run on the exact GEMM's kernel under the same name: ragged N, K of two and of many groups. Weights of few rows take
+# the slim GEMV, five to eight rows over a K past 4096 that or the exact GEMM. Many weight rows over a K of 1024 ... 4096 take the
+# matrix-pipe GEMV (gemv_mfma_kernel; conftest.rows_kernel states where; q4 at five rows and more from 24577 rows on, the slim one below): ragged N, K
+# of 8 / 9 / 16 stages, 3 ... 8 rows, both weight types.
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("m,n,k", [(2, 70, 96), (3, 1001, 1056), (5, 333, 2048), (8, 1030, 14336), (7, 4100, 7200), (4, 9000, 512),
                                    (5, 16390, 256), (8, 20001, 2048), (6, 16384, 4096), (4, 1030, 16384), (3, 300, 32768),
-                                   (5, 70, 4128), (8, 14336, 8192), (5, 14400, 4096), (3, 65600, 2048), (8, 65539, 2304), (4, 14336, 4096), (6, 65552, 4096)])
+                                   (5, 70, 4128), (8, 14336, 8192), (5, 14400, 4096), (3, 65600, 2048), (8, 65539, 2304), (4, 14336, 4096), (6, 65552, 4096),
+                                   (5, 24577, 4096), (6, 24584, 2048)])
 def test_decode_gemv_two_to_eight_rows(gpu, orc, dtype, layout, m, n, k):
     say("gemv rows", dtype, layout, m, n, k)
     blocks, w = make_weight(gpu, orc, dtype, layout, n, k, seed=m * 31 + n + k, std=0.05)
