@@ -462,11 +462,9 @@ int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *
         const char *mname = q8 ? "gemv_q8_mfma" : "gemv_q4_mfma";
         ProfScope scope(ctx, mname);
         const int rc = launch_gemv_mfma(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
-        if (rc == AIONHIP_OK) {
-            LAUNCH_CHECK(ctx, mname);
-            return AIONHIP_OK;
-        }
-        if (rc != -1) return rc;
+        if (rc) return rc;
+        LAUNCH_CHECK(ctx, mname);
+        return AIONHIP_OK;
     }
     const char *name = q8 ? "gemv_q8" : "gemv_q4";
     ProfScope scope(ctx, name);

@@ -17,13 +17,11 @@
 //                        4(g & 1) .. +3 of block kb + (g >> 1): every lane rescales and accumulates real results, and the two
 //                        lane halves are added once per tile.
 //
-// Weights never pass through registers on their way in: every wavefront owns a ring of NSTG stages in LDS, a stage being 8
+// Weights never pass through registers on their way in: every wavefront owns a ring of MF_NSTG stages in LDS, a stage being 8
 // quant blocks of its 16 rows plus their f16 scales, filled by LDS-writing loads (whole 128-byte lines per row) and waited
 // for by count. The 16-byte chunks of a row are XOR-swizzled on the global side so that the operand reads of the 64 lanes
-// fall into distinct banks. The activations (codes, scales, -8 * sums) of the launch's K range sit in LDS once per
+// fall into distinct banks. The activations (codes, scales, -8 * sums) sit in LDS once per
 // workgroup, shared by its four wavefronts and by every tile the workgroup walks (persistent grid).
-// KS wavefronts share a tile when there are few weight rows, each taking every KS-th stage; their partial sums are added in
-// wavefront order through LDS, so the result does not depend on timing.
 #include "common.h"
 
 namespace {
@@ -31,7 +29,8 @@ namespace {
 using i32x4 = __attribute__((ext_vector_type(4))) int;
 using u32x2 = __attribute__((ext_vector_type(2))) unsigned int;
 
-constexpr int MF_ROWS = 16, MF_SB = 8;          // weight rows per tile, quant blocks per stage
+constexpr int MF_ROWS = 16, MF_SB = 8, MF_NSTG = 4;      // weight rows per tile, quant blocks per stage, stages of a wavefront's ring
+constexpr size_t MF_MIN_K = 1024, MF_MAX_K = 4096;
 template <int DT>
 struct MfCfg {
     static constexpr bool Q8 = DT == AIONHIP_Q8_0;
@@ -56,25 +55,22 @@ struct MfBatch {
     int count, tiles;
 };
 
-template <int DT, int NSTG, int KS>
+template <int DT>
 __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32x4 *__restrict__ aq, const float *__restrict__ a_scale,
-                                                        const int *__restrict__ a_sum, int K, int m, int kb0, int kbn, float alpha, float beta) {
+                                                        const int *__restrict__ a_sum, int K, int m, float alpha, float beta) {
     using Cfg = MfCfg<DT>;
     constexpr bool Q8 = Cfg::Q8;
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mf[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n = lane & 15, g = lane >> 4;
     const int KB = K >> 5;
-    // LDS: [wave rings][activation codes: kbn x 8 rows x 32 B][scales: kbn x 8 f32][q4: -8 * sums: kbn x 8 i32][KS > 1: partial sums][16 zero bytes]
-    unsigned char *ring = s_mf + wave * (NSTG * Cfg::STAGE);
-    unsigned char *s_act = s_mf + 4 * NSTG * Cfg::STAGE;
-    float *s_as = (float *)(s_act + (size_t)kbn * 256);
-    int *s_bias = (int *)(s_as + kbn * 8);
+    // LDS: [wave rings][activation codes: KB x 8 rows x 32 B][scales: KB x 8 f32][q4: -8 * sums: KB x 8 i32][16 zero bytes]
+    unsigned char *ring = s_mf + wave * (MF_NSTG * Cfg::STAGE);
+    unsigned char *s_act = s_mf + 4 * MF_NSTG * Cfg::STAGE;
+    float *s_as = (float *)(s_act + (size_t)KB * 256);
+    int *s_bias = (int *)(s_as + KB * 8);
 
-    constexpr int TPW = 4 / KS;                                  // tiles a workgroup works on at once
-    const int kpart = wave % KS;
-    const int stages = kbn / MF_SB;                              // the launcher passes whole stages only
-    const int my_stages = (stages - kpart + KS - 1) / KS;        // stages kpart, kpart + KS, ...
+    const int stages = KB / MF_SB;                               // (K is whole stages)
     const size_t row_bytes = Q8 ? (size_t)K : (size_t)(K >> 1);
 
     // per-lane constants of the loads: instruction j of a stage covers rows j*RPI .. +RPI; lane -> (row, slot);
@@ -83,7 +79,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
     auto swz = [](int row) { return Q8 ? (row & 15) : ((row >> 1) & 7); };
 
     struct Tile {
-        const uint8_t *wrow[Cfg::NLD];      // this lane's row of each load instruction, at the launch's first block
+        const uint8_t *wrow[Cfg::NLD];      // this lane's row of each load instruction
         const unsigned char *srow;          // this lane's piece of the scales: row lane >> 2, blocks 2 * (lane & 3) ..
         int seg, row0, valid;
     };
@@ -102,14 +98,14 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
         for (int j = 0; j < Cfg::NLD; ++j) {
             const int rl = j * Cfg::RPI + l_row;
             const int row = min(t.row0 + rl, N - 1);
-            t.wrow[j] = batch.seg[si].qs + (size_t)row * row_bytes + (size_t)kb0 * (Q8 ? 32 : 16) + ((l_slot ^ swz(rl)) * 16);
+            t.wrow[j] = batch.seg[si].qs + (size_t)row * row_bytes + ((l_slot ^ swz(rl)) * 16);
         }
-        t.srow = (const unsigned char *)(batch.seg[si].sc + (size_t)min(t.row0 + (lane >> 2), N - 1) * KB + kb0) + (lane & 3) * 4;
+        t.srow = (const unsigned char *)(batch.seg[si].sc + (size_t)min(t.row0 + (lane >> 2), N - 1) * KB) + (lane & 3) * 4;
         return t;
     };
-    auto issue_stage = [&](const Tile &t, int k, int slot) {       // k: k-th stage of this wavefront (clamped: a repeat lands in a dead slot)
+    auto issue_stage = [&](const Tile &t, int k, int slot) {       // (clamped: a repeat lands in a dead slot)
 #if defined(__HIP_DEVICE_COMPILE__)
-        const int st = min(kpart + k * KS, stages - 1);
+        const int st = min(k, stages - 1);
         unsigned char *dst = ring + slot * Cfg::STAGE;
 #pragma unroll
         for (int j = 0; j < Cfg::NLD; ++j)
@@ -119,20 +115,19 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
     };
     constexpr int LPS = Cfg::NLD + 1;                             // load instructions per stage
 
-    const int wg_first = blockIdx.x * TPW, tile_stride = gridDim.x * TPW;
-    Tile cur = open_tile(wg_first + wave / KS);
+    const int wg_first = blockIdx.x * 4, tile_stride = gridDim.x * 4;      // a tile to a wavefront
+    Tile cur = open_tile(wg_first + wave);
 
-    // ---- activations of the K range -> LDS, rows m..7 zero. The first batch of their loads is requested, then the first
+    // ---- activations -> LDS, rows m..7 zero. The first batch of their loads is requested, then the first
     // stages of the first tile (both in flight together; the loads retire in order, so the activation data is waited for
     // by count without draining the ring), then the copy goes on.
     // Ring slots are used round robin across tiles: rs is the slot of the next stage to consume.
     int rs = 0;
     {
-        const int chunks = kbn * 2;                               // 16-byte chunks per activation row
-        const int a_chunks = K >> 4;
+        const int chunks = KB * 2;                                // 16-byte chunks per activation row
         const int total = 8 * chunks;
         constexpr int AB = 8, SBT = 2;                            // loads per thread in flight: 8 rows x 4096 codes in one batch
-        const int quads = kbn >> 2, total_q = 8 * quads;          // scales and sums: four consecutive blocks of a row per load
+        const int quads = KB >> 2, total_q = 8 * quads;          // scales and sums: four consecutive blocks of a row per load
         for (int base = 0, base_q = 0; base < total || base_q < total_q; base += 256 * AB, base_q += 256 * SBT) {
             u32x4 v[AB];
             f32x4 sv[SBT];
@@ -142,7 +137,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
                 for (int i = 0; i < AB; ++i) {
                     const int idx = min(base + tid + 256 * i, total - 1);
                     const int b = idx / chunks, c = idx - b * chunks;
-                    v[i] = aq[(size_t)min(b, m - 1) * a_chunks + 2 * kb0 + c];   // unconditional: a load under a branch is waited for on the spot
+                    v[i] = aq[(size_t)min(b, m - 1) * chunks + c];   // unconditional: a load under a branch is waited for on the spot
                 }
             }
             if (base_q < total_q) {
@@ -150,13 +145,13 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
                 for (int i = 0; i < SBT; ++i) {
                     const int idx = min(base_q + tid + 256 * i, total_q - 1);
                     const int b = idx / quads, qd = idx - b * quads;
-                    sv[i] = *(const f32x4 *)(a_scale + (size_t)min(b, m - 1) * KB + kb0 + qd * 4);
-                    if (!Q8) bv[i] = *(const i32x4 *)(a_sum + (size_t)min(b, m - 1) * KB + kb0 + qd * 4);
+                    sv[i] = *(const f32x4 *)(a_scale + (size_t)min(b, m - 1) * KB + qd * 4);
+                    if (!Q8) bv[i] = *(const i32x4 *)(a_sum + (size_t)min(b, m - 1) * KB + qd * 4);
                 }
             }
             if (base == 0) {
 #pragma unroll
-                for (int k = 0; k < NSTG - 1; ++k) issue_stage(cur, k, k);
+                for (int k = 0; k < MF_NSTG - 1; ++k) issue_stage(cur, k, k);
             }
             if (base < total) {
 #pragma unroll
@@ -190,7 +185,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
 
     const int hb = g >> 1, hh = g & 1;                             // which block of a pair this lane's k group and results belong to; which half of it
     const bool a_real = (n >> 3) == hb;                          // block-diagonal A: real codes, or zeros
-    unsigned char *s_zero = (unsigned char *)(s_bias + (Q8 ? 0 : kbn * 8)) + (KS > 1 ? 4096 : 0);      // 16 zero bytes behind everything else
+    unsigned char *s_zero = (unsigned char *)(s_bias + (Q8 ? 0 : KB * 8));      // 16 zero bytes behind everything else
     if (tid < 4) ((unsigned *)s_zero)[tid] = 0u;
     const unsigned char *a_base = a_real ? s_act + (hb * 8 + (n & 7)) * 32 + hh * 16 : s_zero;
     const int a_step = a_real ? 512 : 0;                         // bytes per block pair
@@ -198,22 +193,21 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
     const int w_off = Q8 ? n * Cfg::ROWB : n * Cfg::ROWB + hh * 8;
     const int w_swz = swz(n);
     const int ws_shift = hb * 16;
-    float *red = (float *)(s_bias + (Q8 ? 0 : kbn * 8));           // KS > 1: [wave][lane] partial sums
     __syncthreads();                                             // the zero bytes
 
     for (int it = 0; wg_first + it * tile_stride < batch.tiles; ++it) {      // the same trip count for every wavefront of a workgroup
-        const Tile next = open_tile(wg_first + wave / KS + (it + 1) * tile_stride);
+        const Tile next = open_tile(wg_first + wave + (it + 1) * tile_stride);
         f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < my_stages; ++k) {
-            // keep NSTG - 1 stages in flight: past this tile's last stage, the next tile's first ones
-            const int ahead = k + NSTG - 1;
-            const int ws_slot = rs == 0 ? NSTG - 1 : rs - 1;       // the slot consumed last
-            if (ahead < my_stages) issue_stage(cur, ahead, ws_slot);
-            else issue_stage(next, ahead - my_stages, ws_slot);
-            __builtin_amdgcn_s_waitcnt(vmcnt_imm((NSTG - 1) * LPS));
+        for (int k = 0; k < stages; ++k) {
+            // keep MF_NSTG - 1 stages in flight: past this tile's last stage, the next tile's first ones
+            const int ahead = k + MF_NSTG - 1;
+            const int ws_slot = rs == 0 ? MF_NSTG - 1 : rs - 1;    // the slot consumed last
+            if (ahead < stages) issue_stage(cur, ahead, ws_slot);
+            else issue_stage(next, ahead - stages, ws_slot);
+            __builtin_amdgcn_s_waitcnt(vmcnt_imm((MF_NSTG - 1) * LPS));
             const unsigned char *st = ring + rs * Cfg::STAGE;
-            rs = rs + 1 == NSTG ? 0 : rs + 1;
-            const int kb = (kpart + k * KS) * MF_SB;
+            rs = rs + 1 == MF_NSTG ? 0 : rs + 1;
+            const int kb = k * MF_SB;
             const u32x4 sc8 = *(const u32x4 *)(st + Cfg::W_BYTES + n * 16);
             const unsigned scw[4] = {sc8.x, sc8.y, sc8.z, sc8.w};
             // All of a stage's operands are requested, then its four MFMAs issued, then the rescales: one LDS round trip and
@@ -257,16 +251,7 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
         acc.z += __shfl_xor(acc.z, 32, 64);
         acc.w += __shfl_xor(acc.w, 32, 64);
         // ---- the tile's results: lanes 0..31 (weight row n, group g) hold activation rows 4g .. 4g+3
-        if (KS > 1) {
-            *(f32x4 *)(red + (wave * 64 + lane) * 4) = acc;
-            __syncthreads();
-            if (kpart == 0) {
-#pragma unroll
-                for (int w = 1; w < KS; ++w) acc += *(const f32x4 *)(red + ((wave + w) * 64 + lane) * 4);
-            }
-            __syncthreads();                                     // the partial sums are read before the next tile writes its own
-        }
-        if (cur.valid && kpart == 0 && g < 2) {
+        if (cur.valid && g < 2) {
             const MfSeg &sg = batch.seg[cur.seg];
             const int row = cur.row0 + n;
             if (row < sg.n) {
@@ -287,23 +272,10 @@ __global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));                    // no LDS-writing load may outlive the workgroup
 }
 
-template <int DT, int NSTG, int KS>
-int launch_mf(aionhip_ctx *ctx, const MfBatch &batch, int wgs, size_t lds, const u32x4 *aq, PreparedAct act, int K, int m, int kb0, int kbn,
-              float alpha, float beta) {
-    static size_t attr = 0;                                       // per instantiation: the largest LDS size asked for so far
-    if (lds > 64 * 1024 && lds > attr) {
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemv_mfma_kernel<DT, NSTG, KS>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)(160 * 1024)));
-        attr = 160 * 1024;
-    }
-    launch_k(ctx, gemv_mfma_kernel<DT, NSTG, KS>, dim3((unsigned)wgs), dim3(256), lds, batch, aq, act.scale, act.sum, K, m, kb0, kbn, alpha, beta);
-    return AIONHIP_OK;
-}
-
 template <int DT>
-int launch_mf_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
-                 float alpha, float beta) {
+int launch_mf(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act, float alpha, float beta) {
     using Cfg = MfCfg<DT>;
-    const int K = (int)ws[0]->k, KB = K >> 5, stages_all = KB / MF_SB;
+    const int K = (int)ws[0]->k, KB = K >> 5;
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     MfBatch batch{};
     batch.count = count;
@@ -313,31 +285,20 @@ int launch_mf_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const
         tiles += ((int)ws[i]->n + MF_ROWS - 1) / MF_ROWS;
     }
     batch.tiles = tiles;
-    // wavefronts per tile: one while that gives every CU four tiles, else the K range is shared by two
-    int ks = tiles >= cus * 4 ? 1 : 2;
-    while (ks > 1 && stages_all / ks < 8) ks >>= 1;               // too short a K to share
-    const int wgs_all = (tiles * ks + 3) / 4;
-    // Ring depth: 4 stages when two workgroups share a CU, 8 (q8: 4, a stage is twice the bytes) when a workgroup has the
-    // CU to itself - about 48..56 KB of weight loads in flight per CU either way.
-    const size_t red = (ks > 1 ? 4096 : 0) + 16;                  // partial sums of sibling wavefronts; the zero bytes of the A operand
-    const size_t ring4 = 4 * 4 * (size_t)Cfg::STAGE, ring8 = 4 * 8 * (size_t)Cfg::STAGE;
-    const size_t act_all = (size_t)KB * Cfg::PER_BLOCK;
-    const bool two_per_cu = wgs_all > cus && ring4 + act_all + red <= 80 * 1024;
-    const int nstg = two_per_cu || Cfg::Q8 ? 4 : 8;
-    const size_t ring = nstg == 4 ? ring4 : ring8;
-    // K ranges whose activations fit the LDS left over, as even as possible, whole stages each
-    const size_t budget = (two_per_cu ? 80 : 158) * 1024 - ring - red;
-    const int max_stages = (int)(budget / ((size_t)Cfg::PER_BLOCK * MF_SB));
-    if (max_stages < stages_all) return -1;                      // the activations of the whole K do not fit the LDS left over
-    if (stages_all / ks < nstg - 1) return -1;                   // shorter than the ring: the caller falls back
-    const int wgs = (int)min((long)wgs_all, (long)cus * (two_per_cu ? 2 : 1));
-    const auto *aq = (const u32x4 *)act.q;
-    const int kbn = stages_all * MF_SB;
-    const size_t lds = ring + (size_t)kbn * Cfg::PER_BLOCK + red;
-    if (nstg == 4) return ks == 1 ? launch_mf<DT, 4, 1>(ctx, batch, wgs, lds, aq, act, K, m, 0, kbn, alpha, beta)
-                                  : launch_mf<DT, 4, 2>(ctx, batch, wgs, lds, aq, act, K, m, 0, kbn, alpha, beta);
-    return ks == 1 ? launch_mf<DT, 8, 1>(ctx, batch, wgs, lds, aq, act, K, m, 0, kbn, alpha, beta)
-                   : launch_mf<DT, 8, 2>(ctx, batch, wgs, lds, aq, act, K, m, 0, kbn, alpha, beta);
+    // 36 (q8: 68) KB of rings beside up to 40 KB of activations: two workgroups to a CU, q8 from K = 1536 on one
+    constexpr size_t RINGS = 4 * MF_NSTG * (size_t)Cfg::STAGE, ZERO = 16, MOST = RINGS + (MF_MAX_K / 32) * (size_t)Cfg::PER_BLOCK + ZERO;
+    static_assert(MOST <= 160 * 1024 && (Cfg::Q8 || MOST <= 80 * 1024), "workgroups per CU");
+    const size_t lds = RINGS + (size_t)KB * Cfg::PER_BLOCK + ZERO;
+    const int wgs = (int)min((long)(tiles + 3) / 4, (long)cus * (lds <= 80 * 1024 ? 2 : 1));
+    if (lds > 64 * 1024) {
+        static bool attr = false;                                 // per instantiation
+        if (!attr) {
+            HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemv_mfma_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST));
+            attr = true;
+        }
+    }
+    launch_k(ctx, gemv_mfma_kernel<DT>, dim3((unsigned)wgs), dim3(256), lds, batch, (const u32x4 *)act.q, act.scale, act.sum, K, m, alpha, beta);
+    return AIONHIP_OK;
 }
 
 }  // namespace
@@ -346,9 +307,8 @@ int launch_mf_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const
 // K = 1024 ... 8192, both weight types (us, this kernel against the faster of the other two; columns for 256 CUs): it needs many row
 // tiles to amortise its longer start (ring fill behind the activation copy), and it gains most where the vector ALU is the rows kernel's
 // bound - q4 from five rows on.
-//   q4, 5..8 rows, 56 columns a CU:  65536 x 2048 22 / 25.5, 65536 x 4096 37 / 43, 262144 x 2048 66 / 84; siblings (q/k/v, gate/up) have
-//                      the rows kernel only: 14336 x 4096 19.3 / 19.5, 24576 x 4096 22 / 28. A single weight of up to 32768 rows is
-//                      faster on the exact GEMM's kernel (14336 x 4096 14.2, 24576 x 4096 20.8, 32768 x 4096 level)
+//   q4, 5..8 rows, past 96 columns a CU:  65536 x 2048 22 / 25.5, 65536 x 4096 37 / 43, 262144 x 2048 66 / 84, 32768 x 4096 level with the exact
+//                      GEMM. From 56 to 96 the rule below claims the call for gemv_slim_kernel (launch_gemv_batch, with the figures)
 //     K under 2048, 192:              262144 x 1024 36 / 44, 131072 x 1536 0.61 / 0.67 of the rows kernel, 49152 level; 32768 x 1024 0.85 / 0.74
 //   q4, 3..4 rows, 256:  65536 x 2048 21 / 23, x 1024 14.9 / 15.5, 262144 x 1024 35 / 39; x 2048 65 / 63, 65536 x 4096 level; 32768 x 4096 22.3 / 20.6
 //   q8, 5..8 rows, 256:  65536 x 2048 32 / 34, 262144 x 2048 106 / 117, x 1024 level; 49152 x 4096 51 / 51
@@ -359,7 +319,7 @@ int launch_mf_dt(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const
 bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m) {
     if (m < 3 || m > 8 || count < 1 || count > 4) return false;
     const size_t k = ws[0]->k, cus = ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256;
-    if (k % (MF_SB * 32) != 0 || k < 1024 || k > 4096) return false;
+    if (k % (MF_SB * 32) != 0 || k < MF_MIN_K || k > MF_MAX_K) return false;
     size_t rows = 0;
     for (int i = 0; i < count; ++i) {
         if (ws[i]->k != k || ws[i]->dtype != ws[0]->dtype || ws[i]->n < 1) return false;
@@ -371,9 +331,8 @@ bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, 
     return false;
 }
 
-// returns -1 when the shape does not suit the kernel after all (the caller then takes the vector-ALU kernel)
 int launch_gemv_mfma(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
                      float alpha, float beta) {
-    return ws[0]->dtype == AIONHIP_Q8_0 ? launch_mf_dt<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
-                                        : launch_mf_dt<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
+    return ws[0]->dtype == AIONHIP_Q8_0 ? launch_mf<AIONHIP_Q8_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta)
+                                        : launch_mf<AIONHIP_Q4_0>(ctx, ws, cs, ldcs, count, m, act, alpha, beta);
 }
