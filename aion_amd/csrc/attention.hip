@@ -208,11 +208,8 @@ int launch_flash_split(aionhip_ctx *ctx, AttnArgs &a) {
     if constexpr (!HILO && !RING && !PREPARE)
         if (a.codes) return launch_flash_split<KV, D, HILO, RING, DVS, true>(ctx, a);
     constexpr int LDS = FlashCfg<D, SPLIT_NW, DVS>::LDS_BYTES;
-    static bool attr_split = false;   // per kernel instantiation
-    if (!attr_split) {
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)attn_flash_kernel<KV, D, true, HILO, RING, DVS, PREPARE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
-        attr_split = true;
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)attn_flash_kernel<KV, D, true, HILO, RING, DVS, PREPARE>, LDS)) return rc;
     ProfScope scope(ctx, "attn_flash_split");
     launch_k(ctx, attn_flash_kernel<KV, D, true, HILO, RING, DVS, PREPARE>, dim3((unsigned)(a.row_tiles * a.nseg * DVS), (unsigned)(a.B * a.Hkv)),
              dim3(SPLIT_NW * 64), LDS, a);
@@ -296,11 +293,8 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         return launch_prefill(ctx, a, D);
     } else {
         a.nseg = 1;
-        static bool attr_prefill = false;
-        if (!attr_prefill) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)attn_flash_kernel<KV, D, false, HILO>, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES));
-            attr_prefill = true;
-        }
+        static std::atomic<uint64_t> attr{0};
+        if (const int rc = allow_lds(ctx, attr, (const void *)attn_flash_kernel<KV, D, false, HILO>, Cfg::LDS_BYTES)) return rc;
         ProfScope scope(ctx, "attn_flash_prefill");
         launch_k(ctx, attn_flash_kernel<KV, D, false, HILO>, dim3((unsigned)((a.row_tiles + 3) / 4), (unsigned)units), dim3(256), Cfg::LDS_BYTES, a);
         LAUNCH_CHECK(ctx, "attn_flash_prefill");

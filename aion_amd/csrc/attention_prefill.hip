@@ -6,8 +6,6 @@
 // plain multiply. The other attention kernels (attention.hip) keep the compiler's default register form.
 #include "attention_common.h"
 
-#include <atomic>
-
 namespace {
 using namespace attn;
 
@@ -815,12 +813,8 @@ template <int KV, int D>
 int launch_prefill_prepare(aionhip_ctx *ctx, AttnArgs &a) {
     using PCfg = PrefillCfg<D>;
     auto *kern = attn_prefill_kernel<KV, D, false, false, true>;
-    static std::atomic<uint64_t> attr{0};                        // devices (by number, of the first 64) that have it; per instance
-    const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
-    if (!(attr.load() & bit)) {
-        HIP_TRY(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, PCfg::LDS_BYTES));
-        attr.fetch_or(bit);
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)kern, PCfg::LDS_BYTES)) return rc;
     ProfScope scope(ctx, "attn_prefill");
     launch_k(ctx, kern, dim3((unsigned)((a.rows_total + PF_ROWS - 1) / PF_ROWS), (unsigned)(a.B * a.Hkv)), dim3(256), PCfg::LDS_BYTES, a);
     LAUNCH_CHECK(ctx, "attn_prefill");
@@ -861,13 +855,10 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
         if (rc) return rc;
         a.partial = (float *)ctx->scratch2;
     }
-    static bool attr_pf[2] = {false, false};   // per kernel instantiation
+    static std::atomic<uint64_t> attr[2] = {};
     const bool cap = a.soft_cap > 0.f;
     const void *fn = cap ? (const void *)attn_prefill_kernel<KV, D, true, RING> : (const void *)attn_prefill_kernel<KV, D, false, RING>;
-    if (!attr_pf[cap]) {
-        HIP_TRY(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, PCfg::LDS_BYTES));
-        attr_pf[cap] = true;
-    }
+    if (const int rc = allow_lds(ctx, attr[cap], fn, PCfg::LDS_BYTES)) return rc;
     {
         ProfScope scope(ctx, "attn_prefill");
         const dim3 grid((unsigned)((a.rows_total + PF_ROWS - 1) / PF_ROWS), (unsigned)units, (unsigned)nseg);

@@ -4,6 +4,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_ext.h>
 
+#include <atomic>
 #include <cstdarg>
 #include <cstdint>
 #include <cstdio>
@@ -161,6 +162,16 @@ constexpr size_t STATIC_SCRATCH_BYTES = AIONHIP_STATIC_SCRATCH_BYTES;
         hipError_t e_ = hipGetLastError();                                                          \
         if (e_ != hipSuccess) return set_err((ctx), AIONHIP_EXECUTION_FAILED, "launch %s: %s", (name), hipGetErrorString(e_)); \
     } while (0)
+
+// Dynamic LDS past 64 KB has to be asked for once per kernel and device. `done`: the devices (by number, of the first 64) that have it, a static of the
+// kernel instance's launcher; contexts of several threads may meet here.
+inline int allow_lds(aionhip_ctx *ctx, std::atomic<uint64_t> &done, const void *kernel, size_t bytes) {
+    const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
+    if (bytes <= 64 * 1024 || (done.load() & bit)) return AIONHIP_OK;
+    HIP_TRY(ctx, hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    done.fetch_or(bit);
+    return AIONHIP_OK;
+}
 
 // ---- prepared activations (aion cpu/kernels/matmul_q_i8.zig:187-264) --------------------------
 // Row-major for the GEMV kernels; `tiled` in the order the exact GEMM's operand loads want (gemm_i8_kernel.h): tiles of 32 rows (the

@@ -614,20 +614,14 @@ int launch_gemm_bf16(aionhip_ctx *ctx, const aionhip_weight *w, size_t m, const 
         // kernel variant: 0 = the bf16 copy, 1 = q4 blocks converted while staged, 2 = q8 blocks
         const int var = wcopy ? 0 : (w->dtype == AIONHIP_Q8_0 ? 2 : 1);
         const uint8_t *wp = wcopy ? (const uint8_t *)wcopy : w->qs;
-        static bool attr[3][5] = {};
+        static std::atomic<uint64_t> attr[3][5] = {};
         auto launch = [&](auto kernel, int shape, int lds, int tiles) -> int {
-            if (!attr[var][shape]) {
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-                attr[var][shape] = true;
-            }
+            if (const int status = allow_lds(ctx, attr[var][shape], (const void *)kernel, (size_t)lds)) return status;
             launch_k(ctx, kernel, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, abf, wp, w->sc, c, (int)m, (int)N, (int)K, ldc, alpha, beta, tm, tiles);
             return AIONHIP_OK;
         };
         auto launch_mixed = [&](auto kernel, int lds, int tiles) -> int {
-            if (!attr[var][4]) {
-                HIP_TRY(ctx, hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds));
-                attr[var][4] = true;
-            }
+            if (const int status = allow_lds(ctx, attr[var][4], (const void *)kernel, (size_t)lds)) return status;
             launch_k(ctx, kernel, dim3((unsigned)((tiles + 7) / 8 * 8)), dim3(256), lds, abf, wp, w->sc, c, (int)m, (int)N, (int)K, ldc, alpha, beta,
                      tm, tn_wide, tn_narrow);
             return AIONHIP_OK;

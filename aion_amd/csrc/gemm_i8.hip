@@ -4,7 +4,6 @@
 // launches.
 #include "gemm_i8_kernel.h"
 
-#include <atomic>
 #include <cmath>
 
 namespace {
@@ -170,14 +169,8 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
     static_assert((uint64_t)32 * NT * GEMM_I8_MAX_K <= (uint64_t)1 << 32, "a lane's weight offset and the group's behind it fit 32 bits");
-    if (LDS > 64 * 1024) {
-        static std::atomic<uint64_t> attr{0};                // devices (by number, of the first 64) that have it; per instance
-        const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
-        if (!(attr.load() & bit)) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
-            attr.fetch_or(bit);
-        }
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, LDS)) return rc;
     GemmSegs segs{};
     segs.count = count;
     int tiles = 0;

@@ -7,8 +7,6 @@
 // K is divided among as many wavefronts as the separate launches would divide it (k_split in gemm_i8.hip), so that the results are theirs to the bit.
 #include "gemm_i8_kernel.h"
 
-#include <atomic>
-
 namespace {
 
 template <int EPI, int DT, int MT, int KS, int WGM, int RQ, bool WHOLE, class Segs>
@@ -16,14 +14,8 @@ int launch_kernel(aionhip_ctx *ctx, const Segs &segs, int tiles, size_t k, size_
     constexpr int LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, 2, KS, WGM, 1, RQ>();
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
     auto *kern = gemm_i8_kernel<DT, MT, 2, KS, WGM, 1, RQ, WHOLE, EPI>;
-    if (LDS > 64 * 1024) {
-        static std::atomic<uint64_t> attr{0};                // devices (by number, of the first 64) that have it; per instance
-        const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
-        if (!(attr.load() & bit)) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
-            attr.fetch_or(bit);
-        }
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
     const int row_tiles = (int)((m + 32 * MT * WGM - 1) / (32 * MT * WGM));
     const int one_round = (size_t)tiles * row_tiles <= 2 * (size_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
     launch_k(ctx, kern, dim3((unsigned)(tiles * row_tiles)), dim3(64 * KS * WGM), LDS, segs, (const uint8_t *)in.q, (const float *)in.scale, (int)m,

@@ -290,13 +290,8 @@ int launch_mf(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
     static_assert(MOST <= 160 * 1024 && (Cfg::Q8 || MOST <= 80 * 1024), "workgroups per CU");
     const size_t lds = RINGS + (size_t)KB * Cfg::PER_BLOCK + ZERO;
     const int wgs = (int)min((long)(tiles + 3) / 4, (long)cus * (lds <= 80 * 1024 ? 2 : 1));
-    if (lds > 64 * 1024) {
-        static bool attr = false;                                 // per instantiation
-        if (!attr) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)gemv_mfma_kernel<DT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)MOST));
-            attr = true;
-        }
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)gemv_mfma_kernel<DT>, MOST)) return rc;
     launch_k(ctx, gemv_mfma_kernel<DT>, dim3((unsigned)wgs), dim3(256), lds, batch, (const u32x4 *)act.q, act.scale, act.sum, K, m, alpha, beta);
     return AIONHIP_OK;
 }

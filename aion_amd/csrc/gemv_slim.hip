@@ -10,8 +10,6 @@
 // q4 nibbles stay 0..15 and a second MFMA against a constant -8 supplies their offset, which costs the vector ALU nothing.
 #include "gemm_i8_kernel.h"
 
-#include <atomic>
-
 namespace {
 
 using u32x2 = __attribute__((ext_vector_type(2))) unsigned int;
@@ -234,14 +232,8 @@ int launch_ks(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
     static_assert(LDS <= 160 * 1024 / (16 / KS), "16 wavefronts per CU");
     static_assert(KS * 1024 <= LDS && (KS == 4 || KS == 8 || KS == 16), "partial sums in the rings; one, two or four runs of K to a wavefront");
     auto *kern = gemv_slim_kernel<DT, KS>;
-    if (LDS > 64 * 1024) {
-        static std::atomic<uint64_t> attr{0};                    // devices (by number, of the first 64) that have it; per instance
-        const uint64_t bit = ctx->device < 64 ? (uint64_t)1 << ctx->device : 0;
-        if (!(attr.load() & bit)) {
-            HIP_TRY(ctx, hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
-            attr.fetch_or(bit);
-        }
-    }
+    static std::atomic<uint64_t> attr{0};
+    if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
     GemmSegs segs;
     const int tiles = fill_segs(segs, ws, cs, ldcs, count, SL_ROWS);
     launch_k(ctx, kern, dim3((unsigned)tiles), dim3(64 * KS), LDS, segs, (const uint8_t *)act.q, (const float *)act.scale, (int)act.tiled,
