@@ -254,7 +254,7 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         const float prefill_us = (nseg_p > 1 ? 16.f : 12.f) + (float)((tiles64 + nseg_p - 1) / nseg_p) * per_tile * (float)rounds_p;
         if (prefill_us < split_us) split = false;
     }
-    if (a.codes && (HILO || RING)) return AIONHIP_UNSUPPORTED;
+    if (a.codes && (HILO || RING)) return rows_not_prepared(ctx, HILO ? "the precise mode" : "rolling caches");
     if (split) {
         // key segments: one 32-key tile per wavefront while that leaves the device under-filled,
         // more tiles per wavefront beyond one workgroup per CU (its LDS tiles fill a CU)
@@ -265,7 +265,7 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         int nseg = cus / (units * a.row_tiles);
         nseg = max(1, min(nseg, (tiles + SPLIT_NW - 1) / SPLIT_NW));
         nseg = min(nseg, 256);
-        if (a.codes && nseg != 1) return AIONHIP_UNSUPPORTED;      // (the merge of segments writes f32 rows)
+        if (a.codes && nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
         a.nseg = nseg;
         if (nseg > 1) {
             const size_t bytes = (size_t)units * a.row_tiles * nseg * (16 * D + 32) * sizeof(float);
@@ -353,7 +353,7 @@ int run_attention(aionhip_ctx *ctx, const aionhip_attention *p, const PreparedAc
     a.win_left = p->window_left; a.win_right = p->window_right; a.win_chunk = p->window_chunk;
     a.ring = p->rolling ? a.T : 0;
 
-    if (prepared && a.T == 0) return AIONHIP_UNSUPPORTED;
+    if (prepared && a.T == 0) return rows_not_prepared(ctx, "no keys");
     if (a.T == 0) {
         // no keys at all: every interval is empty -> zeros (cpu/exec/attention.zig:787-815)
         return aionhip_memset(ctx, p->out, 0, 0, p->batch * p->l_q * p->h_q * p->d_v * sizeof(float));
@@ -368,7 +368,7 @@ int run_attention(aionhip_ctx *ctx, const aionhip_attention *p, const PreparedAc
         if (p->kv_dtype == AIONHIP_F16) return launch_flash_d<AIONHIP_F16>(ctx, a, (int)p->d_k);
         return launch_flash_d<AIONHIP_BF16>(ctx, a, (int)p->d_k);
     }
-    if (prepared) return AIONHIP_UNSUPPORTED;
+    if (prepared) return rows_not_prepared(ctx, "the generic kernel");
     const size_t rows = p->batch * p->l_q * p->h_q;
     int rc = ensure_scratch2(ctx, rows * p->t_kv * sizeof(float));
     if (rc) return rc;

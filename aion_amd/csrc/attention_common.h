@@ -29,6 +29,10 @@ struct AttnArgs {
     float *code_scales;
 };
 
+inline int rows_not_prepared(aionhip_ctx *ctx, const char *why) {
+    return set_err(ctx, AIONHIP_UNSUPPORTED, "attention_matmul: the attention step writes f32 rows only (%s)", why);
+}
+
 __device__ __forceinline__ unsigned short f32_to_bf16_bits(float x) {
     unsigned u = __float_as_uint(x);
     u += 0x7FFFu + ((u >> 16) & 1u);

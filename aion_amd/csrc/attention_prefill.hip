@@ -846,7 +846,7 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     int nseg = max(1, min(min(want, key_tiles / seg_tiles), 16));
     a.nseg = nseg;
     if (a.codes) {
-        if (RING || nseg > 1 || a.soft_cap > 0.f) return AIONHIP_UNSUPPORTED;
+        if (RING || nseg > 1 || a.soft_cap > 0.f) return rows_not_prepared(ctx, RING ? "rolling caches" : nseg > 1 ? "keys in segments" : "a soft cap");
         return launch_prefill_prepare<KV, D>(ctx, a);
     }
     if (nseg > 1) {

@@ -427,7 +427,7 @@ def test_exact_gemm_scale_products_keep_their_bits(gpu, orc, dtype, layout, m, n
 # the edges of the 32-, 64- and 128-row tiles and for widths and K that end inside a group of four blocks; a row of zeros among them.
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("rows,hidden,ffn", [(9, 256, 512), (16, 2048, 4128), (17, 2080, 8192), (32, 2048, 544), (33, 96, 8224), (64, 1056, 2048), (65, 2048, 8192),
-                                             (100, 256, 11008), (128, 2048, 8192), (129, 4096, 1056), (300, 672, 2080), (1100, 512, 16416), (2048, 2048, 8192)])
+                                             (100, 256, 11008), (5, 4128, 2080), (8, 4224, 12320), (128, 2048, 8192), (129, 4096, 1056), (300, 672, 2080), (1100, 512, 16416), (2048, 2048, 8192)])
 def test_geglu_block_of_many_rows_is_the_separate_calls(gpu, dtype, layout, rows, hidden, ffn):
     say("geglu rows", dtype, layout, rows, hidden, ffn)
     gpu.set_gemm_mode(be.GEMM_EXACT_I8)
@@ -461,7 +461,7 @@ def test_geglu_block_of_many_rows_is_the_separate_calls(gpu, dtype, layout, rows
 @pytest.mark.parametrize("dtype,layout", CASES)
 @pytest.mark.parametrize("b,s,hidden,heads,kv_heads,d,t_cap", [(1, 9, 512, 8, 1, 64, 40), (1, 128, 2048, 8, 1, 256, 256), (2, 33, 1056, 6, 2, 128, 100),
                                                               (1, 65, 4096, 32, 8, 128, 65), (3, 50, 640, 4, 4, 192, 300), (1, 700, 512, 32, 8, 128, 1024),
-                                                              (1, 17, 2080, 16, 4, 64, 17)])
+                                                              (1, 17, 2080, 16, 4, 64, 17), (1, 8, 4128, 8, 2, 128, 20), (5, 1, 4128, 4, 4, 64, 3)])
 def test_qkv_rope_append_of_many_tokens_is_the_separate_calls(gpu, dtype, layout, b, s, hidden, heads, kv_heads, d, t_cap):
     say("qkv rope rows", dtype, layout, b, s, hidden, heads, kv_heads, d)
     gpu.set_gemm_mode(be.GEMM_EXACT_I8)
@@ -537,4 +537,48 @@ def test_attention_and_its_matmul_is_the_separate_calls(gpu, dtype, layout, b, s
         for x in c:
             x.free()
     for x in (q, k, v, pos, lens, w, out):
+        x.free()
+
+
+# What the row-preparing attention refuses has written nothing and says why: precise mode, a soft cap on the 128-row kernel, rolling caches, keys in
+# segments, no keys, a head size of the generic kernel. A soft cap on the 16-row kernel runs, and so does a short prompt beside a sequence that
+# sees no key (rows of zeros).
+@pytest.mark.parametrize("b,s,t,heads,kv_heads,d,options,why", [
+    (1, 33, 64, 8, 1, 64, {"precise": True}, "precise"), (1, 512, 512, 32, 8, 128, {"soft_cap": 20.0}, "soft cap"), (1, 20, 128, 8, 1, 64, {"rolling": True}, "rolling"),
+    (1, 512, 512, 32, 8, 128, {"rolling": True}, "rolling"), (1, 64, 1500, 4, 1, 64, {}, "segments"), (1, 1000, 1000, 16, 4, 64, {}, "segments"), (1, 20, 0, 8, 1, 64, {}, "no keys"),
+    (1, 20, 40, 8, 1, 96, {}, "generic"), (1, 20, 40, 8, 1, 64, {"soft_cap": 20.0}, None), (4, 17, 70, 8, 2, 128, {"unseen": True}, None),
+    (3, 9, 40, 2, 2, 256, {"unseen": True}, None)])
+def test_attention_matmul_refusals_and_unseen_rows(gpu, b, s, t, heads, kv_heads, d, options, why):
+    say("attention matmul refusals", b, s, t, heads, kv_heads, d, options)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    rng = np.random.default_rng(s + t)
+    n, rows, shape = 96, b * s, (b, s, t, heads, kv_heads, d, d)
+    q = gpu.upload(rng.standard_normal((rows, heads, d)).astype(np.float32))
+    k, v = (gpu.upload(rng.standard_normal((b, max(t, 1), kv_heads, d)).astype(np.float16)) for _ in range(2))
+    lengths = np.full(b, t, np.int32)
+    if options.get("unseen"):
+        lengths[1] = 0
+    pos, lens = gpu.upload((t - s + np.arange(rows) % s).astype(np.int32).reshape(b, s)), gpu.upload(lengths)
+    w = make_weight(gpu, be.Q8_0, be.ROWS_NK, n, heads * d, seed=n)[1]
+    kw = {"query_positions": pos, "kv_lengths": lens, "soft_cap": options.get("soft_cap", 0.0), "rolling": options.get("rolling", False)}
+    c = [gpu.upload(np.full((rows, n), 0.25, np.float32)) for _ in range(2)]
+    out = gpu.alloc(4 * rows * heads * d)
+    gpu.set_attention_precise(options.get("precise", False))
+    try:
+        ran = gpu.step_attention_matmul(w, q, k, v, shape, d ** -0.5, c[1], beta=1.0, **kw)
+        assert ran == (why is None)
+        if not ran:
+            said = gpu._lib.aionhip_last_error(gpu._ctx).decode()
+            assert "attention_matmul" in said and why in said, said
+            assert (gpu.download(c[1], np.float32, (rows, n)) == 0.25).all()
+        else:
+            gpu.step_attention(out, q, k, v, shape, d ** -0.5, **kw)
+            gpu.step_matmul(w, out, rows, c[0], beta=1.0)
+            want, got = (gpu.download(x, np.float32, (rows, n)) for x in c)
+            assert np.array_equal(want.view(np.uint32), got.view(np.uint32))
+            if options.get("unseen"):
+                assert (got.reshape(b, s, n)[1] == 0.25).all() and (got.reshape(b, s, n)[0] != 0.25).any()
+    finally:
+        gpu.set_attention_precise(False)
+    for x in (q, k, v, pos, lens, w, out, *c):
         x.free()
