@@ -369,7 +369,11 @@ int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weigh
         !rows_on_gemm(ctx, in, rows) || !rows_on_gemm(ctx, down, rows) || !gemm_i8_gate_applies(ctx, w_gate, rows))
         return set_err(ctx, AIONHIP_UNSUPPORTED, "geglu_matmul_rows: %zu rows against %zu x %zu do not run on the exact GEMM's gate instances", rows, (size_t)w_gate->n, in.k);
     const size_t in_bytes = (prepared_act_bytes(rows, in.k) + 255) & ~(size_t)255;
-    rc = ensure_scratch(ctx, in_bytes + prepared_act_bytes(rows, down.k));
+    const size_t bytes = in_bytes + prepared_act_bytes(rows, down.k);
+    // (both prepared forms at once: the two calls, which need the larger alone, may fit a recording where these do not)
+    if (ctx->capturing && bytes > ctx->scratch_bytes)
+        return set_err(ctx, AIONHIP_UNSUPPORTED, "geglu_matmul_rows: scratch must grow to %zu bytes while a program is being recorded: run the step once before recording", bytes);
+    rc = ensure_scratch(ctx, bytes);
     if (rc) return rc;
     const PreparedAct act = prepared_act_carve(ctx->scratch, rows, in.k, true), gated = prepared_act_carve((char *)ctx->scratch + in_bytes, rows, down.k, true);
     rc = launch_prepare_rmsnorm(ctx, (const float *)(uintptr_t)x, (const float *)(uintptr_t)gamma, (const float *)(uintptr_t)beta_norm, eps, rows, in.k, act);

@@ -196,7 +196,8 @@ int aionhip_step_rmsnorm_geglu_matmul(aionhip_ctx *ctx, const aionhip_weight *w_
                                       aionhip_handle c, float alpha, float beta);
 /* The same block for any number of rows on the exact GEMM (C [rows, n_down] with row pitch ldc, 0: n_down), in three launches: the results are
  * those of aionhip_step_rmsnorm_matmul + aionhip_step_gate_matmul to the bit. AIONHIP_UNSUPPORTED, with nothing launched, where one of the
- * three matmuls would run on another kernel (a few rows, the bf16 modes, gate and up with a K that is cut into slices): issue the two calls. */
+ * three matmuls would run on another kernel (a few rows, the bf16 modes, gate and up with a K that is cut into slices), or where a program is
+ * being recorded and the scratch memory, which holds both matmuls' prepared rows at once, would have to grow: issue the two calls. */
 int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weight *w_gate, const aionhip_weight *w_up, const aionhip_weight *w_down,
                                            size_t rows, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
                                            aionhip_handle c, size_t ldc, float alpha, float beta);

@@ -582,3 +582,42 @@ def test_attention_matmul_refusals_and_unseen_rows(gpu, b, s, t, heads, kv_heads
         gpu.set_attention_precise(False)
     for x in (q, k, v, pos, lens, w, out, *c):
         x.free()
+
+
+# A context whose scratch memory has grown for the two calls only: in a recording the GeGLU block of many rows, which needs both prepared forms at
+# once, is refused as unsupported with nothing recorded, and the two calls are recorded in its place.
+def test_geglu_block_in_a_recording_leaves_scratch_as_it_is(gpu):
+    del gpu                                                     # (its scratch has long grown)
+    own = be.HipBackend(0)
+    try:
+        rng = np.random.default_rng(3)
+        rows, k = 64, 2048
+        wg, wu, wd = (make_weight(own, be.Q8_0, be.ROWS_NK, k, k, seed=s)[1] for s in range(3))
+        x, gamma = own.upload(rng.standard_normal((rows, k)).astype(np.float32)), own.upload(np.ones(k, np.float32))
+        gate, up, c = (own.alloc(4 * rows * k) for _ in range(3))
+
+        def two_calls():
+            own.step_rmsnorm_matmul([wg, wu], x, gamma, rows, [gate, up], 1e-6)
+            own.step_gate_matmul(wd, gate, up, rows, c)
+
+        two_calls()
+        want = own.download(c, np.uint32, (rows, k))
+        ran = []
+
+        def block():
+            ran.append(own.step_rmsnorm_geglu_matmul_rows(wg, wu, wd, x, gamma, rows, 1e-6, c))
+            if not ran[-1]:
+                two_calls()
+
+        for expected in (False, True):
+            prog = own.record_program(block)
+            assert ran == [expected]
+            for _ in range(3):
+                own.write(c, np.zeros((rows, k), np.float32))
+                own.program_execute(prog)
+                assert np.array_equal(own.download(c, np.uint32, (rows, k)), want)
+            own.program_destroy(prog)
+            assert own.step_rmsnorm_geglu_matmul_rows(wg, wu, wd, x, gamma, rows, 1e-6, c)      # eagerly: it grows the scratch
+            ran.clear()
+    finally:
+        own.close()
