@@ -108,12 +108,12 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
     const int KB = K >> 5, G = (KB + 3) >> 2;
     // (a head's columns: pair tile `head_tile` is its columns 32 head_tile .. and the same of its second half)
     [[maybe_unused]] int head = 0, head_tile = 0, pair_col = ct * 32;
-    size_t second = 0;                           // weight rows from a column of the first tile to its partner's
+    size_t partner = 0;                          // weight rows from a column of the first tile to its partner's
     if constexpr (EPI == GEMM_ROPE) {
         const int per_head = segs.d >> 6;
         head = (ct - segs.first_tile[si]) / per_head;
         head_tile = ct - segs.first_tile[si] - head * per_head;
-        second = (size_t)segs.d >> 1;
+        partner = (size_t)segs.d >> 1;
         pair_col = head * segs.d + head_tile * 32;
     }
     const int n0 = PAIR ? pair_col : (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
@@ -146,8 +146,8 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
         }
         const int nb = min(n0, N - 1);
         const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = (GATE ? segs.qs[1] : qs) + ((size_t)nb + second) * wpitch;      // (used in the device pass only)
-        const __half *sb = (GATE && h ? segs.sc[1] : sc) + ((size_t)nb + (EPI == GEMM_ROPE && h ? second : 0)) * KB;
+        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = (GATE ? segs.qs[1] : qs) + ((size_t)nb + partner) * wpitch;      // (used in the device pass only)
+        const __half *sb = (GATE && h ? segs.sc[1] : sc) + ((size_t)nb + (EPI == GEMM_ROPE && h ? partner : 0)) * KB;
         // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
         constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
         const int w_row = lane / LPR;
@@ -278,13 +278,13 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
         // Of two wavefronts on a SIMD the older goes first wherever both could, ends a quarter of its time ahead and leaves the other to run alone,
         // at little more than half the SIMD's rate (512 x 4096 x 4096: workgroups end between 19 and 25 us). So a wavefront's priority falls as it
         // proceeds. Where more workgroups follow that would hold up the ones about to end: 2048 x 14336 x 512 q8 61.2 -> 66.7 us.
-        const int quarter = (g_hi - g + 4 * KS - 1) / (4 * KS) * KS, second = g + quarter, third = second + quarter, fourth = third + quarter;
+        const int quarter = (g_hi - g + 4 * KS - 1) / (4 * KS) * KS, quarter2 = g + quarter, quarter3 = quarter2 + quarter, quarter4 = quarter3 + quarter;
         if (MT * NT > 1 && one_round) __builtin_amdgcn_s_setprio(3);
         for (; g < g_hi; g += KS) {
             if (MT * NT > 1 && one_round) {
-                if (g == second) __builtin_amdgcn_s_setprio(2);
-                if (g == third) __builtin_amdgcn_s_setprio(1);
-                if (g == fourth) __builtin_amdgcn_s_setprio(0);
+                if (g == quarter2) __builtin_amdgcn_s_setprio(2);
+                if (g == quarter3) __builtin_amdgcn_s_setprio(1);
+                if (g == quarter4) __builtin_amdgcn_s_setprio(0);
             }
             const int gn = g + KS < g_hi ? g + KS : g;      // past the last group it is repeated (never used)
             constexpr int SW = OUTER ? 1 : NT;           // (a lane's own column is what a pair of column tiles wants of it)
@@ -455,7 +455,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
                 if (si == 0) {
                     float *dst = segs.q_out + ((size_t)row * segs.h_q + head) * segs.d + pair;
                     dst[0] = yl;
-                    dst[second] = yh;
+                    dst[partner] = yh;
                     continue;
                 }
                 const int b = row / segs.s_len;
@@ -463,7 +463,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
                 if (t < 0 || t >= segs.t_cap) continue;
                 __half *dst = (si == 1 ? segs.kcache : segs.vcache) + (((size_t)b * segs.t_cap + (size_t)t) * segs.h_kv + head) * segs.d + pair;
                 dst[0] = __float2half_rn(yl);
-                dst[second] = __float2half_rn(yh);
+                dst[partner] = __float2half_rn(yh);
             }
             return;
         }

@@ -621,3 +621,25 @@ def test_geglu_block_in_a_recording_leaves_scratch_as_it_is(gpu):
             ran.clear()
     finally:
         own.close()
+
+
+# The same where products of scales are subnormal (weight scales of 2^-4 .. 2^-9 times row scales down to 2^-135) and where sums cross into them:
+# the matrix pipe's products of scales are the multiply's there too.
+@pytest.mark.parametrize("dtype,layout", CASES)
+@pytest.mark.parametrize("m,n,k", [(512, 4096, 2048), (77, 11008, 672), (300, 5000, 1056), (90, 2100, 4096)])
+def test_exact_gemm_scale_products_keep_their_bits_below_the_normal_range(gpu, orc, dtype, layout, m, n, k):
+    say("subnormal scale products", dtype, layout, m, n, k)
+    gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+    _, w = make_weight(gpu, dtype, layout, n, k, seed=m + k)
+    rng = np.random.default_rng(k + 1)
+    a = np.zeros((m, k // 32, 32), np.float32)
+    at = np.arange(m) * 7 % (k // 32)
+    a[np.arange(m), at] = rng.standard_normal((m, 32)) * 2.0 ** rng.integers(-135, -110, (m, 1))
+    a = a.reshape(m, k)
+    got = gpu.matmul(w, a)
+    assert "gemm_i8" in gpu.last_launch()["kernel"]
+    assert ((np.abs(got) < 2.0 ** -126) & (got != 0)).mean() > 0.05 and (np.abs(got) > 2.0 ** -126).mean() > 0.05
+    for rows in ([0, 1, m // 2, m - 1, *rng.integers(0, m, 8)], rng.integers(0, m, 12)):
+        assert np.array_equal(got[rows].view(np.uint32), gpu.matmul(w, a[rows]).view(np.uint32)), rows
+        assert "gemm_i8" in gpu.last_launch()["kernel"]
+    w.free()
