@@ -279,6 +279,8 @@ int launch_gemm_i8_few_rows(aionhip_ctx *ctx, const aionhip_weight *w, size_t m,
 // how the exact GEMM divides a K among a workgroup's wavefronts (false: it is also cut into slices), and whether four of them to a tile of 64
 // columns are better given 64 rows than 32
 bool gemm_i8_unsliced(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k, int *wavefronts);
+// (and how far the better of those two is behind the best tile of four wavefronts, past 32 rows)
+float gemm_i8_wide_behind_us(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k);
 bool gemm_i8_tall(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k);
 // gate and up projections of m prepared rows, the gate and the preparation of its rows as one launch (gemm_i8_pair.hip); both prepared forms tiled
 bool gemm_i8_gate_applies(const aionhip_ctx *ctx, const aionhip_weight *gate, size_t m);

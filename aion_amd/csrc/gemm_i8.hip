@@ -286,6 +286,12 @@ bool gemm_i8_unsliced(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, siz
     *wavefronts = split.wavefronts;
     return split.slices == 1;
 }
+float gemm_i8_wide_behind_us(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k) {
+    const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
+    float best = 0.f;
+    pick_shape(ctx, dtype, m, ns, count, k, KSplit{4, 1, false}, &best);
+    return fminf(shape_us(ctx, I8_SQUARE4, fits[I8_SQUARE4], m, ns, count, k, 1), shape_us(ctx, I8_WIDE4, fits[I8_WIDE4], m, ns, count, k, 1)) - best;
+}
 bool gemm_i8_tall(const aionhip_ctx *ctx, int dtype, size_t m, const size_t *ns, int count, size_t k) {
     const I8Fit *fits = I8_FITS[fit_set(m, k)][dtype == AIONHIP_Q8_0];
     return m > 32 && shape_us(ctx, I8_SQUARE4, fits[I8_SQUARE4], m, ns, count, k, 1) < shape_us(ctx, I8_WIDE4, fits[I8_WIDE4], m, ns, count, k, 1);

@@ -57,13 +57,26 @@ bool pair_plan(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int coun
     return m <= 0x7FFFFFFFu && ws[0]->k <= GEMM_I8_MAX_K && (*wavefronts >= 4 || m > 64);
 }
 
+constexpr size_t LONG_K = 2560;                  // (between the measured 2048 and 4096)
+size_t cus_of(const aionhip_ctx *ctx) { return ctx->cu_count > 0 ? (size_t)ctx->cu_count : 256; }
+
 }  // namespace
 
+// The launch is worth 2 .. 11 us less (9 .. 512 rows x 4096 .. 14336 x 1024 .. 4096, both block formats, timed behind each other in a stream) but
+// for two places where the separate launches' tiles are the better ones by more than it saves, us separate -> this launch:
+//   a long K, one row tile and between one and one and a half pair tiles per CU, a nearly empty second round where 32 x 32 tiles fill more of theirs: 9 and
+//     16 rows x 11008 x 4096 q4 41.9 -> 43.3, 44.2 -> 45.0, q8 50.7 -> 51.7, 52.2 -> 53.6, x 8704 q8 2.6 and 2.1 us, at 32 rows level; over K = 2048 the
+//     launch is level (q8) or 1 .. 2 us ahead (q4)
+//   where the model of the shapes (gemm_i8.hip) has them ahead by more than 3.25 us: q8, three row tiles as one of 96 rows, 96 x 11008 x 4096 84.2 -> 86.1, x
+//     14336 104.5 -> 105.8; 2.99 us of the model are 41.5 -> 40.4 at 96 x 8192 x 2048
 bool gemm_i8_gate_applies(const aionhip_ctx *ctx, const aionhip_weight *gate, size_t m) {
     int wavefronts = 0;
     bool tall = false;
     const aionhip_weight *ws[2] = {gate, gate};
-    return pair_plan(ctx, ws, 2, m, &wavefronts, &tall);
+    if (!pair_plan(ctx, ws, 2, m, &wavefronts, &tall)) return false;
+    const size_t cus = cus_of(ctx), pairs = (gate->n + 31) / 32, ns[2] = {gate->n, gate->n};
+    if (gate->k > LONG_K && m <= 32 && pairs > cus && pairs * 2 < cus * 3) return false;
+    return wavefronts != 4 || m <= 32 || gemm_i8_wide_behind_us(ctx, gate->dtype, m, ns, 2, gate->k) <= 3.25f;
 }
 
 int launch_gemm_i8_gate(aionhip_ctx *ctx, const aionhip_weight *gate, const aionhip_weight *up, size_t m, PreparedAct in, PreparedAct out) {
@@ -89,14 +102,21 @@ int launch_gemm_i8_gate(aionhip_ctx *ctx, const aionhip_weight *gate, const aion
     return AIONHIP_OK;
 }
 
-// Microseconds of preparation + projections + rotation and append, separate launches -> these (q4 unless said): 128 x 2048 into 8 + 1 + 1 heads of
-// 256 15.7 -> 13.1 (q8 15.5 -> 13.7); hidden 1024 1.25 .. 1.44 times; hidden 4096 into 32 + 8 + 8 heads of 128: 16 rows 16.0 -> 15.8, 64 rows
-// 21.2 -> 17.8, 512 rows 59.5 -> 56.2; the least is q8 at 24 rows of 4096, 18.9 -> 19.4. Where q and k, v divide K differently (q4, hidden 4096, 77 .. 200
-// rows: few columns of k and v) the separate launches stay: one launch for q and one for k and v would be 28.8 -> 31.7 at 100 rows.
+// Microseconds of preparation + projections + rotation and append, separate launches -> these, behind each other in a stream: 128 x 2048 into 8 + 1 + 1
+// heads of 256 q4 15.4 -> 13.5, q8 15.8 -> 14.5; 4096 into 32 + 8 + 8 heads of 128 64 rows 22.5 -> 19.6, 27.0 -> 24.0, 512 rows 61.7 -> 59.4; 512 x 1024 into
+// 16 + 4 + 4 of 64 15.7 -> 13.3. Where q and k, v divide K differently (q4, hidden 4096, 77 .. 200 rows: few columns of k and v) the separate launches
+// stay: one launch for q and one for k and v would be 28.8 -> 31.7 at 100 rows. They stay too where a pair of tiles to a workgroup costs more than the launch:
+//   up to one 32 x 32 tile per CU, which pairs would leave half of the CUs: 32 rows of 4096 into 32 + 8 + 8 of 128 q4 18.2 -> 19.7, q8 21.4 -> 23.2, of 3072
+//     into 24 + 8 + 8 15.2 -> 16.6, 17.1 -> 19.5; 96 x 2048 into 8 + 1 + 1 of 256 12.6 -> 13.2, 13.7 -> 14.4
+//   a long K and more than one pair per CU where wide weights meet few rows, up to 96 of q8 or a K among eight wavefronts: 33 and 64 rows of 4096 into
+//     32 + 32 + 32 of 128 q8 30.8 -> 33.3, 34.1 -> 34.9, q4 28.6 -> 29.8 and 32.1 -> 31.6; q8 96 rows into 32 + 8 + 8 30.0 -> 31.1, 128 rows 33.2 -> 31.7; over
+//     K = 2048 the launch is 1 .. 3 us ahead there
 bool gemm_i8_rope_applies(const aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, size_t d) {
     int wavefronts = 0;
     bool tall = false;
-    return d % 64 == 0 && pair_plan(ctx, qkv, 3, m, &wavefronts, &tall);
+    if (d % 64 != 0 || !pair_plan(ctx, qkv, 3, m, &wavefronts, &tall)) return false;
+    const size_t cus = cus_of(ctx), tiles = (m + 31) / 32 * ((qkv[0]->n + qkv[1]->n + qkv[2]->n) / 32);
+    return tiles > cus && (tiles <= 2 * cus || qkv[0]->k <= LONG_K || (wavefronts < 8 && (qkv[0]->dtype != AIONHIP_Q8_0 || m > 96)));
 }
 
 int launch_gemm_i8_rope(aionhip_ctx *ctx, const aionhip_weight *const *qkv, size_t m, PreparedAct in, float *q_out, RopeAppend rope) {

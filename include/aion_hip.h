@@ -180,7 +180,8 @@ int aionhip_step_rmsnorm_qkv_rope_append(aionhip_ctx *ctx, const aionhip_weight 
 /* The same for b sequences of s new tokens each on the exact GEMM, linear caches, in two launches (positions [b, s], write_index [b], as
  * aionhip_step_rope_append takes them): the results are those of aionhip_step_rmsnorm_matmul + aionhip_step_rope_append to the bit; k, v and the
  * unrotated q are not written out. AIONHIP_UNSUPPORTED, with nothing launched, where the projections would run on another kernel (a few rows,
- * the bf16 modes, a K that is cut into slices) or the head size is no multiple of 64: issue the two calls. */
+ * the bf16 modes, a K that is cut into slices), where the separate launches are the faster ones (rows and columns that leave CUs idle), or
+ * the head size is no multiple of 64: issue the two calls. */
 int aionhip_step_rmsnorm_qkv_rope_append_rows(aionhip_ctx *ctx, const aionhip_weight *wq, const aionhip_weight *wk, const aionhip_weight *wv,
                                               size_t b, size_t s, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
                                               aionhip_handle q_out, aionhip_handle k_cache, aionhip_handle v_cache, aionhip_handle positions,
@@ -196,7 +197,8 @@ int aionhip_step_rmsnorm_geglu_matmul(aionhip_ctx *ctx, const aionhip_weight *w_
                                       aionhip_handle c, float alpha, float beta);
 /* The same block for any number of rows on the exact GEMM (C [rows, n_down] with row pitch ldc, 0: n_down), in three launches: the results are
  * those of aionhip_step_rmsnorm_matmul + aionhip_step_gate_matmul to the bit. AIONHIP_UNSUPPORTED, with nothing launched, where one of the
- * three matmuls would run on another kernel (a few rows, the bf16 modes, gate and up with a K that is cut into slices), or where a program is
+ * three matmuls would run on another kernel (a few rows, the bf16 modes, gate and up with a K that is cut into slices), where the separate
+ * launches are the faster ones, or where a program is
  * being recorded and the scratch memory, which holds both matmuls' prepared rows at once, would have to grow: issue the two calls. */
 int aionhip_step_rmsnorm_geglu_matmul_rows(aionhip_ctx *ctx, const aionhip_weight *w_gate, const aionhip_weight *w_up, const aionhip_weight *w_down,
                                            size_t rows, aionhip_handle x, aionhip_handle gamma, aionhip_handle beta_norm, float eps,
