@@ -493,15 +493,17 @@ __global__ __launch_bounds__(256) void gemm_bf16_mixed_kernel(const unsigned sho
 // In bf16 mode: is the bf16 MFMA kernel expected to beat the exact kernel for this shape? Up to a few hundred rows it
 // is not - it streams a 2-byte copy of every weight (3.5x the q4 bytes), its 256-column tiles leave most CUs idle and
 // one workgroup's K loop is a latency chain - and the exact kernel is then both the faster and the exact one.
-// Modelled times of whole calls in microseconds, the constants below fitted to the bf16 kernel's over ten weight shapes x 16 .. 2048 rows
-// (rms 20 %). Over those, both block formats, the choice costs 1.2 % over always taking the faster kernel; always exact would cost 10 %,
-// always bf16 58 %. (512 x 4096 x 14336 q4: exact 97 us, bf16 168; 2048 x 14336 x 4096 the other way, 356 and 215.)
+// Modelled times of whole calls in microseconds, the constants below fitted to the bf16 kernel's and to the choice over ten weight shapes (1024 ..
+// 16384 x 2048 .. 14336) x 16 .. 2048 rows, both block formats, weights from memory (rms 15 %; the exact kernel's model is in gemm_i8.hip). Over those
+// the choice costs 0.13 % over always taking the faster kernel; always exact would cost 9 %, always bf16 105 %. The constants before were weighed
+// against an exact kernel that has become faster and cost 1.1 %: 256 x 8192 x 2048 q4 ran in bf16, 28.8 us, over 21.1; 1024 x 4096 x 14336 198 over 171.
+// (512 x 4096 x 14336 q4: exact 95 us, bf16 167; 2048 x 14336 x 4096 the other way, 345 and 218.)
 bool gemm_bf16_pays(const aionhip_ctx *ctx, int dtype, size_t m, size_t n, size_t k) {
     const float exact_us = gemm_i8_us(ctx, dtype, m, n, k);
-    const float copy_us = (float)n * (float)k * 2.f / 2.7e6f;                                  // weight bytes at ~2.7 TB/s
-    const float flop_us = 2.f * (float)m * (float)n * (float)k / 9.3e8f;                        // ~930 TFLOP/s
-    const float chain_us = (float)(k / 32) * 0.31f;                                            // one workgroup's K loop
-    const float act_us = (float)m * (float)k * 2.0e-6f;                                         // the bf16 rounding of A
+    const float copy_us = (float)n * (float)k * 2.f / 2.2e6f;                                  // weight bytes at ~2.2 TB/s
+    const float flop_us = 2.f * (float)m * (float)n * (float)k / 9.28e8f;                       // ~928 TFLOP/s
+    const float chain_us = (float)(k / 32) * 0.34f;                                            // one workgroup's K loop
+    const float act_us = 1.1f + (float)m * (float)k * 2.0e-6f;                                  // the bf16 rounding of A, a launch
     const float bf16_us = fmaxf(fmaxf(copy_us, flop_us), chain_us) + act_us;
     return bf16_us < exact_us;
 }

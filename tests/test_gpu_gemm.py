@@ -647,3 +647,17 @@ def test_exact_gemm_scale_products_keep_their_bits_below_the_normal_range(gpu, o
         assert np.array_equal(got[rows].view(np.uint32), gpu.matmul(w, a[rows]).view(np.uint32)), rows
         assert "gemm_i8" in gpu.last_launch()["kernel"]
     w.free()
+
+
+# bf16 mode between the two kernels: the exact one is the faster of the two up to a few hundred rows (256 x 8192 x 2048 21 against 29 us), the bf16 one
+# beyond (512 x 14336 x 4096 73 against 98)
+@pytest.mark.parametrize("m,n,k,kernel", [(256, 8192, 2048, "gemm_i8_q4"), (512, 14336, 4096, "gemm_bf16")])
+def test_bf16_mode_chooses_the_faster_kernel_at_a_few_hundred_rows(gpu, m, n, k, kernel):
+    _, w = make_weight(gpu, be.Q4_0, be.KMAJOR_KN, n, k, seed=m)
+    gpu.set_gemm_mode(be.GEMM_BF16_MFMA)
+    try:
+        gpu.matmul(w, np.random.default_rng(m).standard_normal((m, k)).astype(np.float32))
+        assert gpu.last_kernel() == kernel
+    finally:
+        gpu.set_gemm_mode(be.GEMM_EXACT_I8)
+        w.free()
