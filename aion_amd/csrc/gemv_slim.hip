@@ -245,7 +245,7 @@ int launch_ks(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
 
 // Where it is the fastest kernel, from timing 2..8 rows against every other kernel over K = 512 .. 28672 x N = 256 .. 131072, both block formats,
 // preparation included, weights rotated past the memory-side cache (the kernel it replaces / this one, us):
-//   up to three workgroups per CU (12288 weight rows). q4 4 x 4096 x 14336 16.3 / 14.1, 4 x 9664 x 14336 1.6 times as fast, 3 x 3072 x 11008 1.46; 2 x
+//   up to three workgroups per CU (12288 weight rows). q4 4 x 4096 x 14336 16.3 / 12.8, 4 x 9664 x 14336 1.6 times as fast, 3 x 3072 x 11008 1.46; 2 x
 //     6144 x 8192 1.2; q8 4 x 4096 x 4096 1.2, 4 x 256 x 28672 1.5. Past them it has no fewer workgroups than its rivals have better tiles: 14336 rows
 //     level, 32768 0.85 .. 1.1.
 //   5..8 rows, where the exact GEMM is the rival: K up to 16384 (8 x 2048 x 28672 q4 0.82), and for q4 not between one and two workgroups per CU (8 x

@@ -66,7 +66,7 @@ static bool fused_row_pays(const Batch &b) {
 // (8 x 14336 x 8192: q8 78 against 31 us, q4 65 against 25; 8 x 6144 x 4128 20 / 15, 18 / 11; q8 up to 4096 columns is level there or, below 3072, up to a
 // fifth ahead on the GEMV: 8 x 2048 x 4128 12.8 / 13.6, 8 x 1024 x 5120 12.0 / 14.2), so they run on gemv_slim_kernel where it applies and on the exact GEMM
 // elsewhere. Which of the two is decided weight by weight: the sums of both depend on the weight alone, and a weight has the same bits by itself and
-// beside any siblings. Siblings of both kinds share the preparation, tiled, and are two launches.
+// beside any siblings. Siblings of both kinds share the preparation, tiled, and are two launches or, where gemm_slim_applies, one.
 static bool rows_over_long_k(const Batch &b, size_t m) { return m >= 5 && m <= GEMV_MAX_M && b.k > FUSED_PAYS_K && b.k <= GEMM_I8_MAX_K; }
 static size_t slim_weights(const aionhip_ctx *ctx, const Batch &b, size_t m) {
     size_t slim = 0;

@@ -338,7 +338,7 @@ def run_gemm_headline(gpu, be):
             (be.GEMM_EXACT_I8, "gemm_i8_q4", "int8", "exact_i8",
              "aion's arithmetic (int8 activations per 32-block, exact i32 block dots, f32 scale-accumulate): tolerance class 2e-3, "
              "observed 1e-6. The parity path, not the throughput path: both operands carry a scale per 32-block, so every 32x32x32 "
-             "MFMA is followed by 48 VALU instructions of rescaling, which bounds it near 15 % of the int8 peak")):
+             "MFMA is followed by 32 VALU instructions of rescaling and half an MFMA of scale products, which bounds it well below the int8 peak")):
         gpu.set_gemm_mode(mode)
         gpu.step_matmul(w, x, m, y)
         settle(gpu, lambda i: gpu.step_matmul(w, x, m, y))
