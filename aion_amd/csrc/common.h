@@ -246,9 +246,7 @@ int launch_gate_gelu(aionhip_ctx *ctx, float *out, const float *a, const float *
 // device table f[i] = scale_factor * freq_step^i built with f32 multiplies in sequence (aion cpu/kernels/rope.zig:22-30)
 int rope_table(aionhip_ctx *ctx, int pairs, float freq_step, float scale_factor, const float **out);
 
-// one activation row against one weight with a long reduction axis: K cut into slices, one launch (gemv_ksplit.hip)
-// 3..8 prepared rows against a weight with very many rows, the dots on the matrix pipe (gemv_mfma.hip); launch returns -1 when
-// the shape does not suit the kernel after all
+// 3..8 prepared rows against weights of very many rows, the dots on the matrix pipe (gemv_mfma.hip)
 bool gemv_mfma_applies(const aionhip_ctx *ctx, const aionhip_weight *const *ws, int count, int m);
 int launch_gemv_mfma(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m, PreparedAct act,
                      float alpha, float beta);
@@ -260,6 +258,7 @@ int launch_gemv_slim(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *c
 bool gemm_slim_applies(const aionhip_ctx *ctx, const aionhip_weight *const *gemm, int count, int m);
 int launch_gemm_slim(aionhip_ctx *ctx, const aionhip_weight *const *gemm, float *const *gemm_cs, const size_t *gemm_ldcs, int gemm_count, const aionhip_weight *const *slim,
                      float *const *slim_cs, const size_t *slim_ldcs, int slim_count, int m, PreparedAct act, float alpha, float beta);
+// one activation row against one weight with a long reduction axis: K cut into slices, one launch (gemv_ksplit.hip)
 bool gemv_ksplit_applies(const aionhip_ctx *ctx, const aionhip_weight *w, const float *x);
 int launch_gemv_ksplit(aionhip_ctx *ctx, const aionhip_weight *w, float *c, const float *x, float alpha, float beta);
 int launch_gemv_batch(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int m,
