@@ -229,9 +229,6 @@ struct FusedEpi {
     __half *k_cache, *v_cache;
     int t_cap, h_kv, d, rope_pairs;
     int rolling;         // the caches are rings: logical step t lives in row t % t_cap
-    int *act_q;          // EPI_GATE_QUANT: prepared activation planes of the down projection
-    float *act_scale;
-    int *act_sum;
 };
 constexpr size_t FUSED_MAX_K = 8192;
 // above this K the per-workgroup prologue costs more than a separate preparation launch

@@ -22,8 +22,20 @@ namespace {
 // K bytes of codes, K/32 scales, K/32 code sums, 4 reduction slots.
 // NT = threads per workgroup (K <= 4 * NT * NCH): 256, or more for the plain preparation - the wavefronts of a workgroup
 // share one preparation, and every workgroup reads the whole activation at the same moment.
-template <int DT, int R, int PRO, int NCH, int EPI, int NT = 256>
-__global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn in, int K, float alpha, float beta, FusedEpi epi) {
+// What the first loads need (the first two weights, the activation) are the leading arguments, as plain values: those arrive in SGPRs with the
+// wavefront, while a structure by value - all of them came in one - is read from memory, two dependent round trips before the first load (q4 1 x 14336 x
+// 4096 6.2 -> 5.6 us, 1 x 262144 x 2048 44.6 -> 44.1, a decode step of eight blocks 237 -> 234).
+// The last argument: what nothing waits for at the start. A launch's arguments are written across the bus (240 bytes: 0.75 us of host time) and the
+// smallest calls are bound by their launch, so that a single weight (MANY = false) is told apart from siblings: q8 1 x 2048 x 2048 3.64 -> 3.43 us a
+// call, q4 1 x 4096 x 4096 4.13 -> 3.60 (in a process whose launches cost 4.3 us: 4.37 -> 4.30, 4.46 -> 4.33).
+template <int EPI, bool MANY> struct FusedTail { GemvBatch batch; };
+template <> struct FusedTail<EPI_NONE, false> { float *c; };
+template <bool MANY> struct FusedTail<EPI_ROPE_APPEND, MANY> { GemvBatch batch; FusedEpi epi; };
+template <bool MANY> struct FusedTail<EPI_GATE_QUANT, MANY> { PreparedAct act; };
+
+template <int DT, int R, int PRO, int NCH, int EPI, int NT = 256, bool MANY = true>
+__global__ __launch_bounds__(NT) void gemv_fused_kernel(const u32x4 *qs0, const __half *sc0, const float *x, const float *side, int K, int total_waves, int n0, int first1,
+                                                        const u32x4 *qs1, const __half *sc1, const float *norm_beta, float eps, float alpha, float beta, FusedTail<EPI, MANY> tail) {
     static_assert(EPI == EPI_NONE || R == 8, "the epilogues own 4 + 4 rows per wavefront");
     static_assert(NT == 256 || (PRO == PRO_QUANT && EPI == EPI_NONE), "wide workgroups: plain preparation only");
     extern __shared__ __attribute__((aligned(16))) unsigned char s_mem[];
@@ -52,32 +64,46 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
     };
     auto locate = [&](int gw) {
         Group gr;
-        int si = 0;
-#pragma unroll
-        for (int i = 1; i < 4; ++i)
-            if (i < batch.count && gw >= batch.seg[i].first_wave) si = i;
-        gr.qs = gr.qs2 = batch.seg[si].qs;
-        gr.sc = gr.sc2 = batch.seg[si].sc;
-        gr.c = batch.seg[si].c;
-        gr.n = batch.seg[si].n;
-        gr.seg = si;
-        gr.row0 = (gw - batch.seg[si].first_wave) * R;
-        if (EPI == EPI_ROPE_APPEND) {
-            // task -> (head, first of four pairs): rows head*D + e0 + {0..3} and head*D + D/2 + e0 + {0..3}
-            const int per_head = epi.d >> 3, task = gw - batch.seg[si].first_wave;
-            gr.row0 = (task / per_head) * epi.d + (task % per_head) * 4;
-        }
-        if (EPI == EPI_GATE_QUANT) {
+        gr.seg = 0;
+        gr.qs = qs0;
+        gr.sc = sc0;
+        gr.n = n0;
+        gr.row0 = gw * R;
+        int half = 0;
+        if constexpr (EPI == EPI_GATE_QUANT) {
             // gw = (task * 2 + sub) * 4 + wavefront: outputs j0 .. j0+3 of the gate (rows 0..3) and the up weight (rows 4..7)
+            gr.qs2 = qs1;
+            gr.sc2 = sc1;
             gr.row0 = (gw >> 2) * 16 + (gw & 3) * 4;
-            gr.qs = batch.seg[0].qs;
-            gr.sc = batch.seg[0].sc;
-            gr.qs2 = batch.seg[1].qs;
-            gr.sc2 = batch.seg[1].sc;
+        } else if constexpr (!MANY) {
+            gr.c = tail.c;
+        } else {
+            const GemvBatch &batch = tail.batch;
+            int task = gw;
+            gr.c = batch.seg[0].c;
+            if (gw >= first1) {
+                int si = 1;
+#pragma unroll
+                for (int i = 2; i < 4; ++i)
+                    if (i < batch.count && gw >= batch.seg[i].first_wave) si = i;
+                gr.seg = si;
+                gr.qs = batch.seg[si].qs;
+                gr.sc = batch.seg[si].sc;
+                gr.c = batch.seg[si].c;
+                gr.n = batch.seg[si].n;
+                task = gw - batch.seg[si].first_wave;
+            }
+            gr.row0 = task * R;
+            if constexpr (EPI == EPI_ROPE_APPEND) {
+                // task -> (head, first of four pairs): rows head*D + e0 + {0..3} and head*D + D/2 + e0 + {0..3}
+                const int per_head = tail.epi.d >> 3;
+                gr.row0 = (task / per_head) * tail.epi.d + (task % per_head) * 4;
+                half = tail.epi.d >> 1;
+            }
         }
 #pragma unroll
         for (int r = 0; r < R; ++r) {
-            const int row = EPI == EPI_ROPE_APPEND ? gr.row0 + (r & 3) + (r >> 2) * (epi.d >> 1)
+            const int row = EPI == EPI_ROPE_APPEND ? gr.row0 + (r & 3) + (r >> 2) * half
                           : EPI == EPI_GATE_QUANT ? gr.row0 + (r & 3)
                           : min(gr.row0 + r, gr.n - 1);
             gr.rowq[r] = (size_t)row * chunks;
@@ -85,7 +111,7 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
         }
         return gr;
     };
-    bool active = gwave < batch.total_waves;
+    bool active = gwave < total_waves;
     Group cur = locate(active ? gwave : 0);
     // ---- prologue: activation -> int8 codes, per-block scale and code sum in LDS
     const int n4 = K >> 2;
@@ -95,12 +121,12 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
     for (int i = 0; i < MAX_CH4; ++i) {
         const int c4 = tid + NT * i;
         const bool live = c4 < n4;
-        v[i] = live ? *(const f32x4 *)(in.x + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+        v[i] = live ? *(const f32x4 *)(x + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
         if (PRO == PRO_RMSNORM) {
-            aux[i] = live ? *(const f32x4 *)(in.gamma + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
-            aux2[i] = (live && in.beta) ? *(const f32x4 *)(in.beta + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+            aux[i] = live ? *(const f32x4 *)(side + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+            aux2[i] = (live && norm_beta) ? *(const f32x4 *)(norm_beta + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
         } else if (PRO == PRO_GATE) {
-            aux[i] = live ? *(const f32x4 *)(in.y + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+            aux[i] = live ? *(const f32x4 *)(side + (size_t)c4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
     }
     // first weight chunk of every row: requested right behind the activation operands (loads return
@@ -124,7 +150,7 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
     float inv_rms = 1.f;
     if (PRO == PRO_RMSNORM) {
         ss = block_sum_256(ss, s_red);
-        inv_rms = 1.f / sqrtf(ss * (1.f / (float)K) + in.eps);
+        inv_rms = 1.f / sqrtf(ss * (1.f / (float)K) + eps);
     }
 #pragma unroll
     for (int i = 0; i < MAX_CH4; ++i) {
@@ -233,7 +259,8 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
 
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = wave_sum(acc[r]);
-        if (EPI == EPI_ROPE_APPEND) {
+        if constexpr (EPI == EPI_ROPE_APPEND) {
+            const FusedEpi &epi = tail.epi;
             // every lane holds all eight sums; lane p < 4 finishes pair p (aion cpu/kernels/rope.zig:20-98,
             // cpu/exec/cast.zig, cpu/exec/sequence_append.zig:12-104 - the arithmetic of rope_append_kernel)
             if (lane < 4) {
@@ -259,7 +286,7 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
                     }
                 }
             }
-        } else if (EPI == EPI_GATE_QUANT) {
+        } else if constexpr (EPI == EPI_GATE_QUANT) {
             // lanes 0..3: h_j; after the second 16 outputs the workgroup's 32 values are one quant block
             float *s_h = s_red + 4;
             if (lane < 4) {
@@ -276,10 +303,10 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
                     float scale;
                     prepare_act_block8(v0, v1, v2, v3, word, scale, sq);
                     const int blk = gwave >> 3;                     // task = quant block of the down projection's activation
-                    epi.act_q[blk * 8 + tid] = word;
+                    ((int *)tail.act.q)[blk * 8 + tid] = word;
                     if (tid == 0) {
-                        epi.act_scale[blk] = scale;
-                        epi.act_sum[blk] = sq;
+                        tail.act.scale[blk] = scale;
+                        tail.act.sum[blk] = sq;
                     }
                 }
                 __syncthreads();                                    // s_h is reused by the next task
@@ -294,7 +321,7 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
         }
         if (EPI == EPI_GATE_QUANT) gwave = ((gwave >> 2) & 1) ? gwave - 4 + 8 * (int)gridDim.x : gwave + 4;
         else gwave += wave_stride;
-        active = gwave < batch.total_waves;
+        active = gwave < total_waves;
         if (active) {
             cur = locate(gwave);
 #pragma unroll
@@ -304,6 +331,13 @@ __global__ __launch_bounds__(NT) void gemv_fused_kernel(GemvBatch batch, FusedIn
             }
         }
     }
+}
+
+template <class Tail>
+void launch_fused(aionhip_ctx *ctx, void (*kernel)(const u32x4 *, const __half *, const float *, const float *, int, int, int, int, const u32x4 *, const __half *, const float *, float, float, float, Tail),
+                  dim3 grid, dim3 block, size_t lds, int pro, const GemvBatch &batch, const FusedIn &in, int K, float alpha, float beta, const Tail &tail) {
+    launch_k(ctx, kernel, grid, block, lds, batch.seg[0].qs, batch.seg[0].sc, in.x, pro == PRO_RMSNORM ? in.gamma : in.y, K, batch.total_waves, batch.seg[0].n,
+             batch.count > 1 ? batch.seg[1].first_wave : INT32_MAX, batch.seg[1].qs, batch.seg[1].sc, in.beta, in.eps, alpha, beta, tail);
 }
 
 template <int DT, int PRO, int NCH>
@@ -338,9 +372,14 @@ void launch_r(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
             constexpr int WNT = decltype(nt_tag)::value, WNCH = (NCH * 256 + WNT - 1) / WNT;
             const int wg = (waves + WNT / 64 - 1) / (WNT / 64), cap = cus * 32 / (WNT / 64) * rounds;
             const dim3 wgrid((unsigned)(wg < cap ? wg : cap)), wblock(WNT);
-            if (R == 4) launch_k(ctx, gemv_fused_kernel<DT, 4, PRO_QUANT, WNCH, EPI_NONE, WNT>, wgrid, wblock, lds, batch, in, K, alpha, beta, FusedEpi{});
-            else if (R == 2) launch_k(ctx, gemv_fused_kernel<DT, 2, PRO_QUANT, WNCH, EPI_NONE, WNT>, wgrid, wblock, lds, batch, in, K, alpha, beta, FusedEpi{});
-            else launch_k(ctx, gemv_fused_kernel<DT, 1, PRO_QUANT, WNCH, EPI_NONE, WNT>, wgrid, wblock, lds, batch, in, K, alpha, beta, FusedEpi{});
+            auto with = [&](auto many, const auto &tail) {
+                constexpr bool MANY = decltype(many)::value;
+                if (R == 4) launch_fused(ctx, gemv_fused_kernel<DT, 4, PRO_QUANT, WNCH, EPI_NONE, WNT, MANY>, wgrid, wblock, lds, PRO_QUANT, batch, in, K, alpha, beta, tail);
+                else if (R == 2) launch_fused(ctx, gemv_fused_kernel<DT, 2, PRO_QUANT, WNCH, EPI_NONE, WNT, MANY>, wgrid, wblock, lds, PRO_QUANT, batch, in, K, alpha, beta, tail);
+                else launch_fused(ctx, gemv_fused_kernel<DT, 1, PRO_QUANT, WNCH, EPI_NONE, WNT, MANY>, wgrid, wblock, lds, PRO_QUANT, batch, in, K, alpha, beta, tail);
+            };
+            if (count > 1) with(std::true_type{}, FusedTail<EPI_NONE, true>{batch});
+            else with(std::false_type{}, FusedTail<EPI_NONE, false>{batch.seg[0].c});
         };
         if (nt == 512) go(std::integral_constant<int, 512>{});
         else go(std::integral_constant<int, 1024>{});
@@ -350,9 +389,9 @@ void launch_r(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
         // reduction; 262144x2048 behind an RMSNorm: 50.8 us on this grid, 56.7 us on eight rounds)
         const int wgs = (waves + 3) / 4;
         const dim3 grid((unsigned)(wgs < cus * 8 ? wgs : cus * 8)), block(256);
-        if (R == 4) launch_k(ctx, gemv_fused_kernel<DT, 4, PRO, NCH, EPI_NONE>, grid, block, lds, batch, in, K, alpha, beta, FusedEpi{});
-        else if (R == 2) launch_k(ctx, gemv_fused_kernel<DT, 2, PRO, NCH, EPI_NONE>, grid, block, lds, batch, in, K, alpha, beta, FusedEpi{});
-        else launch_k(ctx, gemv_fused_kernel<DT, 1, PRO, NCH, EPI_NONE>, grid, block, lds, batch, in, K, alpha, beta, FusedEpi{});
+        if (R == 4) launch_fused(ctx, gemv_fused_kernel<DT, 4, PRO, NCH, EPI_NONE>, grid, block, lds, PRO, batch, in, K, alpha, beta, FusedTail<EPI_NONE, true>{batch});
+        else if (R == 2) launch_fused(ctx, gemv_fused_kernel<DT, 2, PRO, NCH, EPI_NONE>, grid, block, lds, PRO, batch, in, K, alpha, beta, FusedTail<EPI_NONE, true>{batch});
+        else launch_fused(ctx, gemv_fused_kernel<DT, 1, PRO, NCH, EPI_NONE>, grid, block, lds, PRO, batch, in, K, alpha, beta, FusedTail<EPI_NONE, true>{batch});
     }
 }
 
@@ -386,7 +425,7 @@ void launch_rope(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *q_out
     batch.total_waves = waves;
     const dim3 grid((unsigned)((waves + 3) / 4)), block(256);
     const size_t lds = (size_t)K + (size_t)(K >> 5) * 8 + 16;
-    launch_k(ctx, gemv_fused_kernel<DT, 8, PRO_RMSNORM, NCH, EPI_ROPE_APPEND>, grid, block, lds, batch, in, K, 1.f, 0.f, epi);
+    launch_fused(ctx, gemv_fused_kernel<DT, 8, PRO_RMSNORM, NCH, EPI_ROPE_APPEND>, grid, block, lds, PRO_RMSNORM, batch, in, K, 1.f, 0.f, FusedTail<EPI_ROPE_APPEND, true>{batch, epi});
 }
 
 template <int DT, int NCH>
@@ -400,11 +439,7 @@ void launch_geglu(aionhip_ctx *ctx, const aionhip_weight *gate, const aionhip_we
     const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
     const dim3 grid((unsigned)(tasks < cus * 8 ? tasks : cus * 8)), block(256);
     const size_t lds = (size_t)K + (size_t)(K >> 5) * 8 + 16 + 32 * sizeof(float);
-    FusedEpi epi{};
-    epi.act_q = (int *)out.q;
-    epi.act_scale = out.scale;
-    epi.act_sum = out.sum;
-    launch_k(ctx, gemv_fused_kernel<DT, 8, PRO_RMSNORM, NCH, EPI_GATE_QUANT>, grid, block, lds, batch, in, K, 1.f, 0.f, epi);
+    launch_fused(ctx, gemv_fused_kernel<DT, 8, PRO_RMSNORM, NCH, EPI_GATE_QUANT>, grid, block, lds, PRO_RMSNORM, batch, in, K, 1.f, 0.f, FusedTail<EPI_GATE_QUANT, true>{out});
 }
 
 }  // namespace
