@@ -110,6 +110,25 @@ void prof_open(aionhip_ctx *ctx, hipEvent_t *start, hipEvent_t *stop) {
     *stop = r.stop;
 }
 
+void launch_params(aionhip_ctx *ctx, const void *kernel, dim3 grid, dim3 block, size_t lds, void **params) {
+    auto it = ctx->functions.find(kernel);
+    if (it == ctx->functions.end()) {
+        // the handle is the current device's: the context's has to be current while it is looked up
+        hipFunction_t f = nullptr;
+        int current = ctx->device;
+        (void)hipGetDevice(&current);
+        if (current != ctx->device) (void)hipSetDevice(ctx->device);
+        const hipError_t e = hipGetFuncBySymbol(&f, kernel);
+        if (current != ctx->device) (void)hipSetDevice(current);
+        if (e != hipSuccess) {
+            (void)hipLaunchKernel(kernel, grid, block, params, lds, ctx->stream);
+            return;
+        }
+        it = ctx->functions.emplace(kernel, f).first;
+    }
+    (void)hipModuleLaunchKernel(it->second, grid.x, grid.y, grid.z, block.x, block.y, block.z, (unsigned)lds, ctx->stream, params, nullptr);
+}
+
 int rope_table(aionhip_ctx *ctx, int pairs, float freq_step, float scale_factor, const float **out) {
     for (const auto &t : ctx->rope_tables)
         if (t.pairs == pairs && t.freq_step == freq_step && t.scale_factor == scale_factor) {
