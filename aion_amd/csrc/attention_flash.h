@@ -36,7 +36,7 @@ constexpr int SPLIT_NW = 8;
 // 8.0 -> 6.75 us; 1531 keys, 8 KV heads of size 128: 7.6 -> 6.0 us (+ 3.6 for the segments' merge); eight sequences over 16384 keys,
 // one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
 template <int KV, int D, bool SPLIT, bool HILO, bool RING, int DVS = 1, class Hooks>
-__device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int block_x, const int block_y, Hooks &hooks,
+__device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int rt_block, const int seg, const int b, const int hk, Hooks &hooks,
                                                 const int slice_dv = 0) {
     const int ring = RING ? a.ring : 0;
     constexpr int NW = SPLIT ? SPLIT_NW : 4;
@@ -49,17 +49,15 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
 
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4;
-    const int unit = block_y;
-    const int b = unit / a.Hkv, hk = unit % a.Hkv;
-    int rt, seg;
-    if (SPLIT) { rt = block_x / a.nseg; seg = block_x % a.nseg; }
-    else { rt = block_x * 4 + wave; seg = 0; }
+    const int unit = b * a.Hkv + hk;
+    const int rt = SPLIT ? rt_block : rt_block * 4 + wave;
 
     // ---- this lane's query row. Loads are requested in dependency order and consumed late: the index
     // operands first, then q (its address needs no loaded value), so one memory round trip covers both.
     const int r = rt * 16 + n;
     const bool row_ok = rt < a.row_tiles && r < a.rows_total;
-    const int li = row_ok ? r / a.groups : 0, gi = row_ok ? r % a.groups : 0;
+    // (one query per sequence: no division, some 20 dependent instructions ahead of the first load)
+    const int li = row_ok && a.L > 1 ? (int)((unsigned)r / (unsigned)a.groups) : 0, gi = row_ok ? r - li * a.groups : 0;
     const int hq = hk * a.groups + gi;
     // The cache length is read with a vector load (a per-lane zero in the address keeps the compiler from
     // turning it into a scalar load, which it would wait for on the spot): it is then in flight together with
@@ -93,7 +91,7 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     } else if (q_shared) {
         const int r2 = rt * 16 + qs_row;
         if (qs_row < 16 && rt < a.row_tiles && r2 < a.rows_total) {
-            const int l2 = r2 / a.groups, g2 = r2 % a.groups;
+            const int l2 = a.L > 1 ? (int)((unsigned)r2 / (unsigned)a.groups) : 0, g2 = r2 - l2 * a.groups;
             const f32x4 *qp = (const f32x4 *)((const float *)a.q + (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g2) * D + qs_col);
             qs0 = qp[0];
             qs1 = qp[1];

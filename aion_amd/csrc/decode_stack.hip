@@ -584,7 +584,7 @@ __global__ __launch_bounds__(DS_NT) void decode_stack_kernel(DsArgs p) {
                 a.win_left = p.win_left; a.win_right = p.win_right; a.win_chunk = p.win_chunk;
                 StackAttnHooks<D> hooks{p, L, qkv_f, tag0 + (unsigned)(l * 8) + 1, tag0 + (unsigned)(l * 8) + 2, unit, rt, new_row, multi_tile, pc};
                 stamp(l, 0);
-                attn_flash_body<AIONHIP_F16, D, true, false, false>(a, lds, rt, unit, hooks);
+                attn_flash_body<AIONHIP_F16, D, true, false, false>(a, lds, rt, 0, 0, unit, hooks);
                 stamp(l, 1);
                 if (hooks.q_at) stamp_at(p, stamp_wg, l, 2, hooks.q_at, tid);
                 hooks_dead = hooks.dead;

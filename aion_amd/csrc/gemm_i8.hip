@@ -169,8 +169,6 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
     static_assert(I8_SHAPES[SHAPE].bm == BM && I8_SHAPES[SHAPE].bn == BN && I8_SHAPES[SHAPE].ks == KS, "shape table order");
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
     static_assert((uint64_t)32 * NT * GEMM_I8_MAX_K <= (uint64_t)1 << 32, "a lane's weight offset and the group's behind it fit 32 bits");
-    static std::atomic<uint64_t> attr{0};
-    if (const int rc = allow_lds(ctx, attr, (const void *)gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, LDS)) return rc;
     GemmSegs segs{};
     segs.count = count;
     int tiles = 0;
@@ -192,14 +190,22 @@ int launch_kernel(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *cons
         if (rc) return rc;
         partial = (float *)ctx->scratch2;
     }
-    // Tiles are dealt out in groups of eight row tiles (256 .. 1024 rows), columns within: the activation rows and weight columns that run on an XCD
+    // The kernel deals tiles out in groups of eight row tiles (256 .. 1024 rows), columns within: the activation rows and weight columns that run on an XCD
     // at the same time then fit its L2 (2048 x 14336 x 4096, 64 x 64 tiles: 409 -> 387 us for q4, 524 -> 465 for q8).
-    const int row_group = row_tiles < 8 ? row_tiles : 8;
     // All workgroups at once, two per CU at most: wavefronts give way to those behind them, see the kernel (128 x 16384 x 2048 q4 22.0 -> 21.3 us, q8
     // 24.2 -> 23.1; q8 512 x 4096 x 4096 35.9 -> 35.0, 256 x 4096 x 4096 23.4 -> 22.8; 48 x 9000 x 2080 q4 14.8 -> 13.9).
     const int one_round = (size_t)tiles * row_tiles * slices <= 2 * (size_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    launch_k(ctx, gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE>, dim3((unsigned)(tiles * row_tiles), 1, (unsigned)slices), dim3(64 * KS * WGM * WGN), LDS, segs,
-             (const uint8_t *)act.q, (const float *)act.scale, (int)m, (int)ws[0]->k, row_tiles, row_group, tiles, one_round, alpha, beta, partial, partial_ld);
+    const auto launch = [&](auto many, const auto &form) {
+        constexpr bool MANY = decltype(many)::value;
+        using Segs = typename GemmSegsOf<GEMM_PLAIN, MANY>::type;
+        auto *kern = gemm_i8_kernel<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE, GEMM_PLAIN, MANY>;
+        static std::atomic<uint64_t> attr{0};
+        if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
+        launch_k(ctx, kern, dim3((unsigned)(tiles * row_tiles), 1, (unsigned)slices), dim3(64 * KS * WGM * WGN), LDS, (const uint8_t *)act.q, (const float *)act.scale, ws[0]->qs,
+                 ws[0]->sc, (int)m, (int)ws[0]->k, (int)ws[0]->n, gemm_i8_form(one_round, slices, tiles), nullptr, GemmTail<Segs>{form, alpha, beta, partial, partial_ld});
+        return (int)AIONHIP_OK;
+    };
+    if (const int rc = count > 1 ? launch(std::true_type{}, segs) : launch(std::false_type{}, GemmOne{{cs[0]}, {ldcs[0]}})) return rc;
     if (slices > 1) {
         const size_t threads = m * (size_t)(partial_ld >> 2);
         launch_k(ctx, gemm_i8_slices_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, segs, partial, (int)m, slices, partial_ld, BN, alpha, beta);

@@ -62,8 +62,25 @@ struct GemmRopeSegs : GemmSegs {
     const float *freq;
     int s_len, t_cap, h_q, h_kv, d, rope_pairs;
 };
-template <int EPI> struct GemmSegsOf { using type = GemmSegs; };
-template <> struct GemmSegsOf<GEMM_ROPE> { using type = GemmRopeSegs; };
+// A launch's arguments. What a wavefront needs for its first loads - the activation, the first weight, the sizes - are plain leading arguments, which
+// arrive in SGPRs with it (14 words do); a structure by value is read from memory, a round trip ahead of the first address, and so is gridDim. The rest is
+// the last argument, in the form that the launch needs: one weight (c, ldc), up to four, the pair launches' own. q4 512 x 4096 x 4096 33.7 -> 33.0 us, q8 77 x
+// 11008 x 4096 25.5 -> 25.1, q4 4 x 4096 x 14336 (gemv_slim_kernel) 11.4 -> 10.9; a 128-token prompt of 26 blocks 1898 -> 1856.
+struct GemmOne {
+    float *c[1];
+    size_t ldc[1];
+};
+template <int EPI, bool MANY> struct GemmSegsOf { using type = GemmSegs; };
+template <> struct GemmSegsOf<GEMM_PLAIN, false> { using type = GemmOne; };
+template <> struct GemmSegsOf<GEMM_ROPE, true> { using type = GemmRopeSegs; };
+template <class Segs> struct GemmTail {
+    Segs segs;
+    float alpha, beta;
+    float *partial;
+    int partial_ld;
+};
+// the sizes that ride in one word: whether all workgroups run at once, the K slices (at most 4), the column tiles of all weights
+inline int gemm_i8_form(int one_round, int slices, int col_tiles) { return one_round | slices << 1 | col_tiles << 4; }
 
 // Prepared activation in the order the kernel's operand loads want: row tiles of 32 rows (the last one may hold fewer), per
 // tile and quant block [h = 0, 1][row][16 codes] - k = 16 h .. 16 h + 15 of the block - so that a wavefront's load of one
@@ -73,10 +90,11 @@ __host__ __device__ __forceinline__ int act_tile_rows(int M, int mt) { return M 
 // LDS of a wavefront: two groups of four blocks, weight codes and activation scales
 template <bool Q8, int MT, int NT> __host__ __device__ constexpr int gemm_i8_wave_lds_bytes() { return 2 * (NT * 32 * (Q8 ? 128 : 64) + MT * 512); }
 
-// workgroup `bid` of the kernel's grid (the K slices, if any, are the grid's z)
-template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI = GEMM_PLAIN>
-__device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::type &segs, int bid, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int M, int K,
-                                             int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta, float *__restrict__ partial, int partial_ld) {
+// workgroup `bid` of the kernel's grid (the K slices, if any, are the grid's z). qs0, sc0, n0: the first weight; qs1: GEMM_GATE's second.
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI, bool MANY>
+__device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI, MANY>::type &segs, int bid, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
+                                             const uint8_t *__restrict__ qs0, const __half *__restrict__ sc0, int M, int K, int n0w, const uint8_t *__restrict__ qs1,
+                                             int col_tiles, int slices, int one_round, float alpha, float beta, float *__restrict__ partial, int partial_ld) {
     constexpr bool Q8 = DT == AIONHIP_Q8_0;
     constexpr bool PAIR = EPI != GEMM_PLAIN, GATE = EPI == GEMM_GATE;
     constexpr int BM = 32 * MT * WGM, BN = 32 * NT * WGN;
@@ -91,19 +109,29 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
     const int ks = wave / (WGM * WGN), wsub = wave % (WGM * WGN), wm = wsub / WGN, wn = wsub % WGN;
     // workgroup -> tile: ids go round-robin over the 8 XCDs; every XCD takes a contiguous run of tiles, row tiles fastest, so that
     // the workgroups that share a weight column tile run on one L2
-    const int tiles = row_tiles * col_tiles;
+    // (row tiles in groups of eight, columns within: see the launcher)
+    const int row_tiles = (M + BM - 1) / BM, row_group = min(row_tiles, 8), tiles = row_tiles * col_tiles;
     const int xcd = bid & 7, slot = bid >> 3;
     const int t = xcd * (tiles >> 3) + min(xcd, tiles & 7) + slot;
-    const int grp = t / (row_group * col_tiles), gr0 = grp * row_group, gr = min(row_group, row_tiles - gr0);
-    const int ct = (t - gr0 * col_tiles) / gr, rt = gr0 + (t - gr0 * col_tiles) - ct * gr;
-    int si = 0;
+    // (up to eight row tiles: one group. Divisions are some 20 dependent instructions each ahead of the first load)
+    const int gr0 = row_tiles <= 8 ? 0 : (int)((unsigned)t / (unsigned)(row_group * col_tiles)) * row_group, gr = min(row_group, row_tiles - gr0);
+    const int in_group = t - gr0 * col_tiles, ct = gr == 1 ? in_group : (int)((unsigned)in_group / (unsigned)gr), rt = gr0 + in_group - ct * gr;
+    int si = 0, first_tile = 0, N = n0w;
+    const uint8_t *__restrict__ qs = qs0;
+    const __half *__restrict__ sc = sc0;
+    if constexpr (MANY && !GATE) {
+        if (ct >= (n0w + BN - 1) / BN) {                 // (the second weight's first tile)
+            si = 1;
 #pragma unroll
-    for (int i = 1; i < 4; ++i)
-        if (!GATE && i < segs.count && ct >= segs.first_tile[i]) si = i;
-    const uint8_t *__restrict__ qs = segs.qs[si];
-    const __half *__restrict__ sc = segs.sc[si];
+            for (int i = 2; i < 4; ++i)
+                if (i < segs.count && ct >= segs.first_tile[i]) si = i;
+            qs = segs.qs[si];
+            sc = segs.sc[si];
+            N = segs.n[si];
+            first_tile = segs.first_tile[si];
+        }
+    }
     float *__restrict__ c = segs.c[si];
-    const int N = segs.n[si];
     size_t ldc = segs.ldc[si];
     const int KB = K >> 5, G = (KB + 3) >> 2;
     // (a head's columns: pair tile `head_tile` is its columns 32 head_tile .. and the same of its second half)
@@ -111,12 +139,12 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
     size_t partner = 0;                          // weight rows from a column of the first tile to its partner's
     if constexpr (EPI == GEMM_ROPE) {
         const int per_head = segs.d >> 6;
-        head = (ct - segs.first_tile[si]) / per_head;
-        head_tile = ct - segs.first_tile[si] - head * per_head;
+        head = (ct - first_tile) / per_head;
+        head_tile = ct - first_tile - head * per_head;
         partner = (size_t)segs.d >> 1;
         pair_col = head * segs.d + head_tile * 32;
     }
-    const int n0 = PAIR ? pair_col : (ct - segs.first_tile[si]) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
+    const int n0 = PAIR ? pair_col : (ct - first_tile) * BN + wn * (32 * NT), m0 = rt * BM + wm * (32 * MT);
 
     Acc acc[MT][NT];
     // q4 dots are 16 times the codes' dots. The 1/16 is taken from the sums, where it is exact down to subnormal products of scales; sums past
@@ -146,8 +174,10 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
         }
         const int nb = min(n0, N - 1);
         const unsigned wpitch = Q8 ? (unsigned)K : (unsigned)K >> 1;
-        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = (GATE ? segs.qs[1] : qs) + ((size_t)nb + partner) * wpitch;      // (used in the device pass only)
-        const __half *sb = (GATE && h ? segs.sc[1] : sc) + ((size_t)nb + (EPI == GEMM_ROPE && h ? partner : 0)) * KB;
+        [[maybe_unused]] const uint8_t *wb = qs + (size_t)nb * wpitch, *wb1 = (GATE ? qs1 : qs) + ((size_t)nb + partner) * wpitch;      // (used in the device pass only)
+        const __half *sb = sc;
+        if constexpr (GATE) sb = h ? segs.sc[1] : sc;
+        sb += ((size_t)nb + (EPI == GEMM_ROPE && h ? partner : 0)) * KB;
         // weights: load l of a tile's group covers 8 (q8) or 16 (q4) rows, the lanes of a row side by side along it
         constexpr int RB = Q8 ? 128 : 64, LPR = RB / 16, WL = LPR / 2;      // bytes of a row per group, lanes per row, loads per 32 rows
         const int w_row = lane / LPR;
@@ -161,7 +191,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
         const unsigned so = (unsigned)(min(n0 + (NT == 2 && !PAIR ? h * 32 : 0) + r, N - 1) - nb) * (unsigned)KB;
 
         // groups of four quant blocks: K slice z takes a contiguous run of them, its KS wavefronts every KS-th group of the run
-        const int g_per = (G + (int)gridDim.z - 1) / (int)gridDim.z;
+        const int g_per = slices == 1 ? G : (G + slices - 1) / slices;
         const int g_lo = (int)blockIdx.z * g_per, g_hi = min(G, g_lo + g_per);
 
         // Registers: the four blocks of a group's activations (reloaded for the next group as each is used up), the next group's weight
@@ -422,7 +452,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
 
     if (partial) {
         // a K slice leaves raw sums; gemm_i8_slices_kernel adds the slices in order and applies alpha and beta
-        c = partial + (size_t)blockIdx.z * M * partial_ld + (size_t)segs.first_tile[si] * BN;
+        c = partial + (size_t)blockIdx.z * M * partial_ld + (size_t)first_tile * BN;
         ldc = partial_ld;
         alpha = 1.f;
         beta = 0.f;
@@ -467,6 +497,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
             }
             return;
         }
+        if constexpr (GATE) {
         const int kb = n0 >> 5, KBN = N >> 5, mt = (m0 >> 5) + i, rows = act_tile_rows(M, mt);
         uint8_t *codes = (uint8_t *)segs.c[0] + ((size_t)mt * 32 * KBN + (size_t)kb * rows) * 32 + (r >> 4) * rows * 16 + (r & 15);
         float *scales = segs.c[1] + (size_t)mt * 32 * KBN + (size_t)kb * rows;
@@ -479,6 +510,7 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
             if (row >= rows) continue;
             codes[row * 16] = (uint8_t)code;
             if (r == 0) scales[row] = scale;
+        }
         }
     };
     if constexpr (PAIR && KS == 1) {
@@ -537,11 +569,12 @@ __device__ __forceinline__ void gemm_i8_body(const typename GemmSegsOf<EPI>::typ
     }
 }
 
-template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI = GEMM_PLAIN>
-__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(typename GemmSegsOf<EPI>::type segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale,
-                                                                         int M, int K, int row_tiles, int row_group, int col_tiles, int one_round, float alpha, float beta,
-                                                                         float *__restrict__ partial, int partial_ld) {
-    gemm_i8_body<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE, EPI>(segs, (int)blockIdx.x, aq, a_scale, M, K, row_tiles, row_group, col_tiles, one_round, alpha, beta, partial, partial_ld);
+template <int DT, int MT, int NT, int KS, int WGM, int WGN, int RQ, bool WHOLE, int EPI, bool MANY>
+__global__ __launch_bounds__(64 * KS * WGM * WGN, MT * NT == 1 ? 4 : 2) void gemm_i8_kernel(const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, const uint8_t *__restrict__ qs0,
+                                                                         const __half *__restrict__ sc0, int M, int K, int n0, int form, const uint8_t *__restrict__ qs1,
+                                                                         GemmTail<typename GemmSegsOf<EPI, MANY>::type> tail) {
+    gemm_i8_body<DT, MT, NT, KS, WGM, WGN, RQ, WHOLE, EPI, MANY>(tail.segs, (int)blockIdx.x, aq, a_scale, qs0, sc0, M, K, n0, qs1, form >> 4, form >> 1 & 7, form & 1, tail.alpha,
+                                                                 tail.beta, tail.partial, tail.partial_ld);
 }
 
 template <bool Q8, int MT, int NT, int KS, int WGM, int WGN, int RQ> constexpr int gemm_i8_lds_bytes() {

@@ -13,13 +13,13 @@ template <int EPI, int DT, int MT, int KS, int WGM, int RQ, bool WHOLE, class Se
 int launch_kernel(aionhip_ctx *ctx, const Segs &segs, int tiles, size_t k, size_t m, PreparedAct in) {
     constexpr int LDS = gemm_i8_lds_bytes<DT == AIONHIP_Q8_0, MT, 2, KS, WGM, 1, RQ>();
     static_assert(LDS <= 80 * 1024, "two workgroups per CU");
-    auto *kern = gemm_i8_kernel<DT, MT, 2, KS, WGM, 1, RQ, WHOLE, EPI>;
+    auto *kern = gemm_i8_kernel<DT, MT, 2, KS, WGM, 1, RQ, WHOLE, EPI, true>;
     static std::atomic<uint64_t> attr{0};
     if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
     const int row_tiles = (int)((m + 32 * MT * WGM - 1) / (32 * MT * WGM));
     const int one_round = (size_t)tiles * row_tiles <= 2 * (size_t)(ctx->cu_count > 0 ? ctx->cu_count : 256);
-    launch_k(ctx, kern, dim3((unsigned)(tiles * row_tiles)), dim3(64 * KS * WGM), LDS, segs, (const uint8_t *)in.q, (const float *)in.scale, (int)m,
-             (int)k, row_tiles, row_tiles < 8 ? row_tiles : 8, tiles, one_round, 1.f, 0.f, (float *)nullptr, 0);
+    launch_k(ctx, kern, dim3((unsigned)(tiles * row_tiles)), dim3(64 * KS * WGM), LDS, (const uint8_t *)in.q, (const float *)in.scale, segs.qs[0], segs.sc[0], (int)m, (int)k,
+             segs.n[0], gemm_i8_form(one_round, 1, tiles), segs.qs[1], GemmTail<Segs>{segs, 1.f, 0.f, nullptr, 0});
     return AIONHIP_OK;
 }
 

@@ -56,8 +56,8 @@ struct MfBatch {
 };
 
 template <int DT>
-__global__ __launch_bounds__(256) void gemv_mfma_kernel(MfBatch batch, const u32x4 *__restrict__ aq, const float *__restrict__ a_scale,
-                                                        const int *__restrict__ a_sum, int K, int m, float alpha, float beta) {
+__global__ __launch_bounds__(256) void gemv_mfma_kernel(const u32x4 *__restrict__ aq, const float *__restrict__ a_scale, const int *__restrict__ a_sum, int K, int m,
+                                                        MfBatch batch, float alpha, float beta) {
     using Cfg = MfCfg<DT>;
     constexpr bool Q8 = Cfg::Q8;
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_mf[];
@@ -292,7 +292,7 @@ int launch_mf(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
     const int wgs = (int)min((long)(tiles + 3) / 4, (long)cus * (lds <= 80 * 1024 ? 2 : 1));
     static std::atomic<uint64_t> attr{0};
     if (const int rc = allow_lds(ctx, attr, (const void *)gemv_mfma_kernel<DT>, MOST)) return rc;
-    launch_k(ctx, gemv_mfma_kernel<DT>, dim3((unsigned)wgs), dim3(256), lds, batch, (const u32x4 *)act.q, act.scale, act.sum, K, m, alpha, beta);
+    launch_k(ctx, gemv_mfma_kernel<DT>, dim3((unsigned)wgs), dim3(256), lds, (const u32x4 *)act.q, act.scale, act.sum, K, m, batch, alpha, beta);
     return AIONHIP_OK;
 }
 

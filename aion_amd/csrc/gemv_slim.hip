@@ -25,19 +25,32 @@ template <int DT> struct SlCfg {
 };
 
 // workgroup `bid` of the kernel's grid (GemmSegs: tiles of SL_ROWS weight rows)
-template <int DT, int KS>
-__device__ __forceinline__ void gemv_slim_body(const GemmSegs &segs, int bid, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int a_tiled, int K, int m,
-                                               float alpha, float beta) {
+template <int DT, int KS, class Segs>
+__device__ __forceinline__ void gemv_slim_body(const Segs &segs, int bid, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, const uint8_t *__restrict__ qs0,
+                                               const __half *__restrict__ sc0, int n0, int a_tiled, int K, int m, float alpha, float beta) {
     using Cfg = SlCfg<DT>;
     constexpr bool Q8 = Cfg::Q8;
     extern __shared__ __attribute__((aligned(1024))) unsigned char s_sl[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, g = lane >> 4, hb = g >> 1, hh = g & 1;
-    int si = 0;
+    int si = 0, first_tile = 0, N = n0;
+    [[maybe_unused]] const uint8_t *__restrict__ qs = qs0;       // (in the device pass only)
+    const __half *__restrict__ sc = sc0;
+    if constexpr (std::is_same<Segs, GemmSegs>::value) {
+        if (bid >= (n0 + SL_ROWS - 1) / SL_ROWS) {       // (the second weight's first workgroup)
+            si = 1;
 #pragma unroll
-    for (int i = 1; i < 4; ++i)
-        if (i < segs.count && bid >= segs.first_tile[i]) si = i;
-    const int N = segs.n[si], row0 = (bid - segs.first_tile[si]) * SL_ROWS;
+            for (int i = 2; i < 4; ++i)
+                if (i < segs.count && bid >= segs.first_tile[i]) si = i;
+            qs = segs.qs[si];
+            sc = segs.sc[si];
+            N = segs.n[si];
+            first_tile = segs.first_tile[si];
+        }
+    }
+    float *__restrict__ c = segs.c[si];
+    const size_t ldc = segs.ldc[si];
+    const int row0 = (bid - first_tile) * SL_ROWS;
     constexpr int RUNS = SL_PARTS / KS;                          // of a wavefront
     const int KB = K >> 5, stages = K >> 7;
     auto run_end = [&](int i) { return (wave * RUNS + i) * stages / SL_PARTS; };
@@ -65,7 +78,7 @@ __device__ __forceinline__ void gemv_slim_body(const GemmSegs &segs, int bid, co
     // where piece p of row n & 7 lies
     const int a_at = a_tiled ? (n & 7) * 16 : (n & 7) * 128, a_mul = a_tiled ? 128 : 16, a_xor = a_tiled ? 0 : n & 7;
 #if defined(__HIP_DEVICE_COMPILE__)   // (buffer loads: a global LDS-writing load makes the compiler wait for everything in flight before the next LDS read)
-    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(segs.qs[si] + (size_t)first * pitch + (size_t)s_lo * Cfg::ROWB), 0, 0xFFFFFFFFu, 0x00027000);
+    const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(qs + (size_t)first * pitch + (size_t)s_lo * Cfg::ROWB), 0, 0xFFFFFFFFu, 0x00027000);
     const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)(aq + (size_t)s_lo * a_step), 0, 0xFFFFFFFFu, 0x00027000);
 #endif
     auto issue = [&](int s, int slot) {                          // (s past the run: its last stage again, never used)
@@ -82,7 +95,7 @@ __device__ __forceinline__ void gemv_slim_body(const GemmSegs &segs, int bid, co
     f32x4 as_next;
     u32x2 ws_next[2];
     const float *asp = a_scale + (a_tiled ? (size_t)a_src : (size_t)a_src * KB);
-    const __half *wsp = segs.sc[si] + (size_t)min(row0 + (lane >> 2), N - 1) * KB;
+    const __half *wsp = sc + (size_t)min(row0 + (lane >> 2), N - 1) * KB;
     auto load_scales = [&](int s) {
         const size_t kb = (size_t)min(s_lo + s + a_stage, stages - 1) * 4;
         if (a_tiled) {
@@ -188,26 +201,28 @@ __device__ __forceinline__ void gemv_slim_body(const GemmSegs &segs, int bid, co
 #pragma unroll
             for (int i = 0; i < 2; ++i) sum[i][w] = sum[i][2 * w] + sum[i][2 * w + 1];
     const float v = alpha * (sum[0][0] + sum[1][0]);
-    float *dst = segs.c[si] + (size_t)row * segs.ldc[si] + row0 + col;
+    float *dst = c + (size_t)row * ldc + row0 + col;
     *dst = beta == 0.f ? v : v + beta * *dst;
 }
 
-template <int DT, int KS>
-__global__ __launch_bounds__(64 * KS, 4) void gemv_slim_kernel(GemmSegs segs, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int a_tiled, int K, int m,
-                                                               float alpha, float beta) {
-    gemv_slim_body<DT, KS>(segs, (int)blockIdx.x, aq, a_scale, a_tiled, K, m, alpha, beta);
+// (the arguments' order: see GemmTail)
+template <int DT, int KS, class Segs>
+__global__ __launch_bounds__(64 * KS, 4) void gemv_slim_kernel(const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, const uint8_t *__restrict__ qs0,
+                                                               const __half *__restrict__ sc0, int K, int m, int n0, int a_tiled, GemmTail<Segs> tail) {
+    gemv_slim_body<DT, KS>(tail.segs, (int)blockIdx.x, aq, a_scale, qs0, sc0, n0, a_tiled, K, m, tail.alpha, tail.beta);
 }
 
 // Siblings of both kinds in one grid, q4: the exact GEMM's tiles of eight wavefronts first, then this kernel's workgroups of as many. Two launches one
 // after the other would leave half of the CUs to each: 8 x (5120 + 1024 + 1024) x 5120 17.6 -> 14.3 us (all
 // three on the exact GEMM 11.2, with other bits for the narrow ones than they have by themselves), 8 x (8192 + 1024 + 1024) x 8192 21.7 -> 19.0 (23.2).
 constexpr int GS_KS = 8;
-__global__ __launch_bounds__(64 * GS_KS, 4) void gemm_slim_q4_kernel(GemmSegs gemm, GemmSegs slim, const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int K, int m,
-                                                                     int gemm_tiles, float alpha, float beta) {
+__global__ __launch_bounds__(64 * GS_KS, 4) void gemm_slim_q4_kernel(const uint8_t *__restrict__ aq, const float *__restrict__ a_scale, int K, int m, int gemm_tiles, float alpha,
+                                                                     float beta, GemmSegs gemm, GemmSegs slim) {
     if ((int)blockIdx.x < gemm_tiles)
-        gemm_i8_body<AIONHIP_Q4_0, 1, 1, GS_KS, 1, 1, 2, true>(gemm, (int)blockIdx.x, aq, a_scale, m, K, 1, 1, gemm_tiles, 0, alpha, beta, nullptr, 0);
+        gemm_i8_body<AIONHIP_Q4_0, 1, 1, GS_KS, 1, 1, 2, true, GEMM_PLAIN, true>(gemm, (int)blockIdx.x, aq, a_scale, gemm.qs[0], gemm.sc[0], m, K, gemm.n[0], nullptr, gemm_tiles, 1, 0,
+                                                                                 alpha, beta, nullptr, 0);
     else
-        gemv_slim_body<AIONHIP_Q4_0, GS_KS>(slim, (int)blockIdx.x - gemm_tiles, aq, a_scale, 1, K, m, alpha, beta);
+        gemv_slim_body<AIONHIP_Q4_0, GS_KS>(slim, (int)blockIdx.x - gemm_tiles, aq, a_scale, slim.qs[0], slim.sc[0], slim.n[0], 1, K, m, alpha, beta);
 }
 
 int fill_segs(GemmSegs &segs, const aionhip_weight *const *ws, float *const *cs, const size_t *ldcs, int count, int rows) {
@@ -231,14 +246,18 @@ int launch_ks(aionhip_ctx *ctx, const aionhip_weight *const *ws, float *const *c
     constexpr int LDS = KS * SlCfg<DT>::WAVE;
     static_assert(LDS <= 160 * 1024 / (16 / KS), "16 wavefronts per CU");
     static_assert(KS * 1024 <= LDS && (KS == 4 || KS == 8 || KS == 16), "partial sums in the rings; one, two or four runs of K to a wavefront");
-    auto *kern = gemv_slim_kernel<DT, KS>;
-    static std::atomic<uint64_t> attr{0};
-    if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
     GemmSegs segs;
     const int tiles = fill_segs(segs, ws, cs, ldcs, count, SL_ROWS);
-    launch_k(ctx, kern, dim3((unsigned)tiles), dim3(64 * KS), LDS, segs, (const uint8_t *)act.q, (const float *)act.scale, (int)act.tiled,
-             (int)ws[0]->k, m, alpha, beta);
-    return AIONHIP_OK;
+    const auto launch = [&](const auto &form) {
+        using Segs = typename std::decay<decltype(form)>::type;
+        auto *kern = gemv_slim_kernel<DT, KS, Segs>;
+        static std::atomic<uint64_t> attr{0};
+        if (const int rc = allow_lds(ctx, attr, (const void *)kern, LDS)) return rc;
+        launch_k(ctx, kern, dim3((unsigned)tiles), dim3(64 * KS), LDS, (const uint8_t *)act.q, (const float *)act.scale, ws[0]->qs, ws[0]->sc, (int)ws[0]->k, m, (int)ws[0]->n,
+                 (int)act.tiled, GemmTail<Segs>{form, alpha, beta, nullptr, 0});
+        return (int)AIONHIP_OK;
+    };
+    return count > 1 ? launch(segs) : launch(GemmOne{{cs[0]}, {ldcs[0]}});
 }
 
 }  // namespace
@@ -294,8 +313,8 @@ int launch_gemm_slim(aionhip_ctx *ctx, const aionhip_weight *const *gemm, float 
     GemmSegs segs, slim_segs;
     const int gemm_tiles = fill_segs(segs, gemm, gemm_cs, gemm_ldcs, gemm_count, 32), slim_tiles = fill_segs(slim_segs, slim, slim_cs, slim_ldcs, slim_count, SL_ROWS);
     ProfScope scope(ctx, "gemm_i8_q4_slim");
-    launch_k(ctx, gemm_slim_q4_kernel, dim3((unsigned)(gemm_tiles + slim_tiles)), dim3(64 * GS_KS), LDS, segs, slim_segs, (const uint8_t *)act.q, (const float *)act.scale,
-             (int)gemm[0]->k, m, gemm_tiles, alpha, beta);
+    launch_k(ctx, gemm_slim_q4_kernel, dim3((unsigned)(gemm_tiles + slim_tiles)), dim3(64 * GS_KS), LDS, (const uint8_t *)act.q, (const float *)act.scale, (int)gemm[0]->k, m,
+             gemm_tiles, alpha, beta, segs, slim_segs);
     LAUNCH_CHECK(ctx, "gemm_i8_q4_slim");
     return AIONHIP_OK;
 }
