@@ -10,8 +10,8 @@
 //   head); each lane's accumulators, running max and sum belong to ONE query row, so the softmax
 //   bookkeeping is per-lane scalar work. Two launch shapes:
 //     split mode (few query rows: decode) - a workgroup is one 16-row tile x one key segment, its
-//       eight wavefronts interleave 32-key tiles and merge through LDS; segments merge in
-//       attn_merge_kernel (the flash-decoding split of cpu/exec/attention.zig:879-962).
+//       eight wavefronts interleave 32-key tiles and merge through LDS; segments are merged by
+//       the workgroup that ends last, many of them by attn_merge_kernel (the flash-decoding split of cpu/exec/attention.zig:879-962).
 //       Where that leaves CUs idle, the value columns are divided over up to D / 64 workgroups as well.
 //     per-wavefront mode - a workgroup is four 16-row tiles, each wavefront walks its own key range; used
 //       for many query rows only when the hi+lo precise mode is on (see attn_prefill_kernel otherwise).
@@ -63,6 +63,7 @@ struct FlashPrepareHooks : FlashKernelHooks {
 // segments, query type << 16. One token over 1531 keys, 8 KV heads of 128, 9.03 -> 8.56 us with the merge. The grid is (row tiles x segments x shares of the value columns, KV heads, sequences).
 struct FlashTail {
     float *out, *partial;
+    unsigned *tickets;
     float scale, soft_cap;
     unsigned win_left, win_right, win_chunk;
     int ring, B;
@@ -91,6 +92,7 @@ __global__ __launch_bounds__(SPLIT ? SPLIT_NW * 64 : 256) void attn_flash_kernel
     a.kv_dtype = KV;
     a.out = tail.out;
     a.partial = tail.partial;
+    a.tickets = tail.tickets;
     a.scale = tail.scale;
     a.soft_cap = tail.soft_cap;
     a.win_left = tail.win_left;
@@ -125,7 +127,7 @@ __global__ __launch_bounds__(SPLIT ? SPLIT_NW * 64 : 256) void attn_flash_kernel
 inline unsigned flash_heads(const AttnArgs &a) { return (unsigned)a.Hkv | (unsigned)a.groups << 16; }
 inline unsigned flash_form(const AttnArgs &a) { return (unsigned)a.nseg | (unsigned)a.q_dtype << 16; }
 inline FlashTail flash_tail(const AttnArgs &a) {
-    return FlashTail{a.out, a.partial, a.scale, a.soft_cap, a.win_left, a.win_right, a.win_chunk, a.ring, a.B, a.codes, a.code_scales};
+    return FlashTail{a.out, a.partial, a.tickets, a.scale, a.soft_cap, a.win_left, a.win_right, a.win_chunk, a.ring, a.B, a.codes, a.code_scales};
 }
 
 // log-sum-exp merge of the key segments: one workgroup per (row tile, 16-wide dv slice, unit).
@@ -272,6 +274,37 @@ int launch_flash_split(aionhip_ctx *ctx, AttnArgs &a) {
     return AIONHIP_OK;
 }
 
+// Whether the segments are merged by the workgroup that ends last instead of a launch of their own: a wavefront of it has a row's segments in flight
+// MEET_UNROLL at a time for each lane of a column, and up to four such rounds cost no more than a launch. us with the merge launch / without: 1531 keys of 8
+// KV heads x 128, 6 segments, 8.6 / 7.0; 8 sequences over 4000 keys of one KV head x 256, 16 segments, 12.6 / 11.1; one over 16384, 64 segments in four shares
+// of the value columns, 12.4 / 11.4; 8 x 16384, 32 in one share (four rounds), 27.7 / 27.4. Past that the one workgroup reads too much: 4 x 16384, 64 in one
+// share, 19.1 / 20.2.
+constexpr int MEET_ROUNDS = 4;
+bool last_merges(const AttnArgs &a, int dv) { return a.nseg <= min(64, MEET_ROUNDS * MEET_UNROLL * (256 / dv)); }
+
+// Key segments of a 16-row tile. A workgroup's eight wavefronts take a 32-key tile each; how fast a short cache is read is what one CU's L1 fills (64 bytes a
+// clock), so that two tiles to a workgroup on more CUs beat eight on fewer as long as the merge stays small: 24 segments, fewer where the workgroups, with the
+// value columns in all their shares, would not fit the CUs at once. us a token, eight tiles / two: 1531 keys of one KV head x 256 8.9 / 6.4, 3000 8.9 / 7.3; of 8 x
+// 128 6.8 / 6.0 and 7.3 / 6.8; 4 sequences over 11378 keys, 1469 visible, 9.0 / 7.4. From 24 eight-tile segments on they stay (8000 keys: 32 segments 9.3, 63 9.4).
+// Up to FEW_TILES of a whole cache they stay too: there a batch of any size that fits the CUs has the same segments, hence a sequence the same bits.
+// as_few: rows that leave prepared want one segment wherever eight tiles allow it.
+constexpr int FEW_TILES = 32;
+int key_segments(const AttnArgs &a, int d, int cus, int units, bool as_few) {
+    // (behind a window there are no more keys than it shows to the call's consecutive queries)
+    long keys = a.T;
+    if (!as_few && a.win_chunk == 0 && a.win_right < (unsigned)a.T && a.win_left < (unsigned)a.T) keys = min(keys, (long)a.win_left + (long)a.win_right + a.L + TILE_KEYS);
+    const int tiles = (int)((keys + TILE_KEYS - 1) / TILE_KEYS), of_eight = (tiles + SPLIT_NW - 1) / SPLIT_NW;
+    const long wgs = (long)units * a.row_tiles;
+    int nseg = of_eight;
+    if (!as_few && of_eight > 1 && (keys < a.T || tiles > FEW_TILES)) {
+        const long full = wgs * (d / 64);
+        nseg = max(nseg, min((tiles + 1) / 2, full * 24 <= cus ? 24 : full * 16 <= cus ? 16 : 12));
+    }
+    // (as many segments as keep the workgroups within one per CU: a second, partial round of workgroups plus the merge
+    // costs more than CUs left idle - 192 row tiles in two segments each took 26 us, in one 13)
+    return min(max(1, (int)min((long)nseg, (long)cus / wgs)), 256);
+}
+
 template <int KV, int D, bool HILO, bool RING = false>
 int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     using Cfg = FlashCfg<D, 4>;
@@ -312,18 +345,22 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     }
     if (a.codes && (HILO || RING)) return rows_not_prepared(ctx, HILO ? "the precise mode" : "rolling caches");
     if (split) {
-        // key segments: one 32-key tile per wavefront while that leaves the device under-filled,
-        // more tiles per wavefront beyond one workgroup per CU (its LDS tiles fill a CU)
-        const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-        const int tiles = (a.T + TILE_KEYS - 1) / TILE_KEYS;
-        // (as many segments as keep the workgroups within one per CU: a second, partial round of workgroups plus the merge
-        // launch costs more than CUs left idle - 192 row tiles in two segments each took 26 us, in one 13)
-        int nseg = cus / (units * a.row_tiles);
-        nseg = max(1, min(nseg, (tiles + SPLIT_NW - 1) / SPLIT_NW));
-        nseg = min(nseg, 256);
+        const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, nseg = key_segments(a, D, cus, units, a.codes != nullptr);
         if (a.codes && nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
         a.nseg = nseg;
-        if (nseg > 1) {
+        const long wgs = (long)units * a.row_tiles * nseg;
+        const int shares = D >= 256 && wgs * (D / 64) <= cus ? D / 64 : D >= 128 && wgs * 2 <= cus ? 2 : 1;      // of the value columns, see below
+        const size_t meetings = (size_t)units * a.row_tiles * shares, ticket_bytes = meetings * MEET_TICKET_WORDS * sizeof(unsigned);
+        const size_t meet_bytes = meetings * nseg * (16 * (D / shares) + 32) * sizeof(float);
+        // (a recording for which the buffers would have to grow keeps the merge launch)
+        const bool meet = nseg > 1 && last_merges(a, D / shares) &&
+                          (!ctx->capturing || (ticket_bytes <= ctx->tickets_bytes && meet_bytes <= ctx->scratch2_bytes));
+        if (meet) {
+            if (const int rc = ensure_scratch2(ctx, meet_bytes)) return rc;
+            if (const int rc = grow_work_buffer(ctx, &ctx->tickets, &ctx->tickets_bytes, ticket_bytes, true, "the tickets")) return rc;
+            a.partial = (float *)ctx->scratch2;
+            a.tickets = (unsigned *)ctx->tickets;
+        } else if (nseg > 1) {
             const size_t bytes = (size_t)units * a.row_tiles * nseg * (16 * D + 32) * sizeof(float);
             int rc = ensure_scratch2(ctx, bytes);
             if (rc) return rc;
@@ -334,13 +371,12 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         // segment) is a chain of latencies in one CU, of which those three were about 2 us of 9.8: one token over 144 keys, one KV
         // head of size 256, 9.8 -> 8.0 us; over 1531 keys, 8 KV heads of size 128, 10.8 -> 10.4 with the segments' merge. Only
         // while the shares fit one workgroup per CU: past that a second round costs more than a share saves.
-        const long wgs = (long)units * a.row_tiles * nseg;
         int rc;
-        if (D >= 256 && wgs * (D / 64) <= cus) rc = launch_flash_split<KV, D, HILO, RING, D / 64>(ctx, a);
-        else if (D >= 128 && wgs * 2 <= cus) rc = launch_flash_split<KV, D, HILO, RING, D >= 128 ? 2 : 1>(ctx, a);
+        if (D >= 256 && shares == D / 64) rc = launch_flash_split<KV, D, HILO, RING, D / 64>(ctx, a);
+        else if (D >= 128 && shares == 2) rc = launch_flash_split<KV, D, HILO, RING, D >= 128 ? 2 : 1>(ctx, a);
         else rc = launch_flash_split<KV, D, HILO, RING, 1>(ctx, a);
         if (rc) return rc;
-        if (nseg > 1) {
+        if (nseg > 1 && !meet) {
             ProfScope scope(ctx, "attn_merge");
             launch_k(ctx, attn_merge_kernel<D>, dim3((unsigned)(a.row_tiles * (D / MERGE_DV)), (unsigned)units), dim3(256), 0, a);
         }

@@ -20,6 +20,7 @@ struct AttnArgs {
     float *out;
     const int *positions, *kv_lengths;
     float *partial;
+    unsigned *tickets;        // not null: the segments are merged by the workgroup that ends last (attn_flash_body), zero between launches
     int B, L, T, Hq, Hkv, groups, rows_total, row_tiles, nseg;
     int ring;      // rolling caches: T (logical key t lives in row t % T); 0: row t is key t
     int q_dtype, kv_dtype;
@@ -140,6 +141,11 @@ __device__ __forceinline__ float groups4_max(float v) {
     v = fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
     x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
+}
+// the value of the lane 32 away
+__device__ __forceinline__ float half_swap(float v) {
+    const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float((__lane_id() & 32) ? x[0] : x[1]);
 }
 __device__ __forceinline__ float groups4_sum(float v) {
     auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);

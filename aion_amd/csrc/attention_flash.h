@@ -21,6 +21,8 @@ struct FlashCfg {
     static constexpr int LDS_BYTES = Q_OFF + 16 * Q_ROW;
 };
 constexpr int SPLIT_NW = 8;
+constexpr int MEET_TICKET_WORDS = 32;      // a ticket has a line of its own: the segments of every tile draw theirs at the same time
+constexpr int MEET_UNROLL = 8;     // segments that a lane of the merging workgroup has in flight
 
 // HILO: q and the probabilities are fed to the MFMAs as a high and a low half-precision part
 // (x = hi + lo, ~2x the mantissa), which keeps an f32 query path at f32-level accuracy; used when
@@ -415,9 +417,19 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     __syncthreads();
     // every thread derives the weights exp2(m_w - m_all) of its own row from the NW maxima (NW LDS reads that
     // the sixteen lanes of a row share, NW exp2): cheaper than a serial pass by sixteen threads and a third barrier
-    // partial slot layout in global memory (read by attn_merge_kernel): [16][D] o, [16] m, [16] l
-    constexpr int PSTRIDE = 16 * D + 32;
+    // partial slot layout in global memory (read by attn_merge_kernel): [16][D] o, [16] m, [16] l; where the last workgroup merges, each share of the value
+    // columns has slots of its own, [16][DV] o, [16] m, [16] l
+    constexpr int PSTRIDE = 16 * D + 32, SSTRIDE = 16 * DV + 32;
     const size_t pslot = ((size_t)(unit * a.row_tiles + rt) * a.nseg + seg) * PSTRIDE;
+    [[maybe_unused]] const unsigned meeting = (unsigned)(unit * a.row_tiles + rt) * DVS + (unsigned)slice_dv;
+    [[maybe_unused]] float *const slots = a.partial + (size_t)meeting * a.nseg * SSTRIDE;
+    const bool last_merges = !Hooks::Q_LATE && a.tickets;
+    // Device-scope accesses: written through, read at the point where the XCDs' caches agree. As buffer accesses: 16 bytes each, and a lane past the last slot
+    // gets zeros without a request.
+    [[maybe_unused]] constexpr int DEVICE_SCOPE = 16;                                // the sc1 bit of a buffer access
+#if defined(__HIP_DEVICE_COMPILE__)
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t slots_rsrc = __builtin_amdgcn_make_buffer_rsrc((void *)slots, 0, (unsigned)(a.nseg * SSTRIDE * 4), 0x00027000);
+#endif
     for (int e = threadIdx.x; e < 16 * DV / 4; e += NW * 64) {
         const int row = e / (DV / 4), col = (e % (DV / 4)) * 4;
         float mw[NW];
@@ -442,12 +454,78 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
                 const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
                 hooks.store_out(a.out, (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g2) * D + dv0 + col, o * inv);
             }
+        } else if (last_merges) {
+            if (rt * 16 + row < a.rows_total) {
+#if defined(__HIP_DEVICE_COMPILE__)
+                const int at = (seg * SSTRIDE + row * DV + col) * 4;
+                __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), slots_rsrc, at, 0, DEVICE_SCOPE);
+                if (col == 0)
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(m_all), __float_as_uint(l_all)}, slots_rsrc, (seg * SSTRIDE + 16 * DV + row * 2) * 4, 0, DEVICE_SCOPE);
+#endif
+            }
         } else if (rt * 16 + row < a.rows_total) {        // (rows past the last query row are padding: nobody reads them)
             *(f32x4 *)(a.partial + pslot + row * D + dv0 + col) = o;
             if (col == 0 && dv0 == 0) {
                 a.partial[pslot + 16 * D + row] = m_all;
                 a.partial[pslot + 16 * D + 16 + row] = l_all;
             }
+        }
+    }
+    if constexpr (!Hooks::Q_LATE) {
+        // The workgroup that ends last merges the segments: each publishes its partial result, waits until the stores have been acknowledged and takes a
+        // ticket; whoever draws the last one finds all of them. Nobody waits for anybody. No device-scope fence: it would write back and
+        // invalidate the L2 of the XCD. The segments are added in order, whoever comes last.
+        if (!last_merges) return;
+        int *s_ticket = (int *)(lds + Cfg::Q_OFF);                  // (the queries are dead)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (threadIdx.x == 0) *s_ticket = (int)__hip_atomic_fetch_add(a.tickets + meeting * MEET_TICKET_WORDS, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        if (*s_ticket != a.nseg - 1) return;
+        if (threadIdx.x == 0) __hip_atomic_store(a.tickets + meeting * MEET_TICKET_WORDS, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        // A wavefront merges a row: lane s has the maximum and sum of segment s (there are at most 64, the launcher sees to that); a lane has four columns
+        // and every G-th segment, the G lanes of a column meet by lane swaps. A column is summed as four runs, segments i, i + 4, .., in whatever number of
+        // lanes: ((0 + 1) + (2 + 3)), so that the bits do not depend on the shares of the value columns.
+        constexpr int TPR = DV / 4, G = 64 / TPR, RUNS = 4 / G;
+        const int grp = lane / TPR, col = (lane % TPR) * 4, rows = min(16, a.rows_total - rt * 16);
+        for (int row = wave; row < rows; row += NW) {
+            u32x2 stat = {};
+#if defined(__HIP_DEVICE_COMPILE__)
+            stat = __builtin_amdgcn_raw_buffer_load_b64(slots_rsrc, (lane * SSTRIDE + 16 * DV + row * 2) * 4, 0, DEVICE_SCOPE);
+#endif
+            f32x4 run[RUNS];
+#pragma unroll
+            for (int i = 0; i < RUNS; ++i) run[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            float f_lane = 0.f, l_all = 0.f;
+            for (int s0 = grp; s0 - grp < a.nseg; s0 += G * MEET_UNROLL) {
+                u32x4 os[MEET_UNROLL] = {};
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+                for (int u = 0; u < MEET_UNROLL; ++u)
+                    os[u] = __builtin_amdgcn_raw_buffer_load_b128(slots_rsrc, ((s0 + u * G) * SSTRIDE + row * DV + col) * 4, 0, DEVICE_SCOPE);
+#endif
+                if (s0 == grp) {
+                    const float m = lane < a.nseg ? __uint_as_float(stat.x) : -INFINITY, m_max = wave_max(m);
+                    f_lane = m > -INFINITY ? __builtin_amdgcn_exp2f((m - m_max) * LOG2E) : 0.f;
+                    l_all = wave_sum(__uint_as_float(stat.y) * f_lane);
+                }
+#pragma unroll
+                for (int u = 0; u < MEET_UNROLL; ++u) {
+                    const float f = __shfl(f_lane, (s0 + u * G) & 63, 64);          // (past the last segment: a factor or zero, times zeros)
+                    run[u % RUNS] += __builtin_bit_cast(f32x4, os[u]) * f;
+                }
+            }
+            f32x4 o;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (G == 4) o[i] = groups4_sum(run[0][i]);
+                else if constexpr (G == 2) o[i] = (run[0][i] + half_swap(run[0][i])) + (run[1][i] + half_swap(run[1][i]));
+                else o[i] = (run[0][i] + run[1][i]) + (run[2][i] + run[3][i]);
+            }
+            if (grp > 0) continue;
+            const int rr = rt * 16 + row, l2 = a.L > 1 ? (int)((unsigned)rr / (unsigned)a.groups) : 0, g2 = rr - l2 * a.groups;
+            const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
+            hooks.store_out(a.out, (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g2) * D + dv0 + col, o * inv);
         }
     }
 }

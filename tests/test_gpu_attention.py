@@ -143,6 +143,30 @@ def test_decode_ragged_lengths_and_stale_cache_tail(gpu, orc):
     attn_err(got, ref, 2e-3)
 
 
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("B,Hq,Hkv,L,T", [(1, 8, 8, 1, 257), (1, 4, 4, 1, 4096), (3, 8, 1, 1, 2048), (2, 8, 2, 1, 4100), (1, 12, 1, 1, 3000), (4, 8, 1, 1, 16384), (2, 4, 4, 5, 700),
+                                          (1, 8, 1, 3, 900), (1, 9, 3, 6, 1300)])
+@pytest.mark.parametrize("precise", [False, True])
+def test_key_segments_merged_by_the_workgroup_that_ends_last(gpu, orc, precise, B, Hq, Hkv, L, T, D):
+    """Two segments and more: rows from one to sixteen of a tile, several tiles, columns in one share or several, as many segments as the last workgroup takes
+    in one round, two, and more than it takes (a launch merges those); segments without a visible key. Repeated calls, also one after another of
+    different shapes, give the same bits: the tickets return to zero."""
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T + D, B, L, T, Hq, Hkv, D, "f16")
+    lens = np.maximum(T - np.arange(B) * (T // 3), L).astype(np.int32)
+    pos = (lens[:, None] - L + np.arange(L)).astype(np.int32)
+    for b in range(B):
+        for x, f in ((k, kf), (v, vf)):
+            x[b, lens[b]:], f[b, lens[b]:] = np.nan, 0
+    gpu.set_attention_precise(precise)
+    try:
+        for window in (be.CAUSAL, (300, 0, 0)):
+            got = [run_attention(gpu, q, k, v, 1 / math.sqrt(D), qd, kd, window=window, positions=pos, kv_lengths=lens) for _ in range(3)]
+            attn_err(got[0], orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D), window=window, positions=pos, kv_lengths=lens), 2e-3)
+            assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    finally:
+        gpu.set_attention_precise(False)
+
+
 @pytest.mark.parametrize("D,precise", [(64, False), (128, False), (256, False), (128, True), (256, True)])
 @pytest.mark.parametrize("T", [200, 600])                         # one key segment, three
 def test_decode_value_columns_divided_or_not(gpu, orc, T, D, precise):
