@@ -26,6 +26,7 @@ struct AttnArgs {
     int q_dtype, kv_dtype;
     float scale, soft_cap;
     unsigned win_left, win_right, win_chunk;
+    int pf_tiles, pf_first;   // 128-row kernel: row tiles; how many of them go out longest first with the unit fastest, 0: unit by unit (see launch_prefill_t)
     int *codes;               // not null: the output leaves as rows prepared for the exact GEMM (PreparedAct::tiled) in place of `out`
     float *code_scales;
 };

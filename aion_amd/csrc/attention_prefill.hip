@@ -112,12 +112,13 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l31 = lane & 31, lh = lane >> 5;
-    const int unit = blockIdx.y, b = unit / a.Hkv, hk = unit % a.Hkv;
+    const unsigned fastest = a.pf_first ? (unsigned)(a.B * a.Hkv) : (unsigned)a.pf_tiles;
+    const unsigned slow = blockIdx.x < fastest ? 0u : blockIdx.x / fastest, fast = blockIdx.x - slow * fastest;      // (one KV head, one sequence: no division)
+    const int unit = (int)(a.pf_first ? fast : slow), place = (int)(a.pf_first ? slow : fast);
+    const int b = unit < a.Hkv ? 0 : (int)((unsigned)unit / (unsigned)a.Hkv), hk = unit - b * a.Hkv;
 
     // ---- this lane's query row (lanes l and l+32 share it)
-    // row tiles in descending order: under a causal mask the last rows see the most keys, and workgroups are
-    // dispatched in index order - the long ones start first and the short ones fill the gaps at the end
-    const int r = ((int)gridDim.x - 1 - (int)blockIdx.x) * PF_ROWS + wave * 32 + l31;
+    const int r = (a.pf_first && place >= a.pf_first ? place - a.pf_first : a.pf_tiles - 1 - place) * PF_ROWS + wave * 32 + l31;
     const bool row_ok = r < a.rows_total;
     const int li = row_ok ? r / a.groups : 0, gi = row_ok ? r % a.groups : 0;
     const int hq = hk * a.groups + gi;
@@ -816,7 +817,7 @@ int launch_prefill_prepare(aionhip_ctx *ctx, AttnArgs &a) {
     static std::atomic<uint64_t> attr{0};
     if (const int rc = allow_lds(ctx, attr, (const void *)kern, PCfg::LDS_BYTES)) return rc;
     ProfScope scope(ctx, "attn_prefill");
-    launch_k(ctx, kern, dim3((unsigned)((a.rows_total + PF_ROWS - 1) / PF_ROWS), (unsigned)(a.B * a.Hkv)), dim3(256), PCfg::LDS_BYTES, a);
+    launch_k(ctx, kern, dim3((unsigned)(a.pf_tiles * a.B * a.Hkv)), dim3(256), PCfg::LDS_BYTES, a);
     LAUNCH_CHECK(ctx, "attn_prefill");
     return AIONHIP_OK;
 }
@@ -845,6 +846,15 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     if (want < 2 && D > 128 && wgs > cus0 && balance_pays && (long)wgs * 10 < (long)cus0 * PF_TWO_SEG_BELOW_TENTHS) want = 2;
     int nseg = max(1, min(min(want, key_tiles / seg_tiles), 16));
     a.nseg = nseg;
+    a.pf_tiles = (a.rows_total + PF_ROWS - 1) / PF_ROWS;
+    // The order of the workgroups, which start in index order, round robin over the XCDs and their CUs. Under a causal mask a row tile's length grows with
+    // its index, so the longest go first. Where there are more workgroups than CUs the unit - a sequence's KV head - is the fastest index: a CU's workgroups
+    // are then of different lengths (unit by unit, two of the longest could meet on one), and an XCD has few units' K and V in its L2. Where two share a CU
+    // and all fit, the rest of the tiles go out shortest first, beside the longest. us unit by unit / so: 32 heads x 128 over 1611 keys 51.7 / 40.6, 4096 216 / 150, two
+    // sequences over 1500 82.5 / 53.6; 32 on 8 x 128 over 4096 194 / 147; 16 on 4 x 64 over 4096 105 / 80; four sequences of 8 on one x 256 over 2000 96 / 77.
+    // A grid of at most one workgroup per CU has nothing to even out and is a little ahead unit by unit (1100 keys, 8 on 2 x 256, 25.8 / 26.9).
+    const long all = (long)wgs * nseg;
+    a.pf_first = all <= cus0 ? 0 : D <= 128 && all <= 2L * cus0 ? min(a.pf_tiles, (cus0 + units - 1) / units) : a.pf_tiles;
     if (a.codes) {
         if (RING || nseg > 1 || a.soft_cap > 0.f) return rows_not_prepared(ctx, RING ? "rolling caches" : nseg > 1 ? "keys in segments" : "a soft cap");
         return launch_prefill_prepare<KV, D>(ctx, a);
@@ -861,7 +871,7 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     if (const int rc = allow_lds(ctx, attr[cap], fn, PCfg::LDS_BYTES)) return rc;
     {
         ProfScope scope(ctx, "attn_prefill");
-        const dim3 grid((unsigned)((a.rows_total + PF_ROWS - 1) / PF_ROWS), (unsigned)units, (unsigned)nseg);
+        const dim3 grid((unsigned)(a.pf_tiles * units), 1, (unsigned)nseg);
         if (cap) launch_k(ctx, attn_prefill_kernel<KV, D, true, RING>, grid, dim3(256), PCfg::LDS_BYTES, a);
         else launch_k(ctx, attn_prefill_kernel<KV, D, false, RING>, grid, dim3(256), PCfg::LDS_BYTES, a);
     }
