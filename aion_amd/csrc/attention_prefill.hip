@@ -166,7 +166,10 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
     const bool live = hi > lo;
     // wavefront: union (which tiles it computes) and intersection (which tiles need no mask)
     const int w_lo = wave_min_i(live ? lo : INT_MAX), w_hi = wave_max_i(live ? hi : 0);
-    const int w_lo_max = wave_max_i(live ? lo : INT_MAX), w_hi_min = wave_min_i(live ? hi : 0);
+    // (rows past the last one take no part: nobody reads what they hold. Counted as rows that see nothing they made every tile of the last row tile, the
+    // longest under a causal mask, pay for the mask: 16 heads on 4 x 64 over 1611 keys 50.2 -> 34.9 us, 32 on 8 x 128 40.4 ->
+    // 36.1, two sequences of 8 on 2 x 256 over 1500 49.0 -> 45.2)
+    const int w_lo_max = wave_max_i(live ? lo : row_ok ? INT_MAX : INT_MIN), w_hi_min = wave_min_i(live ? hi : row_ok ? 0 : INT_MAX);
     // workgroup union through LDS
     int *s_rng = (int *)(lds + 2 * Cfg::STAGE);
     if (lane == 0) { s_rng[wave] = w_lo; s_rng[4 + wave] = w_hi; }
