@@ -345,7 +345,10 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     }
     if (a.codes && (HILO || RING)) return rows_not_prepared(ctx, HILO ? "the precise mode" : "rolling caches");
     if (split) {
-        const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256, nseg = key_segments(a, D, cus, units, a.codes != nullptr);
+        const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+        int nseg = key_segments(a, D, cus, units, a.codes != nullptr);
+        // (a recording for which the scratch memory would have to grow asks for no more segments than eight-tile ones)
+        if (ctx->capturing && (size_t)units * a.row_tiles * nseg * (16 * D + 32) * sizeof(float) > ctx->scratch2_bytes) nseg = key_segments(a, D, cus, units, true);
         if (a.codes && nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
         a.nseg = nseg;
         const long wgs = (long)units * a.row_tiles * nseg;

@@ -35,8 +35,8 @@ constexpr int MEET_UNROLL = 8;     // segments that a lane of the merging workgr
 // a latency; over a long one HBM, with the wavefronts' own chains under it. The chain is kept short: one memory round trip for the
 // index operands and the queries, reductions by DPP and lane swaps instead of LDS permutes, hardware exp2 (the arguments are <= 0 and
 // results under 2^-126 vanish in a sum that holds a 1), V in flight under the scores. One token, one KV head of size 256, 144 keys:
-// 8.0 -> 6.75 us; 1531 keys, 8 KV heads of size 128: 7.6 -> 6.0 us (+ 3.6 for the segments' merge); eight sequences over 16384 keys,
-// one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
+// 8.0 -> 6.75 us, 6.1 with the operands in SGPRs; 1531 keys, 8 KV heads of size 128: 7.6 -> 6.0 us with eight tiles to a segment (+ 3.6 for the merge as a
+// launch), 5.8 with two and the merge inside; eight sequences over 16384 keys, one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
 template <int KV, int D, bool SPLIT, bool HILO, bool RING, int DVS = 1, class Hooks>
 __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int rt_block, const int seg, const int b, const int hk, Hooks &hooks,
                                                 const int slice_dv = 0) {
