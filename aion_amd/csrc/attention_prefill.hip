@@ -848,6 +848,15 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     // 122 -> 116, 320 the same, 352 and more slower).
     if (want < 2 && D > 128 && wgs > cus0 && balance_pays && (long)wgs * 10 < (long)cus0 * PF_TWO_SEG_BELOW_TENTHS) want = 2;
     int nseg = max(1, min(min(want, key_tiles / seg_tiles), 16));
+    // Head size 64: three of its workgroups share a CU, and where there are few of them against a long key range (eight per key tile at most) the longest
+    // tile alone is most of the time. Whole caches only: a window keeps the tiles short. us in one segment (from 32 key tiles on two) / four, past one
+    // workgroup per CU three: 16 heads on 4 x 64 over 1030 keys 24.2 / 20.3, 1611 35.0 / 26.4, 2000 38.6 / 33.4, 2500 50.5 / 41.4, 4096 79.0 / 72.3; with more
+    // workgroups the merge costs more: two sequences over 1300 30.0 / 31.1, over 2500 54.4 / 63.0.
+    // (Rows that leave prepared want one segment, and a recording is not asked for scratch memory that fewer do without.)
+    if (D <= 64 && !a.codes && key_tiles > 16 && wgs <= 8 * key_tiles && wgs <= 2 * cus0 && a.win_left >= (unsigned)a.T && a.win_chunk == 0) {
+        const int few = wgs <= cus0 ? 4 : 3;
+        if (!ctx->capturing || (size_t)units * a.row_tiles * few * pf_partial_bytes(D, pf_half_partials(KV)) <= ctx->scratch2_bytes) nseg = max(nseg, few);
+    }
     a.nseg = nseg;
     a.pf_tiles = (a.rows_total + PF_ROWS - 1) / PF_ROWS;
     // The order of the workgroups, which start in index order, round robin over the XCDs and their CUs. Under a causal mask a row tile's length grows with

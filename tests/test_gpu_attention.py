@@ -112,6 +112,21 @@ def test_prefill_head_256_stale_tail_odd_lengths_and_scales(gpu, orc):
 
 
 @pytest.mark.parametrize("kind,tol", [("f16", 2e-3), ("bf16", 1e-2)])
+@pytest.mark.parametrize("L,T", [(1030, 1030), (1500, 1600), (2100, 2100)])      # four key segments, four, three
+def test_prefill_head_64_in_key_segments(gpu, orc, L, T, kind, tol):
+    """Few row tiles of head size 64 against a long key range: segments, also ones that no row of a tile reaches, and a last row tile that is not full."""
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(L, 1, L, T, 16, 4, 64, kind)
+    end = np.array([L], np.int32)
+    pos = np.arange(L, dtype=np.int32).reshape(1, L)
+    nan = np.float16(np.nan) if kind == "f16" else np.uint16(0x7FC1)
+    for x, f in ((k, kf), (v, vf)):
+        x[:, L:], f[:, L:] = nan, 0
+    got = run_attention(gpu, q, k, v, 1 / 8.0, qd, kd, positions=pos, kv_lengths=end)
+    assert gpu.last_kernel() == "attn_prefill"
+    attn_err(got, orc.attention_f64(qf, kf, vf, 1 / 8.0, positions=pos, kv_lengths=end), tol)
+
+
+@pytest.mark.parametrize("kind,tol", [("f16", 2e-3), ("bf16", 1e-2)])
 @pytest.mark.parametrize("T,B", [(1024, 1), (1024, 8), (4096, 1), (4096, 8), (16384, 1), (16384, 8), (777, 3)])
 def test_decode_split_k(gpu, orc, kind, tol, T, B):
     # BASELINE config 4b, every (T, B) it names: 1 query token at position T-1, 8 q heads / 1 kv head, hd 256
