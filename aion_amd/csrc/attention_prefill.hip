@@ -710,12 +710,20 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
     }
     if (HP && nseg > 1) {
         // f16 accumulators under a per-row power of two: 2^e <= max|acc| < 2^(e+1) (e clamped so that its inverse is a
-        // normal number; a row of zeros takes 1)
+        // normal number; a row of zeros takes 1). Infinite accumulators, of infinite values, take no part: they stay infinite as f16 and their
+        // scale would leave zeros of the row's other columns.
         float amax = 0.f;
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[j][i]));
+        if (__any(amax == INFINITY)) {
+            amax = 0.f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[j][i]) < INFINITY ? fabsf(acc[j][i]) : 0.f);
+        }
         amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
         unsigned e = (__float_as_uint(amax) >> 23) & 0xFFu;
         e = e == 0u ? 127u : min(e, 253u);

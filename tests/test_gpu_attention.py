@@ -72,6 +72,13 @@ def make_qkv(seed, B, L, T, Hq, Hkv, D, kind):
     return (qb, kb, vb, be.BF16, be.BF16), (qf, kf, vf)
 
 
+def launches(gpu, *args, **kw):
+    """run_attention's result and the names of its launches"""
+    gpu.profile_start()
+    got = run_attention(gpu, *args, **kw)
+    return got, [n for n, _ in gpu.profile_stop()]
+
+
 # A prompt with few 128-row workgroups runs on the 16-row split kernel (up to about 80 / 40 / 32 of them at head size
 # 64 / 128 / 256: the smaller the head, the longer the 16-row kernel stays ahead). L = 150 (2 x 2 units x 5 workgroups) is
 # such a prompt at every head size, L = 560 (2 x 2 x 18 = 72) at head size 64 only, L = 1100 (140) at none.
@@ -269,6 +276,21 @@ def test_prefill_bf16_key_segments_empty_segments_and_value_range(gpu, orc):
         got = run_attention(gpu, q, k, vb, 1 / math.sqrt(D), qd, kd)
         assert gpu.last_kernel() == "attn_prefill"
         attn_err(got * np.float32(2.0 ** -e), ref, 1e-2)
+
+
+@pytest.mark.parametrize("D,Hq,Hkv", [(64, 16, 4), (128, 8, 1), (256, 8, 1)])
+@pytest.mark.parametrize("kind", ["f16", "bf16"])
+def test_prefill_key_segments_keep_an_infinite_value_in_its_column(gpu, orc, D, Hq, Hkv, kind):
+    """An infinite value that a row sees makes its own output column infinite; the row's other columns keep their values, also where the segments'
+    partial results are scaled by the row's largest accumulator."""
+    L = 1030
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(D, 1, L, L, Hq, Hkv, D, kind)
+    v[0, 1, :, 5], vf[0, 1, :, 5] = np.float16(np.inf) if kind == "f16" else np.uint16(0x7F80), 0
+    got, names = launches(gpu, q, k, v, 1 / math.sqrt(D), qd, kd)
+    assert names == ["attn_prefill", "attn_merge"]
+    assert (got[0, 1:, :, 5] == np.inf).all()
+    finite = [i for i in range(D) if i != 5]
+    attn_err(got[..., finite], orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D))[..., finite], 1e-2)
 
 
 def test_soft_cap(gpu, orc):
