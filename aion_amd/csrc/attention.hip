@@ -171,8 +171,8 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
             l_loc *= f0;
 #pragma unroll
             for (int u = 0; u < MERGE_UNROLL; ++u) {
-                const bool live = s0 + u * MERGE_SG < a.nseg && ms[u] > -INFINITY;
-                const float f = live ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
+                if (s0 + u * MERGE_SG >= a.nseg) break;             // (the last segment again: zero times an infinite value is no zero)
+                const float f = ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
                 o_loc += os[u] * f;
                 l_loc += ls[u] * f;
             }

@@ -808,8 +808,8 @@ __global__ __launch_bounds__(256) void attn_merge_rows_kernel(AttnArgs a) {
             l_all *= f0;
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
-                const bool live = s0 + u < a.nseg && ms[u] > -INFINITY;
-                const float f = live ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
+                if (s0 + u >= a.nseg) break;                     // (the last segment again: zero times an infinite value is no zero)
+                const float f = ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
                 o += os[u] * f;
                 l_all += ls[u] * f;
             }

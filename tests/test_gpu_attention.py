@@ -293,6 +293,21 @@ def test_prefill_key_segments_keep_an_infinite_value_in_its_column(gpu, orc, D, 
     attn_err(got[..., finite], orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D))[..., finite], 1e-2)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,L,T,D,merge", [(1, 8, 1, 1088, 1088, 128, "attn_prefill"), (1, 8, 1, 1088, 1088, 256, "attn_prefill"), (1, 16, 4, 2112, 2112, 64, "attn_prefill"),
+                                                  (5, 8, 1, 1, 16384, 256, "attn_flash_split"), (1, 2, 1, 1, 16928, 64, "attn_flash_split")])
+def test_merge_launch_with_an_infinite_value_in_the_last_segment(gpu, orc, B, Hq, Hkv, L, T, D, merge):
+    """Segments in numbers that do not fill the merge's rounds of loads, the last one with an infinite value that the last query sees. (Whole key tiles: past
+    the last key of a partial one that key is read again, under a probability of zero.)"""
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T, B, L, T, Hq, Hkv, D, "f16")
+    v[:, T - 1, :, 5], vf[:, T - 1, :, 5] = np.float16(-np.inf), 0
+    pos = np.tile(np.arange(T - L, T, dtype=np.int32), (B, 1))
+    got, names = launches(gpu, q, k, v, 1 / math.sqrt(D), qd, kd, positions=pos)
+    assert names == [merge, "attn_merge"]
+    assert (got[:, L - 1, :, 5] == -np.inf).all()
+    finite = [i for i in range(D) if i != 5]
+    attn_err(got[:1, L - 1:][..., finite], orc.attention_f64(qf[:1, L - 1:], kf[:1], vf[:1], 1 / math.sqrt(D), positions=pos[:1, L - 1:])[..., finite], 2e-3)
+
+
 def test_soft_cap(gpu, orc):
     (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(13, 1, 40, 40, 8, 1, 64, "f16")
     # logits of std ~24 before the cap: the flash kernel feeds q to the MFMA in the K/V element
