@@ -171,9 +171,9 @@ __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
             l_loc *= f0;
 #pragma unroll
             for (int u = 0; u < MERGE_UNROLL; ++u) {
-                if (s0 + u * MERGE_SG >= a.nseg) break;             // (the last segment again: zero times an infinite value is no zero)
-                const float f = ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
-                o_loc += os[u] * f;
+                const bool there = s0 + u * MERGE_SG < a.nseg;      // (else the last segment again: zero times an infinite value is no zero)
+                const float f = there && ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
+                o_loc += (there ? os[u] : f32x4{0.f, 0.f, 0.f, 0.f}) * f;
                 l_loc += ls[u] * f;
             }
             m_loc = m_new;

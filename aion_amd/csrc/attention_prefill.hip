@@ -808,9 +808,9 @@ __global__ __launch_bounds__(256) void attn_merge_rows_kernel(AttnArgs a) {
             l_all *= f0;
 #pragma unroll
             for (int u = 0; u < UN; ++u) {
-                if (s0 + u >= a.nseg) break;                     // (the last segment again: zero times an infinite value is no zero)
-                const float f = ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
-                o += os[u] * f;
+                const bool there = s0 + u < a.nseg;              // (else the last segment again: zero times an infinite value is no zero)
+                const float f = there && ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
+                o += (there ? os[u] : f32x4{0.f, 0.f, 0.f, 0.f}) * f;
                 l_all += ls[u] * f;
             }
             m_all = m_new;
