@@ -27,6 +27,7 @@ struct AttnArgs {
     float scale, soft_cap;
     unsigned win_left, win_right, win_chunk;
     int pf_tiles, pf_first;   // 128-row kernel: row tiles; how many of them go out longest first with the unit fastest, 0: unit by unit (see launch_prefill_t)
+    int pf_half;              // 128-row kernel: the segments' partial accumulators are f16 (pf_half_partials)
     int *codes;               // not null: the output leaves as rows prepared for the exact GEMM (PreparedAct::tiled) in place of `out`
     float *code_scales;
 };

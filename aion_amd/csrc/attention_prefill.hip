@@ -63,7 +63,8 @@ constexpr int pf_unit_end(int k, int nm) {
 // accumulators 11), each row scaled by a power of two so that any bf16 value range fits, with that scale as a third
 // per-row float; the values of a row stand in the order the lanes hold them (position j*32 + h*16 + q*4 + i holds dv
 // j*32 + q*8 + h*4 + i), 32 contiguous bytes per lane and dv tile. Half the bytes written by the tile kernel and read
-// by the merge: both are bound by the bytes they move (the workgroups of a round all store at the same time).
+// by the merge: both are bound by the bytes they move (the workgroups of a round all store at the same time). The segments that head size 64 takes where
+// the other rules want one (see launch_prefill_t) keep f32: AttnArgs::pf_half is their flag.
 constexpr bool pf_half_partials(int kv) { return kv == AIONHIP_BF16; }
 constexpr int pf_partial_bytes(int d, bool half) { return half ? 32 * d + 192 : 64 * d + 128; }
 
@@ -187,8 +188,8 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
         t_end = min(t_end, t_begin + per);
         nothing = t_begin >= t_end;
     }
-    constexpr bool HP = pf_half_partials(KV);
-    constexpr int PART_BYTES = pf_partial_bytes(D, HP);
+    const bool HP = pf_half_partials(KV) && (D > 64 || a.pf_half);
+    const int PART_BYTES = pf_partial_bytes(D, HP);
     unsigned char *part = nullptr;
     if (nseg > 1) part = (unsigned char *)a.partial + ((size_t)(unit * a.row_tiles + (r >> 4)) * nseg + seg) * PART_BYTES;
     float *part_stats = (float *)(part + (HP ? 32 * D : 64 * D));          // [16] maxima, [16] sums, (f16 form) [16] scales
@@ -858,12 +859,14 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     int nseg = max(1, min(min(want, key_tiles / seg_tiles), 16));
     // Head size 64: three of its workgroups share a CU, and where there are few of them against a long key range (eight per key tile at most) the longest
     // tile alone is most of the time. Whole caches only: a window keeps the tiles short. us in one segment (from 32 key tiles on two) / four, past one
-    // workgroup per CU three: 16 heads on 4 x 64 over 1030 keys 24.2 / 20.3, 1611 35.0 / 26.4, 2000 38.6 / 33.4, 2500 50.5 / 41.4, 4096 79.0 / 72.3; with more
+    // workgroup per CU three: 16 heads on 4 x 64 over 1030 keys 24.2 / 23.5, 1611 35.0 / 29.0, 2000 38.6 / 33.8, 2500 50.5 / 43.0, 4096 79.0 / 76.9; with more
     // workgroups the merge costs more: two sequences over 1300 30.0 / 31.1, over 2500 54.4 / 63.0.
-    // (Rows that leave prepared want one segment, and a recording is not asked for scratch memory that fewer do without.)
+    // (Rows that leave prepared want one segment, and a recording is not asked for scratch memory that fewer do without.) Over a bf16 cache these shapes had f32
+    // accumulators all the way in one segment, and keep them in the partial results: us with f16 ones / f32: 1030 keys 20.3 / 23.5, 1611 26.3 / 29.0, 2500 41.5 / 43.0, 4096 73.0 / 76.9.
+    a.pf_half = pf_half_partials(KV) && nseg > 1;
     if (D <= 64 && !a.codes && key_tiles > 16 && wgs <= 8 * key_tiles && wgs <= 2 * cus0 && a.win_left >= (unsigned)a.T && a.win_chunk == 0) {
         const int few = wgs <= cus0 ? 4 : 3;
-        if (!ctx->capturing || (size_t)units * a.row_tiles * few * pf_partial_bytes(D, pf_half_partials(KV)) <= ctx->scratch2_bytes) nseg = max(nseg, few);
+        if (!ctx->capturing || (size_t)units * a.row_tiles * few * pf_partial_bytes(D, a.pf_half) <= ctx->scratch2_bytes) nseg = max(nseg, few);
     }
     a.nseg = nseg;
     a.pf_tiles = (a.rows_total + PF_ROWS - 1) / PF_ROWS;
@@ -880,7 +883,7 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
         return launch_prefill_prepare<KV, D>(ctx, a);
     }
     if (nseg > 1) {
-        const size_t bytes = (size_t)units * a.row_tiles * nseg * pf_partial_bytes(D, pf_half_partials(KV));
+        const size_t bytes = (size_t)units * a.row_tiles * nseg * pf_partial_bytes(D, a.pf_half);
         int rc = ensure_scratch2(ctx, bytes);
         if (rc) return rc;
         a.partial = (float *)ctx->scratch2;
@@ -898,7 +901,9 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     if (nseg > 1) {
         ProfScope scope(ctx, "attn_merge");
         constexpr int RPB = 256 / (D / 4);
-        launch_k(ctx, attn_merge_rows_kernel<D, pf_half_partials(KV)>, dim3((unsigned)((a.rows_total + RPB - 1) / RPB), (unsigned)units), dim3(256), 0, a);
+        const dim3 grid((unsigned)((a.rows_total + RPB - 1) / RPB), (unsigned)units);
+        if (a.pf_half) launch_k(ctx, attn_merge_rows_kernel<D, pf_half_partials(KV)>, grid, dim3(256), 0, a);
+        else launch_k(ctx, attn_merge_rows_kernel<D, false>, grid, dim3(256), 0, a);
     }
     LAUNCH_CHECK(ctx, "attn_prefill");
     return AIONHIP_OK;
