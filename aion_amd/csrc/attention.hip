@@ -10,8 +10,9 @@
 //   head); each lane's accumulators, running max and sum belong to ONE query row, so the softmax
 //   bookkeeping is per-lane scalar work. Two launch shapes:
 //     split mode (few query rows: decode) - a workgroup is one 16-row tile x one key segment, its
-//       eight wavefronts interleave 32-key tiles and merge through LDS; segments are merged by
-//       the workgroup that ends last, many of them by attn_merge_kernel (the flash-decoding split of cpu/exec/attention.zig:879-962).
+//       eight wavefronts interleave 32-key tiles and merge through LDS; where CUs are idle two or four workgroups hold a segment's
+//       eight wavefronts. The parts are merged by the workgroup that ends last, many of them by attn_merge_kernel (the flash-decoding split of
+//       cpu/exec/attention.zig:879-962).
 //       Where that leaves CUs idle, the value columns are divided over up to D / 64 workgroups as well.
 //     per-wavefront mode - a workgroup is four 16-row tiles, each wavefront walks its own key range; used
 //       for many query rows only when the hi+lo precise mode is on (see attn_prefill_kernel otherwise).
@@ -60,7 +61,7 @@ struct FlashPrepareHooks : FlashKernelHooks {
 
 // The leading arguments, 14 words, arrive in SGPRs with the wavefront and are what the index operands, the queries and the first K tile are addressed by;
 // a structure by value (all of AttnArgs came in one) is read from memory first, and so is gridDim. heads: KV heads, query heads of each << 16; form: key
-// segments, query type << 16. One token over 1531 keys, 8 KV heads of 128, 9.03 -> 8.56 us with the merge. The grid is (row tiles x segments x shares of the value columns, KV heads, sequences).
+// segments, their subdivision << 12, query type << 16. One token over 1531 keys, 8 KV heads of 128, 9.03 -> 8.56 us with the merge. The grid is (row tiles x segments x shares of the value columns, KV heads, sequences).
 struct FlashTail {
     float *out, *partial;
     unsigned *tickets;
@@ -87,7 +88,8 @@ __global__ __launch_bounds__(SPLIT ? SPLIT_NW * 64 : 256) void attn_flash_kernel
     a.Hq = a.Hkv * a.groups;
     a.rows_total = L * a.groups;
     a.row_tiles = (a.rows_total + 15) >> 4;
-    a.nseg = (int)(form & 0xFFFFu);
+    a.nseg = (int)(form & 0xFFFu);
+    a.sub = (int)(form >> 12 & 0xFu);
     a.q_dtype = (int)(form >> 16);
     a.kv_dtype = KV;
     a.out = tail.out;
@@ -125,83 +127,80 @@ __global__ __launch_bounds__(SPLIT ? SPLIT_NW * 64 : 256) void attn_flash_kernel
 }
 
 inline unsigned flash_heads(const AttnArgs &a) { return (unsigned)a.Hkv | (unsigned)a.groups << 16; }
-inline unsigned flash_form(const AttnArgs &a) { return (unsigned)a.nseg | (unsigned)a.q_dtype << 16; }
+inline unsigned flash_form(const AttnArgs &a) { return (unsigned)a.nseg | (unsigned)a.sub << 12 | (unsigned)a.q_dtype << 16; }
 inline FlashTail flash_tail(const AttnArgs &a) {
     return FlashTail{a.out, a.partial, a.tickets, a.scale, a.soft_cap, a.win_left, a.win_right, a.win_chunk, a.ring, a.B, a.codes, a.code_scales};
 }
 
-// log-sum-exp merge of the key segments: one workgroup per (row tile, 16-wide dv slice, unit).
-// Thread = (segment group of 4, row of 16, 4 consecutive dv): it folds every fourth segment with all
-// of a round's loads in flight at once, then the four groups fold through LDS.
-constexpr int MERGE_DV = 16, MERGE_SG = 4, MERGE_UNROLL = 8;
+// Merge of the key segments as a launch: one workgroup per (row tile, 16-wide dv slice, unit). A wavefront derives the segments' exact factors for every
+// fourth row, a lane to a segment (there are at most 256); thread = (8 segments of every 32, row of 16, 4 consecutive dv) adds its segments, with all
+// of a round's loads in flight at once, the first round's ahead of the factors, and the four groups meet through LDS - the order of the sums in attn_flash_body.
+constexpr int MERGE_DV = 16, MERGE_SG = MEET_PARTS / 8, MERGE_MOST = 256;
 template <int D>
 __global__ __launch_bounds__(256) void attn_merge_kernel(AttnArgs a) {
     constexpr int WSTRIDE = 16 * D + 32;
     constexpr int SLICES = D / MERGE_DV;
-    __shared__ float s_m[MERGE_SG][16][4], s_l[MERGE_SG][16][4];
-    __shared__ __attribute__((aligned(16))) float s_o[MERGE_SG][16][MERGE_DV];
+    __shared__ float s_f[16][MERGE_MOST], s_l[16];
+    __shared__ __attribute__((aligned(16))) float s_o[MERGE_MOST / MEET_PARTS][MERGE_SG][16][MERGE_DV];
     const int unit = blockIdx.y, rt = blockIdx.x / SLICES, slice = blockIdx.x % SLICES;
     const int b = unit / a.Hkv, hk = unit % a.Hkv;
-    const int tid = threadIdx.x, q4 = tid & 3, row = (tid >> 2) & 15, sg = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, q4 = tid & 3, row = (tid >> 2) & 15, sg = __builtin_amdgcn_readfirstlane(tid >> 6);
     const float *base = a.partial + (size_t)(unit * a.row_tiles + rt) * a.nseg * WSTRIDE;
-    const int dv = slice * MERGE_DV + q4 * 4;
+    const int dv = slice * MERGE_DV + q4 * 4, rows = min(16, a.rows_total - rt * 16);
     // padding rows of the last tile were never stored: their threads read the tile's last real row instead (the same lines
     // its own threads fetch) and drop the result below
-    const int row_ld = min(row, min(16, a.rows_total - rt * 16) - 1);
-    float m_loc = -INFINITY, l_loc = 0.f;
-    f32x4 o_loc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int s0 = sg; s0 < a.nseg; s0 += MERGE_SG * MERGE_UNROLL) {
-        float ms[MERGE_UNROLL], ls[MERGE_UNROLL];
-        f32x4 os[MERGE_UNROLL];
+    const int row_ld = min(row, rows - 1);
+    f32x4 os[8];
+    auto request = [&](int s0) {
 #pragma unroll
-        for (int u = 0; u < MERGE_UNROLL; ++u) {
-            const int sidx = min(s0 + u * MERGE_SG, a.nseg - 1);      // clamped: every load is unconditional
-            const float *p = base + (size_t)sidx * WSTRIDE;
-            ms[u] = p[16 * D + row_ld];
-            ls[u] = p[16 * D + 16 + row_ld];
-            os[u] = *(const f32x4 *)(p + row_ld * D + dv);
+        for (int u = 0; u < 8; ++u)                                   // clamped: every load is unconditional
+            os[u] = *(const f32x4 *)(base + (size_t)min(s0 + sg * 8 + u, a.nseg - 1) * WSTRIDE + row_ld * D + dv);
+    };
+    request(0);
+    for (int r = sg; r < rows; r += 4) {
+        float ref[MERGE_MOST / 64], l[MERGE_MOST / 64], top = REF_NONE, sum = 0.f;
+#pragma unroll
+        for (int j = 0; j < MERGE_MOST / 64; ++j) {
+            const int s = lane + 64 * j;
+            const float *p = base + (size_t)min(s, a.nseg - 1) * WSTRIDE + 16 * D + r;
+            ref[j] = s < a.nseg ? p[0] : REF_NONE;
+            l[j] = s < a.nseg ? p[16] : 0.f;
+            top = fmaxf(top, ref[j]);
         }
-        float m_new = m_loc;
+        top = lanes_max(top);
 #pragma unroll
-        for (int u = 0; u < MERGE_UNROLL; ++u)
-            if (s0 + u * MERGE_SG < a.nseg) m_new = fmaxf(m_new, ms[u]);
-        if (m_new > -INFINITY) {
-            const float f0 = m_loc > -INFINITY ? exp2f((m_loc - m_new) * LOG2E) : 0.f;
-            o_loc *= f0;
-            l_loc *= f0;
-#pragma unroll
-            for (int u = 0; u < MERGE_UNROLL; ++u) {
-                const bool there = s0 + u * MERGE_SG < a.nseg;      // (else the last segment again: zero times an infinite value is no zero)
-                const float f = there && ms[u] > -INFINITY ? exp2f((ms[u] - m_new) * LOG2E) : 0.f;
-                o_loc += (there ? os[u] : f32x4{0.f, 0.f, 0.f, 0.f}) * f;
-                l_loc += ls[u] * f;
-            }
-            m_loc = m_new;
+        for (int j = 0; j < MERGE_MOST / 64; ++j) {
+            const float f = pow4(ref[j] - top);
+            s_f[r][lane + 64 * j] = f;
+            sum += l[j] * f;
         }
+        sum = lanes_sum(sum);
+        if (lane == 0) s_l[r] = sum;
     }
-    s_m[sg][row][q4] = m_loc;
-    s_l[sg][row][q4] = l_loc;
-    *(f32x4 *)&s_o[sg][row][q4 * 4] = o_loc;
     __syncthreads();
-    if (sg == 0) {
-        float m_all = -INFINITY;
+    for (int s0 = 0; s0 < a.nseg; s0 += MEET_PARTS) {
+        if (s0) request(s0);
 #pragma unroll
-        for (int g2 = 0; g2 < MERGE_SG; ++g2) m_all = fmaxf(m_all, s_m[g2][row][q4]);
+        for (int u = 0; u < 8; ++u) {
+            const int s = s0 + sg * 8 + u;                             // (past the last: that one again, and zero times an infinite value is no zero)
+            os[u] = (s < a.nseg ? os[u] : f32x4{0.f, 0.f, 0.f, 0.f}) * s_f[row_ld][s];
+        }
+#pragma unroll
+        for (int i = 1; i < 8; i *= 2)
+#pragma unroll
+            for (int u = 0; u < 8; u += 2 * i) os[u] += os[u + i];
+        *(f32x4 *)&s_o[s0 / MEET_PARTS][sg][row][q4 * 4] = os[0];
+    }
+    __syncthreads();
+    if (sg == 0 && row < rows) {
         f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-        float l_all = 0.f;
-#pragma unroll
-        for (int g2 = 0; g2 < MERGE_SG; ++g2) {
-            const float mg = s_m[g2][row][q4];
-            const float f = mg > -INFINITY ? exp2f((mg - m_all) * LOG2E) : 0.f;
-            o += *(const f32x4 *)&s_o[g2][row][q4 * 4] * f;
-            l_all += s_l[g2][row][q4] * f;
+        for (int c = 0; c * MEET_PARTS < a.nseg; ++c) {
+            auto run = [&](int i) { return *(const f32x4 *)&s_o[c][i][row][q4 * 4]; };
+            o += (run(0) + run(1)) + (run(2) + run(3));
         }
-        const int rr = rt * 16 + row;
-        if (rr < a.rows_total) {
-            const int l2 = rr / a.groups, g3 = rr % a.groups;
-            const float inv = l_all > 0.f ? 1.f / l_all : 0.f;
-            *(f32x4 *)(a.out + (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g3) * D + dv) = o * inv;
-        }
+        const int rr = rt * 16 + row, l2 = rr / a.groups, g3 = rr % a.groups;
+        const float l_all = s_l[row], inv = l_all > 0.f ? 1.f / l_all : 0.f;
+        *(f32x4 *)(a.out + (((size_t)b * a.L + l2) * a.Hq + hk * a.groups + g3) * D + dv) = o * inv;
     }
 }
 
@@ -274,35 +273,32 @@ int launch_flash_split(aionhip_ctx *ctx, AttnArgs &a) {
     return AIONHIP_OK;
 }
 
-// Whether the segments are merged by the workgroup that ends last instead of a launch of their own: a wavefront of it has a row's segments in flight
-// MEET_UNROLL at a time for each lane of a column, and up to four such rounds cost no more than a launch. us with the merge launch / without: 1531 keys of 8
-// KV heads x 128, 6 segments, 8.6 / 7.0; 8 sequences over 4000 keys of one KV head x 256, 16 segments, 12.6 / 11.1; one over 16384, 64 segments in four shares
-// of the value columns, 12.4 / 11.4; 8 x 16384, 32 in one share (four rounds), 27.7 / 27.4. Past that the one workgroup reads too much: 4 x 16384, 64 in one
-// share, 19.1 / 20.2.
-constexpr int MEET_ROUNDS = 4;
-bool last_merges(const AttnArgs &a, int dv) { return a.nseg <= min(64, MEET_ROUNDS * MEET_UNROLL * (256 / dv)); }
+// Whether the parts are merged by the workgroup that ends last instead of a launch of their own: a wavefront of it adds a row's parts, 32 with all of their
+// loads in flight, and as long as those are no more than 256 columns' worth that costs less than a launch. us with the merge launch / without: 1531 keys of 8
+// KV heads x 128, 6 segments, 8.6 / 7.0; 8 sequences over 4000 keys of one KV head x 256, 16 segments, 12.6 / 10.9; one over 16384, 64 segments in four shares
+// of the value columns, 12.4 / 11.0; 8 x 16384, 32 in one share, 27.7 / 27.5. Past that the one workgroup reads too much: 4 x 16384, 64 in one share, 19.1 / 20.2.
+bool last_merges(const AttnArgs &a, int dv) { return a.nseg <= min(64, MEET_PARTS * (256 / dv)); }
 
-// Key segments of a 16-row tile. A workgroup's eight wavefronts take a 32-key tile each; how fast a short cache is read is what one CU's L1 fills (64 bytes a
-// clock), so that two tiles to a workgroup on more CUs beat eight on fewer as long as the merge stays small: 24 segments, fewer where the workgroups, with the
-// value columns in all their shares, would not fit the CUs at once. us a token, eight tiles / two: 1531 keys of one KV head x 256 8.9 / 6.4, 3000 8.9 / 7.3; of 8 x
-// 128 6.8 / 6.0 and 7.3 / 6.8; 4 sequences over 11378 keys, 1469 visible, 9.0 / 7.4. From 24 eight-tile segments on they stay (8000 keys: 32 segments 9.3, 63 9.4).
-// Up to FEW_TILES of a whole cache they stay too: there a batch of any size that fits the CUs has the same segments, hence a sequence the same bits.
-// as_few: rows that leave prepared want one segment wherever eight tiles allow it.
-constexpr int FEW_TILES = 32;
-int key_segments(const AttnArgs &a, int d, int cus, int units, bool as_few) {
-    // (behind a window there are no more keys than it shows to the call's consecutive queries)
+// Key segments of a 16-row tile, eight 32-key tiles each where that leaves no CU with two workgroups: what a row sums to depends on these alone (and a
+// sequence's bits on the batch only from where they no longer fit the CUs). Behind a window there are no more keys than it shows to the call's consecutive queries.
+// sub: a segment's eight wavefronts divided over 2^sub workgroups. How fast a short cache is read is what one CU's L1 fills (64 bytes a clock), so that two
+// or four tiles to a workgroup on more CUs beat eight on fewer as long as the merge stays small: 24 parts, a quarter of a segment each only where the workgroups, with
+// the value columns in all their shares, fit the CUs at once. us a token, whole segments / so: 512 keys of one KV head x 256 8.7 / 6.2, 1531 8.9 / 6.4, 3000 8.9 /
+// 7.3; of 8 x 128 512 keys 6.7 / 5.6, 1531 6.8 / 5.9 (in quarters, 24 parts, 6.6), 3000 7.3 / 7.0; 4 sequences over 11378 keys, 1469 visible, 9.0 / 7.8. From 13
+// segments on they stay whole (8000 keys: 32 parts 9.3, 63 9.4).
+struct KeySegments { int nseg, sub; };
+KeySegments key_segments(const AttnArgs &a, int d, int cus, int units) {
     long keys = a.T;
-    if (!as_few && a.win_chunk == 0 && a.win_right < (unsigned)a.T && a.win_left < (unsigned)a.T) keys = min(keys, (long)a.win_left + (long)a.win_right + a.L + TILE_KEYS);
-    const int tiles = (int)((keys + TILE_KEYS - 1) / TILE_KEYS), of_eight = (tiles + SPLIT_NW - 1) / SPLIT_NW;
+    if (!a.codes && a.win_chunk == 0 && a.win_right < (unsigned)a.T && a.win_left < (unsigned)a.T) keys = min(keys, (long)a.win_left + (long)a.win_right + a.L + TILE_KEYS);
     const long wgs = (long)units * a.row_tiles;
-    int nseg = of_eight;
-    if (!as_few && of_eight > 1 && (keys < a.T || tiles > FEW_TILES)) {
-        const long full = wgs * (d / 64);
-        nseg = max(nseg, min((tiles + 1) / 2, full * 24 <= cus ? 24 : full * 16 <= cus ? 16 : 12));
-    }
     // (as many segments as keep the workgroups within one per CU: a second, partial round of workgroups plus the merge
     // costs more than CUs left idle - 192 row tiles in two segments each took 26 us, in one 13)
-    return min(max(1, (int)min((long)nseg, (long)cus / wgs)), 256);
+    const int room = (int)min((long)cus / wgs, 256L), of_eight = (int)((keys + SPLIT_NW * TILE_KEYS - 1) / (SPLIT_NW * TILE_KEYS));
+    KeySegments ks{max(1, min(room, of_eight)), 0};
+    if (a.codes || ks.nseg == 1) return ks;
+    const long full = wgs * (d / 64);
+    if (ks.nseg * 2 <= min(room, 24)) ks.sub = ks.nseg * 4 <= min(room, full * 24 <= cus ? 24 : full * 16 <= cus ? 16 : 12) ? 2 : 1;
+    return ks;
 }
 
 template <int KV, int D, bool HILO, bool RING = false>
@@ -346,25 +342,29 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     if (a.codes && (HILO || RING)) return rows_not_prepared(ctx, HILO ? "the precise mode" : "rolling caches");
     if (split) {
         const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
-        int nseg = key_segments(a, D, cus, units, a.codes != nullptr);
-        // (a recording for which the scratch memory would have to grow asks for no more segments than eight-tile ones)
-        if (ctx->capturing && (size_t)units * a.row_tiles * nseg * (16 * D + 32) * sizeof(float) > ctx->scratch2_bytes) nseg = key_segments(a, D, cus, units, true);
-        if (a.codes && nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
-        a.nseg = nseg;
-        const long wgs = (long)units * a.row_tiles * nseg;
-        const int shares = D >= 256 && wgs * (D / 64) <= cus ? D / 64 : D >= 128 && wgs * 2 <= cus ? 2 : 1;      // of the value columns, see below
-        const size_t meetings = (size_t)units * a.row_tiles * shares, ticket_bytes = meetings * MEET_TICKET_WORDS * sizeof(unsigned);
-        const size_t meet_bytes = meetings * nseg * (16 * (D / shares) + 32) * sizeof(float);
-        // (a recording for which the buffers would have to grow keeps the merge launch)
-        const bool meet = nseg > 1 && last_merges(a, D / shares) &&
-                          (!ctx->capturing || (ticket_bytes <= ctx->tickets_bytes && meet_bytes <= ctx->scratch2_bytes));
+        const KeySegments ks = key_segments(a, D, cus, units);
+        if (a.codes && ks.nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
+        int shares = 1;      // of the value columns, see below
+        size_t ticket_bytes = 0, meet_bytes = 0;
+        bool meet = false;
+        auto plan = [&](int sub) {
+            a.sub = sub;
+            a.nseg = ks.nseg << sub;
+            const long tiles = (long)units * a.row_tiles, wgs = tiles * a.nseg;
+            shares = D >= 256 && wgs * (D / 64) <= cus ? D / 64 : D >= 128 && wgs * 2 <= cus ? 2 : 1;
+            ticket_bytes = (size_t)tiles * shares * MEET_TICKET_WORDS * sizeof(unsigned);
+            meet_bytes = (size_t)tiles * shares * a.nseg * (16 * (D / shares) + 32) * sizeof(float);
+            meet = a.nseg > 1 && last_merges(a, D / shares) && (!ctx->capturing || (ticket_bytes <= ctx->tickets_bytes && meet_bytes <= ctx->scratch2_bytes));
+        };
+        plan(ks.sub);
+        if (!meet) plan(0);      // (a recording for which the buffers would have to grow keeps whole segments, or the merge launch: the same sums)
         if (meet) {
             if (const int rc = ensure_scratch2(ctx, meet_bytes)) return rc;
             if (const int rc = grow_work_buffer(ctx, &ctx->tickets, &ctx->tickets_bytes, ticket_bytes, true, "the tickets")) return rc;
             a.partial = (float *)ctx->scratch2;
             a.tickets = (unsigned *)ctx->tickets;
-        } else if (nseg > 1) {
-            const size_t bytes = (size_t)units * a.row_tiles * nseg * (16 * D + 32) * sizeof(float);
+        } else if (a.nseg > 1) {
+            const size_t bytes = (size_t)units * a.row_tiles * a.nseg * (16 * D + 32) * sizeof(float);
             int rc = ensure_scratch2(ctx, bytes);
             if (rc) return rc;
             a.partial = (float *)ctx->scratch2;
@@ -379,7 +379,7 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         else if (D >= 128 && shares == 2) rc = launch_flash_split<KV, D, HILO, RING, D >= 128 ? 2 : 1>(ctx, a);
         else rc = launch_flash_split<KV, D, HILO, RING, 1>(ctx, a);
         if (rc) return rc;
-        if (nseg > 1 && !meet) {
+        if (a.nseg > 1 && !meet) {
             ProfScope scope(ctx, "attn_merge");
             launch_k(ctx, attn_merge_kernel<D>, dim3((unsigned)(a.row_tiles * (D / MERGE_DV)), (unsigned)units), dim3(256), 0, a);
         }

@@ -22,6 +22,7 @@ struct AttnArgs {
     float *partial;
     unsigned *tickets;        // not null: the segments are merged by the workgroup that ends last (attn_flash_body), zero between launches
     int B, L, T, Hq, Hkv, groups, rows_total, row_tiles, nseg;
+    int sub;                  // 16-row kernel: the eight wavefronts of a key segment's tiles are divided over 2^sub workgroups, and nseg counts those (attn_flash_body)
     int ring;      // rolling caches: T (logical key t lives in row t % T); 0: row t is key t
     int q_dtype, kv_dtype;
     float scale, soft_cap;
@@ -144,6 +145,15 @@ __device__ __forceinline__ float groups4_max(float v) {
     x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return fmaxf(__uint_as_float(x[0]), __uint_as_float(x[1]));
 }
+// over the 64 lanes, in the order of wave_sum and wave_max, without their two LDS permutes
+__device__ __forceinline__ float lanes_max(float v) {
+    v = fmaxf(v, dpp_f<DPP_QUAD_XOR1>(v));
+    v = fmaxf(v, dpp_f<DPP_QUAD_XOR2>(v));
+    v = fmaxf(v, dpp_f<DPP_ROW_HALF_MIRROR>(v));
+    return groups4_max(fmaxf(v, dpp_f<DPP_ROW_MIRROR>(v)));
+}
+// 4^n for a whole n <= 0: exact, zero below 2^-126
+__device__ __forceinline__ float pow4(float n) { return __builtin_amdgcn_exp2f(2.f * n); }
 // the value of the lane 32 away
 __device__ __forceinline__ float half_swap(float v) {
     const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -154,6 +164,12 @@ __device__ __forceinline__ float groups4_sum(float v) {
     v = __uint_as_float(x[0]) + __uint_as_float(x[1]);
     x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+}
+__device__ __forceinline__ float lanes_sum(float v) {
+    v += dpp_f<DPP_QUAD_XOR1>(v);
+    v += dpp_f<DPP_QUAD_XOR2>(v);
+    v += dpp_f<DPP_ROW_HALF_MIRROR>(v);
+    return groups4_sum(v + dpp_f<DPP_ROW_MIRROR>(v));
 }
 
 using u32x2 = __attribute__((ext_vector_type(2))) unsigned int;

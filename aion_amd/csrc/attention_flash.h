@@ -15,14 +15,15 @@ struct FlashCfg {
     static constexpr int ROW_BYTES = DV * 2;                     // unpadded: the tile is filled by LDS-writing loads
     static constexpr int WAVE_LDS = TILE_KEYS * ROW_BYTES;       // one V tile per wavefront
     static constexpr int WG_LDS = NW * WAVE_LDS;
-    static constexpr int MERGE_LDS = (NW * (16 * (DV + 4) + 32) + 16 * NW + 32) * 4;   // split mode: NW x (acc[16][DV+4], m[16], l[16]) f32 + merge factors
+    static constexpr int MERGE_LDS = NW * (16 * (DV + 4) + 32) * 4;   // split mode: NW x (acc[16][DV+4], ref[16], l[16]) f32
     static constexpr int Q_ROW = D * 2 + 64;                     // split mode: the 16 query rows in the K/V element type
     static constexpr int Q_OFF = WG_LDS > MERGE_LDS ? WG_LDS : MERGE_LDS;
     static constexpr int LDS_BYTES = Q_OFF + 16 * Q_ROW;
 };
 constexpr int SPLIT_NW = 8;
+constexpr float REF_NONE = -3.402823466e38f;      // the reference of what holds no key
 constexpr int MEET_TICKET_WORDS = 32;      // a ticket has a line of its own: the segments of every tile draw theirs at the same time
-constexpr int MEET_UNROLL = 8;     // segments that a lane of the merging workgroup has in flight
+constexpr int MEET_PARTS = 32;     // parts that the merging workgroup adds in one tree, with all of their loads in flight
 
 // HILO: q and the probabilities are fed to the MFMAs as a high and a low half-precision part
 // (x = hi + lo, ~2x the mantissa), which keeps an f32 query path at f32-level accuracy; used when
@@ -36,7 +37,7 @@ constexpr int MEET_UNROLL = 8;     // segments that a lane of the merging workgr
 // index operands and the queries, reductions by DPP and lane swaps instead of LDS permutes, hardware exp2 (the arguments are <= 0 and
 // results under 2^-126 vanish in a sum that holds a 1), V in flight under the scores. One token, one KV head of size 256, 144 keys:
 // 8.0 -> 6.75 us, 6.1 with the operands in SGPRs; 1531 keys, 8 KV heads of size 128: 7.6 -> 6.0 us with eight tiles to a segment (+ 3.6 for the merge as a
-// launch), 5.8 with two and the merge inside; eight sequences over 16384 keys, one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
+// launch), 5.9 with four and the merge inside; eight sequences over 16384 keys, one KV head of size 256: 25.7 -> 23.5 us = 5.7 TB/s.
 template <int KV, int D, bool SPLIT, bool HILO, bool RING, int DVS = 1, class Hooks>
 __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char *lds, const int rt_block, const int seg, const int b, const int hk, Hooks &hooks,
                                                 const int slice_dv = 0) {
@@ -162,15 +163,18 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
+    [[maybe_unused]] float ref_run = REF_NONE, to_ref = 1.f;         // split mode, of the last tile
 
     // ---- key tiles of this wavefront
     int t_begin = 0, t_end = 0, t_step = 1;
     if (uni_hi > uni_lo) {
         const int tb = uni_lo / TILE_KEYS, te = (uni_hi + TILE_KEYS - 1) / TILE_KEYS;
         if (SPLIT) {
-            const int per = (te - tb + a.nseg - 1) / a.nseg;
-            t_begin = tb + seg * per + wave;
-            t_end = min(tb + (seg + 1) * per, te);
+            // a segment's tiles go round robin to eight wavefronts, which 1, 2 or 4 workgroups hold
+            const int segs = a.nseg >> a.sub, mine = NW >> a.sub, whole = seg >> a.sub;
+            const int per = (te - tb + segs - 1) / segs;
+            t_begin = tb + whole * per + (seg - (whole << a.sub)) * mine + wave;
+            t_end = wave < mine ? min(tb + (whole + 1) * per, te) : t_begin;
             t_step = NW;
         } else {
             t_begin = tb;
@@ -328,6 +332,14 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         rowsum = groups4_sum(rowsum);
         l_run = l_run * alpha + rowsum;
         m_run = m_new;
+        if (SPLIT && !more) {
+            // The wavefronts' results meet under references that are powers of four (of two would leave the range of floats before m does), 4^ref >= e^m: to_ref =
+            // e^m / 4^ref, at most one. (Here, under the wait for V. Past 2^24, where floats are coarser than the grid, clamped; without a visible key the sums are
+            // zeros under the lowest reference.)
+            const float half = ceilf(m_run * (0.5f * LOG2E));
+            to_ref = __builtin_amdgcn_exp2f(-2.f * fminf(fmaxf(fmaf(m_run, -0.5f * LOG2E, half), 0.f), 1.f));
+            ref_run = fmaxf(half, REF_NONE);
+        }
         const u32x4 pf = u32x4{pack2<KV>(p[0], p[1]), pack2<KV>(p[2], p[3]), pack2<KV>(p[4], p[5]), pack2<KV>(p[6], p[7])};
         u32x4 pf_lo = u32x4{0u, 0u, 0u, 0u};
         if (HILO) {
@@ -407,18 +419,22 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     __syncthreads();
     float *mg = (float *)lds;
     constexpr int RS = DV + 4;                // padded row stride (floats)
-    constexpr int WSTRIDE = 16 * RS + 32;     // one wavefront's slot: acc[16][RS], m[16], l[16]
+    constexpr int WSTRIDE = 16 * RS + 32;     // one wavefront's slot: acc[16][RS], ref[16], l[16]
+    // From here on a row's reference is 4^ref (see the last tile): the factors between wavefronts and between segments, 4^(ref - ref'), are exact (v_exp_f32 of a
+    // whole number), and what a row sums to depends on the order of the sums alone. That order is one tree - a segment's eight wavefronts pairwise, then the
+    // parts pairwise, a segment's parts being neighbours, 32 of them at a time - whichever workgroups hold the wavefronts and whoever merges: a sequence has the
+    // same bits in every batch whose segments fit the CUs, and in the merge by the last workgroup and by the launch (down to the subnormal numbers).
     {
         float *w = mg + wave * WSTRIDE;
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) *(f32x4 *)(w + n * RS + mt * 16 + g * 4) = acc[mt];
-        if (g == 0) { w[16 * RS + n] = m_run; w[16 * RS + 16 + n] = l_run; }
+        for (int mt = 0; mt < MT; ++mt) *(f32x4 *)(w + n * RS + mt * 16 + g * 4) = acc[mt] * to_ref;
+        if (g == 0) { w[16 * RS + n] = ref_run; w[16 * RS + 16 + n] = l_run * to_ref; }
     }
     __syncthreads();
-    // every thread derives the weights exp2(m_w - m_all) of its own row from the NW maxima (NW LDS reads that
+    // every thread derives the weights 4^(ref_w - ref) of its own row from the NW references (NW LDS reads that
     // the sixteen lanes of a row share, NW exp2): cheaper than a serial pass by sixteen threads and a third barrier
-    // partial slot layout in global memory (read by attn_merge_kernel): [16][D] o, [16] m, [16] l; where the last workgroup merges, each share of the value
-    // columns has slots of its own, [16][DV] o, [16] m, [16] l
+    // partial slot layout in global memory (read by attn_merge_kernel): [16][D] o, [16] ref, [16] l; where the last workgroup merges, each share of the value
+    // columns has slots of its own, [16][DV] o, [16] (ref, l)
     constexpr int PSTRIDE = 16 * D + 32, SSTRIDE = 16 * DV + 32;
     const size_t pslot = ((size_t)(unit * a.row_tiles + rt) * a.nseg + seg) * PSTRIDE;
     [[maybe_unused]] const unsigned meeting = (unsigned)(unit * a.row_tiles + rt) * DVS + (unsigned)slice_dv;
@@ -432,21 +448,29 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
 #endif
     for (int e = threadIdx.x; e < 16 * DV / 4; e += NW * 64) {
         const int row = e / (DV / 4), col = (e % (DV / 4)) * 4;
-        float mw[NW];
-        float m_all = -INFINITY;
+        float ref_w[NW], lw[NW];
+        f32x4 ow[NW];
+        float ref = REF_NONE;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            mw[w] = mg[w * WSTRIDE + 16 * RS + row];
-            m_all = fmaxf(m_all, mw[w]);
+            ref_w[w] = mg[w * WSTRIDE + 16 * RS + row];
+            ref = fmaxf(ref, ref_w[w]);
         }
-        f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
-        float l_all = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) {
-            const float f = mw[w] > -INFINITY ? __builtin_amdgcn_exp2f((mw[w] - m_all) * LOG2E) : 0.f;
-            l_all += mg[w * WSTRIDE + 16 * RS + 16 + row] * f;
-            o += *(const f32x4 *)(mg + w * WSTRIDE + row * RS + col) * f;
+            const float f = pow4(ref_w[w] - ref);
+            lw[w] = mg[w * WSTRIDE + 16 * RS + 16 + row] * f;
+            ow[w] = *(const f32x4 *)(mg + w * WSTRIDE + row * RS + col) * f;
         }
+#pragma unroll
+        for (int s = 1; s < NW; s *= 2)
+#pragma unroll
+            for (int w = 0; w < NW; w += 2 * s) {
+                lw[w] += lw[w + s];
+                ow[w] += ow[w + s];
+            }
+        const f32x4 o = ow[0];
+        const float l_all = lw[0];
         if (a.nseg == 1) {
             const int rr = rt * 16 + row;
             if (rr < a.rows_total) {
@@ -460,13 +484,13 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
                 const int at = (seg * SSTRIDE + row * DV + col) * 4;
                 __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o), slots_rsrc, at, 0, DEVICE_SCOPE);
                 if (col == 0)
-                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(m_all), __float_as_uint(l_all)}, slots_rsrc, (seg * SSTRIDE + 16 * DV + row * 2) * 4, 0, DEVICE_SCOPE);
+                    __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(ref), __float_as_uint(l_all)}, slots_rsrc, (seg * SSTRIDE + 16 * DV + row * 2) * 4, 0, DEVICE_SCOPE);
 #endif
             }
         } else if (rt * 16 + row < a.rows_total) {        // (rows past the last query row are padding: nobody reads them)
             *(f32x4 *)(a.partial + pslot + row * D + dv0 + col) = o;
             if (col == 0 && dv0 == 0) {
-                a.partial[pslot + 16 * D + row] = m_all;
+                a.partial[pslot + 16 * D + row] = ref;
                 a.partial[pslot + 16 * D + 16 + row] = l_all;
             }
         }
@@ -474,7 +498,7 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
     if constexpr (!Hooks::Q_LATE) {
         // The workgroup that ends last merges the segments: each publishes its partial result, waits until the stores have been acknowledged and takes a
         // ticket; whoever draws the last one finds all of them. Nobody waits for anybody. No device-scope fence: it would write back and
-        // invalidate the L2 of the XCD. The segments are added in order, whoever comes last.
+        // invalidate the L2 of the XCD.
         if (!last_merges) return;
         int *s_ticket = (int *)(lds + Cfg::Q_OFF);                  // (the queries are dead)
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -483,9 +507,8 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
         __syncthreads();
         if (*s_ticket != a.nseg - 1) return;
         if (threadIdx.x == 0) __hip_atomic_store(a.tickets + meeting * MEET_TICKET_WORDS, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // A wavefront merges a row: lane s has the maximum and sum of segment s (there are at most 64, the launcher sees to that); a lane has four columns
-        // and every G-th segment, the G lanes of a column meet by lane swaps. A column is summed as four runs, segments i, i + 4, .., in whatever number of
-        // lanes: ((0 + 1) + (2 + 3)), so that the bits do not depend on the shares of the value columns.
+        // A wavefront merges a row: lane s has the reference and sum of part s (there are at most 64, the launcher sees to that); a lane has four columns
+        // and 8 of every 8 G consecutive parts, the G lanes of a column meet by lane swaps.
         constexpr int TPR = DV / 4, G = 64 / TPR, RUNS = 4 / G;
         const int grp = lane / TPR, col = (lane % TPR) * 4, rows = min(16, a.rows_total - rt * 16);
         for (int row = wave; row < rows; row += NW) {
@@ -493,34 +516,51 @@ __device__ __forceinline__ void attn_flash_body(const AttnArgs &a, unsigned char
 #if defined(__HIP_DEVICE_COMPILE__)
             stat = __builtin_amdgcn_raw_buffer_load_b64(slots_rsrc, (lane * SSTRIDE + 16 * DV + row * 2) * 4, 0, DEVICE_SCOPE);
 #endif
-            f32x4 run[RUNS];
-#pragma unroll
-            for (int i = 0; i < RUNS; ++i) run[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
             float f_lane = 0.f, l_all = 0.f;
-            for (int s0 = grp; s0 - grp < a.nseg; s0 += G * MEET_UNROLL) {
-                u32x4 os[MEET_UNROLL] = {};
+            for (int s0 = 0; s0 < a.nseg; s0 += MEET_PARTS) {
+                u32x4 os[RUNS][8] = {};
 #if defined(__HIP_DEVICE_COMPILE__)
 #pragma unroll
-                for (int u = 0; u < MEET_UNROLL; ++u)
-                    os[u] = __builtin_amdgcn_raw_buffer_load_b128(slots_rsrc, ((s0 + u * G) * SSTRIDE + row * DV + col) * 4, 0, DEVICE_SCOPE);
+                for (int c = 0; c < RUNS; ++c)
+                    if (c == 0 || s0 + c * 8 * G < a.nseg) {
+#pragma unroll
+                        for (int u = 0; u < 8; ++u)
+                            os[c][u] = __builtin_amdgcn_raw_buffer_load_b128(slots_rsrc, ((s0 + (c * G + grp) * 8 + u) * SSTRIDE + row * DV + col) * 4, 0, DEVICE_SCOPE);
+                    }
 #endif
-                if (s0 == grp) {
-                    const float m = lane < a.nseg ? __uint_as_float(stat.x) : -INFINITY, m_max = wave_max(m);
-                    f_lane = m > -INFINITY ? __builtin_amdgcn_exp2f((m - m_max) * LOG2E) : 0.f;
-                    l_all = wave_sum(__uint_as_float(stat.y) * f_lane);
+                if (s0 == 0) {
+                    const float ref = lane < a.nseg ? __uint_as_float(stat.x) : REF_NONE;
+                    f_lane = pow4(ref - lanes_max(ref));
+                    l_all = lanes_sum(__uint_as_float(stat.y) * f_lane);
                 }
+                f32x4 run[RUNS];
 #pragma unroll
-                for (int u = 0; u < MEET_UNROLL; ++u) {
-                    const float f = __shfl(f_lane, (s0 + u * G) & 63, 64);          // (past the last segment: a factor or zero, times zeros)
-                    run[u % RUNS] += __builtin_bit_cast(f32x4, os[u]) * f;
+                for (int c = 0; c < RUNS; ++c) {
+                    run[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    if (c == 0 || s0 + c * 8 * G < a.nseg) {
+                        f32x4 part[8];
+#pragma unroll
+                        for (int u = 0; u < 8; ++u) {
+                            const int s = (s0 + (c * G + grp) * 8 + u) & 63;                    // (past the last part: a factor, times zeros)
+                            const float f = G == 1 ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(f_lane), s)) : __shfl(f_lane, s, 64);
+                            part[u] = __builtin_bit_cast(f32x4, os[c][u]) * f;
+                        }
+#pragma unroll
+                        for (int i = 1; i < 8; i *= 2)
+#pragma unroll
+                            for (int u = 0; u < 8; u += 2 * i) part[u] += part[u + i];
+                        run[c] = part[0];
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            if constexpr (G == 4) run[c][i] = groups4_sum(run[c][i]);
+                            else if constexpr (G == 2) run[c][i] += half_swap(run[c][i]);
+                        }
+                    }
                 }
-            }
-            f32x4 o;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if constexpr (G == 4) o[i] = groups4_sum(run[0][i]);
-                else if constexpr (G == 2) o[i] = (run[0][i] + half_swap(run[0][i])) + (run[1][i] + half_swap(run[1][i]));
-                else o[i] = (run[0][i] + run[1][i]) + (run[2][i] + run[3][i]);
+                if constexpr (RUNS == 1) o += run[0];
+                else if constexpr (RUNS == 2) o += run[0] + run[1];
+                else o += (run[0] + run[1]) + (run[2] + run[3]);
             }
             if (grp > 0) continue;
             const int rr = rt * 16 + row, l2 = a.L > 1 ? (int)((unsigned)rr / (unsigned)a.groups) : 0, g2 = rr - l2 * a.groups;

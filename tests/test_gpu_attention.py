@@ -219,6 +219,49 @@ def test_decode_value_columns_divided_or_not(gpu, orc, T, D, precise):
         gpu.set_attention_precise(False)
 
 
+@pytest.mark.parametrize("Hq,Hkv,D,L,T,window,batches", [
+    (32, 8, 128, 1, 1531, be.CAUSAL, (1, 2, 3, 5)), (8, 1, 256, 1, 16384, be.CAUSAL, (1, 2, 4)), (8, 1, 256, 1, 3000, be.CAUSAL, (1, 4, 8, 20)),
+    (16, 4, 64, 1, 2500, be.CAUSAL, (1, 2, 6)), (8, 2, 256, 1, 11378, (1468, 0, 0), (1, 4, 8)), (8, 1, 128, 3, 1100, be.CAUSAL, (1, 3, 16)), (8, 1, 256, 1, 1024, be.CAUSAL, (1, 8, 40))])
+@pytest.mark.parametrize("precise", [False, True])
+def test_a_sequence_has_the_same_bits_in_every_batch_that_fits_the_cus(gpu, orc, precise, Hq, Hkv, D, L, T, window, batches):
+    """The largest batch fills the CUs with whole segments; smaller ones divide a segment over two or four workgroups, the value columns over several, and merge
+    in the kernel instead of by a launch. Every output is the same sum in the same order."""
+    B = batches[-1]
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T + D, B, L, T, Hq, Hkv, D, "f16")
+    lens = np.maximum(T - np.arange(B) * 77, L).astype(np.int32)
+    pos = (lens[:, None] - L + np.arange(L)).astype(np.int32)
+    gpu.set_attention_precise(precise)
+    try:
+        got = {n: run_attention(gpu, q[:n], k[:n], v[:n], 1 / math.sqrt(D), qd, kd, window=window, positions=pos[:n], kv_lengths=lens[:n]) for n in batches}
+        attn_err(got[B][:2], orc.attention_f64(qf[:2], kf[:2], vf[:2], 1 / math.sqrt(D), window=window, positions=pos[:2], kv_lengths=lens[:2]), 1e-5 if precise else 2e-3)
+        for n in batches:
+            assert np.array_equal(got[n], got[B][:n]), n
+    finally:
+        gpu.set_attention_precise(False)
+
+
+@pytest.mark.parametrize("precise", [False, True])
+@pytest.mark.parametrize("offset", [-1.0, 0.0, 1.0])
+@pytest.mark.parametrize("scale", [1e-3, 0.5, 1e2, 1e5, 1e9, 1e36, 1.5e37])
+def test_decode_scores_of_any_magnitude(gpu, orc, scale, offset, precise):
+    """Wavefronts and key segments meet under references that are powers of two: scores around zero and far from it on either side, up to where floats are coarser
+    than a power of two and to the end of their range."""
+    T, Hq, Hkv, D = 1531, 8, 2, 128
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(11, 1, 1, T, Hq, Hkv, D, "f16")
+    q = (q / 8).astype(np.float16).astype(np.float32)
+    k[..., 0], kf[..., 0] = 4.0, 4.0
+    q[..., 0] = 4.0 * offset
+    top = np.abs(np.einsum("hgd,thd->hgt", q.reshape(Hkv, -1, D).astype(np.float64), kf[0])).max() * scale
+    assert top < 3.4e38 and (scale < 1.5e37 or offset == 0.0 or top > 2.4e38), top          # (2.36e38 x log2 e leaves the range)
+    pos = np.array([[T - 1]], np.int32)
+    gpu.set_attention_precise(precise)
+    try:
+        got = run_attention(gpu, q, k, v, scale, qd, kd, positions=pos)
+    finally:
+        gpu.set_attention_precise(False)
+    attn_err(got, orc.attention_f64(q, kf, vf, scale, positions=pos), 2e-3)
+
+
 @pytest.mark.parametrize("kind,tol", [("f16", 2e-3), ("bf16", 1e-2)])
 @pytest.mark.parametrize("D,Hkv", [(64, 1), (128, 2), (256, 1)])
 @pytest.mark.parametrize("T,left", [(1400, 333), (1400, 5000), (333, 31), (40, 7)])   # window starts inside a key tile, or no limit
