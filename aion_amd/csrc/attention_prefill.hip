@@ -718,7 +718,7 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
             for (int i = 0; i < 16; ++i) amax = fmaxf(amax, fabsf(acc[j][i]));
-        if (__any(amax == INFINITY)) {
+        if (__builtin_expect(__any(amax == INFINITY), 0)) {
             amax = 0.f;
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
@@ -763,14 +763,14 @@ __global__ __launch_bounds__(256) void attn_prefill_kernel(AttnArgs a) {
 }
 
 // The same merge for many rows and few segments (the prefill kernel's key segments): one thread per (row, four
-// consecutive dv), so that a wavefront reads whole contiguous rows of every segment's accumulators.
+// consecutive dv), so that a wavefront reads whole contiguous rows of every segment's accumulators, UN segments at a time: rounds of two where there are two (4096
+// keys, 8 heads on one x 256, bf16, 91.4 -> 89.8 us against rounds of four).
 __device__ __forceinline__ float half_bits_to_float(unsigned bits) { return (float)__builtin_bit_cast(_Float16, (unsigned short)bits); }
 
-template <int D, bool HP>
+template <int D, bool HP, int UN>
 __global__ __launch_bounds__(256) void attn_merge_rows_kernel(AttnArgs a) {
     constexpr int PART_BYTES = pf_partial_bytes(D, HP);
     constexpr int TPR = D / 4, RPB = 256 / TPR;          // threads per row, rows per workgroup
-    constexpr int UN = 4;
     const int unit = blockIdx.y, b = unit / a.Hkv, hk = unit % a.Hkv;
     const int rr = blockIdx.x * RPB + (int)threadIdx.x / TPR, dv = ((int)threadIdx.x % TPR) * 4;
     if (rr >= a.rows_total) return;
@@ -902,8 +902,12 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
         ProfScope scope(ctx, "attn_merge");
         constexpr int RPB = 256 / (D / 4);
         const dim3 grid((unsigned)((a.rows_total + RPB - 1) / RPB), (unsigned)units);
-        if (a.pf_half) launch_k(ctx, attn_merge_rows_kernel<D, pf_half_partials(KV)>, grid, dim3(256), 0, a);
-        else launch_k(ctx, attn_merge_rows_kernel<D, false>, grid, dim3(256), 0, a);
+        const auto merge = [&](auto half) {
+            if (nseg == 2) launch_k(ctx, attn_merge_rows_kernel<D, decltype(half)::value, 2>, grid, dim3(256), 0, a);
+            else launch_k(ctx, attn_merge_rows_kernel<D, decltype(half)::value, 4>, grid, dim3(256), 0, a);
+        };
+        if (a.pf_half) merge(std::integral_constant<bool, pf_half_partials(KV)>{});
+        else merge(std::false_type{});
     }
     LAUNCH_CHECK(ctx, "attn_prefill");
     return AIONHIP_OK;
