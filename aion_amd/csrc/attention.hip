@@ -360,7 +360,7 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         if (!meet) plan(0);      // (a recording for which the buffers would have to grow keeps whole segments, or the merge launch: the same sums)
         if (meet) {
             if (const int rc = ensure_scratch2(ctx, meet_bytes)) return rc;
-            if (const int rc = grow_work_buffer(ctx, &ctx->tickets, &ctx->tickets_bytes, ticket_bytes, true, "the tickets")) return rc;
+            if (const int rc = ensure_tickets(ctx, ticket_bytes)) return rc;
             a.partial = (float *)ctx->scratch2;
             a.tickets = (unsigned *)ctx->tickets;
         } else if (a.nseg > 1) {

@@ -22,7 +22,6 @@ struct FlashCfg {
 };
 constexpr int SPLIT_NW = 8;
 constexpr float REF_NONE = -3.402823466e38f;      // the reference of what holds no key
-constexpr int MEET_TICKET_WORDS = 32;      // a ticket has a line of its own: the segments of every tile draw theirs at the same time
 constexpr int MEET_PARTS = 32;     // parts that the merging workgroup adds in one tree, with all of their loads in flight
 
 // HILO: q and the probabilities are fed to the MFMAs as a high and a low half-precision part

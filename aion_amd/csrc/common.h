@@ -55,7 +55,7 @@ struct aionhip_ctx {
     // K-split GEMV: the words in which the partial sums of sibling K slices meet (all zero between launches)
     void *ksplit = nullptr;
     size_t ksplit_bytes = 0;
-    // argmax: one ticket per row (all zero between launches)
+    // tickets (all zero between launches): argmax's, one per row, and those of attention steps whose key segments meet in the kernel
     void *tickets = nullptr;
     size_t tickets_bytes = 0;
     // moves on whenever one of the four buffers above is replaced by a larger one: a program recorded before that holds
@@ -157,6 +157,8 @@ int dev_malloc(aionhip_ctx *ctx, void **out, size_t bytes, const char *what);
 int grow_work_buffer(aionhip_ctx *ctx, void **buf, size_t *have, size_t bytes, bool zeroed, const char *what);
 int ensure_scratch(aionhip_ctx *ctx, size_t bytes);
 int ensure_scratch2(aionhip_ctx *ctx, size_t bytes);
+constexpr unsigned MEET_TICKET_WORDS = 32;      // a ticket of an attention step has a line of its own: the parts of every row tile draw theirs at the same time
+int ensure_tickets(aionhip_ctx *ctx, size_t bytes);      // never fewer than attention steps take, one per CU
 // size of the file-scope device scratch array behind aionhip_step_matmul_static (prepared activations of one call)
 constexpr size_t STATIC_SCRATCH_BYTES = AIONHIP_STATIC_SCRATCH_BYTES;
 

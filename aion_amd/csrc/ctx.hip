@@ -67,7 +67,7 @@ int dev_malloc(aionhip_ctx *ctx, void **out, size_t bytes, const char *what) {
     return AIONHIP_OK;
 }
 
-// Context-owned work buffers (prepared activations, GEMM staging, K-split meeting words, argmax tickets) grow by
+// Context-owned work buffers (prepared activations, GEMM staging and attention's partial results, K-split meeting words, tickets) grow by
 // replacement. A recorded program holds the old address in its launches, so every replacement moves the context's
 // buffer generation on and aionhip_program_execute refuses a program recorded under an earlier one.
 int grow_work_buffer(aionhip_ctx *ctx, void **buf, size_t *have, size_t bytes, bool zeroed, const char *what) {
@@ -92,6 +92,10 @@ int grow_work_buffer(aionhip_ctx *ctx, void **buf, size_t *have, size_t bytes, b
 }
 int ensure_scratch(aionhip_ctx *ctx, size_t bytes) { return grow_work_buffer(ctx, &ctx->scratch, &ctx->scratch_bytes, bytes, false, "scratch"); }
 int ensure_scratch2(aionhip_ctx *ctx, size_t bytes) { return grow_work_buffer(ctx, &ctx->scratch2, &ctx->scratch2_bytes, bytes, false, "GEMM staging"); }
+int ensure_tickets(aionhip_ctx *ctx, size_t bytes) {
+    const size_t attention = (size_t)(ctx->cu_count > 0 ? ctx->cu_count : 256) * MEET_TICKET_WORDS * sizeof(unsigned);
+    return grow_work_buffer(ctx, &ctx->tickets, &ctx->tickets_bytes, bytes > attention ? bytes : attention, true, "the tickets");
+}
 
 static hipEvent_t take_event(aionhip_ctx *ctx) {
     if (!ctx->event_pool.empty()) {

@@ -724,7 +724,7 @@ int aionhip_step_argmax(aionhip_ctx *ctx, aionhip_handle out_i32, aionhip_handle
     if (rows > 65535) return set_err(ctx, AIONHIP_UNSUPPORTED, "argmax: more than 65535 rows");
     int rc = ensure_scratch2(ctx, rows * ARGMAX_PARTS * 8);
     if (rc) return rc;
-    rc = grow_work_buffer(ctx, &ctx->tickets, &ctx->tickets_bytes, rows * sizeof(unsigned), true, "the argmax tickets");
+    rc = ensure_tickets(ctx, rows * sizeof(unsigned));
     if (rc) return rc;
     argmax_kernel<<<dim3(ARGMAX_PARTS, (unsigned)rows), dim3(256), 0, ctx->stream>>>(dp<int>(out_i32), (unsigned long long *)ctx->scratch2, (unsigned *)ctx->tickets,
                                                                                      dp<const float>(x), n);

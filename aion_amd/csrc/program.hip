@@ -81,6 +81,9 @@ int aionhip_program_begin(aionhip_ctx *ctx) {
     if (ctx->capturing) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "program_begin: already recording");
     if (ctx->profiling) return set_err(ctx, AIONHIP_INVALID_ARGUMENT, "program_begin: stop profiling first (events cannot be captured)");
     HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    // The tickets of attention steps are bounded by the CUs. They are there from the first recording on: an eager step of a larger batch would otherwise
+    // replace the buffer, and a program that addresses it - one argmax does - would be stale.
+    if (const int rc = ensure_tickets(ctx, 0)) return rc;
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     ctx->capturing = true;
     return AIONHIP_OK;

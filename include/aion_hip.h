@@ -425,7 +425,8 @@ int aionhip_decoder_stack_set_stamps(aionhip_ctx *ctx, aionhip_decoder_stack *st
  * While recording: no h2d/d2h/free/sync, no profiling, and scratch cannot grow - run the same
  * steps once eagerly first. Per-token inputs must live in device buffers the steps read.
  * Lifetime: a program's launches hold the addresses of the context's work buffers (prepared
- * activations, GEMM staging, K-split words, argmax tickets). When a later eager step needs a
+ * activations, GEMM staging and attention's partial results, K-split words, the tickets of argmax and of
+ * attention steps - these are bounded and there from the first recording on). When a later eager step needs a
  * larger one (a longer prompt, more rows), the buffer is replaced and every program recorded
  * before that is stale: program_execute then returns AIONHIP_INVALID_ARGUMENT without launching
  * anything (aionhip_last_error says "stale program"), and the caller destroys it and records the

@@ -105,3 +105,29 @@ def test_program_recorded_before_a_work_buffer_grows_is_refused(orc):
         w.free()
     finally:
         g.close()
+
+
+def test_a_program_with_an_argmax_outlives_an_attention_step_of_a_larger_batch():
+    """argmax and the attention steps whose key segments meet in the kernel draw tickets from one buffer. Attention's are bounded by the CUs and there from the
+    first recording on, so that a larger batch later does not replace the buffer under a program that holds an argmax only."""
+    from aion_amd import backend as be
+    g = be.HipBackend(0)
+    try:
+        L, D = 2048, 256
+        zeros = g.zeros(L * 8 * D * 4)
+        x = np.random.default_rng(0).standard_normal((1, 1000)).astype(np.float32)
+        x_buf, idx = g.upload(x), g.zeros(4)
+        g.step_attention(zeros, zeros, zeros, zeros, (1, L, L, 8, 1, D, D), 1.0, q_dtype=be.F16, kv_dtype=be.F16)      # the staging buffer, which argmax uses too
+        g.step_argmax(idx, x_buf, 1, 1000)
+        prog = g.record_program(lambda: g.step_argmax(idx, x_buf, 1, 1000))
+        for batch in (2, 64, 85):
+            g.step_attention(zeros, zeros, zeros, zeros, (batch, 1, 600, 1, 1, 64, 64), 1.0, q_dtype=be.F16, kv_dtype=be.F16)
+            assert g.last_kernel() == "attn_flash_split" and g.program_is_current(prog), batch
+        g._check(g._lib.aionhip_memset(g._ctx, idx.handle, 0, 0, 4))
+        g.program_execute(prog)
+        assert g.download(idx, np.int32, (1,))[0] == x.argmax()
+        g.program_destroy(prog)
+        for t in (zeros, x_buf, idx):
+            t.free()
+    finally:
+        g.close()
