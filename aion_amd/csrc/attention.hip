@@ -344,29 +344,18 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
         const int cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
         const KeySegments ks = key_segments(a, D, cus, units);
         if (a.codes && ks.nseg != 1) return rows_not_prepared(ctx, "keys in segments");      // (their merge writes f32 rows)
-        int shares = 1;      // of the value columns, see below
-        size_t ticket_bytes = 0, meet_bytes = 0;
-        bool meet = false;
-        auto plan = [&](int sub) {
-            a.sub = sub;
-            a.nseg = ks.nseg << sub;
-            const long tiles = (long)units * a.row_tiles, wgs = tiles * a.nseg;
-            shares = D >= 256 && wgs * (D / 64) <= cus ? D / 64 : D >= 128 && wgs * 2 <= cus ? 2 : 1;
-            ticket_bytes = (size_t)tiles * shares * MEET_TICKET_WORDS * sizeof(unsigned);
-            meet_bytes = (size_t)tiles * shares * a.nseg * (16 * (D / shares) + 32) * sizeof(float);
-            meet = a.nseg > 1 && last_merges(a, D / shares) && (!ctx->capturing || (ticket_bytes <= ctx->tickets_bytes && meet_bytes <= ctx->scratch2_bytes));
-        };
-        plan(ks.sub);
-        if (!meet) plan(0);      // (a recording for which the buffers would have to grow keeps whole segments, or the merge launch: the same sums)
+        a.sub = ks.sub;
+        a.nseg = ks.nseg << ks.sub;
+        const long tiles = (long)units * a.row_tiles, wgs = tiles * a.nseg;
+        const int shares = D >= 256 && wgs * (D / 64) <= cus ? D / 64 : D >= 128 && wgs * 2 <= cus ? 2 : 1;      // of the value columns, see below
+        const bool meet = a.nseg > 1 && last_merges(a, D / shares);
         if (meet) {
-            if (const int rc = ensure_scratch2(ctx, meet_bytes)) return rc;
-            if (const int rc = ensure_tickets(ctx, ticket_bytes)) return rc;
+            if (const int rc = ensure_scratch2(ctx, (size_t)tiles * shares * a.nseg * (16 * (D / shares) + 32) * sizeof(float))) return rc;
+            if (const int rc = ensure_tickets(ctx, (size_t)tiles * shares * MEET_TICKET_WORDS * sizeof(unsigned))) return rc;
             a.partial = (float *)ctx->scratch2;
             a.tickets = (unsigned *)ctx->tickets;
         } else if (a.nseg > 1) {
-            const size_t bytes = (size_t)units * a.row_tiles * a.nseg * (16 * D + 32) * sizeof(float);
-            int rc = ensure_scratch2(ctx, bytes);
-            if (rc) return rc;
+            if (const int rc = ensure_scratch2(ctx, (size_t)tiles * a.nseg * (16 * D + 32) * sizeof(float))) return rc;
             a.partial = (float *)ctx->scratch2;
         }
         // Workgroups that leave CUs idle divide the value columns as well, down to 64 each: the scores are computed by every share,

@@ -861,12 +861,12 @@ int launch_prefill_t(aionhip_ctx *ctx, AttnArgs &a) {
     // tile alone is most of the time. Whole caches only: a window keeps the tiles short. us in one segment (from 32 key tiles on two) / four, past one
     // workgroup per CU three: 16 heads on 4 x 64 over 1030 keys 24.2 / 23.5, 1611 35.0 / 29.0, 2000 38.6 / 33.8, 2500 50.5 / 43.0, 4096 79.0 / 76.9; with more
     // workgroups the merge costs more: two sequences over 1300 30.0 / 31.1, over 2500 54.4 / 63.0.
-    // (Rows that leave prepared want one segment, and a recording is not asked for scratch memory that fewer do without.) Over a bf16 cache these shapes had f32
+    // (Rows that leave prepared want one segment.) Over a bf16 cache these shapes had f32
     // accumulators all the way in one segment, and keep them in the partial results: us with f16 ones / f32: 1030 keys 20.3 / 23.5, 1611 26.3 / 29.0, 2500 41.5 / 43.0, 4096 73.0 / 76.9.
     a.pf_half = pf_half_partials(KV) && nseg > 1;
     if (D <= 64 && !a.codes && key_tiles > 16 && wgs <= 8 * key_tiles && wgs <= 2 * cus0 && a.win_left >= (unsigned)a.T && a.win_chunk == 0) {
         const int few = wgs <= cus0 ? 4 : 3;
-        if (!ctx->capturing || (size_t)units * a.row_tiles * few * pf_partial_bytes(D, a.pf_half) <= ctx->scratch2_bytes) nseg = max(nseg, few);
+        nseg = max(nseg, few);           // (scratch memory in a recording: prefill_added_scratch)
     }
     a.nseg = nseg;
     a.pf_tiles = (a.rows_total + PF_ROWS - 1) / PF_ROWS;
@@ -928,6 +928,10 @@ int launch_prefill_d(aionhip_ctx *ctx, AttnArgs &a, int d) {
 }  // namespace
 
 namespace attn {
+
+// What the segments that launch_prefill_t adds at head size 64 take of the scratch memory at most: prompts that would run without any otherwise, which a recording
+// therefore finds there (aionhip_program_begin). The 16-row kernel's parts, one workgroup per CU, are less.
+size_t prefill_added_scratch(int cus) { return (size_t)2 * cus * 3 * (PF_ROWS / 16) * pf_partial_bytes(64, false); }
 
 bool prefill_takes(const AttnArgs &a, int d) {
     if (d != 64 && d != 128 && d != 256) return false;

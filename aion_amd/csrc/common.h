@@ -158,6 +158,7 @@ int grow_work_buffer(aionhip_ctx *ctx, void **buf, size_t *have, size_t bytes, b
 int ensure_scratch(aionhip_ctx *ctx, size_t bytes);
 int ensure_scratch2(aionhip_ctx *ctx, size_t bytes);
 constexpr unsigned MEET_TICKET_WORDS = 32;      // a ticket of an attention step has a line of its own: the parts of every row tile draw theirs at the same time
+namespace attn { size_t prefill_added_scratch(int cus); }
 int ensure_tickets(aionhip_ctx *ctx, size_t bytes);      // never fewer than attention steps take, one per CU
 // size of the file-scope device scratch array behind aionhip_step_matmul_static (prepared activations of one call)
 constexpr size_t STATIC_SCRATCH_BYTES = AIONHIP_STATIC_SCRATCH_BYTES;

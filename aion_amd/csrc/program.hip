@@ -84,6 +84,9 @@ int aionhip_program_begin(aionhip_ctx *ctx) {
     // The tickets of attention steps are bounded by the CUs. They are there from the first recording on: an eager step of a larger batch would otherwise
     // replace the buffer, and a program that addresses it - one argmax does - would be stale.
     if (const int rc = ensure_tickets(ctx, 0)) return rc;
+    // So is the scratch memory that attention steps take by their shape alone where they could do with less: a step then has the same segments, and the same bits,
+    // recorded or not, and is recorded without having run before. (52 MB. On a device without them the step itself refuses.)
+    (void)ensure_scratch2(ctx, attn::prefill_added_scratch(ctx->cu_count > 0 ? ctx->cu_count : 256));
     HIP_TRY(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     ctx->capturing = true;
     return AIONHIP_OK;

@@ -423,7 +423,7 @@ int aionhip_decoder_stack_set_stamps(aionhip_ctx *ctx, aionhip_decoder_stack *st
  * (backend/gpu/frame.zig:77-86). Between program_begin and program_end the aionhip_step_* calls
  * are recorded into a HIP graph instead of executed; program_execute replays it (asynchronous).
  * While recording: no h2d/d2h/free/sync, no profiling, and scratch cannot grow - run the same
- * steps once eagerly first. Per-token inputs must live in device buffers the steps read.
+ * steps once eagerly first (program_begin itself sets some 65 MB of it aside). Per-token inputs must live in device buffers the steps read.
  * Lifetime: a program's launches hold the addresses of the context's work buffers (prepared
  * activations, GEMM staging and attention's partial results, K-split words, the tickets of argmax and of
  * attention steps - these are bounded and there from the first recording on). When a later eager step needs a

@@ -602,3 +602,39 @@ def test_prefill_key_segments_with_windows_and_ragged_lengths(gpu, orc, window, 
         ref = orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D), window=window, soft_cap=soft_cap, positions=pos, kv_lengths=ends)
     assert np.isfinite(got).all()
     attn_err(got, ref, 2e-3)
+
+
+@pytest.mark.parametrize("B,L,T,Hq,Hkv,D,window,kind,names", [
+    (1, 1, 1531, 32, 8, 128, be.CAUSAL, "f16", ["attn_flash_split"]), (4, 1, 16384, 8, 1, 256, (1468, 0, 0), "f16", ["attn_flash_split"]),
+    (1, 1, 16384, 8, 1, 256, be.CAUSAL, "bf16", ["attn_flash_split"]), (5, 1, 16384, 8, 1, 256, be.CAUSAL, "bf16", ["attn_flash_split", "attn_merge"]),
+    (2, 1, 700, 8, 1, 256, be.CAUSAL, "f16", ["attn_flash_split"]), (1, 1611, 1611, 16, 4, 64, be.CAUSAL, "f16", ["attn_prefill", "attn_merge"]),
+    (1, 1611, 1611, 16, 4, 64, be.CAUSAL, "bf16", ["attn_prefill", "attn_merge"]), (1, 4096, 4096, 16, 4, 64, be.CAUSAL, "f16", ["attn_prefill", "attn_merge"])])
+def test_recorded_steps_in_key_segments_have_the_eager_bits(B, L, T, Hq, Hkv, D, window, kind, names):
+    """A context that has run nothing records the step and replays it, with the same step eagerly and other shapes in between: the segments, and the form of the merge,
+    follow the shape alone, and the tickets are back at zero after every replay."""
+    g = be.HipBackend(0)
+    try:
+        (q, k, v, qd, kd), _ = make_qkv(T, B, L, T, Hq, Hkv, D, kind)
+        bufs = [g.upload(x) for x in (q, k, v)]
+        pos = g.upload(np.tile(np.arange(T - L, T, dtype=np.int32), (B, 1)))
+        last = g.upload(np.full((1, 1), T - 1, np.int32))
+        out = [g.zeros(B * L * Hq * D * 4) for _ in range(3)]
+
+        def step(o):
+            g.step_attention(o, *bufs, (B, L, T, Hq, Hkv, D, D), 1 / math.sqrt(D), q_dtype=qd, kv_dtype=kd, window=window, query_positions=pos)
+
+        prog = g.record_program(lambda: step(out[0]))
+        got = []
+        for _ in range(3):
+            g.program_execute(prog)
+            got.append(g.download(out[0], np.float32, (B, L, Hq, D)))
+            g.profile_start()
+            step(out[1])
+            assert [n for n, _ in g.profile_stop()] == names
+            got.append(g.download(out[1], np.float32, (B, L, Hq, D)))
+            g.step_attention(out[2], *bufs, (1, 1, T, Hq, Hkv, D, D), 1.0, q_dtype=qd, kv_dtype=kd, query_positions=last)
+            assert g.program_is_current(prog)
+        assert all(np.array_equal(x, got[0]) for x in got), [np.array_equal(x, got[0]) for x in got]
+        g.program_destroy(prog)
+    finally:
+        g.close()
