@@ -90,6 +90,7 @@ struct aionhip_ctx {
     const void *last_fn = nullptr;
     unsigned last_grid[3] = {0, 0, 0}, last_block[3] = {0, 0, 0}, last_lds = 0;
     std::unordered_map<const void *, hipFunction_t> functions;     // host stub -> this device's kernel (launch_params)
+    hipError_t launch_error = hipSuccess;                          // of a launch whose kernel was not found, until LAUNCH_CHECK reports it
     std::vector<ProfRecord> prof;
     std::vector<hipEvent_t> event_pool;
 };
@@ -175,6 +176,8 @@ constexpr size_t STATIC_SCRATCH_BYTES = AIONHIP_STATIC_SCRATCH_BYTES;
     do {                                                                                            \
         (ctx)->last_kernel = (name);                                                                \
         hipError_t e_ = hipGetLastError();                                                          \
+        if ((ctx)->launch_error != hipSuccess) e_ = (ctx)->launch_error;                            \
+        (ctx)->launch_error = hipSuccess;                                                           \
         if (e_ != hipSuccess) return set_err((ctx), AIONHIP_EXECUTION_FAILED, "launch %s: %s", (name), hipGetErrorString(e_)); \
     } while (0)
 

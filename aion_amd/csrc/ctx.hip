@@ -124,8 +124,9 @@ void launch_params(aionhip_ctx *ctx, const void *kernel, dim3 grid, dim3 block, 
         if (current != ctx->device) (void)hipSetDevice(ctx->device);
         const hipError_t e = hipGetFuncBySymbol(&f, kernel);
         if (current != ctx->device) (void)hipSetDevice(current);
-        if (e != hipSuccess) {
-            (void)hipLaunchKernel(kernel, grid, block, params, lds, ctx->stream);
+        if (e != hipSuccess) {          // nothing is launched, and the launch's check says so: a kernel that ran is never reported as failed
+            (void)hipGetLastError();
+            ctx->launch_error = e;
             return;
         }
         it = ctx->functions.emplace(kernel, f).first;

@@ -148,3 +148,37 @@ def test_session_entry_points_reject_null_handles_without_a_gpu():
     assert lib.aionhip_session_retire(None) == hip.INVALID_ARGUMENT
     assert lib.aionhip_session_stats(None, None, None, None) == hip.INVALID_ARGUMENT
     lib.aionhip_session_destroy(None)          # a no-op
+
+
+def test_a_kernel_that_is_not_found_is_not_launched_and_is_reported(tmp_path):
+    """The launch by handle with the HIP calls it makes replaced: the lookup of the kernel fails. Then nothing may run - a step that is reported as failed is
+    repeated by its caller, wrong for one that adds to its output - and the launch's check, this one alone, reports the failure."""
+    import subprocess
+    src = tmp_path / "launch.hip"
+    src.write_text(r"""
+#include "%s/aion_amd/csrc/common.h"
+#include <cstdio>
+static hipError_t last = hipSuccess;
+static int launches = 0;
+extern "C" {
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetFuncBySymbol(hipFunction_t *, const void *) { return last = hipErrorInvalidDeviceFunction; }
+hipError_t hipLaunchKernel(const void *, dim3, dim3, void **, size_t, hipStream_t) { ++launches; return hipSuccess; }
+hipError_t hipModuleLaunchKernel(hipFunction_t, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, unsigned, hipStream_t, void **, void **) { ++launches; return hipSuccess; }
+hipError_t hipGetLastError() { const hipError_t e = last; last = hipSuccess; return e; }
+}
+static int check(aionhip_ctx *ctx) { LAUNCH_CHECK(ctx, "kernel"); return AIONHIP_OK; }
+int main() {
+    aionhip_ctx ctx;
+    int stub = 0;
+    launch_params(&ctx, &stub, dim3(1), dim3(64), 0, nullptr);
+    const int first = check(&ctx), second = check(&ctx);
+    printf("%%d %%d %%d\n", launches, first == AIONHIP_EXECUTION_FAILED, second == AIONHIP_OK);
+}
+""" % ROOT)
+    exe = tmp_path / "launch"
+    lib = os.path.join(ROOT, "aion_amd")
+    subprocess.run(["/opt/rocm/bin/hipcc", "--offload-arch=gfx950", "--offload-host-only", "-std=c++17", "-O0", str(src), "-o", str(exe), "-L" + lib, "-laion_hip", "-Wl,-rpath," + lib],
+                   check=True, capture_output=True, text=True)
+    assert subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout.split() == ["0", "1", "1"]
