@@ -323,8 +323,8 @@ int launch_flash(aionhip_ctx *ctx, AttnArgs &a) {
     // 1 ... 1024 queries x 1024 ... 16384 keys at head sizes 128 and 256: the 16-row kernel 13 us + 0.56 us per 32-key tile a
     // workgroup walks (head size 256; in proportion below), the 128-row kernel 16 us + 1.9 us per 64-key tile (1.2 at head
     // size 128, 0.85 at 64; 0.7 of that while half the CUs stay free). 8 heads x 256, 256 queries over 16384 keys: 159 -> 46 us.
-    // The 16-row kernel has become faster since; over 400 shapes, 16 ... 1024 queries x 1 ... 64 times as many keys, head sizes 64 to 256, the
-    // choice is within 5 % of the faster kernel on 379 and costs at most 20 % (8 heads x 64, 128 queries over 8192 keys 20.7 against 17.2 us).
+    // The 16-row kernel has become faster since, and its segments finer; over 110 shapes, 9 ... 1024 queries x 4 ... 64 times as many keys, head sizes 64 to
+    // 256, the choice is within 5 % of the faster kernel on 108 and costs at most 18 % (8 heads on one x 128, 104 queries over 4992 keys 21.2 against 17.9 us).
     if (!HILO && a.rows_total > 64 && pf_wgs <= pf_min && prefill_takes(a, D) && (long)a.T >= 4L * a.L && a.win_left >= (unsigned)a.T) {
         const float ds = (float)D / 256.f;
         const long wgs16 = (long)units * a.row_tiles;

@@ -128,9 +128,40 @@ def test_prefill_head_64_in_key_segments(gpu, orc, L, T, kind, tol):
     nan = np.float16(np.nan) if kind == "f16" else np.uint16(0x7FC1)
     for x, f in ((k, kf), (v, vf)):
         x[:, L:], f[:, L:] = nan, 0
-    got = run_attention(gpu, q, k, v, 1 / 8.0, qd, kd, positions=pos, kv_lengths=end)
-    assert gpu.last_kernel() == "attn_prefill"
+    got, names = launches(gpu, q, k, v, 1 / 8.0, qd, kd, positions=pos, kv_lengths=end)
+    assert names == ["attn_prefill", "attn_merge"]
     attn_err(got, orc.attention_f64(qf, kf, vf, 1 / 8.0, positions=pos, kv_lengths=end), tol)
+
+
+@pytest.mark.parametrize("rolling", [False, True])
+def test_prefill_head_64_in_key_segments_with_a_soft_cap_and_over_a_ring(gpu, orc, rolling):
+    """The same segments in the kernel's other two instances."""
+    L, T = 1100, 1100
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(5, 1, L, T, 16, 4, 64, "f16")
+    end = np.array([2 * T + 300 if rolling else T], np.int32)
+    pos = np.arange(end[0] - L, end[0], dtype=np.int32).reshape(1, L)
+    got, names = launches(gpu, q, k, v, 1 / 8.0, qd, kd, positions=pos, kv_lengths=end, rolling=rolling, soft_cap=0.0 if rolling else 5.0)
+    assert names == ["attn_prefill", "attn_merge"]
+    if rolling:
+        ref = orc.attention_rolling_f64(qf, kf, vf, 1 / 8.0, be.CAUSAL, pos, end)
+    else:
+        ref = orc.attention_f64(qf, kf, vf, 1 / 8.0, soft_cap=5.0, positions=pos, kv_lengths=end)
+    attn_err(got, ref, 2e-3)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,L,D", [(1, 32, 8, 1100, 128), (2, 16, 4, 1300, 64), (1, 32, 32, 1611, 128), (1, 8, 8, 4100, 256)])
+def test_prefill_every_row_tile_is_computed_in_each_order_of_the_workgroups(gpu, orc, B, Hq, Hkv, L, D):
+    """Prompts of more workgroups than CUs: 280 and 328, where the longer row tiles go out longest first and the rest shortest first beside them, and 416 and 264 of
+    other shapes. One query of every row tile against the reference, and nothing unwritten."""
+    (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(L, B, L, L, Hq, Hkv, D, "f16")
+    got, names = launches(gpu, q, k, v, 1 / math.sqrt(D), qd, kd)
+    assert names[0] == "attn_prefill" and np.isfinite(got).all()
+    per_tile = 128 * Hkv // Hq
+    some = np.unique(np.r_[np.arange(per_tile // 3, L, per_tile), 0, L - 1])
+    pos = np.tile(some.astype(np.int32), (B, 1))
+    attn_err(got[:, some], orc.attention_f64(qf[:, some], kf, vf, 1 / math.sqrt(D), positions=pos), 2e-3)
+    norm = np.abs(got).max(axis=(2, 3))                                                 # (a row that nobody wrote)
+    assert (norm > 0).all()
 
 
 @pytest.mark.parametrize("kind,tol", [("f16", 2e-3), ("bf16", 1e-2)])
@@ -167,11 +198,11 @@ def test_decode_ragged_lengths_and_stale_cache_tail(gpu, orc):
 
 @pytest.mark.parametrize("D", [64, 128, 256])
 @pytest.mark.parametrize("B,Hq,Hkv,L,T", [(1, 8, 8, 1, 257), (1, 4, 4, 1, 4096), (3, 8, 1, 1, 2048), (2, 8, 2, 1, 4100), (1, 12, 1, 1, 3000), (4, 8, 1, 1, 16384), (2, 4, 4, 5, 700),
-                                          (1, 8, 1, 3, 900), (1, 9, 3, 6, 1300)])
+                                          (1, 8, 1, 3, 900), (1, 9, 3, 6, 1300), (1, 8, 1, 1, 17000)])
 @pytest.mark.parametrize("precise", [False, True])
 def test_key_segments_merged_by_the_workgroup_that_ends_last(gpu, orc, precise, B, Hq, Hkv, L, T, D):
-    """Two segments and more: rows from one to sixteen of a tile, several tiles, columns in one share or several, as many segments as the last workgroup takes
-    in one round, two, and more than it takes (a launch merges those); segments without a visible key. Repeated calls, also one after another of
+    """Two segments and more: rows from one to sixteen of a tile, several tiles, columns in one share or several, up to as many parts as the last workgroup takes
+    (32 of 256 columns, 64 of fewer) and more (a launch merges those); segments without a visible key. Repeated calls, also one after another of
     different shapes, give the same bits: the tickets return to zero."""
     (q, k, v, qd, kd), (qf, kf, vf) = make_qkv(T + D, B, L, T, Hq, Hkv, D, "f16")
     lens = np.maximum(T - np.arange(B) * (T // 3), L).astype(np.int32)
@@ -182,7 +213,12 @@ def test_key_segments_merged_by_the_workgroup_that_ends_last(gpu, orc, precise, 
     gpu.set_attention_precise(precise)
     try:
         for window in (be.CAUSAL, (300, 0, 0)):
-            got = [run_attention(gpu, q, k, v, 1 / math.sqrt(D), qd, kd, window=window, positions=pos, kv_lengths=lens) for _ in range(3)]
+            got, names = zip(*[launches(gpu, q, k, v, 1 / math.sqrt(D), qd, kd, window=window, positions=pos, kv_lengths=lens) for _ in range(3)])
+            if window == be.CAUSAL and (T > 64 * 256 or (T == 16384 and D == 256)):
+                assert all(n == ["attn_flash_split", "attn_merge"] for n in names)
+            else:
+                assert all(n == ["attn_flash_split"] for n in names)
+                assert gpu.last_launch()["grid"][0] > -(-L * (Hq // Hkv) // 16) * (D // 64)      # more workgroups than row tiles in all shares of the value columns
             attn_err(got[0], orc.attention_f64(qf, kf, vf, 1 / math.sqrt(D), window=window, positions=pos, kv_lengths=lens), 2e-3)
             assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
     finally:
@@ -635,6 +671,30 @@ def test_recorded_steps_in_key_segments_have_the_eager_bits(B, L, T, Hq, Hkv, D,
             g.step_attention(out[2], *bufs, (1, 1, T, Hq, Hkv, D, D), 1.0, q_dtype=qd, kv_dtype=kd, query_positions=last)
             assert g.program_is_current(prog)
         assert all(np.array_equal(x, got[0]) for x in got), [np.array_equal(x, got[0]) for x in got]
+        g.program_destroy(prog)
+    finally:
+        g.close()
+
+
+def test_a_recording_that_lacks_scratch_memory_refuses_the_step_until_it_has_run():
+    B, L, Hq, Hkv, D = 1, 4096, 8, 1, 256                                                # two segments of f32 partial results: 67.6 MB
+    g = be.HipBackend(0)
+    try:
+        (q, k, v, qd, kd), _ = make_qkv(9, B, L, L, Hq, Hkv, D, "f16")
+        bufs, out = [g.upload(x) for x in (q, k, v)], g.zeros(B * L * Hq * D * 4)
+
+        def step():
+            g.step_attention(out, *bufs, (B, L, L, Hq, Hkv, D, D), 1 / math.sqrt(D), q_dtype=qd, kv_dtype=kd)
+
+        with pytest.raises(be.AionHipError, match="run the steps once before recording"):
+            g.record_program(step)
+        step()
+        want = g.download(out, np.float32, (B, L, Hq, D))
+        prog = g.record_program(step)
+        for _ in range(2):
+            g._check(g._lib.aionhip_memset(g._ctx, out.handle, 0, 0, 4 * B * L * Hq * D))
+            g.program_execute(prog)
+            assert np.array_equal(g.download(out, np.float32, (B, L, Hq, D)), want)
         g.program_destroy(prog)
     finally:
         g.close()
