@@ -13,7 +13,7 @@ FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-result",
     # hipcc -O3 may otherwise form packed-f32 instructions, which have given wrong results on this pool
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # the first 16 dwords of a kernel's arguments arrive in SGPRs with the wavefront instead of through a scalar load: one
+    # a kernel's leading plain arguments arrive in SGPRs with the wavefront (16 dwords asked for, 14 do) instead of through a scalar load: one
     # memory round trip less at the head of every latency-bound kernel
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]

@@ -18,7 +18,8 @@ namespace {
 
 // The leading arguments, 14 words, arrive in SGPRs with the wavefront: the prepared rows, the first weight, the sizes - what the first loads need. A
 // structure by value is read from memory first; the rest of a launch is in the last one, for a single weight (GemvOne) without the siblings. With the
-// attention kernel's arguments in the same order 16 tokens of a 26-block decoder take 11.33 ms instead of 12.0.
+// attention kernel's arguments in the same order 16 tokens of a 26-block decoder take 11.33 ms instead of 12.0. (The kernel of 2..8 rows below, whose first
+// loads are the prepared rows, still takes its weights from a structure.)
 struct GemvOne {
     float *c;
     size_t ldc;

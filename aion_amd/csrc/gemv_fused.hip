@@ -24,10 +24,10 @@ namespace {
 // share one preparation, and every workgroup reads the whole activation at the same moment.
 // What the first loads need (the first two weights, the activation) are the leading arguments, as plain values: those arrive in SGPRs with the
 // wavefront, while a structure by value - all of them came in one - is read from memory, two dependent round trips before the first load (q4 1 x 14336 x
-// 4096 6.2 -> 5.6 us, 1 x 262144 x 2048 44.6 -> 44.1, a decode step of eight blocks 237 -> 234).
-// The last argument: what nothing waits for at the start. A launch's arguments are written across the bus (240 bytes: 0.75 us of host time) and the
-// smallest calls are bound by their launch, so that a single weight (MANY = false) is told apart from siblings: q8 1 x 2048 x 2048 3.64 -> 3.43 us a
-// call, q4 1 x 4096 x 4096 4.13 -> 3.60 (in a process whose launches cost 4.3 us: 4.37 -> 4.30, 4.46 -> 4.33).
+// 4096 7.0 -> 6.3 us, 1 x 262144 x 2048 45.1 -> 44.5, a decode step of eight blocks 237 -> 234).
+// The last argument: what nothing waits for at the start. A launch's arguments are written across the bus (240 bytes: 0.75 us of host time), so that a
+// single weight (MANY = false) is told apart from siblings. The smallest calls, which their launch bounds, do not show it: q8 1 x 2048 x 2048 4.55 -> 4.58 us,
+// q4 1 x 4096 x 4096 4.63 -> 4.59, less than a run differs from the next (3.4 to 4.6, drawn per process).
 template <int EPI, bool MANY> struct FusedTail { GemvBatch batch; };
 template <> struct FusedTail<EPI_NONE, false> { float *c; };
 template <bool MANY> struct FusedTail<EPI_ROPE_APPEND, MANY> { GemvBatch batch; FusedEpi epi; };
